@@ -217,16 +217,9 @@ void set_step(mpm_context* c, const float* dts, float dt_all, bool force_active,
     }
 }
 
-// The CG operator in the handle's mode: four waves per block (a cell's
-// particles split over them) or one wave per block (a lane runs its cell).
-template <int D>
-void launch_operator_as(const mpm_context* c, const mpm::KP& p, int mode, int grid, bool restart, int k, bool one) {
-    if (mode == 1) mpm::launch_cg_force_cell<D>(p, c->stream, grid, restart, k, one);
-    else mpm::launch_cg_force<D>(p, c->stream, grid, restart, k, one);
-}
 template <int D>
 void launch_operator(const mpm_context* c, const mpm::KP& p, bool restart, int k, bool one) {
-    launch_operator_as<D>(c, p, c->op_mode, c->grid_op, restart, k, one);
+    mpm::launch_cg_force<D>(p, c->stream, c->grid_op, restart, k, one);
 }
 
 // ---- stage sequences --------------------------------------------------------
@@ -1243,30 +1236,24 @@ int autotune(mpm_context* c, const float* dts, mpm_launch_config& best) {
     }
     auto no_prep = [] { return MPM_OK; };
     auto reopen = [&] { return reopen_cg(c); };
-    // the CG operator: four waves per block, or one wave per block with a
-    // lane's cell accumulated in registers
+    // the CG operator (one kernel for both operator modes)
     std::vector<int> cand;
     for (int g : {1024, 2048, 4096, 8192, 16384, 32768})
         if (g <= round8(h.nblocks) || g == 1024) cand.push_back(g);
     if (std::find(cand.begin(), cand.end(), cur.block_groups) == cand.end()) cand.push_back(cur.block_groups);
-    std::vector<std::pair<int, int>> ops;
-    for (int g : cand) ops.push_back({0, g});
-    for (int g : {256, 512, 1024, 2048, 4096})
-        if (g <= round8(h.nblocks / 4 + 8) || g == 256) ops.push_back({1, g});
-    if (std::find(ops.begin(), ops.end(), std::make_pair(cur.operator_mode, cur.operator_groups)) == ops.end())
-        ops.push_back({cur.operator_mode, cur.operator_groups});
+    std::vector<int> ops = cand;
+    if (std::find(ops.begin(), ops.end(), cur.operator_groups) == ops.end()) ops.push_back(cur.operator_groups);
     float best_ms = FLT_MAX;
-    for (const auto& og : ops) {
+    for (int g : ops) {
         const mpm::KP p = make_kp(c);
         float ms = 0.0f;
         rc = time_median(c, reopen, [&] {
-            for (int k = 0; k < 8; ++k) launch_operator_as<D>(c, p, og.first, og.second, false, 1, one);
+            for (int k = 0; k < 8; ++k) mpm::launch_cg_force<D>(p, c->stream, g, false, 1, one);
         }, ms);
         if (rc) return rc;
         if (ms < best_ms) {
             best_ms = ms;
-            best.operator_mode = og.first;
-            best.operator_groups = og.second;
+            best.operator_groups = g;
             best.operator_ms = ms;
         }
     }

@@ -74,7 +74,7 @@ struct mpm_context {
     int poll_boundary[2] = {0, 0};
     int poll_older = 0, poll_target = 1, poll_max_it = 0;
     int grid_particle = 0, grid_block = 0, grid_node = 0;
-    int op_mode = 0, grid_op = 0;  // CG operator: 0 four waves per block, 1 one wave per block
+    int op_mode = 0, grid_op = 0;  // CG operator: its mode (0 or 1, one kernel serves both) and work-groups
     size_t nred = 0;           // entries of the reduction partial arrays
     // captured substeps: one graph per particle-buffer parity
     bool graph = false;

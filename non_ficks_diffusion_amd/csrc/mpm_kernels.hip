@@ -738,56 +738,6 @@ constexpr int BWG = 64 * NW;
 // issue order).
 #define MPM_STEP_FENCE() __asm__ __volatile__("" ::: "memory")
 
-// The tile nodes a thread gathers and stores in a D-channel block kernel
-// depend on its thread index only, so the kernel forms them once:
-//   g: gather of tile node threadIdx.x: neighbour | local node << 5 | LDS
-//      index << 11 (~0u for threads past the tile);
-//   s: store of tile values t = threadIdx.x + k BWG (k < 3): the
-//      channel-major LDS index of each, 10 bits apiece.
-template <int D>
-struct TileMaps {
-    unsigned g, s;
-    __device__ void init() {
-        constexpr int TN = Dims<D>::TN, LTN = Dims<D>::LTN;
-        static_assert(D * TN <= 3 * BWG && D * LTN <= 1024, "three 10-bit store slots");
-        g = ~0u;
-        if ((int)threadIdx.x < TN) {
-            int nb, local, tc[D];
-            tile_map<D>(threadIdx.x, nb, local, tc);
-            g = (unsigned)nb | ((unsigned)local << 5) | ((unsigned)lds_index<D>(tc) << 11);
-        }
-        s = 0u;
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            const int t = threadIdx.x + k * BWG;
-            if (t < D * TN) {
-                const int c = t / TN;
-                int nb, local, tc[D];
-                tile_map<D>(t - c * TN, nb, local, tc);
-                s |= (unsigned)(c * LTN + lds_index<D>(tc)) << (10 * k);
-            }
-        }
-    }
-};
-
-// store_wave_tiles<D, D> with the thread's maps
-template <int D>
-__device__ inline void store_wave_tiles_mapped(const KP& p, int b, const float* lds, unsigned smap) {
-    constexpr int TN = Dims<D>::TN, LTN = Dims<D>::LTN;
-    float* dst = p.tiles + (int64_t)b * D * TN;
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        const int t = threadIdx.x + k * BWG;
-        if (t < D * TN) {
-            const int li = (int)((smap >> (10 * k)) & 1023u);
-            float v = 0.0f;
-#pragma unroll
-            for (int w = 0; w < NW; ++w) v += lds[w * D * LTN + li];
-            dst[t] = v;
-        }
-    }
-}
-
 // Sum of the NW wave tiles (C channels each, LDS layout) of block b into
 // its tile slot (compact layout, node (x,y,z) at (x*TE + y)*TE + z).
 template <int D, int C>
@@ -1005,24 +955,20 @@ __device__ inline void apply_pair(float A, float B, float slo, float shi, float 
     ahl = b * tlh + c * thl;
 }
 
-// A = L T from a particle's operator record
+// A = scale L T from a particle's operator record (in registers)
 template <int D>
-__device__ inline void apply_operator(const float* rec, const float* T, float* A) {
+__device__ inline void apply_operator(const float* rec, float scale, const float* T, float* A) {
     constexpr int DD = D * D;
     if constexpr (D == 3) {
-        const float4 r0 = *reinterpret_cast<const float4*>(rec);       // X0 X1 X2 q0
-        const float4 r1 = *reinterpret_cast<const float4*>(rec + 4);   // q1 q2 q3 s0
-        const float4 r2 = *reinterpret_cast<const float4*>(rec + 8);   // s1 s2 A B
-        const float4 r3 = *reinterpret_cast<const float4*>(rec + 12);  // P Q - -
-        const float q[4] = {r0.w, r1.x, r1.y, r1.z};
-        const float s0 = r1.w, s1 = r2.x, s2 = r2.y, a2 = r2.z, bl = r2.w, pj = r3.x, kappa = r3.x + r3.y;
+        const float s0 = rec[7], s1 = rec[8], s2 = rec[9];
+        const float a2 = scale * rec[10], bl = scale * rec[11], pj = scale * rec[12], kappa = fmaf(scale, rec[13], pj);
         float U[9], Th[9], Ah[9];
-        rot_of(q, U);
+        rot_of(rec + 3, U);
         rotate_in(U, T, Th);
-        const float tr = Th[0] + Th[4] + Th[8];
-        Ah[0] = (a2 * s0 * s0 - pj) * Th[0] + kappa * tr;
-        Ah[4] = (a2 * s1 * s1 - pj) * Th[4] + kappa * tr;
-        Ah[8] = (a2 * s2 * s2 - pj) * Th[8] + kappa * tr;
+        const float tr = kappa * (Th[0] + Th[4] + Th[8]);
+        Ah[0] = fmaf(fmaf(a2 * s0, s0, -pj), Th[0], tr);
+        Ah[4] = fmaf(fmaf(a2 * s1, s1, -pj), Th[4], tr);
+        Ah[8] = fmaf(fmaf(a2 * s2, s2, -pj), Th[8], tr);
         apply_pair(a2, bl, s0, s1, s2, Th[1], Th[3], Ah[1], Ah[3]);
         apply_pair(a2, bl, s0, s2, s1, Th[2], Th[6], Ah[2], Ah[6]);
         apply_pair(a2, bl, s1, s2, s0, Th[5], Th[7], Ah[5], Ah[7]);
@@ -1039,6 +985,8 @@ __device__ inline void apply_operator(const float* rec, const float* T, float* A
                 A[r] += v * T[c];
                 if (c != r) A[c] += v * T[r];
             }
+#pragma unroll
+        for (int r = 0; r < DD; ++r) A[r] *= scale;
     }
 }
 
@@ -1065,124 +1013,274 @@ __device__ inline void store_operator_eos(const KP& p, int i, float c, const flo
     for (int k = 0; k < OpRec<D>::W / 4; ++k) dst[k] = make_float4(rec[4 * k], rec[4 * k + 1], rec[4 * k + 2], rec[4 * k + 3]);
 }
 
-// Separable stencil contractions for the CG operator.  With
-// grad w = (dwx wy wz, wx dwy wz, wx wy dwz) the 3^D-node sums factor axis
-// by axis: 270 multiply-adds per particle in 3D instead of ~400 for the
-// node-by-node form.  `base` is the tile index of the particle's stencil
-// corner (its cell - 1 in every axis).
+// ---------------------------------------------------------------------------
+// The CG operator's stencil in difference form.  Per axis the weights of the
+// three stencil nodes sum to one, so a field in a cell is
+//   u = u1 + w0 (u0 - u1) + w2 (u2 - u1),   u' = w0' (u0 - u1) + w2' (u2 - u1):
+// the middle node's weight and derivative drop out.  The differences are
+// formed once per cell (two operations a node triple) and shared by its
+// particles; a particle's gradient then takes 180 operations in 3D instead
+// of 270.  Forces go back through the transpose, moments of the functions
+// {w0, 1, w2}.  The outer weights keep their own products, so a node that
+// carries only a sliver of a particle's weight (and of its mass) gets its
+// force to the same relative accuracy as node by node; a power basis loses
+// that to cancellation (measured: CG solves stall on light nodes).
+// ---------------------------------------------------------------------------
 template <int D>
-__device__ inline void grad_gather(const float (*w)[3], const float (*dw)[3], int base,
-                                   const float (*ut)[Dims<D>::LTN], float* T) {
+struct CellStencil {
+    static constexpr int NC = D == 3 ? 27 : 9;    // functions of a cell
+    static constexpr int MID = NC / 2;            // the constant: no gradient needs it
+    static constexpr int ROWS = D * (NC - 1);     // coefficient rows of a block, [channel][function][cell]
+    static constexpr int PACK = D == 3 ? 20 : 12;  // floats of a packed particle: A, w0, w2, d0
+    __device__ static constexpr int row(int cc, int n) { return cc * (NC - 1) + (n < MID ? n : n - 1); }
+};
+
+// node values -> differences along one axis (u1 stays)
+__device__ inline void diff_of_nodes(float& u0, const float& u1, float& u2) {
+    u0 -= u1;
+    u2 -= u1;
+}
+// its transpose: moments -> node contributions along one axis
+__device__ inline void nodes_of_moments(const float& m0, float& m1, const float& m2) { m1 -= m0 + m2; }
+
+// Coefficients of channel array u (an LDS tile) for the cell whose stencil
+// corner has tile index `base`.
+template <int D>
+__device__ inline void cell_coefficients(const float* u, int base, float* c) {
     constexpr int LX = Dims<D>::LX, LY = Dims<D>::LY;
     if constexpr (D == 3) {
-        float y00[3][3], y10[3][3], y01[3][3];
 #pragma unroll
-        for (int i = 0; i < 3; ++i) {
-#pragma unroll
-            for (int cc = 0; cc < 3; ++cc) y00[i][cc] = y10[i][cc] = y01[i][cc] = 0.0f;
+        for (int i = 0; i < 3; ++i)
 #pragma unroll
             for (int j = 0; j < 3; ++j) {
-                const int t0 = base + i * LX + j * LY;
-                // the row's nine tile values load before its contractions
-                float u[3][3];
+                float* r = c + (i * 3 + j) * 3;
 #pragma unroll
-                for (int cc = 0; cc < 3; ++cc)
-#pragma unroll
-                    for (int k = 0; k < 3; ++k) u[cc][k] = ut[cc][t0 + k];
-#pragma unroll
-                for (int cc = 0; cc < 3; ++cc) {
-                    const float u0 = u[cc][0], u1 = u[cc][1], u2 = u[cc][2];
-                    const float z0 = w[2][0] * u0 + w[2][1] * u1 + w[2][2] * u2;
-                    const float z1 = dw[2][0] * u0 + dw[2][1] * u1 + dw[2][2] * u2;
-                    y00[i][cc] += w[1][j] * z0;
-                    y10[i][cc] += dw[1][j] * z0;
-                    y01[i][cc] += w[1][j] * z1;
-                }
+                for (int k = 0; k < 3; ++k) r[k] = u[base + i * LX + j * LY + k];
+                diff_of_nodes(r[0], r[1], r[2]);
             }
-        }
 #pragma unroll
-        for (int cc = 0; cc < 3; ++cc) {
-            T[0 * 3 + cc] = dw[0][0] * y00[0][cc] + dw[0][1] * y00[1][cc] + dw[0][2] * y00[2][cc];
-            T[1 * 3 + cc] = w[0][0] * y10[0][cc] + w[0][1] * y10[1][cc] + w[0][2] * y10[2][cc];
-            T[2 * 3 + cc] = w[0][0] * y01[0][cc] + w[0][1] * y01[1][cc] + w[0][2] * y01[2][cc];
-        }
+        for (int i = 0; i < 3; ++i)
+#pragma unroll
+            for (int k = 0; k < 3; ++k) diff_of_nodes(c[i * 9 + k], c[i * 9 + 3 + k], c[i * 9 + 6 + k]);
+#pragma unroll
+        for (int k = 0; k < 9; ++k) diff_of_nodes(c[k], c[9 + k], c[18 + k]);
     } else {
-        float z0[3][2], z1[3][2];
 #pragma unroll
         for (int i = 0; i < 3; ++i) {
-            const int t0 = base + i * LX;
 #pragma unroll
-            for (int cc = 0; cc < 2; ++cc) {
-                const float u0 = ut[cc][t0], u1 = ut[cc][t0 + 1], u2 = ut[cc][t0 + 2];
-                z0[i][cc] = w[1][0] * u0 + w[1][1] * u1 + w[1][2] * u2;
-                z1[i][cc] = dw[1][0] * u0 + dw[1][1] * u1 + dw[1][2] * u2;
-            }
+            for (int k = 0; k < 3; ++k) c[i * 3 + k] = u[base + i * LX + k];
+            diff_of_nodes(c[i * 3], c[i * 3 + 1], c[i * 3 + 2]);
         }
 #pragma unroll
-        for (int cc = 0; cc < 2; ++cc) {
-            T[0 * 2 + cc] = dw[0][0] * z0[0][cc] + dw[0][1] * z0[1][cc] + dw[0][2] * z0[2][cc];
-            T[1 * 2 + cc] = w[0][0] * z1[0][cc] + w[0][1] * z1[1][cc] + w[0][2] * z1[2][cc];
+        for (int k = 0; k < 3; ++k) diff_of_nodes(c[k], c[3 + k], c[6 + k]);
+    }
+}
+
+// A particle's outer weights and their derivatives (in cells; the operator
+// scales its result by inv_dx twice) per axis, the weights operation for
+// operation as in bspline_from_offset.
+template <int D>
+struct OuterWeights {
+    float w0[D], w2[D], d0[D], d2[D];
+    __device__ explicit OuterWeights(const float* xo) {
+#pragma unroll
+        for (int a = 0; a < D; ++a) {
+#pragma clang fp contract(off)
+            float x = xo[a];
+            w0[a] = fabsf(0.5f * x * x - 1.5f * x + 1.125f);
+            d0[a] = x - 1.5f;
+            x -= 2.0f;
+            w2[a] = fabsf(0.5f * x * x + 1.5f * x + 1.125f);
+            d2[a] = x + 1.5f;
+        }
+    }
+};
+
+// T[r][cc] = d_r of channel cc at a particle of cell `cell` (per cell), from
+// the block's coefficient rows in LDS: particles of one cell read the same
+// words (broadcast), neighbouring cells neighbouring banks.
+template <int D>
+__device__ inline void stencil_gradient(const OuterWeights<D>& g, const float* coef, int cell, float* T) {
+    using CS = CellStencil<D>;
+    auto val = [](float w0, float w2, float c0, float c1, float c2) { return fmaf(w2, c2, fmaf(w0, c0, c1)); };
+    auto der = [](float d0, float d2, float c0, float c2) { return fmaf(d2, c2, d0 * c0); };
+#pragma unroll
+    for (int cc = 0; cc < D; ++cc) {
+        auto c = [&](int n) { return coef[CS::row(cc, n) * 64 + cell]; };
+        if constexpr (D == 3) {
+            float v[3], dy[3], dz[3];
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                float z[3], s[3];
+#pragma unroll
+                for (int j = 0; j < 3; ++j) {
+                    const int n = (i * 3 + j) * 3;
+                    const bool mid = i == 1 && j == 1;  // its value meets no derivative
+                    const float k0 = c(n), k1 = mid ? 0.0f : c(n + 1), k2 = c(n + 2);
+                    z[j] = mid ? 0.0f : val(g.w0[2], g.w2[2], k0, k1, k2);
+                    s[j] = der(g.d0[2], g.d2[2], k0, k2);
+                }
+                v[i] = i == 1 ? 0.0f : val(g.w0[1], g.w2[1], z[0], z[1], z[2]);
+                dy[i] = der(g.d0[1], g.d2[1], z[0], z[2]);
+                dz[i] = val(g.w0[1], g.w2[1], s[0], s[1], s[2]);
+            }
+            T[0 * 3 + cc] = der(g.d0[0], g.d2[0], v[0], v[2]);
+            T[1 * 3 + cc] = val(g.w0[0], g.w2[0], dy[0], dy[1], dy[2]);
+            T[2 * 3 + cc] = val(g.w0[0], g.w2[0], dz[0], dz[1], dz[2]);
+        } else {
+            float v[3], dy[3];
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                const int n = i * 3;
+                const float k0 = c(n), k2 = c(n + 2);
+                v[i] = i == 1 ? 0.0f : val(g.w0[1], g.w2[1], k0, c(n + 1), k2);
+                dy[i] = der(g.d0[1], g.d2[1], k0, k2);
+            }
+            T[0 * 2 + cc] = der(g.d0[0], g.d2[0], v[0], v[2]);
+            T[1 * 2 + cc] = val(g.w0[0], g.w2[0], dy[0], dy[1], dy[2]);
         }
     }
 }
 
-// q_node[cc] += sum_r A[r][cc] grad_r w_node over the stencil, into a
-// per-wave LDS tile (channel-major, TN floats per channel).  Lanes of a wave
-// hold distinct cells, so one stencil node is read-modified-written by at
-// most one lane per step; the compiler fence keeps the steps in order.
+// A particle as the scatter reads it: the outer weights and w0' per axis
+// (w2' = w0' + 1 exactly, offsets lie in [1/2, 3/2)) and the columns of its
+// force map A, so that the wave of channel cc reads three (2D: two) float4:
+//   3D: w0[3] d0x | w2[3] d0y | A[.][0] d0z | A[.][1] d0z | A[.][2] d0z
+//   2D: w0[2] w2[2] | A[.][0] d0[2] | A[.][1] d0[2]
 template <int D>
-__device__ inline void grad_scatter(const float (*w)[3], const float (*dw)[3], int base, const float* A, float* q) {
-    constexpr int LX = Dims<D>::LX, LY = Dims<D>::LY, TN = Dims<D>::LTN;
+__device__ inline void pack_particle(const OuterWeights<D>& g, const float* A, float* pack) {
+    float4* q = reinterpret_cast<float4*>(pack);
     if constexpr (D == 3) {
+        q[0] = make_float4(g.w0[0], g.w0[1], g.w0[2], g.d0[0]);
+        q[1] = make_float4(g.w2[0], g.w2[1], g.w2[2], g.d0[1]);
+#pragma unroll
+        for (int cc = 0; cc < 3; ++cc) q[2 + cc] = make_float4(A[cc], A[3 + cc], A[6 + cc], g.d0[2]);
+    } else {
+        q[0] = make_float4(g.w0[0], g.w0[1], g.w2[0], g.w2[1]);
+#pragma unroll
+        for (int cc = 0; cc < 2; ++cc) q[1 + cc] = make_float4(A[cc], A[2 + cc], g.d0[0], g.d0[1]);
+    }
+}
+template <int D>
+struct PackedForce {
+    float4 q[D == 3 ? 3 : 2];
+    // pack: the particle's words; cpack: the same shifted by the channel's four
+    __device__ void load(const float* pack, const float* cpack) {
+        q[0] = reinterpret_cast<const float4*>(pack)[0];
+        if constexpr (D == 3) {
+            q[1] = reinterpret_cast<const float4*>(pack)[1];
+            q[2] = reinterpret_cast<const float4*>(cpack)[2];
+        } else {
+            q[1] = reinterpret_cast<const float4*>(cpack)[1];
+        }
+    }
+};
+
+// One packed particle's force on channel cc: M += sum_r A[r][cc] d_r of every
+// function (the transpose of stencil_gradient; the constant's moment stays 0).
+template <int D>
+__device__ inline void add_force_moments(const PackedForce<D>& f4, float* M) {
+    if constexpr (D == 3) {
+        const float4 p = f4.q[0], r = f4.q[1], a = f4.q[2];
+        const float d2x = p.w + 1.0f, d2y = r.w + 1.0f, d2z = a.w + 1.0f;
+        const float e[3] = {p.w * a.x, 0.0f, d2x * a.x};
+        const float f[3] = {p.x * a.y, a.y, r.x * a.y};
+        const float h[3] = {p.x * a.z, a.z, r.x * a.z};
 #pragma unroll
         for (int i = 0; i < 3; ++i) {
-            float x0[3], x1[3], x2[3];
-#pragma unroll
-            for (int cc = 0; cc < 3; ++cc) {
-                x0[cc] = A[0 * 3 + cc] * dw[0][i];
-                x1[cc] = A[1 * 3 + cc] * w[0][i];
-                x2[cc] = A[2 * 3 + cc] * w[0][i];
-            }
+            const float y[3] = {i == 1 ? r.w * f[i] : fmaf(p.y, e[i], r.w * f[i]), e[i],
+                                i == 1 ? d2y * f[i] : fmaf(r.y, e[i], d2y * f[i])};
+            const float z[3] = {p.y * h[i], h[i], r.y * h[i]};
 #pragma unroll
             for (int j = 0; j < 3; ++j) {
-                float ya[3], yb[3];
-#pragma unroll
-                for (int cc = 0; cc < 3; ++cc) {
-                    ya[cc] = fmaf(w[1][j], x0[cc], dw[1][j] * x1[cc]);
-                    yb[cc] = w[1][j] * x2[cc];
-                }
-                const int t0 = base + i * LX + j * LY;
-#pragma unroll
-                for (int k = 0; k < 3; ++k) {
-                    // a step's three reads go out before its writes
-                    float o[3];
-#pragma unroll
-                    for (int cc = 0; cc < 3; ++cc) o[cc] = q[cc * TN + t0 + k];
-#pragma unroll
-                    for (int cc = 0; cc < 3; ++cc) q[cc * TN + t0 + k] = fmaf(w[2][k], ya[cc], fmaf(dw[2][k], yb[cc], o[cc]));
-                    MPM_STEP_FENCE();
+                float* k = M + (i * 3 + j) * 3;
+                if (i != 1 || j != 1) {
+                    k[0] = fmaf(a.w, z[j], fmaf(p.z, y[j], k[0]));
+                    k[1] += y[j];
+                    k[2] = fmaf(d2z, z[j], fmaf(r.z, y[j], k[2]));
+                } else {
+                    k[0] = fmaf(a.w, z[j], k[0]);
+                    k[2] = fmaf(d2z, z[j], k[2]);
                 }
             }
         }
     } else {
+        const float4 p = f4.q[0], a = f4.q[1];
+        const float d2x = a.z + 1.0f, d2y = a.w + 1.0f;
+        const float e[3] = {a.z * a.x, 0.0f, d2x * a.x};
+        const float f[3] = {p.x * a.y, a.y, p.z * a.y};
 #pragma unroll
         for (int i = 0; i < 3; ++i) {
-            float x0[2], x1[2];
-#pragma unroll
-            for (int cc = 0; cc < 2; ++cc) {
-                x0[cc] = A[0 * 2 + cc] * dw[0][i];
-                x1[cc] = A[1 * 2 + cc] * w[0][i];
+            float* k = M + i * 3;
+            if (i != 1) {
+                k[0] = fmaf(a.w, f[i], fmaf(p.y, e[i], k[0]));
+                k[1] += e[i];
+                k[2] = fmaf(d2y, f[i], fmaf(p.w, e[i], k[2]));
+            } else {
+                k[0] = fmaf(a.w, f[i], k[0]);
+                k[2] = fmaf(d2y, f[i], k[2]);
             }
-            const int t0 = base + i * LX;
+        }
+    }
+}
+
+// The value of lane P0..P3 of each group of four lanes (DPP quad_perm).
+template <int P0, int P1, int P2, int P3>
+__device__ inline float quad_perm(float x) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), P0 | (P1 << 2) | (P2 << 4) | (P3 << 6), 0xf, 0xf, true));
+}
+
+// A cell's moments of one channel into its node contributions (the transposed
+// transform), in place.
+template <int D>
+__device__ inline void nodes_of_cell(float* M) {
+    if constexpr (D == 3) {
 #pragma unroll
-            for (int j = 0; j < 3; ++j) {
+        for (int k = 0; k < 9; ++k) nodes_of_moments(M[k], M[9 + k], M[18 + k]);
 #pragma unroll
-                for (int cc = 0; cc < 2; ++cc) {
-                    float* dst = q + cc * TN + t0 + j;
-                    *dst = fmaf(w[1][j], x0[cc], fmaf(dw[1][j], x1[cc], *dst));
-                }
-                MPM_STEP_FENCE();
-            }
+        for (int i = 0; i < 3; ++i)
+#pragma unroll
+            for (int k = 0; k < 3; ++k) nodes_of_moments(M[i * 9 + k], M[i * 9 + 3 + k], M[i * 9 + 6 + k]);
+#pragma unroll
+        for (int r = 0; r < 9; ++r) nodes_of_moments(M[r * 3], M[r * 3 + 1], M[r * 3 + 2]);
+    } else {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) nodes_of_moments(M[k], M[3 + k], M[6 + k]);
+#pragma unroll
+        for (int r = 0; r < 3; ++r) nodes_of_moments(M[r * 3], M[r * 3 + 1], M[r * 3 + 2]);
+    }
+}
+
+// Adds one channel's node contributions M of all cells (lane = cell) to the
+// channel's LDS tile q in ordered read-add-writes in which the lanes' nodes
+// are distinct (the fence keeps the steps in order: a step may read a node
+// that another lane wrote in the step before).  3D: the four cells of a row in
+// z are neighbouring lanes, so their three planes are summed across the lanes
+// first (lane z keeps node z, lanes 2 and 3 also nodes 4 and 5), nine steps
+// instead of 27.
+template <int D>
+__device__ inline void add_cell_nodes(const float* M, int base, int lane, float* q) {
+    constexpr int LX = Dims<D>::LX, LY = Dims<D>::LY;
+    if constexpr (D == 3) {
+        const int lz = lane & 3;
+#pragma unroll
+        for (int r = 0; r < 9; ++r) {
+            const float* n = M + r * 3;
+            const float up1 = quad_perm<0, 0, 1, 2>(n[1]), up2 = quad_perm<0, 1, 0, 1>(n[2]);
+            const float last = quad_perm<3, 3, 3, 3>(n[1]);
+            const float s0 = n[0] + (lz >= 1 ? up1 : 0.0f) + (lz >= 2 ? up2 : 0.0f);
+            const float s1 = n[2] + (lz == 2 ? last : 0.0f);
+            float* d = q + base + (r / 3) * LX + (r % 3) * LY;
+            const float o0 = d[0], o1 = d[2];
+            d[0] = o0 + s0;
+            if (lz >= 2) d[2] = o1 + s1;
+            MPM_STEP_FENCE();
+        }
+    } else {
+#pragma unroll
+        for (int n = 0; n < 9; ++n) {
+            q[base + (n / 3) * LX + n % 3] += M[n];
+            MPM_STEP_FENCE();
         }
     }
 }
@@ -1655,31 +1753,204 @@ __device__ inline bool cg_all_done(const KP& p) { return p.ctr->cg_ndone >= p.cg
 // the other scenes are skipped.
 __device__ inline bool other_scene(const KP& p, int b) { return p.nscenes > 1 && p.block_scene[b] != p.solo; }
 
+// LDS of the CG operator's work-group:
+//   coef  the block's coefficient rows, later the cells' node contributions
+//         (27 x 64 x channels, running on into pack);
+//   pack  the packed particles of a chunk (and one word group past them, read
+//         ahead and unused), before that the node tile the coefficients come
+//         from, after it the force tile;
+//   cell  the cell of every particle of the chunk;
+//   perm  the block's cells by descending particle count.
+template <int D>
+struct OperatorLds {
+    using CS = CellStencil<D>;
+    static constexpr int LTN = Dims<D>::LTN;
+    static constexpr int COEF = CS::ROWS * 64;
+    static constexpr int PACKED = CS::PACK * (BWG + 1);
+    static constexpr int TILE = 1024;  // the force tile's (and before it the sort's) place in pack
+    static_assert(D * LTN <= TILE && TILE + D * LTN <= PACKED && COEF + TILE >= CS::NC * D * 64 && COEF % 4 == 0, "aliases");
+    float coef[COEF + PACKED];
+    unsigned char cell[BWG];
+    unsigned char perm[64];
+    __device__ float* pack() { return coef + COEF; }
+};
+
+// perm: the cells by descending count n (lane = cell) -- a counting sort by
+// one wave; the order among equal counts follows the LDS atomics and decides
+// only which lane sums a cell, never its sum.
+__device__ inline void sort_cells(int n, int lane, int* hist, unsigned char* perm) {
+    const int key = 63 - min(n, 63);
+    hist[lane] = 0;
+    MPM_STEP_FENCE();
+    atomicAdd(&hist[key], 1);
+    MPM_STEP_FENCE();
+    const int h = hist[lane];
+    int x = h;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int y = __shfl_up(x, off);
+        if (lane >= off) x += y;
+    }
+    hist[lane] = x - h;
+    MPM_STEP_FENCE();
+    perm[atomicAdd(&hist[key], 1)] = (unsigned char)lane;
+}
+
+// One block of the operator by one work-group (every thread calls it; all
+// trip counts are uniform).  load(a, n): channel a of node n.
+//
+// Particles are taken twice.  Storage order, one per lane, for the gather and
+// the force map (about 415 operations): every lane is filled whatever the
+// counts of the cells.  For the scatter a lane takes one cell and channel and
+// keeps its 26 moments in registers over all of the cell's particles, so
+// nothing is read, added and written back per particle and only these 70
+// operations wait for the fullest cell of the wave; the cells are dealt to
+// the three waves by descending count, so that a wave's cells are alike.
+template <int D, class Load>
+__device__ inline void operator_block(const KP& p, int b, float inv_dx, OperatorLds<D>& S, Load&& load) {
+    using CS = CellStencil<D>;
+    using Dm = Dims<D>;
+    constexpr int LTN = Dm::LTN, TN = Dm::TN, NBR = Dm::NBR, W = OpRec<D>::W, DD = D * D, TILE = OperatorLds<D>::TILE;
+    static_assert(TN <= BWG && D <= NW - 1 && NW == 4, "thread roles");
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int p0 = p.block_pstart[b], p1 = p.block_pstart[b + 1];
+    const int c0 = p.cell_start[b * 65 + lane], c1 = p.cell_start[b * 65 + lane + 1];
+    float* pack = S.pack();
+    // the first chunk's records load while the tile is gathered
+    const float4* rec4 = reinterpret_cast<const float4*>(p.pop);
+    float4 next[W / 4];
+    auto load_records = [&](int chunk) {
+        const int64_t i = min(chunk + tid, p1 - 1);
+#pragma unroll
+        for (int k = 0; k < W / 4; ++k) next[k] = rec4[i * (W / 4) + k];
+    };
+    auto mark_cells = [&](int chunk) {
+        for (int j = max(c0, chunk); j < min(c1, chunk + BWG); ++j) S.cell[j - chunk] = (unsigned char)lane;
+    };
+    load_records(p0);
+    int li = 0;  // LDS tile index of tile node tid
+    if (tid < TN) {
+        int nb, local, tc[D];
+        tile_map<D>(tid, nb, local, tc);
+        li = lds_index<D>(tc);
+        const int blk = p.block_nbr[(int64_t)b * NBR + nb];
+        const int64_t n = (int64_t)max(blk, 0) * 64 + local;
+        float u[D];
+#pragma unroll
+        for (int a = 0; a < D; ++a) u[a] = load(a, n);
+#pragma unroll
+        for (int a = 0; a < D; ++a) pack[a * LTN + li] = blk >= 0 ? u[a] : 0.0f;
+    }
+    if (wv == NW - 1) {
+        sort_cells(c1 - c0, lane, reinterpret_cast<int*>(pack + TILE), S.perm);
+        mark_cells(p0);
+    }
+    int base;  // tile index of cell `lane`'s stencil corner
+    {
+        int l[D], off0[D];
+        local_coords<D>(lane, l);
+        base = tile_index<D>(l, 0, off0);
+    }
+    __syncthreads();
+    if (wv < D) {
+        float c[CS::NC];
+        cell_coefficients<D>(pack + wv * LTN, base, c);
+#pragma unroll
+        for (int n = 0; n < CS::NC; ++n)
+            if (n != CS::MID) S.coef[CS::row(0, n) * 64 + wv * (CS::NC - 1) * 64 + lane] = c[n];
+    }
+    __syncthreads();
+    // the lane's cell and channel of the scatter
+    const int ch = tid % D, mine = S.perm[min(tid / D, 63)];
+    const int m0 = p.cell_start[b * 65 + mine], m1 = tid < D * 64 ? p.cell_start[b * 65 + mine + 1] : m0;
+    float m[CS::NC];
+#pragma unroll
+    for (int n = 0; n < CS::NC; ++n) m[n] = 0.0f;
+    const float scale = inv_dx * inv_dx;
+    for (int chunk = p0; chunk < p1; chunk += BWG) {
+        if (chunk + tid < p1) {
+            float rec[W];
+#pragma unroll
+            for (int k = 0; k < W / 4; ++k) {
+                rec[4 * k] = next[k].x;
+                rec[4 * k + 1] = next[k].y;
+                rec[4 * k + 2] = next[k].z;
+                rec[4 * k + 3] = next[k].w;
+            }
+            const OuterWeights<D> g(rec);
+            float T[DD], A[DD];  // A = V0 F dP(T^T F)^T
+            stencil_gradient<D>(g, S.coef, S.cell[tid], T);
+            apply_operator<D>(rec, scale, T, A);
+            pack_particle<D>(g, A, pack + tid * CS::PACK);
+        }
+        __syncthreads();
+        if (chunk + BWG < p1) {
+            load_records(chunk + BWG);
+            if (wv == NW - 1) mark_cells(chunk + BWG);
+        }
+        if (wv < D) {
+            // the next particle's words load while the current one is added
+            const int j0 = min(max(m0 - chunk, 0), BWG);
+            int left = min(m1 - chunk, BWG) - j0;
+            const float *a = pack + j0 * CS::PACK, *ac = a + ch * 4;
+            PackedForce<D> f0, f1;
+            f0.load(a, ac);
+            while (left > 0) {
+                a += CS::PACK;
+                ac += CS::PACK;
+                f1.load(a, ac);
+                add_force_moments<D>(f0, m);
+                if (--left <= 0) break;
+                a += CS::PACK;
+                ac += CS::PACK;
+                f0.load(a, ac);
+                add_force_moments<D>(f1, m);
+                --left;
+            }
+        }
+        __syncthreads();
+    }
+    // every cell's node contributions, then the force tile in cell order
+    if (wv < D) {
+        nodes_of_cell<D>(m);
+#pragma unroll
+        for (int n = 0; n < CS::NC; ++n) S.coef[(n * D + ch) * 64 + mine] = m[n];
+    } else if (wv == NW - 1) {
+        for (int t = lane; t < D * LTN; t += 64) pack[TILE + t] = 0.0f;
+    }
+    __syncthreads();
+    if (wv < D) {
+#pragma unroll
+        for (int n = 0; n < CS::NC; ++n) m[n] = S.coef[(n * D + wv) * 64 + lane];
+        add_cell_nodes<D>(m, base, lane, pack + TILE + wv * LTN);
+    }
+    __syncthreads();
+    if (tid < TN) {
+        float* dst = p.tiles + (int64_t)b * D * TN + tid;
+#pragma unroll
+        for (int a = 0; a < D; ++a) dst[a * TN] = pack[TILE + a * LTN + li];
+    }
+    __syncthreads();
+}
+
 // MPM_CG_System::Force (MPM_CG_System.h:150-215) with the linearised operator
 // record: T = sum_i grad w_ip (x) u_i;  A = L T;  q_i += A^T grad w_ip.
 // RESTART applies it to v* (the initial guess); otherwise to the search
 // direction of iteration k, s = r + beta s, formed while gathering.
+//
+// Bound by VALU issue in large scenes, by one block's chain of phases in small
+// ones.  Per launch, against one lane per cell for everything (nodes read per
+// particle, 81 LDS read-add-writes per particle): avalanche of 1.0M particles
+// in 256^3 mid-slide 57 -> 49 us with 4096 work-groups (32.9M -> 19.9M VALU
+// wave instructions), two balls of 243k 24.4 -> 20.0, 3.8k particles 24.0 ->
+// 13.2.  One wave per block with the moments of its cells in registers (255
+// VGPRs, two waves a SIMD) took 61 us: everything then waits for the fullest
+// cell, which holds two to three times the mean.
 template <int D, bool RESTART, bool ONE>
-__global__ __launch_bounds__(BWG) void k_cg_force(KP p, int k) {
-    using Dm = Dims<D>;
-    constexpr int LTN = Dm::LTN, NBR = Dm::NBR, DD = D * D;
-    __shared__ float ut[D][LTN];
-    __shared__ __align__(16) float qt[NW * D * LTN];
-    __shared__ int nbr[NBR];
+__global__ __launch_bounds__(BWG, 4) void k_cg_force(KP p, int k) {
+    __shared__ __align__(16) OperatorLds<D> S;
     if (cg_all_done(p)) return;
-    const int nblocks = p.ctr->nblocks;
-    const int c = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    float* mine = qt + wv * D * LTN;
-    TileMaps<D> tm;
-    tm.init();
-    int l[D];
-    local_coords<D>(c, l);
-    int base;  // tile index of this cell's stencil corner
-    {
-        int off0[D];
-        base = tile_index<D>(l, 0, off0);
-    }
-    const XcdRange xr = xcd_blocks(nblocks);
+    const XcdRange xr = xcd_blocks(p.ctr->nblocks);
     for (int kb = xr.first; kb < xr.end; kb += xr.step) {
         const int b = p.block_order[p.bcap + kb];  // the fullest cells first within the XCD's range
         // one scene: no per-block lookups (its solve is live: cg_all_done above)
@@ -1688,214 +1959,11 @@ __global__ __launch_bounds__(BWG) void k_cg_force(KP p, int k) {
         const SceneParams& sc = p.scn[si];
         if (!sc.active || (!ONE && p.cg[si].done) || block_empty(p, b)) continue;
         const float beta = (RESTART || ONE) ? 0.0f : (float)p.cg[si].beta;
-        if (threadIdx.x < NBR) nbr[threadIdx.x] = p.block_nbr[b * NBR + threadIdx.x];
-        static_assert((NW * D * LTN) % 4 == 0, "float4 zeroing");
-        for (int t = threadIdx.x; t < NW * D * LTN / 4; t += BWG)
-            reinterpret_cast<float4*>(qt)[t] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        __syncthreads();
-        if (tm.g != ~0u) {
-            const int blk = nbr[tm.g & 31u];
-            const int li = (int)(tm.g >> 11);
-            const int64_t n = (int64_t)blk * 64 + (int)((tm.g >> 5) & 63u);
-#pragma unroll
-            for (int a = 0; a < D; ++a) {
-                float u = 0.0f;
-                if (blk >= 0)
-                    u = RESTART ? p.g_vs[a * p.gcap + n]
-                        : ONE   ? p.g_s[a * p.gcap + n]
-                                : cg_direction(p.g_r[a * p.gcap + n], p.g_s[a * p.gcap + n], beta, k);
-                ut[a][li] = u;
-            }
-        }
-        __syncthreads();
-        const int i0 = p.cell_start[b * 65 + c], i1 = p.cell_start[b * 65 + c + 1];
-        for (int i = i0 + wv; i < i1; i += NW) {
-            const float* rec = p.pop + (int64_t)i * OpRec<D>::W;
-            float w[D][3], dw[D][3];
-            {
-                // the record's stencil offsets, formed from the position that
-                // binned the particle into this cell
-                const float4 x4 = *reinterpret_cast<const float4*>(rec);
-                const float xo[3] = {x4.x, x4.y, x4.z};
-#pragma unroll
-                for (int a = 0; a < D; ++a) bspline_from_offset(xo[a], sc.inv_dx, w[a], dw[a]);
-            }
-            float T[DD];
-            grad_gather<D>(w, dw, base, ut, T);
-            float A[DD];  // V0 F dP(T^T F)^T
-            apply_operator<D>(rec, T, A);
-            grad_scatter<D>(w, dw, base, A, mine);
-        }
-        __syncthreads();
-        store_wave_tiles_mapped<D>(p, b, qt, tm.s);
-        __syncthreads();
-    }
-}
-
-// The operator's scatter for one particle, accumulated in registers over the
-// particles of a cell (they share the cell's stencil): acc[node * D + cc],
-// node = (i * 3 + j) * 3 + k.
-template <int D>
-__device__ inline void grad_accumulate(const float (*w)[3], const float (*dw)[3], const float* A, float* acc) {
-    if constexpr (D == 3) {
-#pragma unroll
-        for (int i = 0; i < 3; ++i) {
-            float x0[3], x1[3], x2[3];
-#pragma unroll
-            for (int cc = 0; cc < 3; ++cc) {
-                x0[cc] = A[0 * 3 + cc] * dw[0][i];
-                x1[cc] = A[1 * 3 + cc] * w[0][i];
-                x2[cc] = A[2 * 3 + cc] * w[0][i];
-            }
-#pragma unroll
-            for (int j = 0; j < 3; ++j) {
-                float ya[3], yb[3];
-#pragma unroll
-                for (int cc = 0; cc < 3; ++cc) {
-                    ya[cc] = fmaf(w[1][j], x0[cc], dw[1][j] * x1[cc]);
-                    yb[cc] = w[1][j] * x2[cc];
-                }
-#pragma unroll
-                for (int k = 0; k < 3; ++k)
-#pragma unroll
-                    for (int cc = 0; cc < 3; ++cc) {
-                        float& a = acc[((i * 3 + j) * 3 + k) * 3 + cc];
-                        a = fmaf(w[2][k], ya[cc], fmaf(dw[2][k], yb[cc], a));
-                    }
-            }
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < 3; ++i) {
-            float x0[2], x1[2];
-#pragma unroll
-            for (int cc = 0; cc < 2; ++cc) {
-                x0[cc] = A[0 * 2 + cc] * dw[0][i];
-                x1[cc] = A[1 * 2 + cc] * w[0][i];
-            }
-#pragma unroll
-            for (int j = 0; j < 3; ++j)
-#pragma unroll
-                for (int cc = 0; cc < 2; ++cc) {
-                    float& a = acc[(i * 3 + j) * 2 + cc];
-                    a = fmaf(w[1][j], x0[cc], fmaf(dw[1][j], x1[cc], a));
-                }
-        }
-    }
-}
-
-// Adds a lane's accumulated stencil to the wave's LDS tile: one ordered
-// read-add-write per stencil node (lanes hold distinct cells).
-template <int D>
-__device__ inline void flush_accumulated(int base, const float* acc, float* q) {
-    constexpr int LX = Dims<D>::LX, LY = Dims<D>::LY, TN = Dims<D>::LTN;
-    if constexpr (D == 3) {
-#pragma unroll
-        for (int i = 0; i < 3; ++i)
-#pragma unroll
-            for (int j = 0; j < 3; ++j)
-#pragma unroll
-                for (int k = 0; k < 3; ++k) {
-                    const int t = base + i * LX + j * LY + k;
-#pragma unroll
-                    for (int cc = 0; cc < 3; ++cc) q[cc * TN + t] += acc[((i * 3 + j) * 3 + k) * 3 + cc];
-                    MPM_STEP_FENCE();
-                }
-    } else {
-#pragma unroll
-        for (int i = 0; i < 3; ++i)
-#pragma unroll
-            for (int j = 0; j < 3; ++j) {
-                const int t = base + i * LX + j;
-#pragma unroll
-                for (int cc = 0; cc < 2; ++cc) q[cc * TN + t] += acc[(i * 3 + j) * 2 + cc];
-                MPM_STEP_FENCE();
-            }
-    }
-}
-
-// The same operator with one wave per block: lane c runs every particle of
-// cell c and accumulates the cell's scatter in registers, so a block costs
-// one read-add-write chain per cell instead of one per particle.  The waves
-// of a work-group take different blocks and share nothing (no barriers).
-template <int D, bool RESTART, bool ONE>
-__global__ __launch_bounds__(WG) void k_cg_force_cell(KP p, int k) {
-    using Dm = Dims<D>;
-    constexpr int LTN = Dm::LTN, NBR = Dm::NBR, DD = D * D, TN = Dm::TN, W = WG / 64;
-    __shared__ float ut_all[W][D * LTN];
-    __shared__ float qt_all[W][D * LTN];
-    __shared__ int nbr_all[W][NBR];
-    if (cg_all_done(p)) return;
-    const int c = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    float* ut = ut_all[wv];
-    float* qt = qt_all[wv];
-    int* nbr = nbr_all[wv];
-    int l[D];
-    local_coords<D>(c, l);
-    int base;
-    {
-        int off0[D];
-        base = tile_index<D>(l, 0, off0);
-    }
-    const XcdRange r = xcd_wave_blocks(p.ctr->nblocks);
-    for (int b = r.first; b < r.end; b += r.step) {
-        if (ONE && other_scene(p, b)) continue;
-        const int si = ONE ? p.solo : p.block_scene[b];
-        const SceneParams& sc = p.scn[si];
-        if (!sc.active || (!ONE && p.cg[si].done) || block_empty(p, b)) continue;
-        const float beta = (RESTART || ONE) ? 0.0f : (float)p.cg[si].beta;
-        if (c < NBR) nbr[c] = p.block_nbr[b * NBR + c];
-        for (int t = c; t < D * LTN; t += 64) qt[t] = 0.0f;
-        MPM_STEP_FENCE();
-        for (int t = c; t < TN; t += 64) {
-            int nb, local, tc[D];
-            tile_map<D>(t, nb, local, tc);
-            const int blk = nbr[nb];
-            const int li = lds_index<D>(tc);
-            const int64_t n = (int64_t)blk * 64 + local;
-#pragma unroll
-            for (int a = 0; a < D; ++a) {
-                float u = 0.0f;
-                if (blk >= 0)
-                    u = RESTART ? p.g_vs[a * p.gcap + n]
-                        : ONE   ? p.g_s[a * p.gcap + n]
-                                : cg_direction(p.g_r[a * p.gcap + n], p.g_s[a * p.gcap + n], beta, k);
-                ut[a * LTN + li] = u;
-            }
-        }
-        MPM_STEP_FENCE();
-        float acc[D == 3 ? 81 : 18];
-#pragma unroll
-        for (int t = 0; t < (D == 3 ? 81 : 18); ++t) acc[t] = 0.0f;
-        const int i0 = p.cell_start[b * 65 + c], i1 = p.cell_start[b * 65 + c + 1];
-        const float (*utile)[LTN] = reinterpret_cast<const float (*)[LTN]>(ut);
-        for (int i = i0; i < i1; ++i) {
-            const float* rec = p.pop + (int64_t)i * OpRec<D>::W;
-            float w[D][3], dw[D][3];
-            {
-                // the record's stencil offsets, formed from the position that
-                // binned the particle into this cell
-                const float4 x4 = *reinterpret_cast<const float4*>(rec);
-                const float xo[3] = {x4.x, x4.y, x4.z};
-#pragma unroll
-                for (int a = 0; a < D; ++a) bspline_from_offset(xo[a], sc.inv_dx, w[a], dw[a]);
-            }
-            float T[DD];
-            grad_gather<D>(w, dw, base, utile, T);
-            float A[DD];
-            apply_operator<D>(rec, T, A);
-            grad_accumulate<D>(w, dw, A, acc);
-        }
-        flush_accumulated<D>(base, acc, qt);
-        MPM_STEP_FENCE();
-        float* dst = p.tiles + (int64_t)b * D * TN;
-        for (int t = c; t < D * TN; t += 64) {
-            const int cc = t / TN;
-            int nb, local, tc[D];
-            tile_map<D>(t - cc * TN, nb, local, tc);
-            dst[t] = qt[cc * LTN + lds_index<D>(tc)];
-        }
-        MPM_STEP_FENCE();
+        operator_block<D>(p, b, sc.inv_dx, S, [&](int a, int64_t n) {
+            return RESTART ? p.g_vs[a * p.gcap + n]
+                   : ONE   ? p.g_s[a * p.gcap + n]
+                           : cg_direction(p.g_r[a * p.gcap + n], p.g_s[a * p.gcap + n], beta, k);
+        });
     }
 }
 
@@ -2783,11 +2851,6 @@ template <int D> void launch_cg_force(const KP& p, hipStream_t s, int grid, bool
     else if (one) hipLaunchKernelGGL((k_cg_force<D, false, true>), dim3(grid), dim3(BWG), 0, s, p, k);
     else hipLaunchKernelGGL((k_cg_force<D, false, false>), dim3(grid), dim3(BWG), 0, s, p, k);
 }
-template <int D> void launch_cg_force_cell(const KP& p, hipStream_t s, int grid, bool restart, int k, bool one) {
-    if (restart) hipLaunchKernelGGL((k_cg_force_cell<D, true, false>), dim3(grid), dim3(WG), 0, s, p, 0);
-    else if (one) hipLaunchKernelGGL((k_cg_force_cell<D, false, true>), dim3(grid), dim3(WG), 0, s, p, k);
-    else hipLaunchKernelGGL((k_cg_force_cell<D, false, false>), dim3(grid), dim3(WG), 0, s, p, k);
-}
 template <int D> void launch_cg_restart_node(const KP& p, hipStream_t s, int grid, bool one) {
     if (one) hipLaunchKernelGGL((k_cg_restart_node<D, true>), dim3(grid), dim3(WG), 0, s, p);
     else hipLaunchKernelGGL((k_cg_restart_node<D, false>), dim3(grid), dim3(WG), 0, s, p);
@@ -2821,7 +2884,6 @@ template <int D> void launch_max_speed(const KP& p, hipStream_t s, int grid) { h
     template void launch_particle_force<D>(const KP&, hipStream_t, int, bool, bool);          \
     template void launch_grid_update<D>(const KP&, hipStream_t, int, bool, bool, bool, bool); \
     template void launch_cg_force<D>(const KP&, hipStream_t, int, bool, int, bool);           \
-    template void launch_cg_force_cell<D>(const KP&, hipStream_t, int, bool, int, bool);      \
     template void launch_cg_restart_node<D>(const KP&, hipStream_t, int, bool);               \
     template void launch_cg_update_s<D>(const KP&, hipStream_t, int, int);                    \
     template void launch_cg_node1<D>(const KP&, hipStream_t, int, int, bool);                 \

@@ -1,0 +1,55 @@
+"""The CG operator at the edges of its chunks and cell counts.
+
+A block's particles are taken 256 at a time and its cells are sorted by
+count up to 63: one substep of a scene that packs a given number of
+particles into one cell (next to a sparse neighbourhood that spans blocks)
+must match the FP64 oracle to the one-substep bar, 1e-5 relative L2, per
+field.  The particles carry a velocity gradient, so the operator's result
+reaches every compared field.
+"""
+import numpy as np
+import pytest
+
+import non_ficks_diffusion_amd as M
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def rel(a, b):
+    return float(np.linalg.norm(np.asarray(a, np.float64) - b) / max(np.linalg.norm(b), 1e-30))
+
+
+@pytest.mark.parametrize("dim", [2, 3])
+@pytest.mark.parametrize("n", [1, 63, 64, 255, 256, 257, 513, 700])
+def test_cell_and_chunk_edges(dim, n):
+    r = np.random.default_rng(100 * dim + n)
+    name, counts = ("disk2d", 32) if dim == 2 else ("two_balls", 32)
+    d, _, _, _ = M.scene_generate(name, counts, 0)
+    d.cg_max_iterations = 200
+    dx = 1.0 / counts
+    # n particles in cell 15 of every axis, the last of its block in 2D and 3D
+    cell = (15 + r.uniform(0.02, 0.98, (n, dim))) * dx
+    # two per cell over the six cells around it (several blocks, sparse cells)
+    g = np.stack(np.meshgrid(*[np.arange(12, 18)] * dim, indexing="ij"), -1).reshape(-1, dim)
+    around = (np.repeat(g, 2, axis=0) + r.uniform(0.1, 0.9, (2 * len(g), dim))) * dx
+    x = np.concatenate([cell, around]).astype(np.float32)
+    # a rate of about one per second, with shear
+    v = ((x - 0.5) @ r.uniform(-1.0, 1.0, (dim, dim)) + 0.5).astype(np.float32)
+    m = np.full(len(x), 400.0 * dx ** dim / 8, np.float32)
+    dt = 0.5 * float(d.max_dt)
+    s = M.Scene(d, len(m))
+    s.upload(x, v, m)
+    s.initialize()
+    st = s.substep(dt, stats=True)
+    got = s.download()
+    s.close()
+    o = O.Oracle(d, 8, 4, O.DOT_FP64 | O.SVD_FP64)
+    o.set_particles(x, v, m)
+    o.initialize()
+    o.advance_step(dt)
+    want = o.particles()
+    assert st["cg_converged"] == 1
+    assert np.array_equal(got["ids"], want["ids"])
+    for k in ("x", "v", "F", "Jp"):
+        assert rel(got[k], want[k]) < 1e-5, k
