@@ -110,6 +110,8 @@ mpm::SceneParams scene_params(const mpm_scene_desc& d, int slot_base, int nslots
     return p;
 }
 
+bool cg_in_one_launch(const mpm_context* c);
+
 mpm::KP make_kp(const mpm_context* c) {
     mpm::KP p{};
     p.scn = c->scn;
@@ -118,6 +120,7 @@ mpm::KP make_kp(const mpm_context* c) {
     p.slot_scene = c->slot_scene;
     p.nscenes = c->nscenes;
     p.solo = c->solo >= 0 ? c->solo : 0;
+    p.one_launch = cg_in_one_launch(c) ? 1 : 0;
     p.cg_target = (c->nscenes == 1 || c->solo >= 0) ? 1 : c->nscenes;
     p.pcur = c->pbuf[c->cur];
     p.palt = c->pbuf[c->cur ^ 1];
@@ -260,13 +263,34 @@ constexpr int64_t SOLO_LAUNCHED_MIN = 65536;
 // the first batch's poll and is usually all no-ops
 constexpr int CG_CHUNK = 4;
 constexpr int CG_COVER = 1;
-// A done poll copies Counters::overflow .. cg_iters (five ints) into a slot
-// of POLL_INTS pinned ints: [0] overflow, [1] finished solves, [4] the
-// largest iteration count among them.
+// A done poll copies the first eight counters into a slot of POLL_INTS pinned
+// ints.
 constexpr int POLL_INTS = 8;
-static_assert(offsetof(mpm::Counters, cg_ndone) == offsetof(mpm::Counters, overflow) + sizeof(int) &&
-                  offsetof(mpm::Counters, cg_iters) == offsetof(mpm::Counters, overflow) + 4 * sizeof(int),
+enum { POLL_NBLOCKS = 0, POLL_OVERFLOW = 3, POLL_NDONE = 4, POLL_CG_ITERS = 7 };
+static_assert(offsetof(mpm::Counters, nblocks) == 0 && offsetof(mpm::Counters, overflow) == POLL_OVERFLOW * sizeof(int) &&
+                  offsetof(mpm::Counters, cg_ndone) == POLL_NDONE * sizeof(int) &&
+                  offsetof(mpm::Counters, cg_iters) == POLL_CG_ITERS * sizeof(int),
               "Counters layout of the done poll");
+
+// The solve in one launch (k_cg_solve) for handles of up to this many
+// particles (at eight a cell about 130 blocks that hold some, 350 with their
+// halo).  Measured per frame of 60 fps: 3.8k particles in 32^3 13.3 -> 7.8 ms
+// (captured), 20k in 64^3 (fluid) 5.7 -> 5.4; above, work-groups take more than
+// one block each and the launched kernels win: four requests of 200k particles
+// together 150 -> 219 ms, two balls of 243k 91 -> 153.  The rule reads only what the
+// caller uploaded, so launched, replayed and repeated substeps take the same
+// kernels.
+constexpr int64_t CG_SOLVE_MAX_PARTICLES = 65536;
+bool cg_in_one_launch(const mpm_context* c) {
+    int64_t n = 0;
+    int scenes = 0;
+    for (int s = 0; s < c->nscenes; ++s) {
+        if (c->pool && !c->entry_used[(size_t)s]) continue;
+        n += c->sc[(size_t)s].n_uploaded;
+        ++scenes;
+    }
+    return n <= CG_SOLVE_MAX_PARTICLES && scenes <= mpm::CG_SOLVE_MAX_SCENES;
+}
 
 int max_cg_iterations(const mpm_context* c) {
     if (c->pool) return c->pool_cg_max;
@@ -287,6 +311,21 @@ int stage_cg(mpm_context* c, bool do_init, bool fixed = false) {
     const int gn = c->grid_node;
     if (do_init)
         timed(c, KC_GRID, [&] { mpm::launch_grid_update<D>(p, c->stream, gn, false, false, true, false); });
+    if (cg_in_one_launch(c)) {
+        timed(c, KC_CG_FORCE, [&] { mpm::launch_cg_solve<D>(p, c->stream, mpm::CG_RESIDENT); });
+        if (!fixed) {
+            // read once the rest of the substep is queued (the overflow flag)
+            mpm::launch_poll(p, c->stream, c->d_done);
+            HIPCHECK(hipEventRecord(c->done_ev[0], c->stream));
+            c->poll_open = true;
+            c->poll_older = 0;
+            c->poll_target = one ? 1 : c->nscenes;
+            c->poll_max_it = max_cg_iterations(c);
+            c->poll_pending[0] = true;
+            c->poll_pending[1] = false;
+        }
+        return MPM_OK;
+    }
     timed(c, KC_CG_FORCE, [&] { launch_operator<D>(c, p, true, 0, one); });
     timed(c, KC_CG_NODE, [&] {
         mpm::launch_cg_restart_node<D>(p, c->stream, gn, one);
@@ -335,11 +374,11 @@ int stage_cg(mpm_context* c, bool do_init, bool fixed = false) {
             HIPCHECK(hipEventSynchronize(c->done_ev[slot]));
             pending[slot] = false;
             const int* h = &c->h_done[POLL_INTS * slot];
-            c->overflow_seen = c->overflow_seen || h[0] != 0;
-            if (h[1] >= target) {
+            c->overflow_seen = c->overflow_seen || h[POLL_OVERFLOW] != 0;
+            if (h[POLL_NDONE] >= target) {
                 // the next solve's first batch: this one's iterations (iteration
                 // k's convergence test ends a solve of k updates)
-                c->cg_predict = h[4] + 1;
+                c->cg_predict = h[POLL_CG_ITERS] + 1;
                 finished = true;
                 break;
             }
@@ -375,8 +414,8 @@ int finish_cg_poll(mpm_context* c) {
         c->poll_pending[slot] = false;
         HIPCHECK(hipEventSynchronize(c->done_ev[slot]));
         const int* h = &c->h_done[POLL_INTS * slot];
-        c->overflow_seen = c->overflow_seen || h[0] != 0;
-        if (iters < 0 && h[1] >= c->poll_target) iters = h[4];
+        c->overflow_seen = c->overflow_seen || h[POLL_OVERFLOW] != 0;
+        if (iters < 0 && h[POLL_NDONE] >= c->poll_target) iters = h[POLL_CG_ITERS];
     }
     // seen done: its iterations; never seen done (the cap's test runs after
     // the last poll): the cap
@@ -442,7 +481,7 @@ int substep(mpm_context* c, const float* dts, bool capture = false) {
         int active = 0, last = -1;
         for (int s = 0; s < c->nscenes; ++s)
             if (dts[s] > 0.0f) { ++active; last = s; }
-        if (active == 1) c->solo = last;
+        if (active == 1 && !cg_in_one_launch(c)) c->solo = last;
     }
     if (capture) mpm::launch_set_step_dev(make_kp(c), c->stream, c->d_dt);
     else set_step(c, dts, 0.0f, false, false);
@@ -937,7 +976,7 @@ int download_scene(mpm_context* c, int s, int64_t cap, float* x, float* v, float
 }
 
 void invalidate_graphs(mpm_context* c) {
-    for (int k = 0; k < 2; ++k) {
+    for (int k = 0; k < 4; ++k) {
         if (c->gexec[k]) {
             (void)hipGraphExecDestroy(c->gexec[k]);
             c->gexec[k] = nullptr;
@@ -957,6 +996,9 @@ void invalidate_graphs(mpm_context* c) {
 // even, so a replay leaves the particle buffers at the parity it found.
 constexpr int FRAME_K = 4;
 
+// The captured graph of a buffer parity: one for each form of the CG.
+int graph_slot(const mpm_context* c, int parity) { return parity + (cg_in_one_launch(c) ? 2 : 0); }
+
 int capture_frame_graph(mpm_context* c, int parity) {
     const bool timing = c->timing;
     c->timing = false;
@@ -974,10 +1016,10 @@ int capture_frame_graph(mpm_context* c, int parity) {
         if (g) (void)hipGraphDestroy(g);
         return rc != MPM_OK ? rc : mpm_set_error(MPM_E_HIP, std::string("hipStreamEndCapture: ") + hipGetErrorString(e));
     }
-    const hipError_t ei = hipGraphInstantiate(&c->fexec[parity], g, nullptr, nullptr, 0);
+    const hipError_t ei = hipGraphInstantiate(&c->fexec[graph_slot(c, parity)], g, nullptr, nullptr, 0);
     (void)hipGraphDestroy(g);
     if (ei != hipSuccess) {
-        c->fexec[parity] = nullptr;
+        c->fexec[graph_slot(c, parity)] = nullptr;
         return mpm_set_error(MPM_E_HIP, std::string("hipGraphInstantiate: ") + hipGetErrorString(ei));
     }
     return MPM_OK;
@@ -1006,11 +1048,11 @@ int device_frames(mpm_context* c, const float* time, const float* target, float*
     HIPCHECK(hipMemcpyAsync(c->frame, f.data(), sizeof(mpm::FrameState) * (size_t)n, hipMemcpyHostToDevice, c->stream));
     while (ndone < n) {
         const int parity = c->cur;
-        if (!c->fexec[parity]) {
+        if (!c->fexec[graph_slot(c, parity)]) {
             const int rc = capture_frame_graph(c, parity);
             if (rc) return rc;
         }
-        HIPCHECK(hipGraphLaunch(c->fexec[parity], c->stream));
+        HIPCHECK(hipGraphLaunch(c->fexec[graph_slot(c, parity)], c->stream));
         c->binned = false;
         c->ever_binned = true;
         c->stepped = true;
@@ -1046,7 +1088,7 @@ int graph_substep(mpm_context* c, const float* dts) {
     HIPCHECK(hipEventRecord(c->dt_ev, c->stream));
     c->dt_pending = true;
     const int parity = c->cur;
-    if (!c->gexec[parity]) {
+    if (!c->gexec[graph_slot(c, parity)]) {
         const bool timing = c->timing;
         c->timing = false;
         HIPCHECK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
@@ -1059,14 +1101,14 @@ int graph_substep(mpm_context* c, const float* dts) {
             if (g) (void)hipGraphDestroy(g);
             return rc != MPM_OK ? rc : mpm_set_error(MPM_E_HIP, std::string("hipStreamEndCapture: ") + hipGetErrorString(e));
         }
-        const hipError_t ei = hipGraphInstantiate(&c->gexec[parity], g, nullptr, nullptr, 0);
+        const hipError_t ei = hipGraphInstantiate(&c->gexec[graph_slot(c, parity)], g, nullptr, nullptr, 0);
         (void)hipGraphDestroy(g);
         if (ei != hipSuccess) {
-            c->gexec[parity] = nullptr;
+            c->gexec[graph_slot(c, parity)] = nullptr;
             return mpm_set_error(MPM_E_HIP, std::string("hipGraphInstantiate: ") + hipGetErrorString(ei));
         }
     }
-    HIPCHECK(hipGraphLaunch(c->gexec[parity], c->stream));
+    HIPCHECK(hipGraphLaunch(c->gexec[graph_slot(c, parity)], c->stream));
     c->cur = parity ^ 1;  // the replay binned once
     c->binned = false;
     c->ever_binned = true;
@@ -1080,7 +1122,8 @@ int do_substep(mpm_context* c, const float* dts) {
     int active = 0, last = -1;
     for (int s = 0; s < c->nscenes; ++s)
         if (dts[s] > 0.0f) { ++active; last = s; }
-    const bool solo = c->nscenes > 1 && active == 1 && c->sc[(size_t)last].n_uploaded >= SOLO_LAUNCHED_MIN;
+    const bool small = cg_in_one_launch(c);
+    const bool solo = !small && c->nscenes > 1 && active == 1 && c->sc[(size_t)last].n_uploaded >= SOLO_LAUNCHED_MIN;
     int rc = c->graph && !c->emitted && !solo ? graph_substep(c, dts)
              : c->D == 3                      ? substep<3>(c, dts)
                                               : substep<2>(c, dts);

@@ -60,6 +60,9 @@ struct Counters {
     int slot_hw;        // slots [0, slot_hw) hold every scene's range (the binning scans them)
     int frame_ndone;    // device frame loop: scenes that reached their frame end
     int cg_iters;       // largest iteration count of the solves finished in this substep
+    // k_cg_solve: work-groups that have come (with a bit once the door is
+    // closed) and how many of them share the blocks
+    int door, group;
 };
 
 // Device frame loop of one scene (MPM_Driver::Advance_To_Target_Time,
@@ -77,6 +80,8 @@ struct FrameState {
 struct CGState {
     double rho_hist[2], alpha, beta, conv, rr, sq;
     int iter, done, converged, multiplies;
+    int arrived;  // k_cg_solve: work-groups of the scene counted in, over all its waits
+    int pad;
 };
 
 struct KP {
@@ -87,6 +92,7 @@ struct KP {
     const int* slot_scene;  // per global slot: the scene that owns it, -1 if none
     int nscenes;
     int solo;        // the scene of the single-scene CG kernels (0 for a one-scene context)
+    int one_launch;  // the solve is k_cg_solve
     int cg_target;   // finished solves that end the CG: 1 on the single-scene path, else nscenes
     // particles: field-major arrays of capacity pcap
     float* pcur;
@@ -196,6 +202,11 @@ template <int D> void launch_particle_force(const KP& p, hipStream_t s, int grid
 template <int D> void launch_grid_update(const KP& p, hipStream_t s, int grid, bool force, bool collision, bool cg_init, bool write_f);
 template <int D> void launch_cg_force(const KP& p, hipStream_t s, int grid, bool restart, int k, bool one);
 // `one`: a batch of one scene (per-work-group partials, see k_cg_update_s)
+// the whole solve in one launch (scenes too small to fill the chip; at most
+// CG_SOLVE_MAX_SCENES of them)
+constexpr int CG_SOLVE_MAX_SCENES = 64;
+constexpr int CG_RESIDENT = 512;  // blocks up to which each has a work-group of its own
+template <int D> void launch_cg_solve(const KP& p, hipStream_t s, int grid);
 template <int D> void launch_cg_restart_node(const KP& p, hipStream_t s, int grid, bool one);
 template <int D> void launch_cg_update_s(const KP& p, hipStream_t s, int grid, int k);
 template <int D> void launch_cg_node1(const KP& p, hipStream_t s, int grid, int k, bool one);

@@ -57,6 +57,32 @@ __device__ inline XcdRange xcd_wave_blocks(int n) {
     return {lo + k * W + (int)(threadIdx.x >> 6), hi, (int)(gridDim.x >> 3) * W};
 }
 
+// Accesses of data that work-groups on different XCDs exchange inside one
+// kernel: relaxed atomics at device scope, so that a load never hits a stale
+// line of its XCD's L2 and a store reaches memory without a write-back of the
+// whole cache (a release fence at device scope is one per work-group).
+__device__ inline float ld_agent(const float* a) { return __hip_atomic_load(a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ inline double ld_agent(const double* a) { return __hip_atomic_load(a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ inline int ld_agent(const int* a) { return __hip_atomic_load(a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ inline void st_agent(float* a, float v) { __hip_atomic_store(a, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ inline void st_agent(double* a, double v) { __hip_atomic_store(a, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ inline void st_agent(int* a, int v) { __hip_atomic_store(a, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ inline int add_agent(int* a, int v) { return __hip_atomic_fetch_add(a, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+template <bool AGENT, class T>
+__device__ inline T ld(const T* a) {
+    if constexpr (AGENT) return ld_agent(a);
+    else return *a;
+}
+template <bool AGENT, class T>
+__device__ inline void st(T* a, T v) {
+    if constexpr (AGENT) st_agent(a, v);
+    else *a = v;
+}
+
+// A place for a partial of k_cg_solve that has not been written: a NaN no
+// arithmetic yields.
+constexpr unsigned long long CG_EMPTY = 0x7ff8c0dec0dec0deull;
+
 // Active block b holds no particles (a halo block of its neighbours).
 __device__ inline bool block_empty(const KP& p, int b) { return p.block_pstart[b + 1] == p.block_pstart[b]; }
 
@@ -184,7 +210,7 @@ __device__ inline bool particle_weights(const KP& p, const SceneParams& sc, int 
 // zero) and are absent from the tile neighbour table.  With crop_ghost_x, nodes whose x index is outside [0, counts-1]
 // receive nothing (the reference's slab crop,
 // Tools/Cropped_Influence_Iterator.h:31-42).
-template <int D, int C>
+template <int D, int C, bool AGENT = false>
 __device__ inline void gather_node_tiles(const KP& p, const SceneParams& sc, int n, float* out) {
     using Dm = Dims<D>;
     constexpr int B = Dm::B, TE = Dm::TE, TN = Dm::TN, NBR = Dm::NBR;
@@ -230,7 +256,7 @@ __device__ inline void gather_node_tiles(const KP& p, const SceneParams& sc, int
         if ((m & ~face) == 0) {
             const float* src = p.tiles + (int64_t)max(blk[m], 0) * C * TN + t;
 #pragma unroll
-            for (int c = 0; c < C; ++c) v[m][c] = src[c * TN];
+            for (int c = 0; c < C; ++c) v[m][c] = ld<AGENT>(src + c * TN);
         }
     }
     // the crop test's loads go out with the tile loads (a cropped node sums
@@ -1651,6 +1677,7 @@ __global__ __launch_bounds__(WG) void k_grid_update(KP p) {
             CGState& cg = p.cg[si];
             const int other = p.cg_target == 1 && si != p.solo ? 1 : 0;
             cg.iter = 0;
+            cg.arrived = 0;
             cg.done = other;
             cg.converged = other;
             cg.multiplies = 0;
@@ -1660,7 +1687,16 @@ __global__ __launch_bounds__(WG) void k_grid_update(KP p) {
         if (blockIdx.x == 0 && threadIdx.x == 0) {
             p.ctr->cg_ndone = 0;
             p.ctr->cg_iters = 0;
+            p.ctr->door = 0;
+            p.ctr->group = 0;
         }
+        // k_cg_solve's places for partials (both parities) and tile flags
+        if (p.one_launch)
+            for (int i = blockIdx.x * WG + threadIdx.x; i < 2 * CG_RESIDENT; i += gridDim.x * WG) {
+                const double empty = __longlong_as_double((long long)CG_EMPTY);
+                p.bsum[i] = p.bmax[i] = p.bsq[i] = empty;
+                if (i < min(CG_RESIDENT, p.bcap)) p.bu[i] = 0u;
+            }
     }
     const XcdRange r = xcd_wave_blocks(p.ctr->nblocks);
     const int lane = threadIdx.x & 63;
@@ -1753,26 +1789,34 @@ __device__ inline bool cg_all_done(const KP& p) { return p.ctr->cg_ndone >= p.cg
 // the other scenes are skipped.
 __device__ inline bool other_scene(const KP& p, int b) { return p.nscenes > 1 && p.block_scene[b] != p.solo; }
 
-// LDS of the CG operator's work-group:
-//   coef  the block's coefficient rows, later the cells' node contributions
-//         (27 x 64 x channels, running on into pack);
-//   pack  the packed particles of a chunk (and one word group past them, read
+// LDS of the CG operator's work-group of NT threads:
+//   coef  the block's coefficient rows, later the node contributions of every
+//         part (27 x 64 x channels a part, running on into pack);
+//   pack  the packed particles of a chunk (and a few words past them, read
 //         ahead and unused), before that the node tile the coefficients come
-//         from, after it the force tile;
+//         from;
+//   tile  the force tile, and before it the counting sort's histogram;
 //   cell  the cell of every particle of the chunk;
 //   perm  the block's cells by descending particle count.
-template <int D>
+template <int D, int NT>
 struct OperatorLds {
     using CS = CellStencil<D>;
     static constexpr int LTN = Dims<D>::LTN;
+    static constexpr int TASKS = D * 64;         // cells and channels of a block
+    static constexpr int PARTS = NT / TASKS;     // lanes that share a task's particles
     static constexpr int COEF = CS::ROWS * 64;
-    static constexpr int PACKED = CS::PACK * (BWG + 1);
-    static constexpr int TILE = 1024;  // the force tile's (and before it the sort's) place in pack
-    static_assert(D * LTN <= TILE && TILE + D * LTN <= PACKED && COEF + TILE >= CS::NC * D * 64 && COEF % 4 == 0, "aliases");
-    float coef[COEF + PACKED];
-    unsigned char cell[BWG];
+    static constexpr int PACKED = CS::PACK * (NT + PARTS);
+    static constexpr int NODES = CS::NC * TASKS * PARTS;
+    // the force tile sits past the packed particles' place or the node
+    // contributions, whichever ends last -- inside pack where that has room
+    static constexpr int TILE = NODES > COEF + 1024 ? NODES : COEF + 1024;
+    static constexpr int WORDS = TILE + D * LTN > COEF + PACKED ? TILE + D * LTN : COEF + PACKED;
+    static_assert(D * LTN <= 1024 && COEF % 4 == 0 && TILE % 4 == 0, "aliases");
+    float coef[WORDS];
+    unsigned char cell[NT];
     unsigned char perm[64];
     __device__ float* pack() { return coef + COEF; }
+    __device__ float* tile() { return coef + TILE; }
 };
 
 // perm: the cells by descending count n (lane = cell) -- a counting sort by
@@ -1796,140 +1840,192 @@ __device__ inline void sort_cells(int n, int lane, int* hist, unsigned char* per
     perm[atomicAdd(&hist[key], 1)] = (unsigned char)lane;
 }
 
-// One block of the operator by one work-group (every thread calls it; all
-// trip counts are uniform).  load(a, n): channel a of node n.
+// One block of the operator by one work-group (every thread makes every call;
+// all trip counts are uniform): open, then any number of apply.
 //
 // Particles are taken twice.  Storage order, one per lane, for the gather and
 // the force map (about 415 operations): every lane is filled whatever the
-// counts of the cells.  For the scatter a lane takes one cell and channel and
-// keeps its 26 moments in registers over all of the cell's particles, so
-// nothing is read, added and written back per particle and only these 70
-// operations wait for the fullest cell of the wave; the cells are dealt to
-// the three waves by descending count, so that a wave's cells are alike.
-template <int D, class Load>
-__device__ inline void operator_block(const KP& p, int b, float inv_dx, OperatorLds<D>& S, Load&& load) {
+// counts of the cells.  For the scatter a lane takes one cell and channel (a
+// part of its particles in work-groups of more lanes than tasks) and keeps the
+// 26 moments in registers, so nothing is read, added and written back per
+// particle and only these 70 operations wait for the fullest cell of the
+// wave; the cells are dealt to the waves by descending count, so that a
+// wave's cells are alike.
+template <int D, int NT>
+struct BlockOperator {
     using CS = CellStencil<D>;
     using Dm = Dims<D>;
-    constexpr int LTN = Dm::LTN, TN = Dm::TN, NBR = Dm::NBR, W = OpRec<D>::W, DD = D * D, TILE = OperatorLds<D>::TILE;
-    static_assert(TN <= BWG && D <= NW - 1 && NW == 4, "thread roles");
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int p0 = p.block_pstart[b], p1 = p.block_pstart[b + 1];
-    const int c0 = p.cell_start[b * 65 + lane], c1 = p.cell_start[b * 65 + lane + 1];
-    float* pack = S.pack();
-    // the first chunk's records load while the tile is gathered
-    const float4* rec4 = reinterpret_cast<const float4*>(p.pop);
+    using L = OperatorLds<D, NT>;
+    static constexpr int LTN = Dm::LTN, TN = Dm::TN, NBR = Dm::NBR, W = OpRec<D>::W, DD = D * D;
+    static constexpr int PARTS = L::PARTS, TASKS = L::TASKS, LAST = NT / 64 - 1;
+    static_assert(TN <= NT && D <= LAST, "thread roles");
+
+    const KP& p;
+    L& S;
+    const float4* rec4;
     float4 next[W / 4];
-    auto load_records = [&](int chunk) {
+    int b, tid, lane, wv, p0, p1, c0, c1, base;
+    int li, node;  // tile node tid: its LDS index and grid node (-1: none)
+
+    __device__ BlockOperator(const KP& kp, L& lds)
+        : p(kp), S(lds), rec4(reinterpret_cast<const float4*>(kp.pop)), tid(threadIdx.x), lane(tid & 63), wv(tid >> 6) {
+        int l[D], off0[D];
+        local_coords<D>(lane, l);
+        base = tile_index<D>(l, 0, off0);  // cell `lane`'s stencil corner
+    }
+    __device__ void load_records(int chunk) {
         const int64_t i = min(chunk + tid, p1 - 1);
 #pragma unroll
         for (int k = 0; k < W / 4; ++k) next[k] = rec4[i * (W / 4) + k];
-    };
-    auto mark_cells = [&](int chunk) {
-        for (int j = max(c0, chunk); j < min(c1, chunk + BWG); ++j) S.cell[j - chunk] = (unsigned char)lane;
-    };
-    load_records(p0);
-    int li = 0;  // LDS tile index of tile node tid
-    if (tid < TN) {
-        int nb, local, tc[D];
-        tile_map<D>(tid, nb, local, tc);
-        li = lds_index<D>(tc);
-        const int blk = p.block_nbr[(int64_t)b * NBR + nb];
-        const int64_t n = (int64_t)max(blk, 0) * 64 + local;
-        float u[D];
-#pragma unroll
-        for (int a = 0; a < D; ++a) u[a] = load(a, n);
-#pragma unroll
-        for (int a = 0; a < D; ++a) pack[a * LTN + li] = blk >= 0 ? u[a] : 0.0f;
     }
-    if (wv == NW - 1) {
-        sort_cells(c1 - c0, lane, reinterpret_cast<int*>(pack + TILE), S.perm);
-        mark_cells(p0);
+    __device__ void mark_cells(int chunk) {
+        for (int j = max(c0, chunk); j < min(c1, chunk + NT); ++j) S.cell[j - chunk] = (unsigned char)lane;
     }
-    int base;  // tile index of cell `lane`'s stencil corner
-    {
-        int l[D], off0[D];
-        local_coords<D>(lane, l);
-        base = tile_index<D>(l, 0, off0);
-    }
-    __syncthreads();
-    if (wv < D) {
-        float c[CS::NC];
-        cell_coefficients<D>(pack + wv * LTN, base, c);
-#pragma unroll
-        for (int n = 0; n < CS::NC; ++n)
-            if (n != CS::MID) S.coef[CS::row(0, n) * 64 + wv * (CS::NC - 1) * 64 + lane] = c[n];
-    }
-    __syncthreads();
-    // the lane's cell and channel of the scatter
-    const int ch = tid % D, mine = S.perm[min(tid / D, 63)];
-    const int m0 = p.cell_start[b * 65 + mine], m1 = tid < D * 64 ? p.cell_start[b * 65 + mine + 1] : m0;
-    float m[CS::NC];
-#pragma unroll
-    for (int n = 0; n < CS::NC; ++n) m[n] = 0.0f;
-    const float scale = inv_dx * inv_dx;
-    for (int chunk = p0; chunk < p1; chunk += BWG) {
-        if (chunk + tid < p1) {
-            float rec[W];
-#pragma unroll
-            for (int k = 0; k < W / 4; ++k) {
-                rec[4 * k] = next[k].x;
-                rec[4 * k + 1] = next[k].y;
-                rec[4 * k + 2] = next[k].z;
-                rec[4 * k + 3] = next[k].w;
-            }
-            const OuterWeights<D> g(rec);
-            float T[DD], A[DD];  // A = V0 F dP(T^T F)^T
-            stencil_gradient<D>(g, S.coef, S.cell[tid], T);
-            apply_operator<D>(rec, scale, T, A);
-            pack_particle<D>(g, A, pack + tid * CS::PACK);
+    // Block bi: its ranges, the tile node of this thread, the order of its
+    // cells and the first chunk's records (in flight).
+    __device__ void open(int bi) {
+        b = bi;
+        p0 = p.block_pstart[b];
+        p1 = p.block_pstart[b + 1];
+        c0 = p.cell_start[b * 65 + lane];
+        c1 = p.cell_start[b * 65 + lane + 1];
+        if (p1 > p0) load_records(p0);
+        li = 0;
+        node = -1;
+        if (tid < TN) {
+            int nb, local, tc[D];
+            tile_map<D>(tid, nb, local, tc);
+            li = lds_index<D>(tc);
+            const int blk = p.block_nbr[(int64_t)b * NBR + nb];
+            node = blk >= 0 ? blk * 64 + local : -1;
         }
+        if (wv == LAST) {
+            sort_cells(c1 - c0, lane, reinterpret_cast<int*>(S.tile()), S.perm);
+            mark_cells(p0);
+        }
+    }
+    // The operator of node values u (channels of tile node tid): leaves the
+    // block's force tile in S.tile().  `again`: not the first apply since open.
+    __device__ void apply(float inv_dx, const float* u, bool again) {
+        float* pack = S.pack();
+        if (tid < TN) {
+#pragma unroll
+            for (int a = 0; a < D; ++a) pack[a * LTN + li] = u[a];
+        }
+        if (again && wv == LAST && p1 - p0 > NT) mark_cells(p0);
         __syncthreads();
-        if (chunk + BWG < p1) {
-            load_records(chunk + BWG);
-            if (wv == NW - 1) mark_cells(chunk + BWG);
-        }
         if (wv < D) {
-            // the next particle's words load while the current one is added
-            const int j0 = min(max(m0 - chunk, 0), BWG);
-            int left = min(m1 - chunk, BWG) - j0;
-            const float *a = pack + j0 * CS::PACK, *ac = a + ch * 4;
-            PackedForce<D> f0, f1;
-            f0.load(a, ac);
-            while (left > 0) {
-                a += CS::PACK;
-                ac += CS::PACK;
-                f1.load(a, ac);
-                add_force_moments<D>(f0, m);
-                if (--left <= 0) break;
-                a += CS::PACK;
-                ac += CS::PACK;
-                f0.load(a, ac);
-                add_force_moments<D>(f1, m);
-                --left;
+            float c[CS::NC];
+            cell_coefficients<D>(pack + wv * LTN, base, c);
+#pragma unroll
+            for (int n = 0; n < CS::NC; ++n)
+                if (n != CS::MID) S.coef[CS::row(0, n) * 64 + wv * (CS::NC - 1) * 64 + lane] = c[n];
+        }
+        __syncthreads();
+        // the lane's cell, channel and part of the scatter: particles j, j +
+        // PARTS, ... below m1
+        const int part = tid / TASKS, task = tid - part * TASKS;
+        const bool scatter = part < PARTS;
+        const int ch = task % D, mine = S.perm[task / D];
+        const int m1 = scatter ? p.cell_start[b * 65 + mine + 1] : 0;
+        int j = p.cell_start[b * 65 + mine] + part;
+        float m[CS::NC];
+#pragma unroll
+        for (int n = 0; n < CS::NC; ++n) m[n] = 0.0f;
+        const float scale = inv_dx * inv_dx;
+        for (int chunk = p0; chunk < p1; chunk += NT) {
+            if (chunk + tid < p1) {
+                float rec[W];
+#pragma unroll
+                for (int k = 0; k < W / 4; ++k) {
+                    rec[4 * k] = next[k].x;
+                    rec[4 * k + 1] = next[k].y;
+                    rec[4 * k + 2] = next[k].z;
+                    rec[4 * k + 3] = next[k].w;
+                }
+                const OuterWeights<D> g(rec);
+                float T[DD], A[DD];  // A = V0 F dP(T^T F)^T
+                stencil_gradient<D>(g, S.coef, S.cell[tid], T);
+                apply_operator<D>(rec, scale, T, A);
+                pack_particle<D>(g, A, pack + tid * CS::PACK);
             }
+            __syncthreads();
+            if (chunk + NT < p1) {
+                load_records(chunk + NT);
+                if (wv == LAST) mark_cells(chunk + NT);
+            }
+            // the next particle's words load while the current one is added
+            const int end = min(m1, chunk + NT);
+            if (j < end) {
+                const float *a = pack + (j - chunk) * CS::PACK, *ac = a + ch * 4;
+                PackedForce<D> f0, f1;
+                f0.load(a, ac);
+                for (;;) {
+                    a += CS::PACK * PARTS;
+                    ac += CS::PACK * PARTS;
+                    f1.load(a, ac);
+                    add_force_moments<D>(f0, m);
+                    j += PARTS;
+                    if (j >= end) break;
+                    a += CS::PACK * PARTS;
+                    ac += CS::PACK * PARTS;
+                    f0.load(a, ac);
+                    add_force_moments<D>(f1, m);
+                    j += PARTS;
+                    if (j >= end) break;
+                }
+            }
+            __syncthreads();
+        }
+        // every part's node contributions, then the force tile in cell order
+        if (scatter) {
+            nodes_of_cell<D>(m);
+#pragma unroll
+            for (int n = 0; n < CS::NC; ++n) S.coef[(part * CS::NC + n) * TASKS + ch * 64 + mine] = m[n];
+        }
+        if (wv == LAST)
+            for (int t = lane; t < D * LTN; t += 64) S.tile()[t] = 0.0f;
+        __syncthreads();
+        if (wv < D) {
+            const float* q = S.coef + wv * 64 + lane;
+#pragma unroll
+            for (int n = 0; n < CS::NC; ++n) m[n] = q[n * TASKS];
+#pragma unroll 1
+            for (int k = 1; k < PARTS; ++k) {
+                q += CS::NC * TASKS;
+#pragma unroll
+                for (int n = 0; n < CS::NC; ++n) m[n] += q[n * TASKS];
+            }
+            add_cell_nodes<D>(m, base, lane, S.tile() + wv * LTN);
         }
         __syncthreads();
     }
-    // every cell's node contributions, then the force tile in cell order
-    if (wv < D) {
-        nodes_of_cell<D>(m);
+    // The force tile to the block's place in memory (AGENT: other work-groups
+    // of this kernel read it).
+    template <bool AGENT>
+    __device__ void store() {
+        if (tid < TN) {
+            float* dst = p.tiles + (int64_t)b * D * TN + tid;
 #pragma unroll
-        for (int n = 0; n < CS::NC; ++n) S.coef[(n * D + ch) * 64 + mine] = m[n];
-    } else if (wv == NW - 1) {
-        for (int t = lane; t < D * LTN; t += 64) pack[TILE + t] = 0.0f;
+            for (int a = 0; a < D; ++a) st<AGENT>(dst + a * TN, S.tile()[a * LTN + li]);
+        }
     }
-    __syncthreads();
-    if (wv < D) {
+};
+
+// load(a, n): channel a of node n
+template <int D, int NT, bool AGENT, class Load>
+__device__ inline void operator_block(const KP& p, int b, float inv_dx, OperatorLds<D, NT>& S, Load&& load) {
+    BlockOperator<D, NT> op(p, S);
+    op.open(b);
+    float u[D];
 #pragma unroll
-        for (int n = 0; n < CS::NC; ++n) m[n] = S.coef[(n * D + wv) * 64 + lane];
-        add_cell_nodes<D>(m, base, lane, pack + TILE + wv * LTN);
-    }
-    __syncthreads();
-    if (tid < TN) {
-        float* dst = p.tiles + (int64_t)b * D * TN + tid;
+    for (int a = 0; a < D; ++a) u[a] = 0.0f;
+    if (op.node >= 0) {
 #pragma unroll
-        for (int a = 0; a < D; ++a) dst[a * TN] = pack[TILE + a * LTN + li];
+        for (int a = 0; a < D; ++a) u[a] = load(a, op.node);
     }
+    op.apply(inv_dx, u, false);
+    op.template store<AGENT>();
     __syncthreads();
 }
 
@@ -1948,7 +2044,7 @@ __device__ inline void operator_block(const KP& p, int b, float inv_dx, Operator
 // cell, which holds two to three times the mean.
 template <int D, bool RESTART, bool ONE>
 __global__ __launch_bounds__(BWG, 4) void k_cg_force(KP p, int k) {
-    __shared__ __align__(16) OperatorLds<D> S;
+    __shared__ __align__(16) OperatorLds<D, BWG> S;
     if (cg_all_done(p)) return;
     const XcdRange xr = xcd_blocks(p.ctr->nblocks);
     for (int kb = xr.first; kb < xr.end; kb += xr.step) {
@@ -1959,7 +2055,7 @@ __global__ __launch_bounds__(BWG, 4) void k_cg_force(KP p, int k) {
         const SceneParams& sc = p.scn[si];
         if (!sc.active || (!ONE && p.cg[si].done) || block_empty(p, b)) continue;
         const float beta = (RESTART || ONE) ? 0.0f : (float)p.cg[si].beta;
-        operator_block<D>(p, b, sc.inv_dx, S, [&](int a, int64_t n) {
+        operator_block<D, BWG, false>(p, b, sc.inv_dx, S, [&](int a, int64_t n) {
             return RESTART ? p.g_vs[a * p.gcap + n]
                    : ONE   ? p.g_s[a * p.gcap + n]
                            : cg_direction(p.g_r[a * p.gcap + n], p.g_s[a * p.gcap + n], beta, k);
@@ -2012,25 +2108,26 @@ __device__ inline void wg_partials_store(double* dsum, double* dmax, double sum,
 
 // Sum / max of `count` partials starting at `first`, in a fixed order
 // relative to `first`; the result is broadcast to every thread.
+template <bool AGENT = false, int NT = WG>
 __device__ inline void reduce_range(const double* sums, const double* maxs, int first, int count, double& sum,
                                     double& mx) {
-    constexpr int U = 8;  // eight independent loads in flight per thread
+    constexpr int U = NT == WG ? 8 : 4;  // independent loads in flight per thread
     double sa[U], ma[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) { sa[u] = 0.0; ma[u] = 0.0; }
-    for (int base = (int)threadIdx.x; base < count; base += U * WG) {
+    for (int base = (int)threadIdx.x; base < count; base += U * NT) {
         // the chunk's loads all go out before its first add (an index past
         // the range reads the range's last entry and is not added)
         double vs[U], vm[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int j = min(base + u * WG, count - 1);
-            vs[u] = sums[first + j];
-            vm[u] = maxs ? maxs[first + j] : 0.0;
+            const int j = min(base + u * NT, count - 1);
+            vs[u] = ld<AGENT>(sums + first + j);
+            vm[u] = maxs ? ld<AGENT>(maxs + first + j) : 0.0;
         }
 #pragma unroll
         for (int u = 0; u < U; ++u)
-            if (base + u * WG < count) {
+            if (base + u * NT < count) {
                 sa[u] += vs[u];
                 if (maxs) ma[u] = fmax(ma[u], vm[u]);
             }
@@ -2039,7 +2136,7 @@ __device__ inline void reduce_range(const double* sums, const double* maxs, int 
 #pragma unroll
     for (int u = 0; u < U; ++u) { s += sa[u]; m = fmax(m, ma[u]); }
     wave_reduce2(s, m);
-    __shared__ double ss[WG / 64], sm[WG / 64];
+    __shared__ double ss[NT / 64], sm[NT / 64];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     __syncthreads();
     if (lane == 0) { ss[wave] = s; sm[wave] = m; }
@@ -2047,7 +2144,7 @@ __device__ inline void reduce_range(const double* sums, const double* maxs, int 
     s = 0.0;
     m = 0.0;
 #pragma unroll
-    for (int w = 0; w < WG / 64; ++w) { s += ss[w]; m = fmax(m, sm[w]); }
+    for (int w = 0; w < NT / 64; ++w) { s += ss[w]; m = fmax(m, sm[w]); }
     sum = s;
     mx = m;
 }
@@ -2066,7 +2163,7 @@ struct CGTestIn {
 __device__ inline CGTestIn cg_test_in(const KP& p, int si, int k) {
     const SceneParams& sc = p.scn[si];
     CGTestIn in;
-    in.rho_prev = p.cg[si].rho_hist[(k + 1) & 1];
+    in.rho_prev = ld_agent(&p.cg[si].rho_hist[(k + 1) & 1]);
     in.tol = sc.cg_tol;
     in.cg_min = sc.cg_min;
     in.cg_max = sc.cg_max;
@@ -2089,20 +2186,58 @@ __device__ inline bool cg_test(const KP& p, int si, int k, double rr, double mx,
         cg.rr = rr;
         if (done) {
             cg.converged = (pass || in.empty) ? 1 : 0;
-            cg.done = 1;
+            st_agent(&cg.done, 1);
             atomicMax(&p.ctr->cg_iters, k);
             atomicAdd(&p.ctr->cg_ndone, 1);
         } else {
-            cg.beta = beta;
-            cg.rho_hist[k & 1] = rr;
+            st_agent(&cg.beta, beta);
+            st_agent(&cg.rho_hist[k & 1], rr);
         }
     }
     beta_f = (float)beta;
     return done;
 }
 
-// CG restart: q = dt^2/m q + x (Multiply_Helper), r = b - q, Project(r);
-// partials of r.r (M-weighted) and max |r|^2.
+// CG restart of block b: q = dt^2/m q + x (Multiply_Helper), r = b - q,
+// Project(r); the block's r.r (M-weighted) and max |r|^2.
+template <int D, bool AGENT>
+__device__ inline void cg_restart_block(const KP& p, const SceneParams& sc, int b, int lane, double& sum, double& mx) {
+    const int n = b * 64 + lane;
+    const float sds = sc.dt * sc.dt;
+    const bool interior = (p.g_flags[n] & MPM_FLAG_INTERIOR_DEV) != 0;
+    float q[D], rv[D];
+    gather_node_tiles<D, D, AGENT>(p, sc, n, q);
+#pragma unroll
+    for (int a = 0; a < D; ++a) rv[a] = p.g_r[a * p.gcap + n];
+    if (interior) {
+        const float cm = sds / p.g_m[n];
+#pragma unroll
+        for (int a = 0; a < D; ++a) {
+            q[a] = cm * q[a] + p.g_vs[a * p.gcap + n];
+            rv[a] = rv[a] - q[a];
+        }
+    }
+    if (project_zero<D>(p, sc, n)) {
+#pragma unroll
+        for (int a = 0; a < D; ++a) rv[a] = 0.0f;
+    }
+#pragma unroll
+    for (int a = 0; a < D; ++a) {
+        st<AGENT>(p.g_r + a * p.gcap + n, rv[a]);
+        p.g_q[a * p.gcap + n] = q[a];
+    }
+    sum = 0.0;
+    mx = 0.0;
+    if (interior) {
+        const double m = (double)p.g_m[n];
+#pragma unroll
+        for (int a = 0; a < D; ++a) {
+            sum += (double)rv[a] * ((double)rv[a] * m);
+            mx += (double)rv[a] * (double)rv[a];
+        }
+    }
+    wave_reduce2(sum, mx);
+}
 template <int D, bool ONE>
 __global__ __launch_bounds__(WG) void k_cg_restart_node(KP p) {
     const XcdRange r = xcd_wave_blocks(p.ctr->nblocks);
@@ -2112,40 +2247,8 @@ __global__ __launch_bounds__(WG) void k_cg_restart_node(KP p) {
         if (ONE && other_scene(p, b)) continue;
         const SceneParams& sc = p.scn[ONE ? p.solo : p.block_scene[b]];
         if (!sc.active) continue;
-        const int n = b * 64 + lane;
-        const float sds = sc.dt * sc.dt;
-        const bool interior = (p.g_flags[n] & MPM_FLAG_INTERIOR_DEV) != 0;
-        float q[D], rv[D];
-        gather_node_tiles<D, D>(p, sc, n, q);
-#pragma unroll
-        for (int a = 0; a < D; ++a) rv[a] = p.g_r[a * p.gcap + n];
-        if (interior) {
-            const float cm = sds / p.g_m[n];
-#pragma unroll
-            for (int a = 0; a < D; ++a) {
-                q[a] = cm * q[a] + p.g_vs[a * p.gcap + n];
-                rv[a] = rv[a] - q[a];
-            }
-        }
-        if (project_zero<D>(p, sc, n)) {
-#pragma unroll
-            for (int a = 0; a < D; ++a) rv[a] = 0.0f;
-        }
-#pragma unroll
-        for (int a = 0; a < D; ++a) {
-            p.g_r[a * p.gcap + n] = rv[a];
-            p.g_q[a * p.gcap + n] = q[a];
-        }
-        double sum = 0.0, mx = 0.0;
-        if (interior) {
-            const double m = (double)p.g_m[n];
-#pragma unroll
-            for (int a = 0; a < D; ++a) {
-                sum += (double)rv[a] * ((double)rv[a] * m);
-                mx += (double)rv[a] * (double)rv[a];
-            }
-        }
-        wave_reduce2(sum, mx);
+        double sum, mx;
+        cg_restart_block<D, false>(p, sc, b, lane, sum, mx);
         if (ONE) {
             wsum += sum;
             wmx = fmax(wmx, mx);
@@ -2197,9 +2300,50 @@ __global__ __launch_bounds__(WG) void k_cg_update_s(KP p, int k, int nparts) {
     }
 }
 
-// Tile sum of the operator, q = dt^2/m q + s, Project(q); partials of s.q.
-// Batches form and store this iteration's s = r + beta s (interior nodes);
-// for one scene k_cg_update_s stored it already.
+// Tile sum of the operator, q = dt^2/m q + s, Project(q) on block b; the
+// block's s.q.  Batches form and store this iteration's s = r + beta s
+// (interior nodes); for one scene k_cg_update_s stored it already.
+template <int D, bool ONE, bool AGENT>
+__device__ inline void cg_node1_block(const KP& p, const SceneParams& sc, int b, int lane, float beta, int k, double& sum) {
+    const float sds = sc.dt * sc.dt;
+    const int n = b * 64 + lane;
+    const bool interior = (p.g_flags[n] & MPM_FLAG_INTERIOR_DEV) != 0;
+    float q[D], sv[D], rv[D];
+    // s, r and m load alongside the flags and the tile gather (every node of
+    // an active block has them; only interior ones use them)
+    const float mn = p.g_m[n];
+#pragma unroll
+    for (int a = 0; a < D; ++a) {
+        sv[a] = ld<AGENT>(p.g_s + a * p.gcap + n);
+        if (!ONE) rv[a] = ld<AGENT>(p.g_r + a * p.gcap + n);
+    }
+    gather_node_tiles<D, D, AGENT>(p, sc, n, q);
+    if (interior) {
+        const float cm = sds / mn;
+#pragma unroll
+        for (int a = 0; a < D; ++a) {
+            if (!ONE) {
+                sv[a] = cg_direction(rv[a], sv[a], beta, k);
+                st<AGENT>(p.g_s + a * p.gcap + n, sv[a]);
+            }
+            q[a] = cm * q[a] + sv[a];
+        }
+    }
+    if (project_zero<D>(p, sc, n)) {
+#pragma unroll
+        for (int a = 0; a < D; ++a) q[a] = 0.0f;
+    }
+#pragma unroll
+    for (int a = 0; a < D; ++a) p.g_q[a * p.gcap + n] = q[a];
+    sum = 0.0;
+    double mx = 0.0;
+    if (interior) {
+        const double m = (double)mn;
+#pragma unroll
+        for (int a = 0; a < D; ++a) sum += (double)sv[a] * ((double)q[a] * m);
+    }
+    wave_reduce2(sum, mx);
+}
 template <int D, bool ONE>
 __global__ __launch_bounds__(WG) void k_cg_node1(KP p, int k) {
     if (cg_all_done(p)) return;
@@ -2212,46 +2356,33 @@ __global__ __launch_bounds__(WG) void k_cg_node1(KP p, int k) {
         const SceneParams& sc = p.scn[si];
         if (!sc.active || (!ONE && p.cg[si].done)) continue;
         const float beta = ONE ? 0.0f : (float)p.cg[si].beta;
-        const float sds = sc.dt * sc.dt;
-        const int n = b * 64 + lane;
-        const bool interior = (p.g_flags[n] & MPM_FLAG_INTERIOR_DEV) != 0;
-        float q[D], sv[D], mn = 1.0f;
-        // one scene: s and m load alongside the flags and the tile gather
-        // (every node of an active block has them; only interior ones use them)
-        if (ONE) {
-            mn = p.g_m[n];
-#pragma unroll
-            for (int a = 0; a < D; ++a) sv[a] = p.g_s[a * p.gcap + n];
-        }
-        gather_node_tiles<D, D>(p, sc, n, q);
-        if (interior) {
-            const float cm = sds / (ONE ? mn : p.g_m[n]);
-#pragma unroll
-            for (int a = 0; a < D; ++a) {
-                if (!ONE) {
-                    sv[a] = cg_direction(p.g_r[a * p.gcap + n], p.g_s[a * p.gcap + n], beta, k);
-                    p.g_s[a * p.gcap + n] = sv[a];
-                }
-                q[a] = cm * q[a] + sv[a];
-            }
-        }
-        if (project_zero<D>(p, sc, n)) {
-#pragma unroll
-            for (int a = 0; a < D; ++a) q[a] = 0.0f;
-        }
-#pragma unroll
-        for (int a = 0; a < D; ++a) p.g_q[a * p.gcap + n] = q[a];
-        double sum = 0.0, mx = 0.0;
-        if (interior) {
-            const double m = (double)(ONE ? mn : p.g_m[n]);
-#pragma unroll
-            for (int a = 0; a < D; ++a) sum += (double)sv[a] * ((double)q[a] * m);
-        }
-        wave_reduce2(sum, mx);
+        double sum;
+        cg_node1_block<D, ONE, false>(p, sc, b, lane, beta, k, sum);
         if (ONE) wsum += sum;
         else if (lane == 0) p.bsq[b] = sum;
     }
     if (ONE) wg_partials_store(p.bsq, nullptr, wsum, 0.0);
+}
+
+// x += alpha s, r -= alpha q on block b; its r.r and max |r|^2.
+template <int D, bool AGENT>
+__device__ inline void cg_node2_block(const KP& p, int b, int lane, float alpha, double& sum, double& mx) {
+    const int n = b * 64 + lane;
+    sum = 0.0;
+    mx = 0.0;
+    if ((p.g_flags[n] & MPM_FLAG_INTERIOR_DEV) != 0) {
+        const double m = (double)p.g_m[n];
+#pragma unroll
+        for (int a = 0; a < D; ++a) {
+            const float sv = ld<AGENT>(p.g_s + a * p.gcap + n), q = p.g_q[a * p.gcap + n], xv = p.g_vs[a * p.gcap + n];
+            p.g_vs[a * p.gcap + n] = alpha * sv + xv;
+            const float rv = -alpha * q + ld<AGENT>(p.g_r + a * p.gcap + n);
+            st<AGENT>(p.g_r + a * p.gcap + n, rv);
+            sum += (double)rv * ((double)rv * m);
+            mx += (double)rv * (double)rv;
+        }
+    }
+    wave_reduce2(sum, mx);
 }
 
 // alpha = rho_k / s.q;  x += alpha s, r -= alpha q; partials of r.r and
@@ -2335,11 +2466,11 @@ __global__ __launch_bounds__(WG) void k_cg_node2(KP p, int k, int nparts) {
 
 // Batches: alpha = rho_k / s.q for every scene still iterating (one
 // work-group per scene over the scene's block partials)
-// The CG's done poll: Counters::overflow .. cg_iters (five ints) into the
-// host's pinned poll slot.
+// The CG's done poll: the eight ints from Counters::nblocks to cg_iters into
+// the host's pinned poll slot.
 __global__ __launch_bounds__(64) void k_poll(KP p, int* dst) {
     const int t = (int)threadIdx.x;
-    if (t < 5) dst[t] = (&p.ctr->overflow)[t];
+    if (t < 8) dst[t] = (&p.ctr->nblocks)[t];
 }
 
 __global__ __launch_bounds__(WG) void k_cg_reduce_sq(KP p, int k) {
@@ -2366,6 +2497,449 @@ __global__ __launch_bounds__(WG) void k_cg_reduce_rr(KP p, int k) {
     reduce_range(p.bsum, p.bmax, b0, b1 - b0, rr, mx);
     float beta;
     (void)cg_test(p, si, k, rr, mx, threadIdx.x == 0, beta, tin);
+}
+
+// ============================================================================
+// The whole CG solve of every scene in one launch, for scenes too small to
+// fill the chip: there a launch's work is a few microseconds, and the four or
+// five launches of an iteration cost more than it.  The iterations, their
+// arithmetic and the order of every sum are those of the launched kernels for
+// batches (a partial per block, a scene's partials summed in block order).
+//
+// Work-groups share the blocks and wait for one another.  No wait depends on a
+// work-group that might not run: they enter through a door (cg_enter) that the
+// first of them closes as soon as all that are needed have come, or after
+// 20 us; those that come later leave, and whoever is inside is running until
+// the kernel ends.  The results do not depend on how many they are.  What
+// work-groups exchange goes through device-scope accesses.
+//
+// All inside (the usual case, at most CG_RESIDENT blocks): one block each,
+// its nodes' m, x, r and s in the registers of wave 0 and its tile's s in those
+// of the tile threads (a halo node's s = r + beta s follows from r alone, so
+// only r and the force tiles travel).  An iteration waits three times: for the
+// neighbours' force tiles (a flag per block), for the scene's partials of s.q
+// and for those of r.r.  A partial is its own flag: its place holds a bit
+// pattern that no partial has until it is written, and its owner puts the
+// pattern back once every reader is known to have passed (two places, by
+// parity of the iteration).
+// Otherwise: work-group r of G takes blocks [r n / G, (r + 1) n / G) and counts
+// itself in at its scenes' counters before each wait.
+//
+// Bound by the latency of an iteration's chain (gather, operator phases, three
+// exchanges of about two memory round trips each).  A substep's solve on two
+// balls of 3.8k particles, 13 iterations: 24 us an iteration with every array
+// in memory and counted waits, about 14 resident; the launched kernels need
+// about 30 and, in a captured substep, the launches of all iterations up to
+// the cap.
+// ============================================================================
+constexpr int CG_DOOR_CLOSED = 1 << 30;
+constexpr long long CG_DOOR_TICKS = 2000;  // of the 100 MHz clock
+
+// The work-group's rank among those inside and their number (at most `most`
+// come), false if the door is closed.
+__device__ inline bool cg_enter(const KP& p, int most, int& rank, int& group) {
+    __shared__ int sh[2];
+    if (threadIdx.x == 0) {
+        const int ticket = add_agent(&p.ctr->door, 1);
+        int g = 0;
+        if (ticket == 0) {
+            const long long t0 = wall_clock64();
+            while (ld_agent(&p.ctr->door) < most && wall_clock64() - t0 < CG_DOOR_TICKS) __builtin_amdgcn_s_sleep(1);
+            g = __hip_atomic_fetch_or(&p.ctr->door, CG_DOOR_CLOSED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            st_agent(&p.ctr->group, g);
+        } else if (ticket < CG_DOOR_CLOSED) {
+            while ((g = ld_agent(&p.ctr->group)) == 0) __builtin_amdgcn_s_sleep(1);
+        }
+        sh[0] = ticket;
+        sh[1] = g;
+    }
+    __syncthreads();
+    rank = sh[0];
+    group = sh[1];
+    return group != 0;
+}
+
+// The same value, not known to be: what is computed from it stays inside the
+// loop instead of holding registers across it.
+__device__ inline int opaque(int v) {
+    __asm__ __volatile__("" : "+v"(v));
+    return v;
+}
+
+// Every store of this wave has reached memory.
+__device__ inline void drain_stores() { __asm__ __volatile__("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory"); }
+
+// ---- a partial that is its own flag -----------------------------------------
+__device__ inline void put_partial(double* a, double v) {
+    if (!(v == v)) v = __longlong_as_double(0x7ff8000000000000ll);
+    st_agent(a, v);
+}
+__device__ inline void clear_partial(double* a) { st_agent(a, __longlong_as_double((long long)CG_EMPTY)); }
+// Waits for the count (<= CG_RESIDENT) partials at sums (and maxs), and sums
+// (takes the largest of) them in a fixed order; one wave, result in every lane.
+__device__ inline void await_partials(const double* sums, const double* maxs, int count, int lane, double& sum, double& mx) {
+    constexpr int U = CG_RESIDENT / 64;
+    double vs[U], vm[U];
+    bool waiting;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        vs[u] = u * 64 + lane < count ? __longlong_as_double((long long)CG_EMPTY) : 0.0;
+        vm[u] = maxs ? vs[u] : 0.0;
+    }
+    do {
+        waiting = false;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (u * 64 >= count) break;
+            if ((unsigned long long)__double_as_longlong(vs[u]) == CG_EMPTY) vs[u] = ld_agent(sums + u * 64 + lane);
+            if (maxs && (unsigned long long)__double_as_longlong(vm[u]) == CG_EMPTY) vm[u] = ld_agent(maxs + u * 64 + lane);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            waiting |= (unsigned long long)__double_as_longlong(vs[u]) == CG_EMPTY ||
+                       (unsigned long long)__double_as_longlong(vm[u]) == CG_EMPTY;
+    } while (__any(waiting));
+    sum = 0.0;
+    mx = 0.0;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        sum += vs[u];
+        mx = fmax(mx, vm[u]);
+    }
+    wave_reduce2(sum, mx);
+}
+
+// Work-group of k_cg_solve: one operator launch of blocks that find the chip
+// empty takes 13.2 us with 256 threads a block (56 blocks), 8.9 with 512, 10.2
+// with 1024 (102 dense blocks: 31.5, 17.0, 14.3); 512 lets two share a CU.
+constexpr int CGW = 512;
+// One block's part of its scene's solve (every thread of the work-group).
+template <int D>
+__device__ inline void cg_solve_resident(const KP& p, int b, OperatorLds<D, CGW>& S) {
+    // by parity of the iteration: in a block without particles no other barrier
+    // keeps wave 0 from writing the next ones before every wave has read these
+    __shared__ float sh_beta[2];
+    __shared__ int sh_done[2];
+    // the node state lives in LDS: registers held across the operator would
+    // spill (x, r, s of the block's nodes and the tile's s)
+    __shared__ float nx[D][64], nr[D][64], ns[D][64], nm[64], ts[D][Dims<D>::TN];
+    const int si = p.block_scene[b];
+    const SceneParams& sc = p.scn[si];
+    if (!sc.active) return;
+    const int b0 = p.sst[si].block_begin, nb = p.sst[si].block_end - b0;
+    const int lane0 = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const bool full = !block_empty(p, b), recorder = b == b0 && threadIdx.x == 0;
+    const float inv_dx = sc.inv_dx;
+    BlockOperator<D, CGW> op(p, S);
+    op.open(b);
+    // wave 0: the block's nodes; tile threads: their node's s
+    bool interior = false, zero = false;
+    int tnbr = -1;
+    if (wv == 0) {
+        const int lane = lane0, n = b * 64 + lane;
+        interior = (p.g_flags[n] & MPM_FLAG_INTERIOR_DEV) != 0;
+        nm[lane] = p.g_m[n];
+        zero = project_zero<D>(p, sc, n);
+        if (lane < Dims<D>::NBR) tnbr = p.block_tnbr[(int64_t)b * Dims<D>::NBR + lane];
+        if (tnbr == b) tnbr = -1;
+#pragma unroll
+        for (int a = 0; a < D; ++a) {
+            nx[a][lane] = p.g_vs[a * p.gcap + n];
+            nr[a][lane] = p.g_r[a * p.gcap + n];
+            ns[a][lane] = 0.0f;
+        }
+    }
+    int* flag = reinterpret_cast<int*>(p.bu);
+    // iteration -1 is the restart: the operator on x, r = b - A x
+    double rho = 0.0;
+    for (int k = -1;; ++k) {
+        const int par = (k & 1) * CG_RESIDENT;
+        const int lane = opaque(lane0), n = b * 64 + lane;
+        op.tid = opaque(op.tid);
+        op.node = opaque(op.node);
+        float u[D];
+#pragma unroll
+        for (int a = 0; a < D; ++a) u[a] = 0.0f;
+        if (k < 0) {
+            if (op.node >= 0) {
+#pragma unroll
+                for (int a = 0; a < D; ++a) {
+                    u[a] = p.g_vs[a * p.gcap + op.node];
+                    ts[a][op.tid] = 0.0f;
+                }
+            }
+        } else {
+            if (wv == 0) {
+                // convergence test and beta on the scene's r.r
+                double rr, mx;
+                await_partials(p.bsum + par + b0, p.bmax + par + b0, nb, lane, rr, mx);
+                // every reader of the s.q partials of iteration k - 1 has passed
+                if (lane == 0) clear_partial(p.bsq + (CG_RESIDENT - par) + b);
+                const CGTestIn in{rho, sc.cg_tol, sc.cg_min, sc.cg_max, false};
+                float beta;
+                const bool done = cg_test(p, si, k, rr, mx, recorder, beta, in);
+                rho = rr;
+                if (lane == 0) {
+                    sh_beta[k & 1] = beta;
+                    sh_done[k & 1] = done ? 1 : 0;
+                }
+            }
+            __syncthreads();
+            if (sh_done[k & 1]) break;
+            // s = r + beta s of the tile's nodes and of the block's
+            const float beta = sh_beta[k & 1];
+            if (op.node >= 0) {
+#pragma unroll
+                for (int a = 0; a < D; ++a) {
+                    u[a] = cg_direction(ld_agent(p.g_r + a * p.gcap + op.node), ts[a][op.tid], beta, k);
+                    ts[a][op.tid] = u[a];
+                }
+            }
+            if (interior) {
+#pragma unroll
+                for (int a = 0; a < D; ++a) ns[a][lane] = cg_direction(nr[a][lane], ns[a][lane], beta, k);
+            }
+        }
+        if (full) {
+            op.apply(inv_dx, u, k >= 0);
+            op.template store<true>();
+            drain_stores();
+            __syncthreads();
+            if (threadIdx.x == 0) st_agent(flag + b, k + 2);
+            op.load_records(op.p0);  // for the next time
+        }
+        if (wv != 0) continue;
+        // the neighbours' tiles, and this block's nodes
+        while (__any(tnbr >= 0 && ld_agent(flag + max(tnbr, 0)) < k + 2)) __builtin_amdgcn_s_sleep(1);
+        __asm__ __volatile__("" ::: "memory");
+        float q[D], r[D];
+        gather_node_tiles<D, D, true>(p, sc, n, q);
+        const double m = (double)nm[lane];
+        const float cm = sc.dt * sc.dt / nm[lane];
+        double sum = 0.0, mx = 0.0;
+        if (k < 0) {
+#pragma unroll
+            for (int a = 0; a < D; ++a) {
+                r[a] = nr[a][lane];
+                if (interior) {
+                    q[a] = cm * q[a] + nx[a][lane];
+                    r[a] = r[a] - q[a];
+                }
+                if (zero) r[a] = 0.0f;
+            }
+        } else {
+            float s[D];
+#pragma unroll
+            for (int a = 0; a < D; ++a) {
+                s[a] = ns[a][lane];
+                if (interior) q[a] = cm * q[a] + s[a];
+                if (zero) q[a] = 0.0f;
+                if (interior) sum += (double)s[a] * ((double)q[a] * m);
+            }
+            double sq;
+            wave_reduce2(sum, mx);
+            if (lane == 0) put_partial(p.bsq + par + b, sum);
+            await_partials(p.bsq + par + b0, nullptr, nb, lane, sq, mx);
+            // every reader of this iteration's r.r partials has passed
+            if (lane == 0) {
+                clear_partial(p.bsum + par + b);
+                clear_partial(p.bmax + par + b);
+            }
+            const double alpha_d = sq != 0.0 ? rho / sq : (double)FLT_MAX;
+            if (recorder) {
+                CGState& cg = p.cg[si];
+                cg.sq = sq;
+                cg.alpha = alpha_d;
+                cg.multiplies += 1;
+            }
+            const float alpha = (float)alpha_d;
+#pragma unroll
+            for (int a = 0; a < D; ++a) {
+                r[a] = nr[a][lane];
+                if (interior) {
+                    nx[a][lane] = alpha * s[a] + nx[a][lane];
+                    r[a] = -alpha * q[a] + r[a];
+                }
+            }
+        }
+        // r and its partials
+        sum = 0.0;
+        mx = 0.0;
+#pragma unroll
+        for (int a = 0; a < D; ++a) {
+            if (interior) {
+                sum += (double)r[a] * ((double)r[a] * m);
+                mx += (double)r[a] * (double)r[a];
+            }
+            nr[a][lane] = r[a];
+            st_agent(p.g_r + a * p.gcap + n, r[a]);
+            p.g_q[a * p.gcap + n] = q[a];
+        }
+        wave_reduce2(sum, mx);
+        drain_stores();
+        if (lane == 0) {
+            put_partial(p.bsum + (CG_RESIDENT - par) + b, sum);
+            put_partial(p.bmax + (CG_RESIDENT - par) + b, mx);
+        }
+    }
+    if (wv == 0) {
+        const int lane = lane0, n = b * 64 + lane;
+#pragma unroll
+        for (int a = 0; a < D; ++a) {
+            p.g_vs[a * p.gcap + n] = nx[a][lane];
+            p.g_s[a * p.gcap + n] = ns[a][lane];
+        }
+    }
+}
+
+// ---- fewer work-groups than blocks -------------------------------------------
+// The work-group that owns block b of n when g (<= n) share them.
+__device__ inline int cg_owner(int b, int n, int g) { return (int)((((int64_t)b + 1) * g - 1) / n); }
+
+// A run is the part of one scene's blocks that a work-group owns.  f(si, e,
+// r, b): run r of scene si is blocks [b, e).
+template <class F>
+__device__ inline void for_runs(const KP& p, int w0, int w1, F&& f) {
+    int r = 0;
+    for (int b = w0; b < w1; ++r) {
+        const int si = p.block_scene[b], e = min(w1, p.sst[si].block_end);
+        f(si, e, r, b);
+        b = e;
+    }
+}
+
+// Waits until every work-group that owns blocks of the scenes still running
+// here (runs not in `done`) has come; `phase` counts the waits from 1.
+__device__ inline void cg_wait(const KP& p, int w0, int w1, int n, int g, unsigned long long done, int phase) {
+    drain_stores();  // before the work-group is counted
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for_runs(p, w0, w1, [&](int si, int, int r, int) {
+            if (!((done >> r) & 1)) add_agent(&p.cg[si].arrived, 1);
+        });
+        for_runs(p, w0, w1, [&](int si, int, int r, int) {
+            if ((done >> r) & 1) return;
+            const int b0 = p.sst[si].block_begin, b1 = p.sst[si].block_end;
+            const int target = (cg_owner(b1 - 1, n, g) - cg_owner(b0, n, g) + 1) * phase;
+            while (ld_agent(&p.cg[si].arrived) < target) __builtin_amdgcn_s_sleep(1);
+        });
+    }
+    __syncthreads();
+    __asm__ __volatile__("" ::: "memory");
+}
+
+static_assert(CG_SOLVE_MAX_SCENES <= 64, "a work-group holds at most that many runs, a bit each");
+// Blocks [w0, w1) of n, work-groups g.
+template <int D>
+__device__ inline void cg_solve_shared(const KP& p, int w0, int w1, int n, int g, OperatorLds<D, CGW>& S) {
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    unsigned long long done = 0, all = 0;
+    for_runs(p, w0, w1, [&](int si, int, int r, int) {
+        all |= 1ull << r;
+        if (!p.scn[si].active) done |= 1ull << r;
+    });
+    if (done == all) return;
+    int phase = 0;
+    for (int k = -1;; ++k) {
+        // convergence test and beta of every scene, then its operator
+        // (iteration -1: the restart, the operator on x, r = b - A x)
+        for_runs(p, w0, w1, [&](int si, int e, int r, int b) {
+            if ((done >> r) & 1) return;
+            float beta = 0.0f;
+            if (k >= 0) {
+                const int b0 = p.sst[si].block_begin, b1 = p.sst[si].block_end;
+                const CGTestIn in = cg_test_in(p, si, k);
+                double rr, mx;
+                reduce_range<true, CGW>(p.bsum, p.bmax, b0, b1 - b0, rr, mx);
+                if (cg_test(p, si, k, rr, mx, b == b0 && threadIdx.x == 0, beta, in)) {
+                    done |= 1ull << r;
+                    return;
+                }
+            }
+            for (; b < e; ++b)
+                if (!block_empty(p, b))
+                    operator_block<D, CGW, true>(p, b, p.scn[si].inv_dx, S, [&](int a, int64_t nd) {
+                        return k < 0 ? p.g_vs[a * p.gcap + nd]
+                                     : cg_direction(ld_agent(p.g_r + a * p.gcap + nd), ld_agent(p.g_s + a * p.gcap + nd), beta, k);
+                    });
+        });
+        if (k < 0) {
+            cg_wait(p, w0, w1, n, g, done, ++phase);
+            for_runs(p, w0, w1, [&](int si, int e, int r, int b) {
+                if ((done >> r) & 1) return;
+                for (b += wv; b < e; b += CGW / 64) {
+                    double sum, mx;
+                    cg_restart_block<D, true>(p, p.scn[si], b, lane, sum, mx);
+                    if (lane == 0) {
+                        st_agent(p.bsum + b, sum);
+                        st_agent(p.bmax + b, mx);
+                    }
+                }
+            });
+            cg_wait(p, w0, w1, n, g, done, ++phase);
+            continue;
+        }
+        if (done == all) return;
+        cg_wait(p, w0, w1, n, g, done, ++phase);
+        // q = A s and s itself, s.q
+        for_runs(p, w0, w1, [&](int si, int e, int r, int b) {
+            if ((done >> r) & 1) return;
+            const float beta = (float)ld_agent(&p.cg[si].beta);
+            for (b += wv; b < e; b += CGW / 64) {
+                double sum;
+                cg_node1_block<D, false, true>(p, p.scn[si], b, lane, beta, k, sum);
+                if (lane == 0) st_agent(p.bsq + b, sum);
+            }
+        });
+        cg_wait(p, w0, w1, n, g, done, ++phase);
+        // alpha, x and r, r.r
+        for_runs(p, w0, w1, [&](int si, int e, int r, int b) {
+            if ((done >> r) & 1) return;
+            const int b0 = p.sst[si].block_begin, b1 = p.sst[si].block_end;
+            const double rho = ld_agent(&p.cg[si].rho_hist[k & 1]);
+            double sq, unused;
+            reduce_range<true, CGW>(p.bsq, nullptr, b0, b1 - b0, sq, unused);
+            const double alpha = sq != 0.0 ? rho / sq : (double)FLT_MAX;
+            if (b == b0 && threadIdx.x == 0) {
+                CGState& cg = p.cg[si];
+                cg.sq = sq;
+                cg.alpha = alpha;
+                cg.multiplies += 1;
+            }
+            for (b += wv; b < e; b += CGW / 64) {
+                double sum, mx;
+                cg_node2_block<D, true>(p, b, lane, (float)alpha, sum, mx);
+                if (lane == 0) {
+                    st_agent(p.bsum + b, sum);
+                    st_agent(p.bmax + b, mx);
+                }
+            }
+        });
+        cg_wait(p, w0, w1, n, g, done, ++phase);
+    }
+}
+
+template <int D>
+__global__ __launch_bounds__(CGW, 4) void k_cg_solve(KP p) {
+    __shared__ __align__(16) OperatorLds<D, CGW> S;
+    const int n = p.ctr->nblocks, most = min(n, (int)gridDim.x);
+    if ((int)blockIdx.x == 0) {
+        // scenes without blocks or at rest are done at once
+        for (int si = threadIdx.x; si < p.nscenes; si += CGW) {
+            const CGTestIn in = cg_test_in(p, si, 0);
+            float beta;
+            if (in.empty) (void)cg_test(p, si, 0, 0.0, 0.0, true, beta, in);
+        }
+    }
+    if ((int)blockIdx.x >= most) return;
+    int rank, group;
+    if (!cg_enter(p, most, rank, group)) return;
+    if (group == n && n <= CG_RESIDENT) {
+        cg_solve_resident<D>(p, (int)blockIdx.x, S);
+    } else {
+        const int w0 = (int)((int64_t)rank * n / group), w1 = (int)((int64_t)(rank + 1) * n / group);
+        cg_solve_shared<D>(p, w0, w1, n, group, S);
+    }
 }
 
 // ============================================================================
@@ -2851,6 +3425,9 @@ template <int D> void launch_cg_force(const KP& p, hipStream_t s, int grid, bool
     else if (one) hipLaunchKernelGGL((k_cg_force<D, false, true>), dim3(grid), dim3(BWG), 0, s, p, k);
     else hipLaunchKernelGGL((k_cg_force<D, false, false>), dim3(grid), dim3(BWG), 0, s, p, k);
 }
+template <int D> void launch_cg_solve(const KP& p, hipStream_t s, int grid) {
+    hipLaunchKernelGGL(k_cg_solve<D>, dim3(grid), dim3(CGW), 0, s, p);
+}
 template <int D> void launch_cg_restart_node(const KP& p, hipStream_t s, int grid, bool one) {
     if (one) hipLaunchKernelGGL((k_cg_restart_node<D, true>), dim3(grid), dim3(WG), 0, s, p);
     else hipLaunchKernelGGL((k_cg_restart_node<D, false>), dim3(grid), dim3(WG), 0, s, p);
@@ -2884,6 +3461,7 @@ template <int D> void launch_max_speed(const KP& p, hipStream_t s, int grid) { h
     template void launch_particle_force<D>(const KP&, hipStream_t, int, bool, bool);          \
     template void launch_grid_update<D>(const KP&, hipStream_t, int, bool, bool, bool, bool); \
     template void launch_cg_force<D>(const KP&, hipStream_t, int, bool, int, bool);           \
+    template void launch_cg_solve<D>(const KP&, hipStream_t, int);                            \
     template void launch_cg_restart_node<D>(const KP&, hipStream_t, int, bool);               \
     template void launch_cg_update_s<D>(const KP&, hipStream_t, int, int);                    \
     template void launch_cg_node1<D>(const KP&, hipStream_t, int, int, bool);                 \

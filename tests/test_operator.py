@@ -53,3 +53,42 @@ def test_cell_and_chunk_edges(dim, n):
     assert np.array_equal(got["ids"], want["ids"])
     for k in ("x", "v", "F", "Jp"):
         assert rel(got[k], want[k]) < 1e-5, k
+
+
+@pytest.mark.parametrize("graph", [False, True])
+@pytest.mark.parametrize("scenes", [1, 3])
+def test_solve_with_more_blocks_than_work_groups(scenes, graph):
+    """Scattered particles: over a thousand active blocks for a few thousand
+    particles, so a work-group of the one-launch solve takes several blocks
+    (and, in a batch, blocks of two scenes)."""
+    counts, n = 64, 700
+    descs, parts = [], []
+    for k in range(scenes):
+        r = np.random.default_rng(7 + k)
+        d, _, _, _ = M.scene_generate("two_balls", counts, 0)
+        d.cg_max_iterations = 200
+        x = r.uniform(0.15, 0.85, (n, 3)).astype(np.float32)
+        x = np.concatenate([x, x + r.uniform(-0.5, 0.5, x.shape).astype(np.float32) / counts]).astype(np.float32)
+        v = ((x - 0.5) @ r.uniform(-1.0, 1.0, (3, 3)) + 0.5).astype(np.float32)
+        descs.append(d)
+        parts.append((x, v, np.full(len(x), 400.0 / counts ** 3 / 8, np.float32)))
+    dt = 0.5 * float(descs[0].max_dt)
+    b = M.Batch(descs, [2 * n] * scenes)
+    for k, (x, v, m) in enumerate(parts):
+        b.upload(k, x, v, m)
+    b.initialize()
+    b.use_graph(graph)
+    for _ in range(2):
+        b.substep(dt)
+    assert sum(b.stats(k)["active_blocks"] for k in range(scenes)) > 1000
+    for k, (x, v, m) in enumerate(parts):
+        o = O.Oracle(descs[k], 8, 4, O.DOT_FP64 | O.SVD_FP64)
+        o.set_particles(x, v, m)
+        o.initialize()
+        for _ in range(2):
+            o.advance_step(dt)
+        got, want = b.download(k), o.particles()
+        assert np.array_equal(got["ids"], want["ids"])
+        for f in ("x", "v", "F", "Jp"):
+            assert rel(got[f], want[f]) < 1e-5, (k, f)
+    b.close()
