@@ -915,6 +915,63 @@ int upload_max_speed(mpm_context* c) {
     return check_launch("max speed");
 }
 
+// The live particles of scene s by id, ordered and transposed on the device in
+// the buffers that only a binning uses: the idle particle copy takes the
+// particle-major arrays, the binning's scratch the ids' index.  false: the
+// scene's ids outgrew that scratch (they are not reused, so particles added to
+// a scene that keeps losing others can pass the capacity).
+bool pack_fits(const mpm_context* c, int64_t nid) {
+    return nid > 0 && nid <= c->pcap && mpm::pack_tiles(nid) + 1 <= c->pcap;
+}
+int download_packed(mpm_context* c, int s, int64_t b0, int64_t b1, int64_t cap, float* x, float* v, float* F, float* Jp,
+                    float* mass, float* volume, int32_t* ids, int64_t* n_out, int32_t* material) {
+    const mpm::KP p = make_kp(c);
+    const int D = c->D;
+    mpm::PackArgs a{};
+    a.scene = s;
+    a.first = b0;
+    a.last = b1;
+    a.nid = c->sc[(size_t)s].n_uploaded;
+    a.inv = c->cell_order;
+    a.part = c->prank;
+    mpm::launch_pack_count(p, c->stream, a);
+    int live = 0;
+    HIPCHECK(hipStreamSynchronize(c->stream));
+    HIPCHECK(hipMemcpy(&live, a.part + mpm::pack_tiles(a.nid), sizeof(int), hipMemcpyDeviceToHost));
+    if (n_out) *n_out = live;
+    if (live > cap) return mpm_set_error(MPM_E_CAPACITY, "mpm_download_particles: cap too small");
+    if (live == 0) return MPM_OK;
+    float* out = p.palt;
+    const auto take = [&](const void* wanted, int64_t words) {
+        float* at = wanted ? out : nullptr;
+        out += words * live;
+        return at;
+    };
+    a.x = take(x, D);
+    a.v = take(v, D);
+    a.F = take(F, D * D);
+    a.Jp = take(Jp, 1);
+    a.mass = take(mass, 1);
+    a.volume = take(volume, 1);
+    a.material = reinterpret_cast<int*>(take(material, 1));
+    a.ids = ids ? p.idalt : nullptr;
+    if (D == 3) mpm::launch_pack_write<3>(p, c->stream, a);
+    else mpm::launch_pack_write<2>(p, c->stream, a);
+    HIPCHECK(hipStreamSynchronize(c->stream));
+    const auto get = [&](void* dst, const void* src, int64_t words) {
+        return dst ? hipMemcpy(dst, src, (size_t)(words * live) * 4, hipMemcpyDeviceToHost) : hipSuccess;
+    };
+    HIPCHECK(get(x, a.x, D));
+    HIPCHECK(get(v, a.v, D));
+    HIPCHECK(get(F, a.F, D * D));
+    HIPCHECK(get(Jp, a.Jp, 1));
+    HIPCHECK(get(mass, a.mass, 1));
+    HIPCHECK(get(volume, a.volume, 1));
+    HIPCHECK(get(material, a.material, 1));
+    HIPCHECK(get(ids, a.ids, 1));
+    return check_launch("download");
+}
+
 int download_scene(mpm_context* c, int s, int64_t cap, float* x, float* v, float* F, float* Jp, float* mass,
                    float* volume, int32_t* ids, int64_t* n_out, int32_t* material = nullptr) {
     mpm::Counters hc{};
@@ -934,6 +991,8 @@ int download_scene(mpm_context* c, int s, int64_t cap, float* x, float* v, float
         b0 = c->sc[(size_t)s].pbase;
         b1 = b0 + c->sc[(size_t)s].capacity;
     }
+    if (pack_fits(c, c->sc[(size_t)s].n_uploaded))
+        return download_packed(c, s, b0, std::max(b0, b1), cap, x, v, F, Jp, mass, volume, ids, n_out, material);
     const int D = c->D, NF = nfields(D);
     const int64_t n = std::max<int64_t>(b1 - b0, 0);
     std::vector<float> h((size_t)NF * (size_t)std::max<int64_t>(n, 1));

@@ -180,6 +180,18 @@ struct NoallocOut {
     int* valid;  // 1: binned and inside the domain after G2P; 0: removed
 };
 
+// Download of one scene: the index and number of every id, and where the
+// particle-major arrays go (device memory; null: not wanted).
+struct PackArgs {
+    int scene;
+    int64_t first, last;  // its particles in the current buffer lie in [first, last)
+    int64_t nid;          // ids are below this
+    int* inv;             // nid entries
+    int* part;            // a count per tile of ids, and their total
+    float *x, *v, *F, *Jp, *mass, *volume;
+    int *ids, *material;
+};
+
 // launchers (host)
 void launch_set_step(const KP& p, hipStream_t s, const StepArgs& a);
 void launch_set_step_dev(const KP& p, hipStream_t s, const float* dt);
@@ -194,6 +206,9 @@ template <int D> void launch_block_setup(const KP& p, hipStream_t s, int grid);
 // block order, scene ranges and the in-cell order scatter (cell_groups work-groups)
 void launch_setup_order(const KP& p, hipStream_t s, int cell_groups);
 void launch_poll(const KP& p, hipStream_t s, int* dst);
+int pack_tiles(int64_t nid);
+void launch_pack_count(const KP& p, hipStream_t s, const PackArgs& a);  // fills inv and part
+template <int D> void launch_pack_write(const KP& p, hipStream_t s, const PackArgs& a);
 template <int D> void launch_reorder(const KP& p, hipStream_t s, int grid);
 template <int D> void launch_p2g(const KP& p, hipStream_t s, int grid);
 template <int D> void launch_normalize(const KP& p, hipStream_t s, int grid);

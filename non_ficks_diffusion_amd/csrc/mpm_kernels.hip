@@ -25,6 +25,7 @@
 // and a one-work-group-per-scene kernel sums a scene's block partials in a
 // fixed order.
 #include "mpm_kernels.h"
+#include <algorithm>
 
 namespace mpm {
 
@@ -3193,6 +3194,90 @@ __global__ __launch_bounds__(WG) void k_max_speed(KP p) {
     }
 }
 
+// ============================================================================
+// Download: the live particles of one scene by id, particle-major as the
+// caller's arrays are.  Every id finds its particle (k_pack_mark), the ids that
+// found one are numbered by a scan over tiles of PACK_TILE ids (k_pack_count,
+// k_pack_top), and each particle is written at its number (k_pack_write).
+// Bound by the copy to the host, then by the gathers of k_pack_write, whose
+// particles are in cell order (most of its loads take a line each).  A download
+// of 1.0M particles, host copy included: 180 -> 7.3 ms, 2M: 370 -> 18, 20k: 1.3
+// -> 0.25, against copying the fields and sorting and transposing on the host.
+// ============================================================================
+constexpr int PACK_PER_THREAD = 4, PACK_TILE = WG * PACK_PER_THREAD;
+__global__ __launch_bounds__(WG) void k_pack_clear(PackArgs a) {
+    for (int64_t i = (int64_t)blockIdx.x * WG + threadIdx.x; i < a.nid; i += (int64_t)gridDim.x * WG) a.inv[i] = -1;
+}
+__global__ __launch_bounds__(WG) void k_pack_mark(KP p, PackArgs a) {
+    for (int64_t i = a.first + (int64_t)blockIdx.x * WG + threadIdx.x; i < a.last; i += (int64_t)gridDim.x * WG) {
+        const int id = p.idcur[i];
+        if (p.keycur[i] >= 0 && p.scur[i] == a.scene && id >= 0 && id < a.nid) a.inv[id] = (int)i;
+    }
+}
+__global__ __launch_bounds__(WG) void k_pack_count(PackArgs a) {
+    const int64_t base = (int64_t)blockIdx.x * PACK_TILE + threadIdx.x * PACK_PER_THREAD;
+    int c = 0;
+#pragma unroll
+    for (int k = 0; k < PACK_PER_THREAD; ++k) c += base + k < a.nid && a.inv[base + k] >= 0 ? 1 : 0;
+    int total;
+    wg_exclusive_scan(c, total);
+    if (threadIdx.x == 0) a.part[blockIdx.x] = total;
+}
+// one work-group: exclusive scan of the tiles' counts, their total behind them
+__global__ __launch_bounds__(WG) void k_pack_top(PackArgs a, int tiles) {
+    const int per = (tiles + WG - 1) / WG;
+    const int64_t t0 = (int64_t)threadIdx.x * per;
+    int sum = 0;
+    for (int k = 0; k < per; ++k)
+        if (t0 + k < tiles) sum += a.part[t0 + k];
+    int total;
+    int run = wg_exclusive_scan(sum, total);
+    for (int k = 0; k < per; ++k)
+        if (t0 + k < tiles) {
+            const int c = a.part[t0 + k];
+            a.part[t0 + k] = run;
+            run += c;
+        }
+    if (threadIdx.x == 0) a.part[tiles] = total;
+}
+template <int D>
+__global__ __launch_bounds__(WG) void k_pack_write(KP p, PackArgs a) {
+    const int64_t base = (int64_t)blockIdx.x * PACK_TILE + threadIdx.x * PACK_PER_THREAD;
+    int from[PACK_PER_THREAD], c = 0;
+#pragma unroll
+    for (int k = 0; k < PACK_PER_THREAD; ++k) {
+        from[k] = base + k < a.nid ? a.inv[base + k] : -1;
+        c += from[k] >= 0 ? 1 : 0;
+    }
+    int total;
+    int64_t to = wg_exclusive_scan(c, total) + a.part[blockIdx.x];
+#pragma unroll
+    for (int k = 0; k < PACK_PER_THREAD; ++k) {
+        if (from[k] < 0) continue;
+        float f[PF<D>::N];
+#pragma unroll
+        for (int q = 0; q < PF<D>::N; ++q) f[q] = p.pcur[q * p.pcap + from[k]];
+        if (a.x) {
+#pragma unroll
+            for (int q = 0; q < D; ++q) a.x[to * D + q] = f[PF<D>::X + q];
+        }
+        if (a.v) {
+#pragma unroll
+            for (int q = 0; q < D; ++q) a.v[to * D + q] = f[PF<D>::V + q];
+        }
+        if (a.F) {
+#pragma unroll
+            for (int q = 0; q < D * D; ++q) a.F[to * D * D + q] = f[PF<D>::F + q];
+        }
+        if (a.Jp) a.Jp[to] = f[PF<D>::J];
+        if (a.mass) a.mass[to] = f[PF<D>::M];
+        if (a.volume) a.volume[to] = f[PF<D>::VOL];
+        if (a.material) a.material[to] = __float_as_int(f[PF<D>::MAT]);
+        if (a.ids) a.ids[to] = (int)(base + k);
+        ++to;
+    }
+}
+
 // dt and activity of scenes [first, first + n) for the next substep
 __global__ __launch_bounds__(WG) void k_set_step(KP p, StepArgs a) {
     const int i = blockIdx.x * WG + threadIdx.x;
@@ -3402,6 +3487,20 @@ void launch_setup_order(const KP& p, hipStream_t s, int cell_groups) {
     const int grid = ORDER_GROUPS + (p.nscenes + WG - 1) / WG + cell_groups;
     hipLaunchKernelGGL(k_setup_order, dim3(grid), dim3(WG), 0, s, p);
 }
+int pack_tiles(int64_t nid) { return (int)((nid + PACK_TILE - 1) / PACK_TILE); }
+void launch_pack_count(const KP& p, hipStream_t s, const PackArgs& a) {
+    const auto groups = [](int64_t n) { return dim3((unsigned)std::min<int64_t>(std::max<int64_t>((n + WG - 1) / WG, 1), 8192)); };
+    const int tiles = pack_tiles(a.nid);
+    hipLaunchKernelGGL(k_pack_clear, groups(a.nid), dim3(WG), 0, s, a);
+    hipLaunchKernelGGL(k_pack_mark, groups(a.last - a.first), dim3(WG), 0, s, p, a);
+    hipLaunchKernelGGL(k_pack_count, dim3(tiles), dim3(WG), 0, s, a);
+    hipLaunchKernelGGL(k_pack_top, dim3(1), dim3(WG), 0, s, a, tiles);
+}
+template <int D> void launch_pack_write(const KP& p, hipStream_t s, const PackArgs& a) {
+    hipLaunchKernelGGL(k_pack_write<D>, dim3(pack_tiles(a.nid)), dim3(WG), 0, s, p, a);
+}
+template void launch_pack_write<2>(const KP&, hipStream_t, const PackArgs&);
+template void launch_pack_write<3>(const KP&, hipStream_t, const PackArgs&);
 void launch_poll(const KP& p, hipStream_t s, int* dst) { hipLaunchKernelGGL(k_poll, dim3(1), dim3(64), 0, s, p, dst); }
 template <int D> void launch_reorder(const KP& p, hipStream_t s, int grid) { hipLaunchKernelGGL(k_reorder<D>, dim3(grid), dim3(WG), 0, s, p); }
 template <int D> void launch_p2g(const KP& p, hipStream_t s, int grid) { hipLaunchKernelGGL(k_p2g<D>, dim3(grid), dim3(BWG), 0, s, p); }
