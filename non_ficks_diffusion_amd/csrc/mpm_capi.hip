@@ -274,12 +274,12 @@ static_assert(offsetof(mpm::Counters, nblocks) == 0 && offsetof(mpm::Counters, o
 
 // The solve in one launch (k_cg_solve) for handles of up to this many
 // particles (at eight a cell about 130 blocks that hold some, 350 with their
-// halo).  Measured per frame of 60 fps: 3.8k particles in 32^3 13.3 -> 7.8 ms
-// (captured), 20k in 64^3 (fluid) 5.7 -> 5.4; above, work-groups take more than
-// one block each and the launched kernels win: four requests of 200k particles
-// together 150 -> 219 ms, two balls of 243k 91 -> 153.  The rule reads only what the
-// caller uploaded, so launched, replayed and repeated substeps take the same
-// kernels.
+// halo).  Measured per frame of 60 fps: 3.8k particles in 32^3 13.3 -> 7.7 ms
+// (captured), twelve scenes of 48k together 26 -> 19; above, more blocks of
+// particles meet in a work-group and the launched kernels win: two balls of
+// 243k 73 -> 104 ms, a dense slab of 333k 45 -> 81, four requests of 200k
+// together 139 either way.  The rule reads only what the caller uploaded, so
+// launched, replayed and repeated substeps take the same kernels.
 constexpr int64_t CG_SOLVE_MAX_PARTICLES = 65536;
 bool cg_in_one_launch(const mpm_context* c) {
     int64_t n = 0;
@@ -312,7 +312,7 @@ int stage_cg(mpm_context* c, bool do_init, bool fixed = false) {
     if (do_init)
         timed(c, KC_GRID, [&] { mpm::launch_grid_update<D>(p, c->stream, gn, false, false, true, false); });
     if (cg_in_one_launch(c)) {
-        timed(c, KC_CG_FORCE, [&] { mpm::launch_cg_solve<D>(p, c->stream, mpm::CG_RESIDENT); });
+        timed(c, KC_CG_FORCE, [&] { mpm::launch_cg_solve<D>(p, c->stream); });
         if (!fixed) {
             // read once the rest of the substep is queued (the overflow flag)
             mpm::launch_poll(p, c->stream, c->d_done);

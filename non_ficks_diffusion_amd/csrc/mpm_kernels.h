@@ -220,8 +220,9 @@ template <int D> void launch_cg_force(const KP& p, hipStream_t s, int grid, bool
 // the whole solve in one launch (scenes too small to fill the chip; at most
 // CG_SOLVE_MAX_SCENES of them)
 constexpr int CG_SOLVE_MAX_SCENES = 64;
-constexpr int CG_RESIDENT = 512;  // blocks up to which each has a work-group of its own
-template <int D> void launch_cg_solve(const KP& p, hipStream_t s, int grid);
+constexpr int CG_GROUPS = 512;     // its work-groups (two fit a CU)
+constexpr int CG_RESIDENT = 2 * CG_GROUPS;  // blocks up to which their state stays in the work-groups
+template <int D> void launch_cg_solve(const KP& p, hipStream_t s);
 template <int D> void launch_cg_restart_node(const KP& p, hipStream_t s, int grid, bool one);
 template <int D> void launch_cg_update_s(const KP& p, hipStream_t s, int grid, int k);
 template <int D> void launch_cg_node1(const KP& p, hipStream_t s, int grid, int k, bool one);

@@ -2514,10 +2514,10 @@ __global__ __launch_bounds__(WG) void k_cg_reduce_rr(KP p, int k) {
 // the kernel ends.  The results do not depend on how many they are.  What
 // work-groups exchange goes through device-scope accesses.
 //
-// All inside (the usual case, at most CG_RESIDENT blocks): one block each,
-// its nodes' m, x, r and s in the registers of wave 0 and its tile's s in those
-// of the tile threads (a halo node's s = r + beta s follows from r alone, so
-// only r and the force tiles travel).  An iteration waits three times: for the
+// All inside (the usual case, at most CG_RESIDENT blocks): one block each, or
+// two, their nodes' m, x, r and s and their tiles' s in LDS for the whole solve
+// (a halo node's s = r + beta s follows from r alone, so only r and the force
+// tiles travel).  An iteration waits three times: for the
 // neighbours' force tiles (a flag per block), for the scene's partials of s.q
 // and for those of r.r.  A partial is its own flag: its place holds a bit
 // pattern that no partial has until it is written, and its owner puts the
@@ -2576,10 +2576,11 @@ __device__ inline void put_partial(double* a, double v) {
     st_agent(a, v);
 }
 __device__ inline void clear_partial(double* a) { st_agent(a, __longlong_as_double((long long)CG_EMPTY)); }
-// Waits for the count (<= CG_RESIDENT) partials at sums (and maxs), and sums
-// (takes the largest of) them in a fixed order; one wave, result in every lane.
+// Waits for the count (<= MOST) partials at sums (and maxs), and sums (takes
+// the largest of) them in a fixed order; one wave, result in every lane.
+template <int MOST>
 __device__ inline void await_partials(const double* sums, const double* maxs, int count, int lane, double& sum, double& mx) {
-    constexpr int U = CG_RESIDENT / 64;
+    constexpr int U = MOST / 64;
     double vs[U], vm[U];
     bool waiting;
 #pragma unroll
@@ -2614,40 +2615,57 @@ __device__ inline void await_partials(const double* sums, const double* maxs, in
 // empty takes 13.2 us with 256 threads a block (56 blocks), 8.9 with 512, 10.2
 // with 1024 (102 dense blocks: 31.5, 17.0, 14.3); 512 lets two share a CU.
 constexpr int CGW = 512;
-// One block's part of its scene's solve (every thread of the work-group).
-template <int D>
-__device__ inline void cg_solve_resident(const KP& p, int b, OperatorLds<D, CGW>& S) {
+// K blocks' part of their scenes' solves (every thread of the work-group);
+// a negative one is none.
+template <int D, int K>
+__device__ inline void cg_solve_resident(const KP& p, int blk0, int blk1, OperatorLds<D, CGW>& S) {
+    constexpr int TN = Dims<D>::TN, NBR = Dims<D>::NBR, MOST = K * CG_GROUPS;
     // by parity of the iteration: in a block without particles no other barrier
-    // keeps wave 0 from writing the next ones before every wave has read these
-    __shared__ float sh_beta[2];
-    __shared__ int sh_done[2];
+    // keeps wave j from writing the next ones before every wave has read these
+    __shared__ float sh_beta[2][K];
+    __shared__ int sh_done[2][K];
     // the node state lives in LDS: registers held across the operator would
-    // spill (x, r, s of the block's nodes and the tile's s)
-    __shared__ float nx[D][64], nr[D][64], ns[D][64], nm[64], ts[D][Dims<D>::TN];
-    const int si = p.block_scene[b];
-    const SceneParams& sc = p.scn[si];
-    if (!sc.active) return;
-    const int b0 = p.sst[si].block_begin, nb = p.sst[si].block_end - b0;
-    const int lane0 = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const bool full = !block_empty(p, b), recorder = b == b0 && threadIdx.x == 0;
-    const float inv_dx = sc.inv_dx;
+    // spill (x, r, s of the blocks' nodes and the tiles' s)
+    __shared__ float nx[K][D][64], nr[K][D][64], ns[K][D][64], nm[K][64], ts[K][D][TN];
+    // the wave's number as a scalar: its block's and scene's data stay scalar
+    const int lane0 = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     BlockOperator<D, CGW> op(p, S);
-    op.open(b);
-    // wave 0: the block's nodes; tile threads: their node's s
+    // wave j: the nodes of block j; tile threads: their node's s in every tile.
+    // full, done: a bit per block.
     bool interior = false, zero = false;
-    int tnbr = -1;
-    if (wv == 0) {
+    int tnbr = -1, b = -1, si = 0, b0 = 0, nb = 0;
+    unsigned full = 0, done = 0;
+    for (int j = 0; j < K; ++j) {
+        const int bj = j == 0 ? blk0 : blk1;
+        const int sj = bj >= 0 ? p.block_scene[bj] : 0;
+        if (bj < 0 || !p.scn[sj].active) {
+            done |= 1u << j;
+            continue;
+        }
+        if (!block_empty(p, bj)) full |= 1u << j;
+        if (wv == j) {
+            b = bj;
+            si = sj;
+        }
+    }
+    constexpr unsigned ALL = (1u << K) - 1u;
+    if (done == ALL) return;
+    if (K == 1 && full) op.open(blk0);
+    const SceneParams& sc = p.scn[si];
+    if (b >= 0) {
         const int lane = lane0, n = b * 64 + lane;
+        b0 = p.sst[si].block_begin;
+        nb = p.sst[si].block_end - b0;
         interior = (p.g_flags[n] & MPM_FLAG_INTERIOR_DEV) != 0;
-        nm[lane] = p.g_m[n];
+        nm[wv][lane] = p.g_m[n];
         zero = project_zero<D>(p, sc, n);
-        if (lane < Dims<D>::NBR) tnbr = p.block_tnbr[(int64_t)b * Dims<D>::NBR + lane];
+        if (lane < NBR) tnbr = p.block_tnbr[(int64_t)b * NBR + lane];
         if (tnbr == b) tnbr = -1;
 #pragma unroll
         for (int a = 0; a < D; ++a) {
-            nx[a][lane] = p.g_vs[a * p.gcap + n];
-            nr[a][lane] = p.g_r[a * p.gcap + n];
-            ns[a][lane] = 0.0f;
+            nx[wv][a][lane] = p.g_vs[a * p.gcap + n];
+            nr[wv][a][lane] = p.g_r[a * p.gcap + n];
+            ns[wv][a][lane] = 0.0f;
         }
     }
     int* flag = reinterpret_cast<int*>(p.bu);
@@ -2657,97 +2675,100 @@ __device__ inline void cg_solve_resident(const KP& p, int b, OperatorLds<D, CGW>
         const int par = (k & 1) * CG_RESIDENT;
         const int lane = opaque(lane0), n = b * 64 + lane;
         op.tid = opaque(op.tid);
-        op.node = opaque(op.node);
-        float u[D];
-#pragma unroll
-        for (int a = 0; a < D; ++a) u[a] = 0.0f;
-        if (k < 0) {
-            if (op.node >= 0) {
-#pragma unroll
-                for (int a = 0; a < D; ++a) {
-                    u[a] = p.g_vs[a * p.gcap + op.node];
-                    ts[a][op.tid] = 0.0f;
-                }
-            }
-        } else {
-            if (wv == 0) {
+        if (k >= 0) {
+            if (b >= 0 && !((done >> wv) & 1u)) {
                 // convergence test and beta on the scene's r.r
                 double rr, mx;
-                await_partials(p.bsum + par + b0, p.bmax + par + b0, nb, lane, rr, mx);
+                await_partials<MOST>(p.bsum + par + b0, p.bmax + par + b0, nb, lane, rr, mx);
                 // every reader of the s.q partials of iteration k - 1 has passed
                 if (lane == 0) clear_partial(p.bsq + (CG_RESIDENT - par) + b);
                 const CGTestIn in{rho, sc.cg_tol, sc.cg_min, sc.cg_max, false};
                 float beta;
-                const bool done = cg_test(p, si, k, rr, mx, recorder, beta, in);
+                const bool fin = cg_test(p, si, k, rr, mx, b == b0 && lane == 0, beta, in);
                 rho = rr;
                 if (lane == 0) {
-                    sh_beta[k & 1] = beta;
-                    sh_done[k & 1] = done ? 1 : 0;
+                    sh_beta[k & 1][wv] = beta;
+                    sh_done[k & 1][wv] = fin ? 1 : 0;
                 }
             }
             __syncthreads();
-            if (sh_done[k & 1]) break;
-            // s = r + beta s of the tile's nodes and of the block's
-            const float beta = sh_beta[k & 1];
+            for (int j = 0; j < K; ++j)
+                if (!((done >> j) & 1u) && sh_done[k & 1][j]) done |= 1u << j;
+            if (done == ALL) break;
+        }
+#pragma unroll 1
+        for (int j = 0; j < K; ++j) {
+            if (!((full & ~done) >> j & 1u)) continue;
+            const int bj = j == 0 ? blk0 : blk1;
+            if (K > 1) op.open(bj);
+            op.node = opaque(op.node);
+            // s = r + beta s of the tile's nodes
+            float u[D];
+#pragma unroll
+            for (int a = 0; a < D; ++a) u[a] = 0.0f;
             if (op.node >= 0) {
 #pragma unroll
                 for (int a = 0; a < D; ++a) {
-                    u[a] = cg_direction(ld_agent(p.g_r + a * p.gcap + op.node), ts[a][op.tid], beta, k);
-                    ts[a][op.tid] = u[a];
+                    if (k < 0) {
+                        u[a] = p.g_vs[a * p.gcap + op.node];
+                        ts[j][a][op.tid] = 0.0f;
+                    } else {
+                        u[a] = cg_direction(ld_agent(p.g_r + a * p.gcap + op.node), ts[j][a][op.tid], sh_beta[k & 1][j], k);
+                        ts[j][a][op.tid] = u[a];
+                    }
                 }
             }
-            if (interior) {
-#pragma unroll
-                for (int a = 0; a < D; ++a) ns[a][lane] = cg_direction(nr[a][lane], ns[a][lane], beta, k);
-            }
-        }
-        if (full) {
-            op.apply(inv_dx, u, k >= 0);
+            op.apply(p.scn[p.block_scene[bj]].inv_dx, u, K == 1 && k >= 0);
             op.template store<true>();
             drain_stores();
             __syncthreads();
-            if (threadIdx.x == 0) st_agent(flag + b, k + 2);
-            op.load_records(op.p0);  // for the next time
+            if (threadIdx.x == 0) st_agent(flag + bj, k + 2);
+            if (K == 1) op.load_records(op.p0);  // for the next time
         }
-        if (wv != 0) continue;
+        if (b < 0 || ((done >> wv) & 1u)) continue;
         // the neighbours' tiles, and this block's nodes
         while (__any(tnbr >= 0 && ld_agent(flag + max(tnbr, 0)) < k + 2)) __builtin_amdgcn_s_sleep(1);
         __asm__ __volatile__("" ::: "memory");
         float q[D], r[D];
         gather_node_tiles<D, D, true>(p, sc, n, q);
-        const double m = (double)nm[lane];
-        const float cm = sc.dt * sc.dt / nm[lane];
+        const double m = (double)nm[wv][lane];
+        const float cm = sc.dt * sc.dt / nm[wv][lane];
         double sum = 0.0, mx = 0.0;
         if (k < 0) {
 #pragma unroll
             for (int a = 0; a < D; ++a) {
-                r[a] = nr[a][lane];
+                r[a] = nr[wv][a][lane];
                 if (interior) {
-                    q[a] = cm * q[a] + nx[a][lane];
+                    q[a] = cm * q[a] + nx[wv][a][lane];
                     r[a] = r[a] - q[a];
                 }
                 if (zero) r[a] = 0.0f;
             }
         } else {
+            const float beta = sh_beta[k & 1][wv];
             float s[D];
 #pragma unroll
             for (int a = 0; a < D; ++a) {
-                s[a] = ns[a][lane];
-                if (interior) q[a] = cm * q[a] + s[a];
+                s[a] = ns[wv][a][lane];
+                if (interior) {
+                    s[a] = cg_direction(nr[wv][a][lane], s[a], beta, k);
+                    ns[wv][a][lane] = s[a];
+                    q[a] = cm * q[a] + s[a];
+                }
                 if (zero) q[a] = 0.0f;
                 if (interior) sum += (double)s[a] * ((double)q[a] * m);
             }
             double sq;
             wave_reduce2(sum, mx);
             if (lane == 0) put_partial(p.bsq + par + b, sum);
-            await_partials(p.bsq + par + b0, nullptr, nb, lane, sq, mx);
+            await_partials<MOST>(p.bsq + par + b0, nullptr, nb, lane, sq, mx);
             // every reader of this iteration's r.r partials has passed
             if (lane == 0) {
                 clear_partial(p.bsum + par + b);
                 clear_partial(p.bmax + par + b);
             }
             const double alpha_d = sq != 0.0 ? rho / sq : (double)FLT_MAX;
-            if (recorder) {
+            if (b == b0 && lane == 0) {
                 CGState& cg = p.cg[si];
                 cg.sq = sq;
                 cg.alpha = alpha_d;
@@ -2756,9 +2777,9 @@ __device__ inline void cg_solve_resident(const KP& p, int b, OperatorLds<D, CGW>
             const float alpha = (float)alpha_d;
 #pragma unroll
             for (int a = 0; a < D; ++a) {
-                r[a] = nr[a][lane];
+                r[a] = nr[wv][a][lane];
                 if (interior) {
-                    nx[a][lane] = alpha * s[a] + nx[a][lane];
+                    nx[wv][a][lane] = alpha * s[a] + nx[wv][a][lane];
                     r[a] = -alpha * q[a] + r[a];
                 }
             }
@@ -2772,7 +2793,7 @@ __device__ inline void cg_solve_resident(const KP& p, int b, OperatorLds<D, CGW>
                 sum += (double)r[a] * ((double)r[a] * m);
                 mx += (double)r[a] * (double)r[a];
             }
-            nr[a][lane] = r[a];
+            nr[wv][a][lane] = r[a];
             st_agent(p.g_r + a * p.gcap + n, r[a]);
             p.g_q[a * p.gcap + n] = q[a];
         }
@@ -2783,12 +2804,12 @@ __device__ inline void cg_solve_resident(const KP& p, int b, OperatorLds<D, CGW>
             put_partial(p.bmax + (CG_RESIDENT - par) + b, mx);
         }
     }
-    if (wv == 0) {
+    if (b >= 0) {
         const int lane = lane0, n = b * 64 + lane;
 #pragma unroll
         for (int a = 0; a < D; ++a) {
-            p.g_vs[a * p.gcap + n] = nx[a][lane];
-            p.g_s[a * p.gcap + n] = ns[a][lane];
+            p.g_vs[a * p.gcap + n] = nx[wv][a][lane];
+            p.g_s[a * p.gcap + n] = ns[wv][a][lane];
         }
     }
 }
@@ -2920,11 +2941,15 @@ __device__ inline void cg_solve_shared(const KP& p, int w0, int w1, int n, int g
     }
 }
 
+// One resident block a work-group up to CG_GROUPS blocks; above, up to
+// CG_RESIDENT, two, heaviest with lightest within an XCD's range of the block
+// order, so that a block of particles is paired with a halo block wherever
+// there are as many.
 template <int D>
 __global__ __launch_bounds__(CGW, 4) void k_cg_solve(KP p) {
     __shared__ __align__(16) OperatorLds<D, CGW> S;
-    const int n = p.ctr->nblocks, most = min(n, (int)gridDim.x);
-    if ((int)blockIdx.x == 0) {
+    const int n = p.ctr->nblocks, bid = (int)blockIdx.x;
+    if (bid == 0) {
         // scenes without blocks or at rest are done at once
         for (int si = threadIdx.x; si < p.nscenes; si += CGW) {
             const CGTestIn in = cg_test_in(p, si, 0);
@@ -2932,14 +2957,30 @@ __global__ __launch_bounds__(CGW, 4) void k_cg_solve(KP p) {
             if (in.empty) (void)cg_test(p, si, 0, 0.0, 0.0, true, beta, in);
         }
     }
-    if ((int)blockIdx.x >= most) return;
+    const bool pairs = n > CG_GROUPS && n <= CG_RESIDENT;
+    int blk0 = bid, blk1 = -1, most = min(n, CG_GROUPS);
+    bool mine = bid < most;
+    if (pairs) {
+        const auto lo = [&](int x) { return (int)(((int64_t)n * x) >> 3); };
+        most = 0;
+        for (int x = 0; x < 8; ++x) most += (lo(x + 1) - lo(x) + 1) / 2;
+        const int i = lo(bid & 7) + (bid >> 3), e = lo((bid & 7) + 1) - 1 - (bid >> 3);
+        mine = i <= e;
+        blk0 = mine ? p.block_order[p.bcap + i] : -1;
+        blk1 = i < e ? p.block_order[p.bcap + e] : -1;
+    }
+    if (!mine) return;
     int rank, group;
     if (!cg_enter(p, most, rank, group)) return;
-    if (group == n && n <= CG_RESIDENT) {
-        cg_solve_resident<D>(p, (int)blockIdx.x, S);
+    if (group == most && n <= CG_GROUPS) {
+        cg_solve_resident<D, 1>(p, blk0, -1, S);
+    } else if (group == most && pairs) {
+        cg_solve_resident<D, 2>(p, blk0, blk1, S);
     } else {
-        const int w0 = (int)((int64_t)rank * n / group), w1 = (int)((int64_t)(rank + 1) * n / group);
-        cg_solve_shared<D>(p, w0, w1, n, group, S);
+        const int g = min(group, n);
+        if (rank >= g) return;
+        const int w0 = (int)((int64_t)rank * n / g), w1 = (int)((int64_t)(rank + 1) * n / g);
+        cg_solve_shared<D>(p, w0, w1, n, g, S);
     }
 }
 
@@ -3524,8 +3565,8 @@ template <int D> void launch_cg_force(const KP& p, hipStream_t s, int grid, bool
     else if (one) hipLaunchKernelGGL((k_cg_force<D, false, true>), dim3(grid), dim3(BWG), 0, s, p, k);
     else hipLaunchKernelGGL((k_cg_force<D, false, false>), dim3(grid), dim3(BWG), 0, s, p, k);
 }
-template <int D> void launch_cg_solve(const KP& p, hipStream_t s, int grid) {
-    hipLaunchKernelGGL(k_cg_solve<D>, dim3(grid), dim3(CGW), 0, s, p);
+template <int D> void launch_cg_solve(const KP& p, hipStream_t s) {
+    hipLaunchKernelGGL((k_cg_solve<D>), dim3(CG_GROUPS), dim3(CGW), 0, s, p);
 }
 template <int D> void launch_cg_restart_node(const KP& p, hipStream_t s, int grid, bool one) {
     if (one) hipLaunchKernelGGL((k_cg_restart_node<D, true>), dim3(grid), dim3(WG), 0, s, p);
@@ -3560,7 +3601,7 @@ template <int D> void launch_max_speed(const KP& p, hipStream_t s, int grid) { h
     template void launch_particle_force<D>(const KP&, hipStream_t, int, bool, bool);          \
     template void launch_grid_update<D>(const KP&, hipStream_t, int, bool, bool, bool, bool); \
     template void launch_cg_force<D>(const KP&, hipStream_t, int, bool, int, bool);           \
-    template void launch_cg_solve<D>(const KP&, hipStream_t, int);                            \
+    template void launch_cg_solve<D>(const KP&, hipStream_t);                                 \
     template void launch_cg_restart_node<D>(const KP&, hipStream_t, int, bool);               \
     template void launch_cg_update_s<D>(const KP&, hipStream_t, int, int);                    \
     template void launch_cg_node1<D>(const KP&, hipStream_t, int, int, bool);                 \

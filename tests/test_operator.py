@@ -55,13 +55,15 @@ def test_cell_and_chunk_edges(dim, n):
         assert rel(got[k], want[k]) < 1e-5, k
 
 
+# active blocks (all scenes) of the scattered particles below: 322, 606 (a pair of
+# blocks per work-group), 1271; 638 and 1741 for two and three scenes of a batch
 @pytest.mark.parametrize("graph", [False, True])
-@pytest.mark.parametrize("scenes", [1, 3])
-def test_solve_with_more_blocks_than_work_groups(scenes, graph):
-    """Scattered particles: over a thousand active blocks for a few thousand
-    particles, so a work-group of the one-launch solve takes several blocks
-    (and, in a batch, blocks of two scenes)."""
-    counts, n = 64, 700
+@pytest.mark.parametrize("scenes,n,blocks", [(1, 100, 322), (1, 200, 606), (1, 700, 1271), (2, 100, 638), (3, 200, 1741)])
+def test_solve_by_number_of_blocks(scenes, n, blocks, graph):
+    """Scattered particles make hundreds of active blocks of a few hundred
+    particles: the one-launch solve keeps one block, then two, to a
+    work-group, then lets each take a range (of two scenes, in a batch)."""
+    counts = 64
     descs, parts = [], []
     for k in range(scenes):
         r = np.random.default_rng(7 + k)
@@ -78,9 +80,9 @@ def test_solve_with_more_blocks_than_work_groups(scenes, graph):
         b.upload(k, x, v, m)
     b.initialize()
     b.use_graph(graph)
-    for _ in range(2):
-        b.substep(dt)
-    assert sum(b.stats(k)["active_blocks"] for k in range(scenes)) > 1000
+    b.substep(dt)
+    assert sum(b.stats(k)["active_blocks"] for k in range(scenes)) == blocks
+    b.substep(dt)
     for k, (x, v, m) in enumerate(parts):
         o = O.Oracle(descs[k], 8, 4, O.DOT_FP64 | O.SVD_FP64)
         o.set_particles(x, v, m)
