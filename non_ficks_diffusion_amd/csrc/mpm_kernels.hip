@@ -1866,6 +1866,7 @@ struct BlockOperator {
     const float4* rec4;
     float4 next[W / 4];
     int b, tid, lane, wv, p0, p1, c0, c1, base;
+    int chunks;  // particle p0 + t chunks + c sits at place t of chunk c
     int li, node;  // tile node tid: its LDS index and grid node (-1: none)
 
     __device__ BlockOperator(const KP& kp, L& lds)
@@ -1874,13 +1875,21 @@ struct BlockOperator {
         local_coords<D>(lane, l);
         base = tile_index<D>(l, 0, off0);  // cell `lane`'s stencil corner
     }
-    __device__ void load_records(int chunk) {
-        const int64_t i = min(chunk + tid, p1 - 1);
+    // A block of more than NT particles is taken in chunks of every chunks-th
+    // one, so that each chunk holds a like part of every cell: in consecutive
+    // chunks most cells would have none, and their lanes nothing to sum.
+    __device__ void load_records(int c) {
+        const int64_t i = min(p0 + tid * chunks + c, p1 - 1);
 #pragma unroll
         for (int k = 0; k < W / 4; ++k) next[k] = rec4[i * (W / 4) + k];
     }
-    __device__ void mark_cells(int chunk) {
-        for (int j = max(c0, chunk); j < min(c1, chunk + NT); ++j) S.cell[j - chunk] = (unsigned char)lane;
+    // the first place of chunk c whose particle is m or later
+    __device__ int place(int m, int c) const {
+        const unsigned d = (unsigned)max(m - p0 - c, 0);
+        return chunks == 1 ? (int)d : (int)((d + (unsigned)chunks - 1u) / (unsigned)chunks);
+    }
+    __device__ void mark_cells(int c) {
+        for (int t = place(c0, c), e = place(c1, c); t < e; ++t) S.cell[t] = (unsigned char)lane;
     }
     // Block bi: its ranges, the tile node of this thread, the order of its
     // cells and the first chunk's records (in flight).
@@ -1890,7 +1899,8 @@ struct BlockOperator {
         p1 = p.block_pstart[b + 1];
         c0 = p.cell_start[b * 65 + lane];
         c1 = p.cell_start[b * 65 + lane + 1];
-        if (p1 > p0) load_records(p0);
+        chunks = max(1, (p1 - p0 + NT - 1) / NT);
+        if (p1 > p0) load_records(0);
         li = 0;
         node = -1;
         if (tid < TN) {
@@ -1902,7 +1912,7 @@ struct BlockOperator {
         }
         if (wv == LAST) {
             sort_cells(c1 - c0, lane, reinterpret_cast<int*>(S.tile()), S.perm);
-            mark_cells(p0);
+            mark_cells(0);
         }
     }
     // The operator of node values u (channels of tile node tid): leaves the
@@ -1913,7 +1923,7 @@ struct BlockOperator {
 #pragma unroll
             for (int a = 0; a < D; ++a) pack[a * LTN + li] = u[a];
         }
-        if (again && wv == LAST && p1 - p0 > NT) mark_cells(p0);
+        if (again && wv == LAST && chunks > 1) mark_cells(0);
         __syncthreads();
         if (wv < D) {
             float c[CS::NC];
@@ -1923,19 +1933,17 @@ struct BlockOperator {
                 if (n != CS::MID) S.coef[CS::row(0, n) * 64 + wv * (CS::NC - 1) * 64 + lane] = c[n];
         }
         __syncthreads();
-        // the lane's cell, channel and part of the scatter: particles j, j +
-        // PARTS, ... below m1
+        // the lane's cell, channel and part of the scatter
         const int part = tid / TASKS, task = tid - part * TASKS;
         const bool scatter = part < PARTS;
         const int ch = task % D, mine = S.perm[task / D];
-        const int m1 = scatter ? p.cell_start[b * 65 + mine + 1] : 0;
-        int j = p.cell_start[b * 65 + mine] + part;
+        const int m0 = p.cell_start[b * 65 + mine], m1 = scatter ? p.cell_start[b * 65 + mine + 1] : m0;
         float m[CS::NC];
 #pragma unroll
         for (int n = 0; n < CS::NC; ++n) m[n] = 0.0f;
         const float scale = inv_dx * inv_dx;
-        for (int chunk = p0; chunk < p1; chunk += NT) {
-            if (chunk + tid < p1) {
+        for (int c = 0; c < chunks; ++c) {
+            if (p0 + tid * chunks + c < p1) {
                 float rec[W];
 #pragma unroll
                 for (int k = 0; k < W / 4; ++k) {
@@ -1951,14 +1959,15 @@ struct BlockOperator {
                 pack_particle<D>(g, A, pack + tid * CS::PACK);
             }
             __syncthreads();
-            if (chunk + NT < p1) {
-                load_records(chunk + NT);
-                if (wv == LAST) mark_cells(chunk + NT);
+            if (c + 1 < chunks) {
+                load_records(c + 1);
+                if (wv == LAST) mark_cells(c + 1);
             }
             // the next particle's words load while the current one is added
-            const int end = min(m1, chunk + NT);
+            int j = place(m0, c) + part;
+            const int end = place(m1, c);
             if (j < end) {
-                const float *a = pack + (j - chunk) * CS::PACK, *ac = a + ch * 4;
+                const float *a = pack + j * CS::PACK, *ac = a + ch * 4;
                 PackedForce<D> f0, f1;
                 f0.load(a, ac);
                 for (;;) {
@@ -2038,9 +2047,10 @@ __device__ inline void operator_block(const KP& p, int b, float inv_dx, Operator
 // Bound by VALU issue in large scenes, by one block's chain of phases in small
 // ones.  Per launch, against one lane per cell for everything (nodes read per
 // particle, 81 LDS read-add-writes per particle): avalanche of 1.0M particles
-// in 256^3 mid-slide 57 -> 49 us with 4096 work-groups (32.9M -> 19.9M VALU
-// wave instructions), two balls of 243k 24.4 -> 20.0, 3.8k particles 24.0 ->
-// 13.2.  One wave per block with the moments of its cells in registers (255
+// in 256^3 mid-slide 57 -> 49 us with chunks of consecutive particles, 42 with
+// chunks that hold a part of every cell (32.9M, 19.9M, 16.7M VALU wave
+// instructions); two balls of 243k 24.4, 20.0, 16.6; 3.8k particles 24.0, 13.2,
+// 11.0.  One wave per block with the moments of its cells in registers (255
 // VGPRs, two waves a SIMD) took 61 us: everything then waits for the fullest
 // cell, which holds two to three times the mean.
 template <int D, bool RESTART, bool ONE>
@@ -2723,7 +2733,7 @@ __device__ inline void cg_solve_resident(const KP& p, int blk0, int blk1, Operat
             drain_stores();
             __syncthreads();
             if (threadIdx.x == 0) st_agent(flag + bj, k + 2);
-            if (K == 1) op.load_records(op.p0);  // for the next time
+            if (K == 1) op.load_records(0);  // for the next time
         }
         if (b < 0 || ((done >> wv) & 1u)) continue;
         // the neighbours' tiles, and this block's nodes
