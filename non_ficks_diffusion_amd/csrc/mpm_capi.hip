@@ -220,9 +220,21 @@ void set_step(mpm_context* c, const float* dts, float dt_all, bool force_active,
     }
 }
 
+// Work-groups of the kernels that take a block each: no more than the blocks
+// of the last binning the host has seen (a done poll, or the initialisation)
+// with a quarter on top, four times them in a captured sequence, which keeps its
+// grid for later substeps.  More blocks than that are taken in further rounds,
+// so the count only matters for speed: the avalanche's 3,340 blocks leave 4,850
+// of 8,192 work-groups without one, which cost an operator launch 5 us.
+int block_groups(const mpm_context* c, int configured) {
+    if (c->blocks_seen <= 0) return configured;
+    const int64_t want = c->capturing ? 4 * (int64_t)c->blocks_seen + 256 : c->blocks_seen + c->blocks_seen / 4 + 64;
+    return (int)std::min<int64_t>(configured, (want + 7) / 8 * 8);
+}
+
 template <int D>
 void launch_operator(const mpm_context* c, const mpm::KP& p, bool restart, int k, bool one) {
-    mpm::launch_cg_force<D>(p, c->stream, c->grid_op, restart, k, one);
+    mpm::launch_cg_force<D>(p, c->stream, block_groups(c, c->grid_op), restart, k, one);
 }
 
 // ---- stage sequences --------------------------------------------------------
@@ -232,7 +244,7 @@ void stage_bin(mpm_context* c) {
     timed(c, KC_BIN, [&] { mpm::launch_bin<D>(p, c->stream, c->grid_particle); });
     timed(c, KC_SCAN, [&] { mpm::launch_scan(p, c->stream); });
     timed(c, KC_SETUP, [&] {
-        mpm::launch_block_setup<D>(p, c->stream, c->grid_block);
+        mpm::launch_block_setup<D>(p, c->stream, block_groups(c, c->grid_block));
         mpm::launch_setup_order(p, c->stream, c->grid_particle);
     });
     timed(c, KC_REORDER, [&] { mpm::launch_reorder<D>(p, c->stream, c->grid_particle); });
@@ -245,14 +257,14 @@ void stage_bin(mpm_context* c) {
 template <int D>
 void stage_p2g(mpm_context* c) {
     mpm::KP p = make_kp(c);
-    timed(c, KC_P2G, [&] { mpm::launch_p2g<D>(p, c->stream, c->grid_block); });
+    timed(c, KC_P2G, [&] { mpm::launch_p2g<D>(p, c->stream, block_groups(c, c->grid_block)); });
     timed(c, KC_NORMALIZE, [&] { mpm::launch_normalize<D>(p, c->stream, c->grid_node); });
 }
 
 template <int D>
 void stage_waiting(mpm_context* c) {
     mpm::KP p = make_kp(c);
-    timed(c, KC_INIT_VOLUME, [&] { mpm::launch_init_volume<D>(p, c->stream, c->grid_block); });
+    timed(c, KC_INIT_VOLUME, [&] { mpm::launch_init_volume<D>(p, c->stream, block_groups(c, c->grid_block)); });
 }
 
 // particles from which a batch substep with one active scene is launched
@@ -375,6 +387,7 @@ int stage_cg(mpm_context* c, bool do_init, bool fixed = false) {
             pending[slot] = false;
             const int* h = &c->h_done[POLL_INTS * slot];
             c->overflow_seen = c->overflow_seen || h[POLL_OVERFLOW] != 0;
+            c->blocks_seen = h[POLL_NBLOCKS];
             if (h[POLL_NDONE] >= target) {
                 // the next solve's first batch: this one's iterations (iteration
                 // k's convergence test ends a solve of k updates)
@@ -415,6 +428,7 @@ int finish_cg_poll(mpm_context* c) {
         HIPCHECK(hipEventSynchronize(c->done_ev[slot]));
         const int* h = &c->h_done[POLL_INTS * slot];
         c->overflow_seen = c->overflow_seen || h[POLL_OVERFLOW] != 0;
+        c->blocks_seen = h[POLL_NBLOCKS];
         if (iters < 0 && h[POLL_NDONE] >= c->poll_target) iters = h[POLL_CG_ITERS];
     }
     // seen done: its iterations; never seen done (the cap's test runs after
@@ -426,7 +440,7 @@ int finish_cg_poll(mpm_context* c) {
 template <int D>
 void stage_g2p(mpm_context* c) {
     mpm::KP p = make_kp(c);
-    timed(c, KC_G2P, [&] { mpm::launch_g2p<D>(p, c->stream, c->grid_block); });
+    timed(c, KC_G2P, [&] { mpm::launch_g2p<D>(p, c->stream, block_groups(c, c->grid_block)); });
     c->binned = false;
 }
 
@@ -443,11 +457,11 @@ int run_stage(mpm_context* c, int stage, float dt) {
             set_step(c, nullptr, dt, true, true);
             break;
         case MPM_STAGE_CONSTITUTIVE:
-            timed(c, KC_PFORCE, [&] { mpm::launch_particle_force<D>(p, c->stream, c->grid_block, true, false); });
+            timed(c, KC_PFORCE, [&] { mpm::launch_particle_force<D>(p, c->stream, block_groups(c, c->grid_block), true, false); });
             c->records_fresh = c->binned;
             break;
         case MPM_STAGE_EXPLICIT_FORCE:
-            timed(c, KC_PFORCE, [&] { mpm::launch_particle_force<D>(p, c->stream, c->grid_block, false, true); });
+            timed(c, KC_PFORCE, [&] { mpm::launch_particle_force<D>(p, c->stream, block_groups(c, c->grid_block), false, true); });
             timed(c, KC_GRID, [&] { mpm::launch_grid_update<D>(p, c->stream, c->grid_node, true, false, false, true); });
             break;
         case MPM_STAGE_COLLISION:
@@ -483,6 +497,11 @@ int substep(mpm_context* c, const float* dts, bool capture = false) {
             if (dts[s] > 0.0f) { ++active; last = s; }
         if (active == 1 && !cg_in_one_launch(c)) c->solo = last;
     }
+    struct Capturing {
+        mpm_context* c;
+        ~Capturing() { c->capturing = false; }
+    } capturing{c};
+    c->capturing = capture;
     if (capture) mpm::launch_set_step_dev(make_kp(c), c->stream, c->d_dt);
     else set_step(c, dts, 0.0f, false, false);
     c->overflow_seen = false;
@@ -494,7 +513,7 @@ int substep(mpm_context* c, const float* dts, bool capture = false) {
     if (c->pool || c->emitted) {
         // scenes attached or particles added since the last substep:
         // Process_Waiting_Particles (every other scene's blocks return at once)
-        timed(c, KC_INIT_VOLUME, [&] { mpm::launch_init_volume<D>(p, c->stream, c->grid_block); });
+        timed(c, KC_INIT_VOLUME, [&] { mpm::launch_init_volume<D>(p, c->stream, block_groups(c, c->grid_block)); });
         mpm::launch_clear_waiting(p, c->stream);
         if (!capture) {
             c->emitted = false;
@@ -504,7 +523,7 @@ int substep(mpm_context* c, const float* dts, bool capture = false) {
             }
         }
     }
-    timed(c, KC_PFORCE, [&] { mpm::launch_particle_force<D>(p, c->stream, c->grid_block, true, true); });
+    timed(c, KC_PFORCE, [&] { mpm::launch_particle_force<D>(p, c->stream, block_groups(c, c->grid_block), true, true); });
     c->records_fresh = true;
     timed(c, KC_GRID, [&] { mpm::launch_grid_update<D>(p, c->stream, c->grid_node, true, true, true, false); });
     int rc = stage_cg<D>(c, false, capture);
@@ -1329,9 +1348,9 @@ int autotune(mpm_context* c, const float* dts, mpm_launch_config& best) {
     // a grid and CG set-up on the binned particles
     {
         mpm::KP p = make_kp(c);
-        mpm::launch_p2g<D>(p, c->stream, c->grid_block);
+        mpm::launch_p2g<D>(p, c->stream, block_groups(c, c->grid_block));
         mpm::launch_normalize<D>(p, c->stream, c->grid_node);
-        mpm::launch_particle_force<D>(p, c->stream, c->grid_block, false, true);
+        mpm::launch_particle_force<D>(p, c->stream, block_groups(c, c->grid_block), false, true);
         mpm::launch_grid_update<D>(p, c->stream, c->grid_node, true, true, true, false);
         launch_operator<D>(c, p, true, 0, one);
         mpm::launch_cg_restart_node<D>(p, c->stream, c->grid_node, one);
@@ -1769,6 +1788,7 @@ int mpm_initialize(mpm_handle c) {
     mpm::Counters h{};
     rc = read_counters(c, h);
     if (rc) return rc;
+    c->blocks_seen = h.nblocks;
     // the particles need more active blocks than the handle stores: nothing
     // was built, and the handle waits for an upload that fits
     if (h.overflow) return mpm_set_error(MPM_E_CAPACITY, "mpm_initialize: active blocks exceed the block capacity");
@@ -2378,6 +2398,7 @@ int noalloc_substep(NoallocDevice& nd, const mpm_scene_desc& d, int64_t n, float
     c->pool = false;
     c->graph = false;
     c->timing = false;
+    c->blocks_seen = 0;
     c->emitted = true;  // every call runs Process_Waiting_Particles for particles of volume 0
     c->ever_binned = true;
     size_t off = 0;

@@ -73,11 +73,13 @@ struct mpm_context {
     bool poll_pending[2] = {false, false};
     int poll_boundary[2] = {0, 0};
     int poll_older = 0, poll_target = 1, poll_max_it = 0;
+    int blocks_seen = 0;   // active blocks of the last binning whose counters the host has read (0: none)
     int grid_particle = 0, grid_block = 0, grid_node = 0;
     int op_mode = 0, grid_op = 0;  // CG operator: its mode (0 or 1, one kernel serves both) and work-groups
     size_t nred = 0;           // entries of the reduction partial arrays
     // captured substeps: one graph per particle-buffer parity
     bool graph = false;
+    bool capturing = false;  // the launches are being captured (or stand for any later state)
     // (entries 0, 1: launched CG iterations; 2, 3: the solve in one launch)
     hipGraphExec_t gexec[4] = {nullptr, nullptr, nullptr, nullptr};
     float* d_dt = nullptr;     // per-scene dt read by a replayed graph
