@@ -349,6 +349,11 @@ int mpm_substep_noalloc(const mpm_scene_desc* desc, int64_t n, float* x, float* 
 int mpm_get_launch_config(mpm_handle h, mpm_launch_config* cfg);
 /* Sets the launch shapes (results do not depend on them). */
 int mpm_set_launch_config(mpm_handle h, const mpm_launch_config* cfg);
+/* How long the CG's work-groups, which exchange sums within a launch, wait for
+ * the last of their launch to start before those that run share its work (in
+ * 10 ns; the default, 5000, is far above the time a free device takes).
+ * Results do not depend on it. */
+int mpm_set_wait_limit(mpm_handle h, int32_t ticks);
 /* Autotuner: times candidate work-group counts for the per-block,
  * per-node and per-particle kernels on the handle's current particles
  * (re-binned, with the grid and CG set up for dt; nscenes dts, or one dt for

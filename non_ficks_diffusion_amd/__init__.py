@@ -165,6 +165,7 @@ SIGNATURES = {
     "mpm_set_launch_config": (ctypes.c_int, [_H, ctypes.POINTER(LaunchConfig)]),
     "mpm_autotune": (ctypes.c_int, [_H, _FP, ctypes.c_int32, ctypes.POINTER(LaunchConfig)]),
     "mpm_set_graph": (ctypes.c_int, [_H, ctypes.c_int32]),
+    "mpm_set_wait_limit": (ctypes.c_int, [_H, ctypes.c_int32]),
     "mpm_serve_create": (ctypes.c_int, [ctypes.POINTER(ServeConfig), ctypes.POINTER(_H)]),
     "mpm_serve_destroy": (ctypes.c_int, [_H]),
     "mpm_serve_arena": (ctypes.c_int, [_H, _LP, _LP, _LP, _LP]),
@@ -347,6 +348,11 @@ class _LaunchControl:
         g = LaunchConfig()
         _check(lib().mpm_autotune(self._h, _fp(d), MPM_TUNE_CACHED if cached else 0, ctypes.byref(g)))
         return g.as_dict()
+
+    def set_wait_limit(self, ticks: int) -> None:
+        """How long (10 ns ticks) the CG's work-groups wait for the last of
+        their launch to start; results do not depend on it."""
+        _check(lib().mpm_set_wait_limit(self._h, ticks))
 
     def use_graph(self, on: bool = True) -> None:
         """Each substep replays a captured HIP graph of its launch sequence."""

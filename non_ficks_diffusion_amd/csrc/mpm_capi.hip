@@ -119,9 +119,9 @@ mpm::KP make_kp(const mpm_context* c) {
     p.cg = c->cg;
     p.slot_scene = c->slot_scene;
     p.nscenes = c->nscenes;
-    p.solo = c->solo >= 0 ? c->solo : 0;
     p.one_launch = cg_in_one_launch(c) ? 1 : 0;
-    p.cg_target = (c->nscenes == 1 || c->solo >= 0) ? 1 : c->nscenes;
+    p.one_active = c->one_active ? 1 : 0;
+    p.door_ticks = c->door_ticks;
     p.pcur = c->pbuf[c->cur];
     p.palt = c->pbuf[c->cur ^ 1];
     p.idcur = c->idbuf[c->cur];
@@ -233,8 +233,12 @@ int block_groups(const mpm_context* c, int configured) {
 }
 
 template <int D>
-void launch_operator(const mpm_context* c, const mpm::KP& p, bool restart, int k, bool one) {
-    mpm::launch_cg_force<D>(p, c->stream, block_groups(c, c->grid_op), restart, k, one);
+void launch_operator(const mpm_context* c, const mpm::KP& p, bool restart) {
+    mpm::launch_cg_force<D>(p, c->stream, block_groups(c, c->grid_op), restart);
+}
+template <int D>
+void launch_node_pass(const mpm_context* c, const mpm::KP& p, int k, bool restart) {
+    mpm::launch_cg_node<D>(p, c->stream, block_groups(c, c->bcap), k, restart);
 }
 
 // ---- stage sequences --------------------------------------------------------
@@ -268,7 +272,7 @@ void stage_waiting(mpm_context* c) {
 }
 
 // particles from which a batch substep with one active scene is launched
-// (single-scene CG kernels, polled) rather than replayed from the batch graph
+// (polled: no iterations past its end) rather than replayed
 constexpr int64_t SOLO_LAUNCHED_MIN = 65536;
 // iterations per launch batch of the polled CG after the first; the batch
 // right after the first (the predicted count) covers the host's reading of
@@ -319,10 +323,8 @@ int max_cg_iterations(const mpm_context* c) {
 template <int D>
 int stage_cg(mpm_context* c, bool do_init, bool fixed = false) {
     mpm::KP p = make_kp(c);
-    const bool one = c->nscenes == 1 || c->solo >= 0;
-    const int gn = c->grid_node;
     if (do_init)
-        timed(c, KC_GRID, [&] { mpm::launch_grid_update<D>(p, c->stream, gn, false, false, true, false); });
+        timed(c, KC_GRID, [&] { mpm::launch_grid_update<D>(p, c->stream, c->grid_node, false, false, true, false); });
     if (cg_in_one_launch(c)) {
         timed(c, KC_CG_FORCE, [&] { mpm::launch_cg_solve<D>(p, c->stream); });
         if (!fixed) {
@@ -331,33 +333,23 @@ int stage_cg(mpm_context* c, bool do_init, bool fixed = false) {
             HIPCHECK(hipEventRecord(c->done_ev[0], c->stream));
             c->poll_open = true;
             c->poll_older = 0;
-            c->poll_target = one ? 1 : c->nscenes;
+            c->poll_target = c->nscenes;
             c->poll_max_it = max_cg_iterations(c);
             c->poll_pending[0] = true;
             c->poll_pending[1] = false;
         }
         return MPM_OK;
     }
-    timed(c, KC_CG_FORCE, [&] { launch_operator<D>(c, p, true, 0, one); });
-    timed(c, KC_CG_NODE, [&] {
-        mpm::launch_cg_restart_node<D>(p, c->stream, gn, one);
-        if (!one) mpm::launch_cg_reduce_rr(p, c->stream, 0);
-    });
+    timed(c, KC_CG_FORCE, [&] { launch_operator<D>(c, p, true); });
+    timed(c, KC_CG_NODE, [&] { launch_node_pass<D>(c, p, 0, true); });
     const int max_it = max_cg_iterations(c);
     auto iteration = [&](int k) {
-        if (one) timed(c, KC_CG_NODE, [&] { mpm::launch_cg_update_s<D>(p, c->stream, gn, k); });
-        timed(c, KC_CG_FORCE, [&] { launch_operator<D>(c, p, false, k, one); });
-        timed(c, KC_CG_NODE, [&] {
-            mpm::launch_cg_node1<D>(p, c->stream, gn, k, one);
-            if (!one) mpm::launch_cg_reduce_sq(p, c->stream, k);
-            mpm::launch_cg_node2<D>(p, c->stream, gn, k, one);
-            if (!one) mpm::launch_cg_reduce_rr(p, c->stream, k + 1);
-        });
+        timed(c, KC_CG_FORCE, [&] { launch_operator<D>(c, p, false); });
+        timed(c, KC_CG_NODE, [&] { launch_node_pass<D>(c, p, k, false); });
     };
     if (fixed) {
         // captured substeps: every iteration up to the largest cap, no polling
         for (int k = 0; k < max_it; ++k) iteration(k);
-        if (one) mpm::launch_cg_update_s<D>(p, c->stream, gn, max_it);
         return MPM_OK;
     }
     // Iterations after every solve is done return at once, so launching a few
@@ -365,7 +357,7 @@ int stage_cg(mpm_context* c, bool do_init, bool fixed = false) {
     // count; after it the host polls the done count one chunk behind the GPU
     // (double-buffered events), so the queue never runs dry while it waits.
     const int first = std::min(max_it, std::max(c->cg_predict, CG_CHUNK));
-    const int target = one ? 1 : c->nscenes;
+    const int target = c->nscenes;
     int slot = 0, launched = 0;
     int boundary[2] = {0, 0};
     bool pending[2] = {false, false};
@@ -398,8 +390,6 @@ int stage_cg(mpm_context* c, bool do_init, bool fixed = false) {
         }
     }
     if (!finished) {
-        // one scene: the convergence test after the last iteration (batches ran it in reduce_rr)
-        if (one) timed(c, KC_CG_NODE, [&] { mpm::launch_cg_update_s<D>(p, c->stream, gn, max_it); });
         // the polls still in flight are read once the rest of the substep is queued
         c->poll_open = true;
         c->poll_older = slot;  // the slot written first of the two
@@ -446,7 +436,7 @@ void stage_g2p(mpm_context* c) {
 
 template <int D>
 int run_stage(mpm_context* c, int stage, float dt) {
-    c->solo = -1;
+    c->one_active = false;
     set_step(c, nullptr, dt, true, false);
     mpm::KP p = make_kp(c);
     switch (stage) {
@@ -483,19 +473,12 @@ int run_stage(mpm_context* c, int stage, float dt) {
 // capture: the launch sequence of a graph (dts from d_dt, fixed CG count).
 template <int D>
 int substep(mpm_context* c, const float* dts, bool capture = false) {
-    // a batch or arena substep with one active scene runs the single-scene
-    // CG kernels on it (captured substeps keep the batch kernels: their
-    // active set changes between replays)
-    c->solo = -1;
-    struct SoloReset {  // only this substep's launches see the solo scene
-        mpm_context* c;
-        ~SoloReset() { c->solo = -1; }
-    } solo_reset{c};
-    if (!capture && c->nscenes > 1) {
-        int active = 0, last = -1;
-        for (int s = 0; s < c->nscenes; ++s)
-            if (dts[s] > 0.0f) { ++active; last = s; }
-        if (active == 1 && !cg_in_one_launch(c)) c->solo = last;
+    if (!capture) {
+        int active = 0;
+        for (int k = 0; k < c->nscenes; ++k) active += dts[k] > 0.0f ? 1 : 0;
+        c->one_active = c->nscenes > 1 && active == 1;
+    } else {
+        c->one_active = false;
     }
     struct Capturing {
         mpm_context* c;
@@ -600,8 +583,8 @@ int fill_stats(mpm_context* c, int s, mpm_step_stats* out) {
 void size_context(mpm_context* c) {
     c->gcap = (int64_t)c->bcap * 64;
     c->nparts = (c->nslots + mpm::SCAN_TILE - 1) / mpm::SCAN_TILE;
-    // reduction partials: per block (batches) or per node work-group (one scene)
-    c->nred = (size_t)std::max(c->bcap, MAX_NODE_GROUPS);
+    // CG partials: one per block, or the node pass's pairs per group of blocks and scene
+    c->nred = (size_t)std::max(std::max(c->bcap, MAX_NODE_GROUPS), 2 * (c->bcap / 8 + 1 + c->nscenes));
     c->grid_particle = (int)std::min<int64_t>(((c->pcap + mpm::WG - 1) / mpm::WG + 7) / 8 * 8, 4096);
     c->grid_block = (int)std::min<int64_t>(((int64_t)c->bcap + 7) / 8 * 8, 8192);
     c->grid_op = c->grid_block;
@@ -1196,7 +1179,7 @@ int graph_substep(mpm_context* c, const float* dts) {
 int do_substep(mpm_context* c, const float* dts) {
     // a substep after mpm_add_particles runs launched: it adds the waiting
     // pass; so does a batch substep with one large active scene, which then
-    // takes the single-scene CG kernels with the CG's done poll
+    // stops at the CG's done poll instead of its cap
     int active = 0, last = -1;
     for (int s = 0; s < c->nscenes; ++s)
         if (dts[s] > 0.0f) { ++active; last = s; }
@@ -1342,7 +1325,6 @@ int autotune(mpm_context* c, const float* dts, mpm_launch_config& best) {
     int rc = read_counters(c, h);
     if (rc) return rc;
     if (h.overflow) return mpm_set_error(MPM_E_CAPACITY, "mpm_autotune: active blocks exceed the block capacity");
-    const bool one = c->nscenes == 1;
     mpm_launch_config cur = current_config(c);
     best = cur;
     // a grid and CG set-up on the binned particles
@@ -1352,8 +1334,8 @@ int autotune(mpm_context* c, const float* dts, mpm_launch_config& best) {
         mpm::launch_normalize<D>(p, c->stream, c->grid_node);
         mpm::launch_particle_force<D>(p, c->stream, block_groups(c, c->grid_block), false, true);
         mpm::launch_grid_update<D>(p, c->stream, c->grid_node, true, true, true, false);
-        launch_operator<D>(c, p, true, 0, one);
-        mpm::launch_cg_restart_node<D>(p, c->stream, c->grid_node, one);
+        launch_operator<D>(c, p, true);
+        launch_node_pass<D>(c, p, 0, true);
     }
     auto no_prep = [] { return MPM_OK; };
     auto reopen = [&] { return reopen_cg(c); };
@@ -1369,7 +1351,7 @@ int autotune(mpm_context* c, const float* dts, mpm_launch_config& best) {
         const mpm::KP p = make_kp(c);
         float ms = 0.0f;
         rc = time_median(c, reopen, [&] {
-            for (int k = 0; k < 8; ++k) mpm::launch_cg_force<D>(p, c->stream, g, false, 1, one);
+            for (int k = 0; k < 8; ++k) mpm::launch_cg_force<D>(p, c->stream, g, false);
         }, ms);
         if (rc) return rc;
         if (ms < best_ms) {
@@ -1403,7 +1385,6 @@ int autotune(mpm_context* c, const float* dts, mpm_launch_config& best) {
         rc = time_median(c, no_prep, [&] {
             mpm::launch_normalize<D>(p, c->stream, g);
             mpm::launch_grid_update<D>(p, c->stream, g, true, true, true, false);
-            for (int k = 0; k < 8; ++k) mpm::launch_cg_restart_node<D>(p, c->stream, g, one);
         }, ms);
         if (rc) return rc;
         if (ms < best_ms) { best_ms = ms; best.node_groups = g; best.node_ms = ms; }
@@ -2061,8 +2042,8 @@ int mpm_time_cg_operator(mpm_handle c, int32_t reps, float* avg_ms) {
     mpm::KP p = make_kp(c);
     HIPCHECK(hipEventRecord(e0, c->stream));
     for (int r = 0; r < reps; ++r) {
-        if (c->D == 3) launch_operator<3>(c, p, false, 1, c->nscenes == 1);
-        else launch_operator<2>(c, p, false, 1, c->nscenes == 1);
+        if (c->D == 3) launch_operator<3>(c, p, false);
+        else launch_operator<2>(c, p, false);
     }
     HIPCHECK(hipEventRecord(e1, c->stream));
     HIPCHECK(hipEventSynchronize(e1));
@@ -2230,6 +2211,15 @@ int mpm_set_graph(mpm_handle c, int32_t on) {
     return MPM_OK;
 }
 
+int mpm_set_wait_limit(mpm_handle c, int32_t ticks) {
+    if (!c) return mpm_set_error(MPM_E_INVALID, "mpm_set_wait_limit: null handle");
+    if (ticks < 0) return mpm_set_error(MPM_E_INVALID, "mpm_set_wait_limit: negative limit");
+    HIPCHECK(hipStreamSynchronize(c->stream));
+    if (ticks != c->door_ticks) invalidate_graphs(c);
+    c->door_ticks = ticks;
+    return MPM_OK;
+}
+
 const char* mpm_kernel_class_name(int32_t cls) { return (cls >= 0 && cls < KC_COUNT) ? kClassNames[cls] : ""; }
 int32_t mpm_kernel_class_count(void) { return KC_COUNT; }
 
@@ -2394,7 +2384,7 @@ int noalloc_substep(NoallocDevice& nd, const mpm_scene_desc& d, int64_t n, float
     c->sc[0].n_uploaded = n;
     c->sc[0].uploaded = true;
     c->cur = 0;
-    c->solo = -1;
+    c->one_active = false;
     c->pool = false;
     c->graph = false;
     c->timing = false;

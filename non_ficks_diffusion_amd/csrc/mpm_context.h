@@ -39,7 +39,8 @@ struct mpm_context {
     int* keybuf[2] = {nullptr, nullptr};
     int* scbuf[2] = {nullptr, nullptr};
     int cur = 0;
-    int solo = -1;  // batch or arena substep with one active scene: it takes the single-scene CG
+    bool one_active = false;  // the launched batch substep has one scene that is not at rest
+    int door_ticks = 5000;  // KP::door_ticks
     int* prank = nullptr;
     int* cell_order = nullptr;  // per particle: index scattered by binning rank (stable in-cell order)
     float* rcache = nullptr;

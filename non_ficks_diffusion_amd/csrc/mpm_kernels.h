@@ -63,6 +63,9 @@ struct Counters {
     // k_cg_solve: work-groups that have come (with a bit once the door is
     // closed) and how many of them share the blocks
     int door, group;
+    int again;         // node pass: work-groups that start again
+    int doors[8][32];  // node pass: each XCD's door, on a line of its own
+    int live;          // scenes whose solve went on at the last operator launch
 };
 
 // Device frame loop of one scene (MPM_Driver::Advance_To_Target_Time,
@@ -81,7 +84,7 @@ struct CGState {
     double rho_hist[2], alpha, beta, conv, rr, sq;
     int iter, done, converged, multiplies;
     int arrived;  // k_cg_solve: work-groups of the scene counted in, over all its waits
-    int pad;
+    int closed;   // done, as of the last operator launch
 };
 
 struct KP {
@@ -91,9 +94,9 @@ struct KP {
     CGState* cg;
     const int* slot_scene;  // per global slot: the scene that owns it, -1 if none
     int nscenes;
-    int solo;        // the scene of the single-scene CG kernels (0 for a one-scene context)
     int one_launch;  // the solve is k_cg_solve
-    int cg_target;   // finished solves that end the CG: 1 on the single-scene path, else nscenes
+    int one_active;  // a launched batch substep of one scene (the others count no operator applications)
+    int door_ticks;  // how long work-groups that exchange wait for the others to start (100 MHz clock)
     // particles: field-major arrays of capacity pcap
     float* pcur;
     float* palt;
@@ -140,9 +143,11 @@ struct KP {
     float* tiles;    // per active block, (D+1) * (B+2)^D floats
     // control
     Counters* ctr;
-    double* bsum;    // partial sums of r.r, per active block (per work-group for one scene)
-    double* bmax;    // partial max |r|^2, same layout
-    double* bsq;     // partial sums of s.q, same layout
+    // partials of the CG: k_cg_solve a place per active block (r.r, max |r|^2,
+    // s.q); the node pass as described there
+    double* bsum;
+    double* bmax;
+    double* bsq;
     unsigned* bu;    // 2 * bcap: per block max |V|^2 bits | removals (G2P)
 };
 
@@ -215,20 +220,15 @@ template <int D> void launch_normalize(const KP& p, hipStream_t s, int grid);
 template <int D> void launch_init_volume(const KP& p, hipStream_t s, int grid);
 template <int D> void launch_particle_force(const KP& p, hipStream_t s, int grid, bool constitutive, bool force);
 template <int D> void launch_grid_update(const KP& p, hipStream_t s, int grid, bool force, bool collision, bool cg_init, bool write_f);
-template <int D> void launch_cg_force(const KP& p, hipStream_t s, int grid, bool restart, int k, bool one);
-// `one`: a batch of one scene (per-work-group partials, see k_cg_update_s)
+template <int D> void launch_cg_force(const KP& p, hipStream_t s, int grid, bool restart);
+// the node pass after it, with enough work-groups for `blocks` of them
+template <int D> void launch_cg_node(const KP& p, hipStream_t s, int blocks, int k, bool restart);
 // the whole solve in one launch (scenes too small to fill the chip; at most
 // CG_SOLVE_MAX_SCENES of them)
 constexpr int CG_SOLVE_MAX_SCENES = 64;
 constexpr int CG_GROUPS = 512;     // its work-groups (two fit a CU)
 constexpr int CG_RESIDENT = 2 * CG_GROUPS;  // blocks up to which their state stays in the work-groups
 template <int D> void launch_cg_solve(const KP& p, hipStream_t s);
-template <int D> void launch_cg_restart_node(const KP& p, hipStream_t s, int grid, bool one);
-template <int D> void launch_cg_update_s(const KP& p, hipStream_t s, int grid, int k);
-template <int D> void launch_cg_node1(const KP& p, hipStream_t s, int grid, int k, bool one);
-template <int D> void launch_cg_node2(const KP& p, hipStream_t s, int grid, int k, bool one);
-void launch_cg_reduce_sq(const KP& p, hipStream_t s, int k);
-void launch_cg_reduce_rr(const KP& p, hipStream_t s, int k);
 template <int D> void launch_g2p(const KP& p, hipStream_t s, int grid);
 template <int D> void launch_max_speed(const KP& p, hipStream_t s, int grid);
 template <int D> void launch_noalloc_load(const KP& p, hipStream_t s, int grid, const SceneParams& sp, const NoallocIn& a);

@@ -1672,24 +1672,29 @@ __global__ __launch_bounds__(BWG) void k_particle_force(KP p) {
 template <int D, bool FORCE, bool COLL, bool CGINIT, bool WRITE_F>
 __global__ __launch_bounds__(WG) void k_grid_update(KP p) {
     if (CGINIT) {
-        // a new solve for every scene (inactive scenes finish at the first
-        // test; on the single-scene path the others are finished here)
-        for (int si = blockIdx.x * WG + threadIdx.x; si < p.nscenes; si += gridDim.x * WG) {
-            CGState& cg = p.cg[si];
-            const int other = p.cg_target == 1 && si != p.solo ? 1 : 0;
-            cg.iter = 0;
-            cg.arrived = 0;
-            cg.done = other;
-            cg.converged = other;
-            cg.multiplies = 0;
-            cg.rho_hist[0] = cg.rho_hist[1] = 0.0;
-            cg.alpha = cg.beta = cg.conv = cg.rr = cg.sq = 0.0;
-        }
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
-            p.ctr->cg_ndone = 0;
-            p.ctr->cg_iters = 0;
-            p.ctr->door = 0;
-            p.ctr->group = 0;
+        // a new solve for every scene; one at rest or without blocks is done
+        if (blockIdx.x == 0) {
+            __shared__ int rest;
+            if (threadIdx.x == 0) rest = 0;
+            __syncthreads();
+            for (int si = threadIdx.x; si < p.nscenes; si += WG) {
+                CGState& cg = p.cg[si];
+                const int idle = !p.scn[si].active || p.sst[si].block_end <= p.sst[si].block_begin ? 1 : 0;
+                cg.iter = 0;
+                cg.arrived = 0;
+                cg.done = cg.closed = cg.converged = idle;
+                cg.multiplies = p.one_active ? 0 : idle;
+                cg.rho_hist[0] = cg.rho_hist[1] = 0.0;
+                cg.alpha = cg.beta = cg.conv = cg.rr = cg.sq = 0.0;
+                if (idle) atomicAdd(&rest, 1);
+            }
+            __syncthreads();
+            if (threadIdx.x == 0) {
+                p.ctr->cg_ndone = rest;
+                p.ctr->cg_iters = 0;
+                p.ctr->door = 0;
+                p.ctr->group = 0;
+            }
         }
         // k_cg_solve's places for partials (both parities) and tile flags
         if (p.one_launch)
@@ -1771,24 +1776,28 @@ __global__ __launch_bounds__(WG) void k_grid_update(KP p) {
 // CG (Apply_Force's solve, MPM_Example.cpp:700-711) for every scene of the
 // batch at once: Hestenes-Stiefel CG in the M inner product with a restart
 // at iteration 0.  Launch order per solve:
-//   grid_update<CGINIT>, cg_force<RESTART>, cg_restart_node, cg_reduce_rr(0),
-//   then for k = 0, 1, ...: cg_force(k), cg_node1(k), cg_reduce_sq(k),
-//   cg_node2, cg_reduce_rr(k + 1).
+//   grid_update<CGINIT>, cg_force<RESTART>, cg_node<RESTART>,
+//   then for k = 0, 1, ...: cg_force(k), cg_node(k).
 // A scene whose solve is finished is skipped by every kernel; when all are,
 // the kernels return at once.
 // ============================================================================
 
-// s = r (k = 0) or r + beta s: the one formula shared by the operator's
-// on-the-fly gather and node1's store, so both see identical bits
+// s = r (k = 0) or r + beta s
 __device__ inline float cg_direction(float r, float s, float beta, int k) {
     return k == 0 ? r : fmaf(beta, s, r);
 }
 
-__device__ inline bool cg_all_done(const KP& p) { return p.ctr->cg_ndone >= p.cg_target; }
-
-// Single-scene CG kernels in a batch or arena (one active scene): blocks of
-// the other scenes are skipped.
-__device__ inline bool other_scene(const KP& p, int b) { return p.nscenes > 1 && p.block_scene[b] != p.solo; }
+// The node pass's work-groups: NGB blocks, a wave each.  What they exchange:
+//   bsq   the runs' partials of s.q,
+//   bsum  the runs' partials of r.r and max |r|^2, in pairs,
+//   bmax  for scenes of many runs the sums over chunks of CG_CHUNK_RUNS of
+//         them, s.q and then the pairs, a copy per XCD.
+constexpr int NGW = 512, NGB = NGW / 64;
+constexpr int CG_NODE_GROUPS = 768;  // three of 512 threads a CU: all fit at once
+constexpr int CG_CHUNK_RUNS = 64, CG_DIRECT_RUNS = 192;  // (scenes of up to so many runs are summed directly)
+__device__ inline int cg_groups(int nblocks) { return (nblocks + NGB - 1) / NGB; }
+__device__ inline int cg_places(const KP& p, int ng) { return ng + p.nscenes; }
+__device__ inline int cg_chunk_places(int ng) { return (ng / (CG_CHUNK_RUNS / 2) + 17) / 16 * 16; }
 
 // LDS of the CG operator's work-group of NT threads:
 //   coef  the block's coefficient rows, later the node contributions of every
@@ -2053,23 +2062,37 @@ __device__ inline void operator_block(const KP& p, int b, float inv_dx, Operator
 // 11.0.  One wave per block with the moments of its cells in registers (255
 // VGPRs, two waves a SIMD) took 61 us: everything then waits for the fullest
 // cell, which holds two to three times the mean.
-template <int D, bool RESTART, bool ONE>
-__global__ __launch_bounds__(BWG, 4) void k_cg_force(KP p, int k) {
+//
+// It also readies what the node pass after it exchanges: empty places for the
+// partials, open doors, and which scenes are still live.
+template <int D, bool RESTART>
+__global__ __launch_bounds__(BWG, 4) void k_cg_force(KP p) {
     __shared__ __align__(16) OperatorLds<D, BWG> S;
-    if (cg_all_done(p)) return;
+    const int live = p.nscenes - p.ctr->cg_ndone;
+    if (blockIdx.x == 0) {
+        for (int si = threadIdx.x; si < p.nscenes; si += BWG) p.cg[si].closed = p.cg[si].done;
+        if (threadIdx.x < 8) p.ctr->doors[threadIdx.x][0] = 0;
+        if (threadIdx.x == 0) {
+            p.ctr->live = live;
+            p.ctr->again = 0;
+        }
+    }
+    if (live <= 0) return;
+    const int ng = cg_groups(p.ctr->nblocks), places = cg_places(p, ng), chunks = 24 * cg_chunk_places(ng);
+    for (int i = (int)blockIdx.x * BWG + (int)threadIdx.x; i < max(2 * places, chunks); i += (int)gridDim.x * BWG) {
+        const double empty = __longlong_as_double((long long)CG_EMPTY);
+        if (i < places) p.bsq[i] = empty;
+        if (i < 2 * places) p.bsum[i] = empty;
+        if (i < chunks) p.bmax[i] = empty;
+    }
     const XcdRange xr = xcd_blocks(p.ctr->nblocks);
     for (int kb = xr.first; kb < xr.end; kb += xr.step) {
         const int b = p.block_order[p.bcap + kb];  // the fullest cells first within the XCD's range
-        // one scene: no per-block lookups (its solve is live: cg_all_done above)
-        if (ONE && other_scene(p, b)) continue;
-        const int si = ONE ? p.solo : p.block_scene[b];
+        const int si = p.nscenes == 1 ? 0 : p.block_scene[b];
         const SceneParams& sc = p.scn[si];
-        if (!sc.active || (!ONE && p.cg[si].done) || block_empty(p, b)) continue;
-        const float beta = (RESTART || ONE) ? 0.0f : (float)p.cg[si].beta;
+        if (!sc.active || (p.nscenes > 1 && p.cg[si].done) || block_empty(p, b)) continue;
         operator_block<D, BWG, false>(p, b, sc.inv_dx, S, [&](int a, int64_t n) {
-            return RESTART ? p.g_vs[a * p.gcap + n]
-                   : ONE   ? p.g_s[a * p.gcap + n]
-                           : cg_direction(p.g_r[a * p.gcap + n], p.g_s[a * p.gcap + n], beta, k);
+            return RESTART ? p.g_vs[a * p.gcap + n] : p.g_s[a * p.gcap + n];
         });
     }
 }
@@ -2094,35 +2117,12 @@ __device__ inline void wave_reduce2(double& sum, double& mx) {
     }
 }
 
-// Two reduction layouts.  Batches (ONE = false): node kernels write one
-// partial per block and a one-work-group-per-scene kernel reduces each
-// scene's partials.  A batch of one scene (ONE = true): node kernels write
-// one partial per work-group and every work-group of the consuming kernel
-// reduces all of them itself (same values, same order, same result), which
-// saves the two reducer launches per CG iteration.
-
-// Writes this wave's partials (ONE: accumulated over its blocks) -- per block
-// in batches, per work-group for one scene.
-__device__ inline void wg_partials_store(double* dsum, double* dmax, double sum, double mx) {
-    __shared__ double ws[WG / 64], wm[WG / 64];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    if (lane == 0) { ws[wave] = sum; wm[wave] = mx; }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double s = 0.0, m = 0.0;
-#pragma unroll
-        for (int w = 0; w < WG / 64; ++w) { s += ws[w]; m = fmax(m, wm[w]); }
-        dsum[blockIdx.x] = s;
-        if (dmax) dmax[blockIdx.x] = m;
-    }
-}
-
 // Sum / max of `count` partials starting at `first`, in a fixed order
 // relative to `first`; the result is broadcast to every thread.
-template <bool AGENT = false, int NT = WG>
+template <int NT>
 __device__ inline void reduce_range(const double* sums, const double* maxs, int first, int count, double& sum,
                                     double& mx) {
-    constexpr int U = NT == WG ? 8 : 4;  // independent loads in flight per thread
+    constexpr int U = 4;  // independent loads in flight per thread
     double sa[U], ma[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) { sa[u] = 0.0; ma[u] = 0.0; }
@@ -2133,8 +2133,8 @@ __device__ inline void reduce_range(const double* sums, const double* maxs, int 
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int j = min(base + u * NT, count - 1);
-            vs[u] = ld<AGENT>(sums + first + j);
-            vm[u] = maxs ? ld<AGENT>(maxs + first + j) : 0.0;
+            vs[u] = ld_agent(sums + first + j);
+            vm[u] = maxs ? ld_agent(maxs + first + j) : 0.0;
         }
 #pragma unroll
         for (int u = 0; u < U; ++u)
@@ -2209,9 +2209,65 @@ __device__ inline bool cg_test(const KP& p, int si, int k, double rr, double mx,
     return done;
 }
 
-// CG restart of block b: q = dt^2/m q + x (Multiply_Helper), r = b - q,
-// Project(r); the block's r.r (M-weighted) and max |r|^2.
+// ---- what work-groups of one launch exchange ---------------------------------
+constexpr int CG_DOOR_CLOSED = 1 << 30;
+
+// Every store of this wave has reached memory.
+__device__ inline void drain_stores() { __asm__ __volatile__("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory"); }
+
+// ---- a partial that is its own flag -----------------------------------------
+__device__ inline void put_partial(double* a, double v) {
+    if (!(v == v)) v = __longlong_as_double(0x7ff8000000000000ll);
+    st_agent(a, v);
+}
+__device__ inline void clear_partial(double* a) { st_agent(a, __longlong_as_double((long long)CG_EMPTY)); }
+// The node values of one lane of a wave that holds a block.
 template <int D, bool AGENT>
+struct NodeRows {
+    float x[D], r[D], s[D], q[D], m;
+    bool interior;
+    __device__ void load(const KP& p, int n) {
+        interior = (p.g_flags[n] & MPM_FLAG_INTERIOR_DEV) != 0;
+        m = p.g_m[n];
+#pragma unroll
+        for (int a = 0; a < D; ++a) {
+            s[a] = ld<AGENT>(p.g_s + a * p.gcap + n);
+            q[a] = p.g_q[a * p.gcap + n];
+            x[a] = p.g_vs[a * p.gcap + n];
+            r[a] = ld<AGENT>(p.g_r + a * p.gcap + n);
+        }
+    }
+    // the block's r.r (M-weighted) and max |r|^2
+    __device__ void residual(double& sum, double& mx) {
+        sum = 0.0;
+        mx = 0.0;
+        if (interior) {
+#pragma unroll
+            for (int a = 0; a < D; ++a) {
+                sum += (double)r[a] * ((double)r[a] * (double)m);
+                mx += (double)r[a] * (double)r[a];
+            }
+        }
+        wave_reduce2(sum, mx);
+    }
+    // x += alpha s, r -= alpha q on block b; its r.r and max |r|^2
+    __device__ void step(const KP& p, int n, float alpha, double& sum, double& mx) {
+        if (interior) {
+#pragma unroll
+            for (int a = 0; a < D; ++a) {
+                p.g_vs[a * p.gcap + n] = alpha * s[a] + x[a];
+                r[a] = -alpha * q[a] + r[a];
+                st<AGENT>(p.g_r + a * p.gcap + n, r[a]);
+            }
+        }
+        residual(sum, mx);
+    }
+};
+
+// CG restart of block b: q = dt^2/m q + x (Multiply_Helper), r = b - q,
+// Project(r); the block's r.r (M-weighted) and max |r|^2.  r goes to g_r, or
+// with TO_S (where the pass may be taken again) to g_s.
+template <int D, bool AGENT, bool TO_S>
 __device__ inline void cg_restart_block(const KP& p, const SceneParams& sc, int b, int lane, double& sum, double& mx) {
     const int n = b * 64 + lane;
     const float sds = sc.dt * sc.dt;
@@ -2220,8 +2276,9 @@ __device__ inline void cg_restart_block(const KP& p, const SceneParams& sc, int 
     gather_node_tiles<D, D, AGENT>(p, sc, n, q);
 #pragma unroll
     for (int a = 0; a < D; ++a) rv[a] = p.g_r[a * p.gcap + n];
+    const float mn = p.g_m[n];
     if (interior) {
-        const float cm = sds / p.g_m[n];
+        const float cm = sds / mn;
 #pragma unroll
         for (int a = 0; a < D; ++a) {
             q[a] = cm * q[a] + p.g_vs[a * p.gcap + n];
@@ -2234,88 +2291,26 @@ __device__ inline void cg_restart_block(const KP& p, const SceneParams& sc, int 
     }
 #pragma unroll
     for (int a = 0; a < D; ++a) {
-        st<AGENT>(p.g_r + a * p.gcap + n, rv[a]);
+        st<AGENT>((TO_S ? p.g_s : p.g_r) + a * p.gcap + n, rv[a]);
         p.g_q[a * p.gcap + n] = q[a];
     }
     sum = 0.0;
     mx = 0.0;
     if (interior) {
-        const double m = (double)p.g_m[n];
 #pragma unroll
         for (int a = 0; a < D; ++a) {
-            sum += (double)rv[a] * ((double)rv[a] * m);
+            sum += (double)rv[a] * ((double)rv[a] * (double)mn);
             mx += (double)rv[a] * (double)rv[a];
         }
     }
     wave_reduce2(sum, mx);
 }
-template <int D, bool ONE>
-__global__ __launch_bounds__(WG) void k_cg_restart_node(KP p) {
-    const XcdRange r = xcd_wave_blocks(p.ctr->nblocks);
-    const int lane = threadIdx.x & 63;
-    double wsum = 0.0, wmx = 0.0;
-    for (int b = r.first; b < r.end; b += r.step) {
-        if (ONE && other_scene(p, b)) continue;
-        const SceneParams& sc = p.scn[ONE ? p.solo : p.block_scene[b]];
-        if (!sc.active) continue;
-        double sum, mx;
-        cg_restart_block<D, false>(p, sc, b, lane, sum, mx);
-        if (ONE) {
-            wsum += sum;
-            wmx = fmax(wmx, mx);
-        } else if (lane == 0) {
-            p.bsum[b] = sum;
-            p.bmax[b] = mx;
-        }
-    }
-    if (ONE) wg_partials_store(p.bsum, p.bmax, wsum, wmx);
-}
-
-// One scene: convergence test of iteration k on the r.r partials (every
-// work-group reduces them; work-group 0 records the state), then
-// s = r (k = 0) or r + beta s on the interior nodes.
-template <int D>
-__global__ __launch_bounds__(WG) void k_cg_update_s(KP p, int k, int nparts) {
-    const XcdRange r = xcd_wave_blocks(p.ctr->nblocks);
-    const int lane = threadIdx.x & 63;
-    // the wave's first block: r and s load while the partials are reduced
-    // (a wave without blocks loads block 0's nodes and uses nothing)
-    float r0[D], s0[D];
-    const bool has = r.first < r.end;
-    const bool mine = has && !other_scene(p, r.first);
-    const int n0 = (has ? r.first : 0) * 64 + lane;
-    const unsigned flags0 = p.g_flags[n0];
-#pragma unroll
-    for (int a = 0; a < D; ++a) {
-        r0[a] = p.g_r[a * p.gcap + n0];
-        s0[a] = p.g_s[a * p.gcap + n0];
-    }
-    if (cg_all_done(p)) return;
-    // the test's inputs load alongside the partials
-    const CGTestIn tin = cg_test_in(p, p.solo, k);
-    double rr, mx;
-    reduce_range(p.bsum, p.bmax, 0, nparts, rr, mx);
-    float beta;
-    if (cg_test(p, p.solo, k, rr, mx, blockIdx.x == 0 && threadIdx.x == 0, beta, tin)) return;
-    if (mine && (flags0 & MPM_FLAG_INTERIOR_DEV) != 0) {
-#pragma unroll
-        for (int a = 0; a < D; ++a) p.g_s[a * p.gcap + n0] = cg_direction(r0[a], s0[a], beta, k);
-    }
-    for (int b = r.first + r.step; b < r.end; b += r.step) {
-        if (other_scene(p, b)) continue;
-        const int n = b * 64 + lane;
-        if (!(p.g_flags[n] & MPM_FLAG_INTERIOR_DEV)) continue;
-#pragma unroll
-        for (int a = 0; a < D; ++a)
-            p.g_s[a * p.gcap + n] = cg_direction(p.g_r[a * p.gcap + n], p.g_s[a * p.gcap + n], beta, k);
-    }
-}
 
 // Tile sum of the operator, q = dt^2/m q + s, Project(q) on block b; the
-// block's s.q.  Batches form and store this iteration's s = r + beta s
-// (interior nodes); for one scene k_cg_update_s stored it already.
-template <int D, bool ONE, bool AGENT>
-__device__ inline void cg_node1_block(const KP& p, const SceneParams& sc, int b, int lane, float beta, int k, double& sum) {
+// block's s.q.  FORM: this iteration's s = r + beta s is formed and stored
+// first (interior nodes).
+template <int D, bool FORM, bool AGENT>
+__device__ inline void cg_product_block(const KP& p, const SceneParams& sc, int b, int lane, float beta, int k, double& sum) {
     const float sds = sc.dt * sc.dt;
     const int n = b * 64 + lane;
     const bool interior = (p.g_flags[n] & MPM_FLAG_INTERIOR_DEV) != 0;
@@ -2326,14 +2321,14 @@ __device__ inline void cg_node1_block(const KP& p, const SceneParams& sc, int b,
 #pragma unroll
     for (int a = 0; a < D; ++a) {
         sv[a] = ld<AGENT>(p.g_s + a * p.gcap + n);
-        if (!ONE) rv[a] = ld<AGENT>(p.g_r + a * p.gcap + n);
+        if (FORM) rv[a] = ld<AGENT>(p.g_r + a * p.gcap + n);
     }
     gather_node_tiles<D, D, AGENT>(p, sc, n, q);
     if (interior) {
         const float cm = sds / mn;
 #pragma unroll
         for (int a = 0; a < D; ++a) {
-            if (!ONE) {
+            if (FORM) {
                 sv[a] = cg_direction(rv[a], sv[a], beta, k);
                 st<AGENT>(p.g_s + a * p.gcap + n, sv[a]);
             }
@@ -2355,159 +2350,336 @@ __device__ inline void cg_node1_block(const KP& p, const SceneParams& sc, int b,
     }
     wave_reduce2(sum, mx);
 }
-template <int D, bool ONE>
-__global__ __launch_bounds__(WG) void k_cg_node1(KP p, int k) {
-    if (cg_all_done(p)) return;
-    const XcdRange r = xcd_wave_blocks(p.ctr->nblocks);
-    const int lane = threadIdx.x & 63;
-    double wsum = 0.0;
-    for (int b = r.first; b < r.end; b += r.step) {
-        if (ONE && other_scene(p, b)) continue;
-        const int si = ONE ? p.solo : p.block_scene[b];
-        const SceneParams& sc = p.scn[si];
-        if (!sc.active || (!ONE && p.cg[si].done)) continue;
-        const float beta = ONE ? 0.0f : (float)p.cg[si].beta;
-        double sum;
-        cg_node1_block<D, ONE, false>(p, sc, b, lane, beta, k, sum);
-        if (ONE) wsum += sum;
-        else if (lane == 0) p.bsq[b] = sum;
-    }
-    if (ONE) wg_partials_store(p.bsq, nullptr, wsum, 0.0);
+
+// alpha = rho_k / s.q
+__device__ inline double cg_alpha(double rho, double sq) { return sq != 0.0 ? rho / sq : (double)FLT_MAX; }
+__device__ inline void cg_record_alpha(CGState& cg, double sq, double alpha) {
+    cg.sq = sq;
+    cg.alpha = alpha;
+    cg.multiplies += 1;
 }
 
-// x += alpha s, r -= alpha q on block b; its r.r and max |r|^2.
-template <int D, bool AGENT>
-__device__ inline void cg_node2_block(const KP& p, int b, int lane, float alpha, double& sum, double& mx) {
-    const int n = b * 64 + lane;
-    sum = 0.0;
-    mx = 0.0;
-    if ((p.g_flags[n] & MPM_FLAG_INTERIOR_DEV) != 0) {
-        const double m = (double)p.g_m[n];
-#pragma unroll
-        for (int a = 0; a < D; ++a) {
-            const float sv = ld<AGENT>(p.g_s + a * p.gcap + n), q = p.g_q[a * p.gcap + n], xv = p.g_vs[a * p.gcap + n];
-            p.g_vs[a * p.gcap + n] = alpha * sv + xv;
-            const float rv = -alpha * q + ld<AGENT>(p.g_r + a * p.gcap + n);
-            st<AGENT>(p.g_r + a * p.gcap + n, rv);
-            sum += (double)rv * ((double)rv * m);
-            mx += (double)rv * (double)rv;
-        }
+// ---- the node pass -----------------------------------------------------------
+// Everything of an iteration but the operator, in one launch: q = A s and s.q;
+// alpha, x and r, r.r; the convergence test, beta and s.  Its work-groups
+// exchange the two sums inside the launch.
+//
+// Groups of NGB consecutive blocks, a wave each.  A run is the part of one
+// scene's blocks in one group: its partial is the sum over them in block
+// order, formed and read by the wave of its first block.  A partial's place is
+// its own flag: it holds CG_EMPTY until the partial is there, the operator
+// launch before empties it.  A scene of many runs is summed in chunks first, by
+// the wave of a chunk's first run: everybody reading everybody's partials was
+// most of the pass (420 work-groups: 3 and 5 us for the two sums).  The order
+// of every sum is fixed, so the result depends neither on the grid nor on who
+// computes a group.
+//
+// Work-groups wait for one another, so all that take part have to be running.
+// Each takes a ticket at its XCD's door when it starts.  Before anything is
+// changed that the pass reads, every one waits until all tickets are out; one
+// that has waited for too long while some are missing closes the doors.  Then
+// those that hold a ticket wait for one another, share all groups by ticket and
+// start again (the partials that are there already are the same), and those
+// that come later leave.  (A door is one word: tickets taken, and once it is
+// closed a bit and how many had been taken by then.  The first door to close
+// does so while one of its tickets is missing, so that nobody ever sees all of
+// them taken; the others follow.)
+//
+// Bound by latency: the gather of the tiles (2.4 to 3.5 us), two sums that each
+// take two or three memory round trips, the start and end of a launch.  Per
+// iteration, against three launches for one scene (s; q and s.q; x, r and r.r,
+// each reducing the partials of the one before) and four for a batch: avalanche
+// of 1.0M particles (3,360 blocks) 18.6 -> 17.0 us, of 2.0M (6,500) 24.1 ->
+// 22.2, two balls of 243k (1,100) 14.1 -> 10.9, twelve scenes (2,000 blocks)
+// 18.9 -> 13.4; and a captured substep holds half the launches.  Work-groups
+// of 256 threads take 18.0, of 1024 15.9 us on the first, 11.4 and 12.9 on the
+// third.
+// Waits until the doors are settled: 0 if all have come that own groups of the
+// ng, else the number of those that have, all of them here now, and `rank`
+// among them of the one with `ticket`.  (One wave.)
+__device__ inline int cg_settle(const KP& p, int ng, long long t0, int ticket, int lane, int& rank) {
+    int* const word = p.ctr->doors[lane & 7];
+    const auto close = [&](int v) {
+        return __hip_atomic_compare_exchange_strong(word, &v, v | v << 16 | CG_DOOR_CLOSED, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                    __HIP_MEMORY_SCOPE_AGENT);
+    };
+    const int x = lane & 7;
+    const int most = min((int)(gridDim.x >> 3), (int)(((int64_t)ng * (x + 1)) >> 3) - (int)(((int64_t)ng * x) >> 3));
+    int v;
+    for (;;) {
+        v = ld_agent(word);
+        if (__any(v >= CG_DOOR_CLOSED)) break;
+        const unsigned long long missing = __ballot(v < most);
+        if (missing == 0) return 0;
+        if (wall_clock64() - t0 >= p.door_ticks && __any(lane == __ffsll(missing) - 1 && close(v))) break;
+        __builtin_amdgcn_s_sleep(1);
     }
-    wave_reduce2(sum, mx);
+    while ((v = ld_agent(word)) < CG_DOOR_CLOSED)
+        if (lane < 8) (void)close(v);
+    const int taken = (v & ~CG_DOOR_CLOSED) >> 16;
+    int group = 0;
+    rank = ticket;
+#pragma unroll
+    for (int y = 0; y < 8; ++y) {
+        const int t = __shfl(taken, y);
+        if (y < (int)(blockIdx.x & 7)) rank += t;
+        group += t;
+    }
+    if (lane == 0) {
+        add_agent(&p.ctr->again, 1);
+        while (ld_agent(&p.ctr->again) < group) __builtin_amdgcn_s_sleep(1);
+    }
+    return group;
 }
 
-// alpha = rho_k / s.q;  x += alpha s, r -= alpha q; partials of r.r and
-// max |r|^2.  One scene: every work-group reduces the s.q partials itself
-// (work-group 0 records alpha); batches read alpha from k_cg_reduce_sq.
-template <int D, bool ONE>
-__global__ __launch_bounds__(WG) void k_cg_node2(KP p, int k, int nparts) {
-    const XcdRange r = xcd_wave_blocks(p.ctr->nblocks);
-    const int lane = threadIdx.x & 63;
-    // one scene: the wave's first block's node values load while the s.q
-    // partials are reduced
-    float pre_s[D], pre_q[D], pre_x[D], pre_r[D], pre_m = 0.0f;
-    unsigned pre_flags = 0u;
-    if (ONE && r.first < r.end) {
-        const int n = r.first * 64 + lane;
-        pre_flags = p.g_flags[n];
-        pre_m = p.g_m[n];
+// A partial, W = 1 or 2 values: sums are added, the second is a maximum.
+template <int W>
+__device__ inline void put_values(double* at, const double* v) {
 #pragma unroll
-        for (int a = 0; a < D; ++a) {
-            pre_s[a] = p.g_s[a * p.gcap + n];
-            pre_q[a] = p.g_q[a * p.gcap + n];
-            pre_x[a] = p.g_vs[a * p.gcap + n];
-            pre_r[a] = p.g_r[a * p.gcap + n];
+    for (int w = 0; w < W; ++w) put_partial(at + w, v[w]);
+}
+// Waits for `count` partials, the i-th at(i), and reduces them; one wave, result
+// in every lane.  `late` is asked while it waits: nonzero ends the wait and is
+// returned.
+template <int W, int U, class At, class F>
+__device__ inline int await_values(At&& at, int count, int lane, double* v, F&& late) {
+#pragma unroll
+    for (int w = 0; w < W; ++w) v[w] = 0.0;
+    for (int base = 0; base < count; base += U * 64) {
+        double u[U][W];
+#pragma unroll
+        for (int j = 0; j < U; ++j)
+#pragma unroll
+            for (int w = 0; w < W; ++w)
+                u[j][w] = base + j * 64 + lane < count ? __longlong_as_double((long long)CG_EMPTY) : 0.0;
+        for (;;) {
+            bool waiting = false;
+#pragma unroll
+            for (int j = 0; j < U; ++j) {
+                if (base + j * 64 >= count) break;
+                const double* from = at(base + j * 64 + lane);
+#pragma unroll
+                for (int w = 0; w < W; ++w)
+                    if ((unsigned long long)__double_as_longlong(u[j][w]) == CG_EMPTY) u[j][w] = ld_agent(from + w);
+            }
+#pragma unroll
+            for (int j = 0; j < U; ++j)
+#pragma unroll
+                for (int w = 0; w < W; ++w) waiting |= (unsigned long long)__double_as_longlong(u[j][w]) == CG_EMPTY;
+            if (!__any(waiting)) break;
+            if (const int group = late()) return group;
+        }
+#pragma unroll
+        for (int j = 0; j < U; ++j) {
+            v[0] += u[j][0];
+            if (W > 1) v[W - 1] = fmax(v[W - 1], u[j][W - 1]);
         }
     }
-    if (cg_all_done(p)) return;
-    float alpha1 = 0.0f;
-    if (ONE) {
-        // the scene's done flag and rho load alongside the partials (a
-        // finished solve writes nothing)
-        CGState& cg = p.cg[p.solo];
-        const bool stop = cg.done != 0;
-        const double rho = cg.rho_hist[k & 1];
-        double sq, unused;
-        reduce_range(p.bsq, nullptr, 0, nparts, sq, unused);
-        if (stop) return;
-        const double alpha_d = sq != 0.0 ? rho / sq : (double)FLT_MAX;
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
-            cg.sq = sq;
-            cg.alpha = alpha_d;
-            cg.multiplies += 1;
+    double mx = W > 1 ? v[W - 1] : 0.0;
+    wave_reduce2(v[0], mx);
+    if (W > 1) v[W - 1] = mx;
+    return 0;
+}
+
+template <int D, bool RESTART>
+__global__ __launch_bounds__(NGW, 6) void k_cg_node(KP p, int k) {
+    __shared__ double ws[NGB], wm[NGB];  // a block's partials
+    __shared__ float sh_alpha[NGB], sh_beta[NGB];
+    __shared__ int sh_fin[NGB], sh_ticket, sh_group, sh_rank;
+    if (p.ctr->live == 0) return;
+    const long long t0 = wall_clock64();
+    const int n = p.ctr->nblocks, ng = cg_groups(n), cp = cg_chunk_places(ng);
+    const XcdRange xr = xcd_blocks(ng);
+    if (xr.first >= xr.end) return;
+    int ticket = 0;
+    if (threadIdx.x == 0) ticket = add_agent(p.ctr->doors[blockIdx.x & 7], 1);
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const bool batch = p.nscenes > 1;
+    // the wave's block in group g (b < 0: none), its scene's blocks [b0, b1),
+    // its run's first wave and number, its scene's number of runs
+    int b, si, b0, b1, head, run, runs;
+    const auto take = [&](int g) {
+        b = g * NGB + wv;
+        si = 0;
+        b0 = 0;
+        b1 = n;
+        if (b < n && batch) {
+            si = p.block_scene[b];
+            b0 = p.sst[si].block_begin;
+            b1 = p.sst[si].block_end;
         }
-        alpha1 = (float)alpha_d;
+        if (b >= n || p.cg[si].closed) b = -1;
+        head = max(b0 - g * NGB, 0);
+        run = g - b0 / NGB;
+        runs = (b1 - 1) / NGB - b0 / NGB + 1;
+    };
+    const auto place = [&](int i) { return i == 0 ? ng + si : b0 / NGB + i; };
+    const auto chunk_place = [&](int c) { return b0 / NGB / (CG_CHUNK_RUNS / 2) + c; };
+    // the run's partial, the chunk's sum (from the wave of the first run), and
+    // the scene's
+    const auto publish = [&](auto width, double* sums, int g) {
+        constexpr int W = decltype(width)::value;
+        const int len = min(b1, (g + 1) * NGB) - b;
+        double v[2] = {0.0, 0.0};
+        for (int w = 0; w < len; ++w) {
+            v[0] += ws[wv + w];
+            v[1] = fmax(v[1], wm[wv + w]);
+        }
+        if (lane == 0) put_values<W>(sums + W * place(run), v);
+    };
+    const auto lead = [&](auto width, const double* sums, double* chunks, auto&& late) {
+        constexpr int W = decltype(width)::value;
+        if (runs <= CG_DIRECT_RUNS || run % CG_CHUNK_RUNS != 0) return 0;
+        double c[W];
+        const int group = await_values<W, 1>([&](int i) { return sums + W * place(run + i); }, min(CG_CHUNK_RUNS, runs - run), lane,
+                                             c, late);
+        if (group == 0 && lane < 8) put_values<W>(chunks + W * (lane * cp + chunk_place(run / CG_CHUNK_RUNS)), c);
+        return group;
+    };
+    const auto total = [&](auto width, const double* sums, const double* chunks, double* t, auto&& late) {
+        constexpr int W = decltype(width)::value;
+        if (runs <= CG_DIRECT_RUNS)
+            return await_values<W, CG_DIRECT_RUNS / 64>([&](int i) { return sums + W * place(i); }, runs, lane, t, late);
+        const double* copy = chunks + W * (int)(blockIdx.x & 7) * cp;
+        return await_values<W, 1>([&](int i) { return copy + W * chunk_place(i); }, (runs + CG_CHUNK_RUNS - 1) / CG_CHUNK_RUNS, lane,
+                                  t, late);
+    };
+    using One = std::integral_constant<int, 1>;
+    using Two = std::integral_constant<int, 2>;
+    using First = std::integral_constant<int, RESTART ? 2 : 1>;  // the launch's first sum: s.q, at the restart r.r
+    double* const rr_chunks = p.bmax + 8 * cp;
+    double* const first_sums = RESTART ? p.bsum : p.bsq;
+    double* const first_chunks = RESTART ? rr_chunks : p.bmax;
+    const auto never = [] { return 0; };
+
+    int first = xr.first, step = xr.step, end = xr.end;
+    NodeRows<D, false> v;
+    double t[2];  // the scene's sum (a run's first wave)
+    for (bool settled = false;; settled = true) {
+        // q and s.q (restart: r, kept in g_s, and r.r)
+        for (int g = first; g < end; g += step) {
+            take(g);
+            if (b >= 0) {
+                const SceneParams& sc = p.scn[si];
+                double sum, mx = 0.0;
+                if (RESTART) cg_restart_block<D, false, true>(p, sc, b, lane, sum, mx);
+                else cg_product_block<D, false, false>(p, sc, b, lane, 0.0f, k, sum);
+                if (lane == 0) {
+                    ws[wv] = sum;
+                    wm[wv] = mx;
+                }
+            }
+            if (threadIdx.x == 0) {
+                sh_ticket = ticket;
+                sh_group = 0;
+            }
+            __syncthreads();
+            if (sh_ticket >= CG_DOOR_CLOSED) return;
+            if (b >= 0 && wv == head) publish(First{}, first_sums, g);
+            __syncthreads();
+        }
+        // The sum of one scene is complete only if everybody has come: it
+        // settles the doors by itself, and they are looked at when it is late.
+        // In a batch the last wave settles them while the sums are awaited.
+        const auto settle = [&] {
+            int rank;
+            const int group = cg_settle(p, ng, t0, sh_ticket, lane, rank);
+            if (group != 0 && lane == 0) {
+                sh_rank = rank;
+                __hip_atomic_store(&sh_group, group, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            }
+            return group;
+        };
+        const auto late = [&] {
+            if (settled) return 0;
+            if (batch) return __hip_atomic_load(&sh_group, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            return wall_clock64() - t0 < p.door_ticks ? 0 : settle();
+        };
+        int group = batch && !settled && wv == NGB - 1 ? settle() : 0;
+        for (int g = first; g < end && group == 0; g += step) {
+            if (first + step < end) take(g);
+            if (b >= 0 && wv == head) group = lead(First{}, first_sums, first_chunks, late);
+        }
+        if (first + step < end) take(first);
+        if (b >= 0) {
+            v.load(p, b * 64 + lane);
+            if (wv == head && group == 0) (void)total(First{}, first_sums, first_chunks, t, late);
+        }
+        __syncthreads();
+        if (sh_group == 0) break;
+        first = sh_rank;
+        step = sh_group;
+        end = ng;
+        __syncthreads();
     }
-    double wsum = 0.0, wmx = 0.0;
-    for (int b = r.first; b < r.end; b += r.step) {
-        if (ONE && other_scene(p, b)) continue;
-        const int si = ONE ? p.solo : p.block_scene[b];
-        const SceneParams& sc = p.scn[si];
-        if (!sc.active || (!ONE && p.cg[si].done)) continue;
-        const float alpha = ONE ? alpha1 : (float)p.cg[si].alpha;
-        const int n = b * 64 + lane;
-        const bool pre = ONE && b == r.first;
-        const bool interior = ((pre ? pre_flags : p.g_flags[n]) & MPM_FLAG_INTERIOR_DEV) != 0;
-        double sum = 0.0, mx = 0.0;
-        if (interior) {
-            const double m = (double)(pre ? pre_m : p.g_m[n]);
-#pragma unroll
-            for (int a = 0; a < D; ++a) {
-                const float sv = pre ? pre_s[a] : p.g_s[a * p.gcap + n];
-                const float q = pre ? pre_q[a] : p.g_q[a * p.gcap + n];
-                const float xv = pre ? pre_x[a] : p.g_vs[a * p.gcap + n];
-                p.g_vs[a * p.gcap + n] = alpha * sv + xv;
-                const float rv = -alpha * q + (pre ? pre_r[a] : p.g_r[a * p.gcap + n]);
-                p.g_r[a * p.gcap + n] = rv;
-                sum += (double)rv * ((double)rv * m);
-                mx += (double)rv * (double)rv;
+    const bool several = first + step < end;
+    if (!RESTART) {
+        // alpha, x and r, r.r
+        for (int g = first; g < end; g += step) {
+            if (g != first) {
+                take(g);
+                if (b >= 0) {
+                    v.load(p, b * 64 + lane);
+                    if (wv == head) (void)total(One{}, p.bsq, p.bmax, t, never);
+                }
+            }
+            if (b >= 0 && wv == head && lane == 0) {
+                const double alpha = cg_alpha(p.cg[si].rho_hist[k & 1], t[0]);
+                if (b == b0) cg_record_alpha(p.cg[si], t[0], alpha);
+                sh_alpha[wv] = (float)alpha;
+            }
+            __syncthreads();
+            if (b >= 0) {
+                double sum, mx;
+                v.step(p, b * 64 + lane, sh_alpha[head], sum, mx);
+                if (lane == 0) {
+                    ws[wv] = sum;
+                    wm[wv] = mx;
+                }
+            }
+            __syncthreads();
+            if (b >= 0 && wv == head) publish(Two{}, p.bsum, g);
+        }
+        for (int g = first; g < end; g += step) {
+            if (several) take(g);
+            if (b >= 0 && wv == head) (void)lead(Two{}, p.bsum, rr_chunks, never);
+        }
+    }
+    // convergence test of the next iteration, beta and s
+    const int kn = RESTART ? 0 : k + 1;
+    for (int g = first; g < end; g += step) {
+        if (several) {
+            take(g);
+            if (b >= 0) v.load(p, b * 64 + lane);
+        }
+        if (b >= 0 && wv == head) {
+            const CGTestIn in = cg_test_in(p, si, kn);
+            if (!RESTART || g != first) (void)total(Two{}, p.bsum, rr_chunks, t, never);
+            float beta;
+            const bool fin = cg_test(p, si, kn, t[0], t[1], b == b0 && lane == 0, beta, in);
+            if (lane == 0) {
+                sh_beta[wv] = beta;
+                sh_fin[wv] = fin ? 1 : 0;
             }
         }
-        wave_reduce2(sum, mx);
-        if (ONE) {
-            wsum += sum;
-            wmx = fmax(wmx, mx);
-        } else if (lane == 0) {
-            p.bsum[b] = sum;
-            p.bmax[b] = mx;
+        __syncthreads();
+        if (b >= 0 && RESTART) {
+#pragma unroll
+            for (int a = 0; a < D; ++a) p.g_r[a * p.gcap + b * 64 + lane] = v.s[a];
+        } else if (b >= 0 && !sh_fin[head] && v.interior) {
+#pragma unroll
+            for (int a = 0; a < D; ++a)
+                p.g_s[a * p.gcap + b * 64 + lane] = cg_direction(v.r[a], v.s[a], sh_beta[head], kn);
         }
+        if (several) __syncthreads();
     }
-    if (ONE) wg_partials_store(p.bsum, p.bmax, wsum, wmx);
 }
 
-// Batches: alpha = rho_k / s.q for every scene still iterating (one
-// work-group per scene over the scene's block partials)
 // The CG's done poll: the eight ints from Counters::nblocks to cg_iters into
 // the host's pinned poll slot.
 __global__ __launch_bounds__(64) void k_poll(KP p, int* dst) {
     const int t = (int)threadIdx.x;
     if (t < 8) dst[t] = (&p.ctr->nblocks)[t];
-}
-
-__global__ __launch_bounds__(WG) void k_cg_reduce_sq(KP p, int k) {
-    const int si = blockIdx.x;
-    CGState& cg = p.cg[si];
-    if (cg.done) return;
-    const int b0 = p.sst[si].block_begin, b1 = p.sst[si].block_end;
-    double sq, unused;
-    reduce_range(p.bsq, nullptr, b0, b1 - b0, sq, unused);
-    if (threadIdx.x == 0) {
-        cg.sq = sq;
-        cg.alpha = sq != 0.0 ? cg.rho_hist[k & 1] / sq : (double)FLT_MAX;
-        cg.multiplies += 1;
-    }
-}
-
-// Batches: convergence test of iteration k and beta per scene
-__global__ __launch_bounds__(WG) void k_cg_reduce_rr(KP p, int k) {
-    const int si = blockIdx.x;
-    if (p.cg[si].done) return;
-    const int b0 = p.sst[si].block_begin, b1 = p.sst[si].block_end;
-    const CGTestIn tin = cg_test_in(p, si, k);
-    double rr, mx;
-    reduce_range(p.bsum, p.bmax, b0, b1 - b0, rr, mx);
-    float beta;
-    (void)cg_test(p, si, k, rr, mx, threadIdx.x == 0, beta, tin);
 }
 
 // ============================================================================
@@ -2543,9 +2715,6 @@ __global__ __launch_bounds__(WG) void k_cg_reduce_rr(KP p, int k) {
 // about 30 and, in a captured substep, the launches of all iterations up to
 // the cap.
 // ============================================================================
-constexpr int CG_DOOR_CLOSED = 1 << 30;
-constexpr long long CG_DOOR_TICKS = 2000;  // of the 100 MHz clock
-
 // The work-group's rank among those inside and their number (at most `most`
 // come), false if the door is closed.
 __device__ inline bool cg_enter(const KP& p, int most, int& rank, int& group) {
@@ -2555,7 +2724,7 @@ __device__ inline bool cg_enter(const KP& p, int most, int& rank, int& group) {
         int g = 0;
         if (ticket == 0) {
             const long long t0 = wall_clock64();
-            while (ld_agent(&p.ctr->door) < most && wall_clock64() - t0 < CG_DOOR_TICKS) __builtin_amdgcn_s_sleep(1);
+            while (ld_agent(&p.ctr->door) < most && wall_clock64() - t0 < p.door_ticks) __builtin_amdgcn_s_sleep(1);
             g = __hip_atomic_fetch_or(&p.ctr->door, CG_DOOR_CLOSED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             st_agent(&p.ctr->group, g);
         } else if (ticket < CG_DOOR_CLOSED) {
@@ -2577,15 +2746,6 @@ __device__ inline int opaque(int v) {
     return v;
 }
 
-// Every store of this wave has reached memory.
-__device__ inline void drain_stores() { __asm__ __volatile__("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory"); }
-
-// ---- a partial that is its own flag -----------------------------------------
-__device__ inline void put_partial(double* a, double v) {
-    if (!(v == v)) v = __longlong_as_double(0x7ff8000000000000ll);
-    st_agent(a, v);
-}
-__device__ inline void clear_partial(double* a) { st_agent(a, __longlong_as_double((long long)CG_EMPTY)); }
 // Waits for the count (<= MOST) partials at sums (and maxs), and sums (takes
 // the largest of) them in a fixed order; one wave, result in every lane.
 template <int MOST>
@@ -2882,7 +3042,7 @@ __device__ inline void cg_solve_shared(const KP& p, int w0, int w1, int n, int g
                 const int b0 = p.sst[si].block_begin, b1 = p.sst[si].block_end;
                 const CGTestIn in = cg_test_in(p, si, k);
                 double rr, mx;
-                reduce_range<true, CGW>(p.bsum, p.bmax, b0, b1 - b0, rr, mx);
+                reduce_range<CGW>(p.bsum, p.bmax, b0, b1 - b0, rr, mx);
                 if (cg_test(p, si, k, rr, mx, b == b0 && threadIdx.x == 0, beta, in)) {
                     done |= 1ull << r;
                     return;
@@ -2901,7 +3061,7 @@ __device__ inline void cg_solve_shared(const KP& p, int w0, int w1, int n, int g
                 if ((done >> r) & 1) return;
                 for (b += wv; b < e; b += CGW / 64) {
                     double sum, mx;
-                    cg_restart_block<D, true>(p, p.scn[si], b, lane, sum, mx);
+                    cg_restart_block<D, true, false>(p, p.scn[si], b, lane, sum, mx);
                     if (lane == 0) {
                         st_agent(p.bsum + b, sum);
                         st_agent(p.bmax + b, mx);
@@ -2919,7 +3079,7 @@ __device__ inline void cg_solve_shared(const KP& p, int w0, int w1, int n, int g
             const float beta = (float)ld_agent(&p.cg[si].beta);
             for (b += wv; b < e; b += CGW / 64) {
                 double sum;
-                cg_node1_block<D, false, true>(p, p.scn[si], b, lane, beta, k, sum);
+                cg_product_block<D, true, true>(p, p.scn[si], b, lane, beta, k, sum);
                 if (lane == 0) st_agent(p.bsq + b, sum);
             }
         });
@@ -2930,7 +3090,7 @@ __device__ inline void cg_solve_shared(const KP& p, int w0, int w1, int n, int g
             const int b0 = p.sst[si].block_begin, b1 = p.sst[si].block_end;
             const double rho = ld_agent(&p.cg[si].rho_hist[k & 1]);
             double sq, unused;
-            reduce_range<true, CGW>(p.bsq, nullptr, b0, b1 - b0, sq, unused);
+            reduce_range<CGW>(p.bsq, nullptr, b0, b1 - b0, sq, unused);
             const double alpha = sq != 0.0 ? rho / sq : (double)FLT_MAX;
             if (b == b0 && threadIdx.x == 0) {
                 CGState& cg = p.cg[si];
@@ -2940,7 +3100,9 @@ __device__ inline void cg_solve_shared(const KP& p, int w0, int w1, int n, int g
             }
             for (b += wv; b < e; b += CGW / 64) {
                 double sum, mx;
-                cg_node2_block<D, true>(p, b, lane, (float)alpha, sum, mx);
+                NodeRows<D, true> v;
+                v.load(p, b * 64 + lane);
+                v.step(p, b * 64 + lane, (float)alpha, sum, mx);
                 if (lane == 0) {
                     st_agent(p.bsum + b, sum);
                     st_agent(p.bmax + b, mx);
@@ -2959,14 +3121,6 @@ template <int D>
 __global__ __launch_bounds__(CGW, 4) void k_cg_solve(KP p) {
     __shared__ __align__(16) OperatorLds<D, CGW> S;
     const int n = p.ctr->nblocks, bid = (int)blockIdx.x;
-    if (bid == 0) {
-        // scenes without blocks or at rest are done at once
-        for (int si = threadIdx.x; si < p.nscenes; si += CGW) {
-            const CGTestIn in = cg_test_in(p, si, 0);
-            float beta;
-            if (in.empty) (void)cg_test(p, si, 0, 0.0, 0.0, true, beta, in);
-        }
-    }
     const bool pairs = n > CG_GROUPS && n <= CG_RESIDENT;
     int blk0 = bid, blk1 = -1, most = min(n, CG_GROUPS);
     bool mine = bid < most;
@@ -3570,31 +3724,18 @@ template <int D> void launch_grid_update(const KP& p, hipStream_t s, int grid, b
     else if (!force && !collision && cg_init) hipLaunchKernelGGL((k_grid_update<D, false, false, true, false>), dim3(grid), dim3(WG), 0, s, p);
     else hipLaunchKernelGGL((k_grid_update<D, true, true, true, false>), dim3(grid), dim3(WG), 0, s, p);
 }
-template <int D> void launch_cg_force(const KP& p, hipStream_t s, int grid, bool restart, int k, bool one) {
-    if (restart) hipLaunchKernelGGL((k_cg_force<D, true, false>), dim3(grid), dim3(BWG), 0, s, p, 0);
-    else if (one) hipLaunchKernelGGL((k_cg_force<D, false, true>), dim3(grid), dim3(BWG), 0, s, p, k);
-    else hipLaunchKernelGGL((k_cg_force<D, false, false>), dim3(grid), dim3(BWG), 0, s, p, k);
+template <int D> void launch_cg_force(const KP& p, hipStream_t s, int grid, bool restart) {
+    if (restart) hipLaunchKernelGGL((k_cg_force<D, true>), dim3(grid), dim3(BWG), 0, s, p);
+    else hipLaunchKernelGGL((k_cg_force<D, false>), dim3(grid), dim3(BWG), 0, s, p);
+}
+template <int D> void launch_cg_node(const KP& p, hipStream_t s, int blocks, int k, bool restart) {
+    const int grid = std::min(CG_NODE_GROUPS, ((blocks + NGB - 1) / NGB + 7) / 8 * 8);
+    if (restart) hipLaunchKernelGGL((k_cg_node<D, true>), dim3(grid), dim3(NGW), 0, s, p, 0);
+    else hipLaunchKernelGGL((k_cg_node<D, false>), dim3(grid), dim3(NGW), 0, s, p, k);
 }
 template <int D> void launch_cg_solve(const KP& p, hipStream_t s) {
     hipLaunchKernelGGL((k_cg_solve<D>), dim3(CG_GROUPS), dim3(CGW), 0, s, p);
 }
-template <int D> void launch_cg_restart_node(const KP& p, hipStream_t s, int grid, bool one) {
-    if (one) hipLaunchKernelGGL((k_cg_restart_node<D, true>), dim3(grid), dim3(WG), 0, s, p);
-    else hipLaunchKernelGGL((k_cg_restart_node<D, false>), dim3(grid), dim3(WG), 0, s, p);
-}
-template <int D> void launch_cg_update_s(const KP& p, hipStream_t s, int grid, int k) {
-    hipLaunchKernelGGL(k_cg_update_s<D>, dim3(grid), dim3(WG), 0, s, p, k, grid);
-}
-template <int D> void launch_cg_node1(const KP& p, hipStream_t s, int grid, int k, bool one) {
-    if (one) hipLaunchKernelGGL((k_cg_node1<D, true>), dim3(grid), dim3(WG), 0, s, p, k);
-    else hipLaunchKernelGGL((k_cg_node1<D, false>), dim3(grid), dim3(WG), 0, s, p, k);
-}
-template <int D> void launch_cg_node2(const KP& p, hipStream_t s, int grid, int k, bool one) {
-    if (one) hipLaunchKernelGGL((k_cg_node2<D, true>), dim3(grid), dim3(WG), 0, s, p, k, grid);
-    else hipLaunchKernelGGL((k_cg_node2<D, false>), dim3(grid), dim3(WG), 0, s, p, k, grid);
-}
-void launch_cg_reduce_sq(const KP& p, hipStream_t s, int k) { hipLaunchKernelGGL(k_cg_reduce_sq, dim3(p.nscenes), dim3(WG), 0, s, p, k); }
-void launch_cg_reduce_rr(const KP& p, hipStream_t s, int k) { hipLaunchKernelGGL(k_cg_reduce_rr, dim3(p.nscenes), dim3(WG), 0, s, p, k); }
 template <int D> void launch_g2p(const KP& p, hipStream_t s, int grid) {
     hipLaunchKernelGGL(k_g2p<D>, dim3(grid), dim3(BWG), 0, s, p);
     hipLaunchKernelGGL(k_g2p_reduce, dim3(p.nscenes), dim3(WG), 0, s, p);
@@ -3610,12 +3751,9 @@ template <int D> void launch_max_speed(const KP& p, hipStream_t s, int grid) { h
     template void launch_init_volume<D>(const KP&, hipStream_t, int);                         \
     template void launch_particle_force<D>(const KP&, hipStream_t, int, bool, bool);          \
     template void launch_grid_update<D>(const KP&, hipStream_t, int, bool, bool, bool, bool); \
-    template void launch_cg_force<D>(const KP&, hipStream_t, int, bool, int, bool);           \
+    template void launch_cg_force<D>(const KP&, hipStream_t, int, bool);                      \
+    template void launch_cg_node<D>(const KP&, hipStream_t, int, int, bool);                  \
     template void launch_cg_solve<D>(const KP&, hipStream_t);                                 \
-    template void launch_cg_restart_node<D>(const KP&, hipStream_t, int, bool);               \
-    template void launch_cg_update_s<D>(const KP&, hipStream_t, int, int);                    \
-    template void launch_cg_node1<D>(const KP&, hipStream_t, int, int, bool);                 \
-    template void launch_cg_node2<D>(const KP&, hipStream_t, int, int, bool);                 \
     template void launch_g2p<D>(const KP&, hipStream_t, int);                                 \
     template void launch_max_speed<D>(const KP&, hipStream_t, int);
 MPM_INSTANTIATE(2)

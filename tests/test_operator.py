@@ -94,3 +94,59 @@ def test_solve_by_number_of_blocks(scenes, n, blocks, graph):
         for f in ("x", "v", "F", "Jp"):
             assert rel(got[f], want[f]) < 1e-5, (k, f)
     b.close()
+
+
+def scattered(dim, counts, n, seed, lo=0.15, hi=0.85):
+    r = np.random.default_rng(seed)
+    name = "disk2d" if dim == 2 else "two_balls"
+    d, _, _, _ = M.scene_generate(name, counts, 0)
+    d.cg_max_iterations = 30
+    x = r.uniform(lo, hi, (n, dim)).astype(np.float32)
+    v = ((x - 0.5) @ r.uniform(-1.0, 1.0, (dim, dim)) + 0.5).astype(np.float32)
+    return d, x, v, np.full(n, 400.0 / counts ** dim / 8, np.float32)
+
+
+# (dimension, cells, particles and part of the domain of each scene, graph): a few
+# groups of blocks; more than 192 of them; more than the launch has
+# work-groups; the same in 2D; scenes that share groups, one of them with few blocks
+@pytest.mark.parametrize("dim,counts,scenes,graph", [
+    (3, 64, [(66000, 0.4, 0.6)], False),
+    (3, 128, [(66000, 0.35, 0.65)], True),
+    (3, 128, [(66000, 0.2, 0.8)], False),
+    (2, 512, [(66000, 0.05, 0.95)], False),
+    (3, 64, [(500, 0.4, 0.6), (66000, 0.2, 0.8), (300, 0.45, 0.5)], False),
+    (3, 64, [(500, 0.4, 0.6), (66000, 0.2, 0.8), (300, 0.45, 0.5)], True),
+])
+def test_node_pass_work_groups(dim, counts, scenes, graph):
+    """The node pass of launched solves (over 65,536 particles): one substep
+    against the oracle, and two bit for bit the same with a wait limit of zero,
+    where those that happen to run share the groups."""
+    parts = [scattered(dim, counts, n, 40 + k, lo, hi) for k, (n, lo, hi) in enumerate(scenes)]
+    dt = 0.5 * float(parts[0][0].max_dt)
+    got = []
+    for limit in (None, 0):
+        b = M.Batch([q[0] for q in parts], [3 * len(q[1]) for q in parts])  # (a block per 16 places)
+        if limit is not None:
+            b.set_wait_limit(limit)
+        for k, (_, x, v, m) in enumerate(parts):
+            b.upload(k, x, v, m)
+        b.initialize()
+        b.use_graph(graph)
+        b.substep(dt)
+        once = [b.download(k) for k in range(len(parts))]
+        b.substep(dt)
+        got.append([(b.download(k), b.stats(k)) for k in range(len(parts))])
+        b.close()
+    for k, (d, x, v, m) in enumerate(parts):
+        (a, sa), (c, sc) = got[0][k], got[1][k]
+        assert sa["cg_iterations"] == sc["cg_iterations"] and sa["cg_multiplies"] == sc["cg_multiplies"]
+        for f in ("x", "v", "F", "Jp", "ids"):
+            assert np.array_equal(a[f], c[f]), f
+        o = O.Oracle(d, 8, 4, O.DOT_FP64 | O.SVD_FP64)
+        o.set_particles(x, v, m)
+        o.initialize()
+        o.advance_step(dt)
+        want = o.particles()
+        assert np.array_equal(once[k]["ids"], want["ids"])
+        for f in ("x", "v", "F", "Jp"):
+            assert rel(once[k][f], want[f]) < 1e-5, (k, f)
