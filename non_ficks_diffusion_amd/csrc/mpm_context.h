@@ -64,7 +64,9 @@ struct mpm_context {
     double *bsum = nullptr, *bmax = nullptr, *bsq = nullptr;
     unsigned* bu = nullptr;
     int cg_predict = 0;    // the next solve's first launch batch: the last solve's iterations plus one
-    int* h_done = nullptr;  // pinned: per poll slot (8 ints), Counters::overflow .. cg_iters
+    // pinned: per poll slot (8 ints) Counters::nblocks .. cg_iters; then the
+    // overflow flag and every scene's max |V|^2 (max_velocities)
+    int* h_done = nullptr;
     int* d_done = nullptr;  // the device's address of h_done
     bool overflow_seen = false;  // the last substep's poll saw a block-capacity overflow
     hipEvent_t done_ev[2] = {nullptr, nullptr};

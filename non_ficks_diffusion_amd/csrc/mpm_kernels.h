@@ -211,6 +211,7 @@ template <int D> void launch_block_setup(const KP& p, hipStream_t s, int grid);
 // block order, scene ranges and the in-cell order scatter (cell_groups work-groups)
 void launch_setup_order(const KP& p, hipStream_t s, int cell_groups);
 void launch_poll(const KP& p, hipStream_t s, int* dst);
+void launch_read_speeds(const KP& p, hipStream_t s, int* dst);
 int pack_tiles(int64_t nid);
 void launch_pack_count(const KP& p, hipStream_t s, const PackArgs& a);  // fills inv and part
 template <int D> void launch_pack_write(const KP& p, hipStream_t s, const PackArgs& a);

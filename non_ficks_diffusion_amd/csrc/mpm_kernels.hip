@@ -2682,6 +2682,13 @@ __global__ __launch_bounds__(64) void k_poll(KP p, int* dst) {
     if (t < 8) dst[t] = (&p.ctr->nblocks)[t];
 }
 
+// The overflow flag and the bits of every scene's max |V|^2, likewise: the
+// host's dt rule reads them after every substep of a launched frame.
+__global__ __launch_bounds__(WG) void k_read_speeds(KP p, int* dst) {
+    if (threadIdx.x == 0) dst[0] = p.ctr->overflow;
+    for (int s = (int)threadIdx.x; s < p.nscenes; s += WG) dst[1 + s] = (int)p.sst[s].max_v2;
+}
+
 // ============================================================================
 // The whole CG solve of every scene in one launch, for scenes too small to
 // fill the chip: there a launch's work is a few microseconds, and the four or
@@ -3706,6 +3713,7 @@ template <int D> void launch_pack_write(const KP& p, hipStream_t s, const PackAr
 }
 template void launch_pack_write<2>(const KP&, hipStream_t, const PackArgs&);
 template void launch_pack_write<3>(const KP&, hipStream_t, const PackArgs&);
+void launch_read_speeds(const KP& p, hipStream_t s, int* dst) { hipLaunchKernelGGL(k_read_speeds, dim3(1), dim3(WG), 0, s, p, dst); }
 void launch_poll(const KP& p, hipStream_t s, int* dst) { hipLaunchKernelGGL(k_poll, dim3(1), dim3(64), 0, s, p, dst); }
 template <int D> void launch_reorder(const KP& p, hipStream_t s, int grid) { hipLaunchKernelGGL(k_reorder<D>, dim3(grid), dim3(WG), 0, s, p); }
 template <int D> void launch_p2g(const KP& p, hipStream_t s, int grid) { hipLaunchKernelGGL(k_p2g<D>, dim3(grid), dim3(BWG), 0, s, p); }
