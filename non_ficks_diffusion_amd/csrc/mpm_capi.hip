@@ -161,6 +161,7 @@ mpm::KP make_kp(const mpm_context* c) {
     p.g_flags = c->g_flags;
     p.gcap = c->gcap;
     p.tiles = c->tiles;
+    p.cg_tiles = c->cg_tiles;
     p.ctr = c->ctr;
     p.bsum = c->bsum;
     p.bmax = c->bmax;
@@ -626,6 +627,7 @@ void layout_buffers(mpm_context* c, Take&& take) {
     take(&c->cell_count, nslots * 64);
     take(&c->cell_start, bcap * 65 + 1);
     take(&c->tiles, bcap * (D + 1) * (D == 3 ? 216 : 100));
+    take(&c->cg_tiles, 2 * std::min(bcap, (size_t)mpm::CG_RESIDENT) * D * (D == 3 ? 216 : 100));
     take(&c->scan_part, (size_t)2 * c->nparts);
     take(&c->g_m, gcap);
     take(&c->g_v, (size_t)D * gcap);
@@ -2336,7 +2338,7 @@ namespace {
 // runs the entry point holds its own copy until the process ends.  In host
 // code the array's name is a host-side stand-in and never a kernel argument:
 // its device address comes from hipGetSymbolAddress, once per device.
-constexpr size_t NOALLOC_SCRATCH_BYTES = (size_t)40 << 20;
+constexpr size_t NOALLOC_SCRATCH_BYTES = (size_t)46 << 20;
 static __device__ __align__(256) unsigned char scratch[NOALLOC_SCRATCH_BYTES];
 static_assert(MPM_NOALLOC_MAX_BLOCKS <= 2048 && MPM_NOALLOC_MAX_COUNTS <= 64 && MPM_NOALLOC_MAX_PARTICLES <= 65536,
               "the scratch size is computed for these limits");

@@ -141,6 +141,7 @@ struct KP {
     unsigned* g_flags;
     int64_t gcap;
     float* tiles;    // per active block, (D+1) * (B+2)^D floats
+    float* cg_tiles;  // k_cg_solve: per block and parity of the iteration, D * (B+2)^D floats
     // control
     Counters* ctr;
     // partials of the CG: k_cg_solve a place per active block (r.r, max |r|^2,

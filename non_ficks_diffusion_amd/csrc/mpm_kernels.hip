@@ -83,6 +83,16 @@ __device__ inline void st(T* a, T v) {
 // A place for a partial of k_cg_solve that has not been written: a NaN no
 // arithmetic yields.
 constexpr unsigned long long CG_EMPTY = 0x7ff8c0dec0dec0deull;
+// The same for a float that is its own flag; what is stored there goes through
+// `flagged`.
+constexpr unsigned CG_EMPTY_FLOAT = 0x7fc0dec0u;
+__device__ inline bool is_empty(float v) { return __float_as_uint(v) == CG_EMPTY_FLOAT; }
+__device__ inline float flagged(float v) { return v == v ? v : __uint_as_float(0x7fc00000u); }
+// k_cg_solve's force tile of block b in an iteration of parity k
+template <int D>
+__device__ inline float* cg_tile(const KP& p, int k, int b) {
+    return p.cg_tiles + ((int64_t)(k & 1) * min(p.bcap, CG_RESIDENT) + b) * (D * Dims<D>::TN);
+}
 
 // Active block b holds no particles (a halo block of its neighbours).
 __device__ inline bool block_empty(const KP& p, int b) { return p.block_pstart[b + 1] == p.block_pstart[b]; }
@@ -211,10 +221,12 @@ __device__ inline bool particle_weights(const KP& p, const SceneParams& sc, int 
 // zero) and are absent from the tile neighbour table.  With crop_ghost_x, nodes whose x index is outside [0, counts-1]
 // receive nothing (the reference's slab crop,
 // Tools/Cropped_Influence_Iterator.h:31-42).
-template <int D, int C, bool AGENT = false>
-__device__ inline void gather_node_tiles(const KP& p, const SceneParams& sc, int n, float* out) {
+// tile_of(o): entry o of that table for the node's block.  WAIT: the tiles
+// (k_cg_solve's) are written meanwhile, a value is there once it is not empty.
+template <int D, int C, bool AGENT, bool WAIT, class TileOf>
+__device__ inline void gather_tiles(const KP& p, const SceneParams& sc, int n, const float* tiles, TileOf&& tile_of, float* out) {
     using Dm = Dims<D>;
-    constexpr int B = Dm::B, TE = Dm::TE, TN = Dm::TN, NBR = Dm::NBR;
+    constexpr int B = Dm::B, TE = Dm::TE, TN = Dm::TN;
     const int b = n >> 6;
     int lc[D];
     local_coords<D>(n & 63, lc);
@@ -233,33 +245,44 @@ __device__ inline void gather_node_tiles(const KP& p, const SceneParams& sc, int
     // candidate m takes option 1 on the axes of its set bits, and the sum
     // runs over the candidates in lexicographic option order
     constexpr int NC = 1 << D;
-    const int* nbr = p.block_tnbr + (int64_t)b * NBR;
     int blk[NC];
 #pragma unroll
     for (int m = 0; m < NC; ++m) {
         int o = 0;
 #pragma unroll
         for (int a = 0; a < D; ++a) o = o * 3 + (((m >> (D - 1 - a)) & 1) ? od1[a] : 1);
-        const int e = nbr[o];  // o is an entry of the table whether or not it is used
+        const int e = tile_of(o);  // o is an entry of the table whether or not it is used
         blk[m] = (m & ~face) == 0 ? e : -1;
     }
     // a candidate on the node's faces loads even where its block wrote no
     // tile (from block 0's slot, in bounds, and not summed), so that no sum
     // shares its load's condition and none is scheduled ahead of the loads
     float v[NC][C];
+    bool waiting;
+    do {
 #pragma unroll
-    for (int m = 0; m < NC; ++m) {
-        int t = 0;
+        for (int m = 0; m < NC; ++m) {
+            int t = 0;
 #pragma unroll
-        for (int a = 0; a < D; ++a) t = t * TE + (((m >> (D - 1 - a)) & 1) ? td1[a] : td0[a]);
+            for (int a = 0; a < D; ++a) t = t * TE + (((m >> (D - 1 - a)) & 1) ? td1[a] : td0[a]);
 #pragma unroll
-        for (int c = 0; c < C; ++c) v[m][c] = 0.0f;
-        if ((m & ~face) == 0) {
-            const float* src = p.tiles + (int64_t)max(blk[m], 0) * C * TN + t;
+            for (int c = 0; c < C; ++c) v[m][c] = 0.0f;
+            if ((m & ~face) == 0) {
+                const float* src = tiles + (int64_t)max(blk[m], 0) * C * TN + t;
 #pragma unroll
-            for (int c = 0; c < C; ++c) v[m][c] = ld<AGENT>(src + c * TN);
+                for (int c = 0; c < C; ++c) v[m][c] = ld<AGENT>(src + c * TN);
+            }
         }
-    }
+        waiting = false;
+        if (WAIT) {
+#pragma unroll
+            for (int m = 0; m < NC; ++m)
+#pragma unroll
+                for (int c = 0; c < C; ++c) waiting |= blk[m] >= 0 && is_empty(v[m][c]);
+        }
+        // (a short rest: polling without one slowed the stores it waits for)
+        if (WAIT && __any(waiting)) __builtin_amdgcn_s_sleep(4);
+    } while (WAIT && __any(waiting));
     // the crop test's loads go out with the tile loads (a cropped node sums
     // nothing)
     bool keep = true;
@@ -278,6 +301,11 @@ __device__ inline void gather_node_tiles(const KP& p, const SceneParams& sc, int
 #pragma unroll
             for (int c = 0; c < C; ++c) out[c] += v[m][c];
         }
+}
+template <int D, int C, bool AGENT = false>
+__device__ inline void gather_node_tiles(const KP& p, const SceneParams& sc, int n, float* out) {
+    const int* nbr = p.block_tnbr + (int64_t)(n >> 6) * Dims<D>::NBR;
+    gather_tiles<D, C, AGENT, false>(p, sc, n, p.tiles, [&](int o) { return nbr[o]; }, out);
 }
 
 __device__ inline bool inside_plane(const SceneParams& sc, int id, const float* x, int D) {
@@ -1696,12 +1724,11 @@ __global__ __launch_bounds__(WG) void k_grid_update(KP p) {
                 p.ctr->group = 0;
             }
         }
-        // k_cg_solve's places for partials (both parities) and tile flags
+        // k_cg_solve's places for partials (both parities)
         if (p.one_launch)
             for (int i = blockIdx.x * WG + threadIdx.x; i < 2 * CG_RESIDENT; i += gridDim.x * WG) {
                 const double empty = __longlong_as_double((long long)CG_EMPTY);
                 p.bsum[i] = p.bmax[i] = p.bsq[i] = empty;
-                if (i < min(CG_RESIDENT, p.bcap)) p.bu[i] = 0u;
             }
     }
     const XcdRange r = xcd_wave_blocks(p.ctr->nblocks);
@@ -1766,8 +1793,11 @@ __global__ __launch_bounds__(WG) void k_grid_update(KP p) {
 #pragma unroll
             for (int a = 0; a < D; ++a) {
                 p.g_r[a * p.gcap + n] = interior ? vs[a] : 0.0f;
-                p.g_s[a * p.gcap + n] = 0.0f;
+                p.g_s[a * p.gcap + n] = p.one_launch ? __uint_as_float(CG_EMPTY_FLOAT) : 0.0f;
             }
+            if (p.one_launch && (n >> 6) < min(p.bcap, CG_RESIDENT))
+                for (int i = n & 63; i < D * Dims<D>::TN; i += 64)
+                    cg_tile<D>(p, 0, n >> 6)[i] = cg_tile<D>(p, 1, n >> 6)[i] = __uint_as_float(CG_EMPTY_FLOAT);
         }
     }
 }
@@ -2019,14 +2049,16 @@ struct BlockOperator {
         }
         __syncthreads();
     }
-    // The force tile to the block's place in memory (AGENT: other work-groups
-    // of this kernel read it).
-    template <bool AGENT>
-    __device__ void store() {
+    // The force tile to its place in memory (AGENT: other work-groups of this
+    // kernel read it, FLAG: as values that are their own flags).
+    template <bool AGENT, bool FLAG = false>
+    __device__ void store(float* tile) {
         if (tid < TN) {
-            float* dst = p.tiles + (int64_t)b * D * TN + tid;
 #pragma unroll
-            for (int a = 0; a < D; ++a) st<AGENT>(dst + a * TN, S.tile()[a * LTN + li]);
+            for (int a = 0; a < D; ++a) {
+                const float f = S.tile()[a * LTN + li];
+                st<AGENT>(tile + tid + a * TN, FLAG ? flagged(f) : f);
+            }
         }
     }
 };
@@ -2044,7 +2076,7 @@ __device__ inline void operator_block(const KP& p, int b, float inv_dx, Operator
         for (int a = 0; a < D; ++a) u[a] = load(a, op.node);
     }
     op.apply(inv_dx, u, false);
-    op.template store<AGENT>();
+    op.template store<AGENT>(p.tiles + (int64_t)b * D * Dims<D>::TN);
     __syncthreads();
 }
 
@@ -2212,6 +2244,11 @@ __device__ inline bool cg_test(const KP& p, int si, int k, double rr, double mx,
 // ---- what work-groups of one launch exchange ---------------------------------
 constexpr int CG_DOOR_CLOSED = 1 << 30;
 
+// A value that is the same in every lane, in scalar registers.
+__device__ inline double scalar(double v) {
+    const int lo = __builtin_amdgcn_readfirstlane(__double2loint(v)), hi = __builtin_amdgcn_readfirstlane(__double2hiint(v));
+    return __hiloint2double(hi, lo);
+}
 // Every store of this wave has reached memory.
 __device__ inline void drain_stores() { __asm__ __volatile__("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory"); }
 
@@ -2265,8 +2302,8 @@ struct NodeRows {
 };
 
 // CG restart of block b: q = dt^2/m q + x (Multiply_Helper), r = b - q,
-// Project(r); the block's r.r (M-weighted) and max |r|^2.  r goes to g_r, or
-// with TO_S (where the pass may be taken again) to g_s.
+// Project(r); the block's r.r (M-weighted) and max |r|^2.  r goes to g_r and
+// s = 0, or with TO_S (where the pass may be taken again) r goes to g_s.
 template <int D, bool AGENT, bool TO_S>
 __device__ inline void cg_restart_block(const KP& p, const SceneParams& sc, int b, int lane, double& sum, double& mx) {
     const int n = b * 64 + lane;
@@ -2292,6 +2329,7 @@ __device__ inline void cg_restart_block(const KP& p, const SceneParams& sc, int 
 #pragma unroll
     for (int a = 0; a < D; ++a) {
         st<AGENT>((TO_S ? p.g_s : p.g_r) + a * p.gcap + n, rv[a]);
+        if (!TO_S) st<AGENT>(p.g_s + a * p.gcap + n, 0.0f);
         p.g_q[a * p.gcap + n] = q[a];
     }
     sum = 0.0;
@@ -2691,36 +2729,37 @@ __global__ __launch_bounds__(WG) void k_read_speeds(KP p, int* dst) {
 
 // ============================================================================
 // The whole CG solve of every scene in one launch, for scenes too small to
-// fill the chip: there a launch's work is a few microseconds, and the four or
-// five launches of an iteration cost more than it.  The iterations, their
-// arithmetic and the order of every sum are those of the launched kernels for
-// batches (a partial per block, a scene's partials summed in block order).
+// fill the chip: there a launch's work is a few microseconds, and the launches
+// of an iteration cost more than it.  The iterations and their arithmetic are
+// those of the launched kernels (a partial per block, a scene's partials summed
+// in block order).
 //
 // Work-groups share the blocks and wait for one another.  No wait depends on a
 // work-group that might not run: they enter through a door (cg_enter) that the
-// first of them closes as soon as all that are needed have come, or after
-// 20 us; those that come later leave, and whoever is inside is running until
+// first of them closes as soon as all that are needed have come, or at the
+// wait limit; those that come later leave, and whoever is inside is running until
 // the kernel ends.  The results do not depend on how many they are.  What
 // work-groups exchange goes through device-scope accesses.
 //
 // All inside (the usual case, at most CG_RESIDENT blocks): one block each, or
 // two, their nodes' m, x, r and s and their tiles' s in LDS for the whole solve
 // (a halo node's s = r + beta s follows from r alone, so only r and the force
-// tiles travel).  An iteration waits three times: for the
-// neighbours' force tiles (a flag per block), for the scene's partials of s.q
-// and for those of r.r.  A partial is its own flag: its place holds a bit
-// pattern that no partial has until it is written, and its owner puts the
-// pattern back once every reader is known to have passed (two places, by
-// parity of the iteration).
+// tiles travel).  An iteration waits three times: for the neighbours' force
+// tiles, for the scene's partials of s.q and, with r of the tile's nodes, for
+// those of r.r.  Everything that travels is its own flag: a place holds a bit
+// pattern that no value has until it is written, and its owner puts the pattern
+// back once every reader is known to have passed (two places, by parity of the
+// iteration; it is back before the owner's next s.q is out).
 // Otherwise: work-group r of G takes blocks [r n / G, (r + 1) n / G) and counts
 // itself in at its scenes' counters before each wait.
 //
 // Bound by the latency of an iteration's chain (gather, operator phases, three
-// exchanges of about two memory round trips each).  A substep's solve on two
-// balls of 3.8k particles, 13 iterations: 24 us an iteration with every array
-// in memory and counted waits, about 14 resident; the launched kernels need
-// about 30 and, in a captured substep, the launches of all iterations up to
-// the cap.
+// exchanges of a store and a load that has to find it).  Two balls of 3.8k
+// particles, captured, a frame: 18.1 ms with launched kernels, 7.7 resident with
+// a flag per force tile and r waited for before r.r goes out (stores drained,
+// then the flag, then the values: three round trips for one), 7.2 now; 2D scene
+// of 3.0k 18.3 -> 17.0, twelve scenes of 48k 19.3 -> 18.6, and the disk of 512
+// 0.77 -> 0.74 ms for four substeps.
 // ============================================================================
 // The work-group's rank among those inside and their number (at most `most`
 // come), false if the door is closed.
@@ -2797,20 +2836,24 @@ constexpr int CGW = 512;
 template <int D, int K>
 __device__ inline void cg_solve_resident(const KP& p, int blk0, int blk1, OperatorLds<D, CGW>& S) {
     constexpr int TN = Dims<D>::TN, NBR = Dims<D>::NBR, MOST = K * CG_GROUPS;
+    // the wave of block j's nodes: NODES + j, after those with tile nodes
+    constexpr int NODES = (TN + 63) / 64;
+    static_assert(NODES + K < CGW / 64, "wave roles");
     // by parity of the iteration: in a block without particles no other barrier
-    // keeps wave j from writing the next ones before every wave has read these
+    // keeps a wave from writing the next ones before every wave has read these
     __shared__ float sh_beta[2][K];
     __shared__ int sh_done[2][K];
+    __shared__ int tnbr[K][NBR];
     // the node state lives in LDS: registers held across the operator would
     // spill (x, r, s of the blocks' nodes and the tiles' s)
     __shared__ float nx[K][D][64], nr[K][D][64], ns[K][D][64], nm[K][64], ts[K][D][TN];
     // the wave's number as a scalar: its block's and scene's data stay scalar
-    const int lane0 = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane0 = threadIdx.x & 63, nw = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) - NODES;
     BlockOperator<D, CGW> op(p, S);
-    // wave j: the nodes of block j; tile threads: their node's s in every tile.
-    // full, done: a bit per block.
-    bool interior = false, zero = false;
-    int tnbr = -1, b = -1, si = 0, b0 = 0, nb = 0;
+    // wave NODES + j: the nodes of block j; tile threads: their node's s in
+    // every tile.  full, done: a bit per block.
+    unsigned long long interiors = 0, zeros = 0;  // a bit per lane (scalar)
+    int b = -1, si = 0, b0 = 0, nb = 0;
     unsigned full = 0, done = 0;
     for (int j = 0; j < K; ++j) {
         const int bj = j == 0 ? blk0 : blk1;
@@ -2820,7 +2863,7 @@ __device__ inline void cg_solve_resident(const KP& p, int blk0, int blk1, Operat
             continue;
         }
         if (!block_empty(p, bj)) full |= 1u << j;
-        if (wv == j) {
+        if (nw == j) {
             b = bj;
             si = sj;
         }
@@ -2829,31 +2872,47 @@ __device__ inline void cg_solve_resident(const KP& p, int blk0, int blk1, Operat
     if (done == ALL) return;
     if (K == 1 && full) op.open(blk0);
     const SceneParams& sc = p.scn[si];
+    // r of iteration k travels in one of two arrays, by parity
+    // (an offset: a choice between the two pointers became a table in scratch)
+    const int64_t apart = (int64_t)(reinterpret_cast<uintptr_t>(p.g_s) - reinterpret_cast<uintptr_t>(p.g_r)) / (int64_t)sizeof(float);
+    const auto r_place = [&](int k) { return p.g_r + (k & 1) * apart; };
     if (b >= 0) {
         const int lane = lane0, n = b * 64 + lane;
         b0 = p.sst[si].block_begin;
         nb = p.sst[si].block_end - b0;
-        interior = (p.g_flags[n] & MPM_FLAG_INTERIOR_DEV) != 0;
-        nm[wv][lane] = p.g_m[n];
-        zero = project_zero<D>(p, sc, n);
-        if (lane < NBR) tnbr = p.block_tnbr[(int64_t)b * NBR + lane];
-        if (tnbr == b) tnbr = -1;
+        interiors = __ballot((p.g_flags[n] & MPM_FLAG_INTERIOR_DEV) != 0);
+        nm[nw][lane] = p.g_m[n];
+        zeros = __ballot(project_zero<D>(p, sc, n));
+        if (lane < NBR) tnbr[nw][lane] = p.block_tnbr[(int64_t)b * NBR + lane];
 #pragma unroll
         for (int a = 0; a < D; ++a) {
-            nx[wv][a][lane] = p.g_vs[a * p.gcap + n];
-            nr[wv][a][lane] = p.g_r[a * p.gcap + n];
-            ns[wv][a][lane] = 0.0f;
+            nx[nw][a][lane] = p.g_vs[a * p.gcap + n];
+            nr[nw][a][lane] = p.g_r[a * p.gcap + n];
+            ns[nw][a][lane] = 0.0f;
+            st_agent(r_place(0) + a * p.gcap + n, __uint_as_float(CG_EMPTY_FLOAT));
         }
     }
-    int* flag = reinterpret_cast<int*>(p.bu);
     // iteration -1 is the restart: the operator on x, r = b - A x
     double rho = 0.0;
     for (int k = -1;; ++k) {
         const int par = (k & 1) * CG_RESIDENT;
         const int lane = opaque(lane0), n = b * 64 + lane;
         op.tid = opaque(op.tid);
+        // r of tile node `node`
+        float rn[D];
+        const auto await_r = [&](int node) {
+            bool waiting;
+            do {
+                waiting = false;
+#pragma unroll
+                for (int a = 0; a < D; ++a) rn[a] = ld_agent(r_place(k - 1) + a * p.gcap + node);
+#pragma unroll
+                for (int a = 0; a < D; ++a) waiting |= is_empty(rn[a]);
+                if (waiting) __builtin_amdgcn_s_sleep(4);
+            } while (waiting);
+        };
         if (k >= 0) {
-            if (b >= 0 && !((done >> wv) & 1u)) {
+            if (b >= 0 && !((done >> nw) & 1u)) {
                 // convergence test and beta on the scene's r.r
                 double rr, mx;
                 await_partials<MOST>(p.bsum + par + b0, p.bmax + par + b0, nb, lane, rr, mx);
@@ -2862,11 +2921,13 @@ __device__ inline void cg_solve_resident(const KP& p, int blk0, int blk1, Operat
                 const CGTestIn in{rho, sc.cg_tol, sc.cg_min, sc.cg_max, false};
                 float beta;
                 const bool fin = cg_test(p, si, k, rr, mx, b == b0 && lane == 0, beta, in);
-                rho = rr;
+                rho = scalar(rr);
                 if (lane == 0) {
-                    sh_beta[k & 1][wv] = beta;
-                    sh_done[k & 1][wv] = fin ? 1 : 0;
+                    sh_beta[k & 1][nw] = beta;
+                    sh_done[k & 1][nw] = fin ? 1 : 0;
                 }
+            } else if (K == 1 && full && op.node >= 0) {
+                await_r(op.node);  // meanwhile
             }
             __syncthreads();
             for (int j = 0; j < K; ++j)
@@ -2884,52 +2945,56 @@ __device__ inline void cg_solve_resident(const KP& p, int blk0, int blk1, Operat
 #pragma unroll
             for (int a = 0; a < D; ++a) u[a] = 0.0f;
             if (op.node >= 0) {
+                if (K > 1 && k >= 0) await_r(op.node);
 #pragma unroll
                 for (int a = 0; a < D; ++a) {
                     if (k < 0) {
                         u[a] = p.g_vs[a * p.gcap + op.node];
                         ts[j][a][op.tid] = 0.0f;
                     } else {
-                        u[a] = cg_direction(ld_agent(p.g_r + a * p.gcap + op.node), ts[j][a][op.tid], sh_beta[k & 1][j], k);
+                        u[a] = cg_direction(rn[a], ts[j][a][op.tid], sh_beta[k & 1][j], k);
                         ts[j][a][op.tid] = u[a];
                     }
                 }
             }
+            // every reader of the tile of iteration k - 1 has passed
+            if (k >= 0 && op.tid < TN) {
+#pragma unroll
+                for (int a = 0; a < D; ++a) st_agent(cg_tile<D>(p, k - 1, bj) + op.tid + a * TN, __uint_as_float(CG_EMPTY_FLOAT));
+            }
             op.apply(p.scn[p.block_scene[bj]].inv_dx, u, K == 1 && k >= 0);
-            op.template store<true>();
-            drain_stores();
+            drain_stores();  // places emptied in this iteration: before its s.q is out
+            op.template store<true, true>(cg_tile<D>(p, k, bj));
             __syncthreads();
-            if (threadIdx.x == 0) st_agent(flag + bj, k + 2);
             if (K == 1) op.load_records(0);  // for the next time
         }
-        if (b < 0 || ((done >> wv) & 1u)) continue;
+        if (b < 0 || ((done >> nw) & 1u)) continue;
         // the neighbours' tiles, and this block's nodes
-        while (__any(tnbr >= 0 && ld_agent(flag + max(tnbr, 0)) < k + 2)) __builtin_amdgcn_s_sleep(1);
-        __asm__ __volatile__("" ::: "memory");
+        const bool interior = (interiors >> lane) & 1, zero = (zeros >> lane) & 1;
         float q[D], r[D];
-        gather_node_tiles<D, D, true>(p, sc, n, q);
-        const double m = (double)nm[wv][lane];
-        const float cm = sc.dt * sc.dt / nm[wv][lane];
+        gather_tiles<D, D, true, true>(p, sc, n, cg_tile<D>(p, k, 0), [&](int o) { return tnbr[nw][o]; }, q);
+        const double m = (double)nm[nw][lane];
+        const float cm = sc.dt * sc.dt / nm[nw][lane];
         double sum = 0.0, mx = 0.0;
         if (k < 0) {
 #pragma unroll
             for (int a = 0; a < D; ++a) {
-                r[a] = nr[wv][a][lane];
+                r[a] = nr[nw][a][lane];
                 if (interior) {
-                    q[a] = cm * q[a] + nx[wv][a][lane];
+                    q[a] = cm * q[a] + nx[nw][a][lane];
                     r[a] = r[a] - q[a];
                 }
                 if (zero) r[a] = 0.0f;
             }
         } else {
-            const float beta = sh_beta[k & 1][wv];
+            const float beta = sh_beta[k & 1][nw];
             float s[D];
 #pragma unroll
             for (int a = 0; a < D; ++a) {
-                s[a] = ns[wv][a][lane];
+                s[a] = ns[nw][a][lane];
                 if (interior) {
-                    s[a] = cg_direction(nr[wv][a][lane], s[a], beta, k);
-                    ns[wv][a][lane] = s[a];
+                    s[a] = cg_direction(nr[nw][a][lane], s[a], beta, k);
+                    ns[nw][a][lane] = s[a];
                     q[a] = cm * q[a] + s[a];
                 }
                 if (zero) q[a] = 0.0f;
@@ -2937,26 +3002,25 @@ __device__ inline void cg_solve_resident(const KP& p, int blk0, int blk1, Operat
             }
             double sq;
             wave_reduce2(sum, mx);
+            drain_stores();
             if (lane == 0) put_partial(p.bsq + par + b, sum);
             await_partials<MOST>(p.bsq + par + b0, nullptr, nb, lane, sq, mx);
-            // every reader of this iteration's r.r partials has passed
+            // every reader of this iteration's r.r partials and of r of
+            // iteration k - 1 has passed
             if (lane == 0) {
                 clear_partial(p.bsum + par + b);
                 clear_partial(p.bmax + par + b);
             }
-            const double alpha_d = sq != 0.0 ? rho / sq : (double)FLT_MAX;
-            if (b == b0 && lane == 0) {
-                CGState& cg = p.cg[si];
-                cg.sq = sq;
-                cg.alpha = alpha_d;
-                cg.multiplies += 1;
-            }
+#pragma unroll
+            for (int a = 0; a < D; ++a) st_agent(r_place(k - 1) + a * p.gcap + n, __uint_as_float(CG_EMPTY_FLOAT));
+            const double alpha_d = cg_alpha(rho, sq);
+            if (b == b0 && lane == 0) cg_record_alpha(p.cg[si], sq, alpha_d);
             const float alpha = (float)alpha_d;
 #pragma unroll
             for (int a = 0; a < D; ++a) {
-                r[a] = nr[wv][a][lane];
+                r[a] = nr[nw][a][lane];
                 if (interior) {
-                    nx[wv][a][lane] = alpha * s[a] + nx[wv][a][lane];
+                    nx[nw][a][lane] = alpha * s[a] + nx[nw][a][lane];
                     r[a] = -alpha * q[a] + r[a];
                 }
             }
@@ -2966,16 +3030,15 @@ __device__ inline void cg_solve_resident(const KP& p, int blk0, int blk1, Operat
         mx = 0.0;
 #pragma unroll
         for (int a = 0; a < D; ++a) {
+            st_agent(r_place(k) + a * p.gcap + n, flagged(r[a]));
             if (interior) {
                 sum += (double)r[a] * ((double)r[a] * m);
                 mx += (double)r[a] * (double)r[a];
             }
-            nr[wv][a][lane] = r[a];
-            st_agent(p.g_r + a * p.gcap + n, r[a]);
+            nr[nw][a][lane] = r[a];
             p.g_q[a * p.gcap + n] = q[a];
         }
         wave_reduce2(sum, mx);
-        drain_stores();
         if (lane == 0) {
             put_partial(p.bsum + (CG_RESIDENT - par) + b, sum);
             put_partial(p.bmax + (CG_RESIDENT - par) + b, mx);
@@ -2985,8 +3048,9 @@ __device__ inline void cg_solve_resident(const KP& p, int blk0, int blk1, Operat
         const int lane = lane0, n = b * 64 + lane;
 #pragma unroll
         for (int a = 0; a < D; ++a) {
-            p.g_vs[a * p.gcap + n] = nx[wv][a][lane];
-            p.g_s[a * p.gcap + n] = ns[wv][a][lane];
+            p.g_vs[a * p.gcap + n] = nx[nw][a][lane];
+            p.g_r[a * p.gcap + n] = flagged(nr[nw][a][lane]);
+            p.g_s[a * p.gcap + n] = flagged(ns[nw][a][lane]);
         }
     }
 }
