@@ -1512,30 +1512,28 @@ __global__ __launch_bounds__(BWG) void k_init_volume(KP p) {
 }
 
 // ============================================================================
-// Explicit force of one particle into its wave's tile:
-// f_i += g m w_i - A grad w_i, A = V0 P F^T (MPM_Example.cpp:774-784).
+// Explicit force of one particle, added to its cell's 3^D nodes:
+// f_i += g m w_i - A grad w_i, A = V0 P F^T (MPM_Example.cpp:774-784).  The
+// sums over all but the last axis are shared by the three nodes along it.
 template <int D>
-__device__ inline void scatter_force(const SceneParams& sc, const int* l, const float (*w)[3], const float (*dw)[3],
-                                     const float* A, float m, float* mine) {
-    constexpr int LTN = Dims<D>::LTN, ST = Dims<D>::ST;
+__device__ inline void add_explicit_force(const SceneParams& sc, const float (*w)[3], const float (*dw)[3], const float* A,
+                                          float m, float (*acc)[D]) {
     float gm[D];
 #pragma unroll
     for (int a = 0; a < D; ++a) gm[a] = sc.gravity[a] * m;
 #pragma unroll
-    for (int s = 0; s < ST; ++s) {
-        int off[D];
-        const int t = tile_index<D>(l, s, off);
-        float g[D];
-        stencil_grad<D>(w, dw, off, g);
-        const float wt = stencil_weight<D>(w, off);
+    for (int r = 0; r < (D == 3 ? 9 : 3); ++r) {
+        const int i = D == 3 ? r / 3 : r, j = r % 3;
+        const float wr = D == 3 ? w[0][i] * w[1][j] : w[0][i];
+        const float gx = D == 3 ? dw[0][i] * w[1][j] : dw[0][i], gy = D == 3 ? w[0][i] * dw[1][j] : 0.0f;
 #pragma unroll
         for (int a = 0; a < D; ++a) {
-            float inner = 0.0f;
+            float even = gm[a] * wr - A[a * D] * gx;
+            if (D == 3) even -= A[a * D + 1] * gy;
+            const float odd = A[a * D + D - 1] * wr;
 #pragma unroll
-            for (int k = 0; k < D; ++k) inner += A[a * D + k] * g[k];
-            mine[a * LTN + t] += gm[a] * wt - inner;
+            for (int k = 0; k < 3; ++k) acc[r * 3 + k][a] += even * w[D - 1][k] - odd * dw[D - 1][k];
         }
-        MPM_STEP_FENCE();
     }
 }
 
@@ -1629,20 +1627,26 @@ __device__ __forceinline__ void particle_stress(const KP& p, const SceneParams& 
 // material table, each pass taking the particles of that entry (a single
 // pass without a check in a one-material scene): the material's parameters
 // stay scalar operands.  With FORCE the chunk's stress terms go to LDS and
-// are then scattered cell by cell (lane = cell, waves interleave a cell's
-// particles) into the wave tiles.
+// are then summed cell by cell (lane = cell, waves interleave a cell's
+// particles) in registers and added to the wave tiles once per chunk.  Bound by
+// the FP64 SVD.  Against adding every particle to the tile (81 ordered
+// read-add-writes each): avalanche of 1.0M particles 138 -> 129 us, two balls of
+// 243k 57.6 -> 52.2, twelve scenes 103 -> 96, fluid of 20k 42 -> 29, balls of
+// 3.8k 26.7 -> 22.3.  Loading the next particle ahead takes the kernel over 168
+// registers, to two waves a SIMD (1.0M: 160 us).
 constexpr int PF_CHUNK = 2 * BWG;
 template <int D, bool CONST, bool FORCE>
 __global__ __launch_bounds__(BWG) void k_particle_force(KP p) {
     using Dm = Dims<D>;
-    constexpr int LTN = Dm::LTN, DD = D * D;
+    constexpr int LTN = Dm::LTN, DD = D * D, ST = Dm::ST;
     __shared__ __align__(16) float tile[NW * D * LTN];
     __shared__ float stress[DD][PF_CHUNK];
     const int nblocks = p.ctr->nblocks;
     const int c = threadIdx.x & 63, wv = threadIdx.x >> 6;
     float* mine = tile + wv * D * LTN;
-    int l[D];
+    int l[D], off0[D];
     local_coords<D>(c, l);
+    const int base = tile_index<D>(l, 0, off0);  // cell c's stencil corner
     const XcdRange xr = xcd_blocks(nblocks);
     for (int kb = xr.first; kb < xr.end; kb += xr.step) {
         const int b = p.block_order[kb];  // heavy blocks first within the XCD's range
@@ -1673,13 +1677,26 @@ __global__ __launch_bounds__(BWG) void k_particle_force(KP p) {
             if (FORCE) {
                 __syncthreads();  // the chunk's stress terms (and, first, the zeroed tiles)
                 const int lo = max(c0, chunk), hi = min(c1, chunk + PF_CHUNK);
+                float acc[ST][D];
+#pragma unroll
+                for (int n = 0; n < ST; ++n)
+#pragma unroll
+                    for (int a = 0; a < D; ++a) acc[n][a] = 0.0f;
                 for (int j = lo + wv; j < hi; j += NW) {
                     float w[D][3], dw[D][3], X[D];
                     if (!cell_particle<D>(p, sc, j, bb, l, w, dw, X)) continue;
                     float A[DD];
 #pragma unroll
                     for (int k = 0; k < DD; ++k) A[k] = stress[k][j - chunk];
-                    scatter_force<D>(sc, l, w, dw, A, p.pcur[PF<D>::M * p.pcap + j], mine);
+                    add_explicit_force<D>(sc, w, dw, A, p.pcur[PF<D>::M * p.pcap + j], acc);
+                }
+                // (lanes hold distinct cells: at one node of the stencil no two write the same place)
+#pragma unroll
+                for (int n = 0; n < ST; ++n) {
+                    const int t = D == 3 ? base + (n / 9) * Dm::LX + ((n / 3) % 3) * Dm::LY + n % 3 : base + (n / 3) * Dm::LX + n % 3;
+#pragma unroll
+                    for (int a = 0; a < D; ++a) mine[a * LTN + t] += acc[n][a];
+                    MPM_STEP_FENCE();
                 }
                 __syncthreads();  // before the next chunk overwrites the stress terms
             }
