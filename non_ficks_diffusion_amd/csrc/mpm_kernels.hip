@@ -811,19 +811,6 @@ __device__ inline void store_wave_tiles(const KP& p, int b, const float* lds) {
     }
 }
 
-// Weights of particle i; false if it is not in cell l of block bb (only after
-// particles moved without re-binning: the particle is skipped).
-template <int D>
-__device__ inline bool cell_particle(const KP& p, const SceneParams& sc, int i, const int* bb, const int* l,
-                                     float (*w)[3], float (*dw)[3], float* X) {
-    int lp[D];
-    if (!particle_weights<D>(p, sc, i, bb, w, dw, lp, X)) return false;
-    bool same = true;
-#pragma unroll
-    for (int a = 0; a < D; ++a) same = same && lp[a] == l[a];
-    return same;
-}
-
 // The record of an EOS particle: its CG force V0 K gamma rho^(gamma-1)
 // (grad w . u) grad w (MPM_CG_System.h:169-174, 205-207) is A = c tr(T) I,
 // taking the reference's matrix-plus-scalar as adding to the diagonal.  In
@@ -1340,22 +1327,37 @@ __device__ inline void add_cell_nodes(const float* M, int base, int lane, float*
     }
 }
 
+// Weights of particle i; false if it is not in cell l of block bb (only after
+// particles moved without re-binning: the particle is skipped).
+template <int D>
+__device__ inline bool cell_particle(const KP& p, const SceneParams& sc, int i, const int* bb, const int* l,
+                                     float (*w)[3], float (*dw)[3], float* X) {
+    int lp[D];
+    if (!particle_weights<D>(p, sc, i, bb, w, dw, lp, X)) return false;
+    bool same = true;
+#pragma unroll
+    for (int a = 0; a < D; ++a) same = same && lp[a] == l[a];
+    return same;
+}
+
 // ============================================================================
 // P2G (Rasterize, MPM_Example.cpp:520-537): m_i += w m_p, (mv)_i += w m_p V_p.
-// One wave per block (the waves of a work-group take different blocks and
-// share nothing).  Lane c runs every particle of cell c, summing the cell's
-// 3^D-node contribution in registers (the particles of a cell share its
-// stencil), then adds it to the wave's LDS tile in 3^D ordered
-// read-add-write steps (lanes hold distinct cells) and the wave stores the
-// tile.  LDS traffic is one stencil per cell instead of one per particle.
+// Lane c runs the particles of cell c, summing the cell's 3^D-node contribution
+// in registers (the particles of a cell share its stencil), then adds it to the
+// wave's LDS tile in 3^D ordered read-add-write steps (lanes hold distinct
+// cells).  LDS traffic is one stencil per cell instead of one per particle.
+// One wave per block (the waves of a work-group take different blocks and share
+// nothing); SPLIT: a work-group per block, its waves taking every NW-th
+// particle of a cell, where there are too few blocks to fill the chip and the
+// fullest cell's particles, one after another, are the time (P2G_SPLIT_MAX).
 // ============================================================================
-template <int D>
+template <int D, bool SPLIT>
 __global__ __launch_bounds__(BWG) void k_p2g(KP p) {
     using Dm = Dims<D>;
     constexpr int LTN = Dm::LTN, C = D + 1, TN = Dm::TN, LX = Dm::LX, LY = Dm::LY;
-    constexpr int NS = D == 3 ? 27 : 9;
+    constexpr int NS = D == 3 ? 27 : 9, EACH = SPLIT ? NW : 1;
     __shared__ float tile_all[NW][C * LTN];
-    const int c = threadIdx.x & 63;
+    const int c = threadIdx.x & 63, first = SPLIT ? (int)(threadIdx.x >> 6) : 0;
     float* mine = tile_all[threadIdx.x >> 6];
     int l[D];
     local_coords<D>(c, l);
@@ -1364,7 +1366,7 @@ __global__ __launch_bounds__(BWG) void k_p2g(KP p) {
         int off0[D];
         base = tile_index<D>(l, 0, off0);
     }
-    const XcdRange xr = xcd_wave_blocks(p.ctr->nblocks);
+    const XcdRange xr = SPLIT ? xcd_blocks(p.ctr->nblocks) : xcd_wave_blocks(p.ctr->nblocks);
     for (int kb = xr.first; kb < xr.end; kb += xr.step) {
         // one scene: heavy blocks first within the XCD's range; batches keep
         // slot order, measured faster there (small blocks of many scenes, and
@@ -1380,8 +1382,8 @@ __global__ __launch_bounds__(BWG) void k_p2g(KP p) {
         for (int n = 0; n < NS; ++n)
 #pragma unroll
             for (int ch = 0; ch < C; ++ch) acc[n][ch] = 0.0f;
-        const int i0 = p.cell_start[b * 65 + c], i1 = p.cell_start[b * 65 + c + 1];
-        for (int i = i0; i < i1; ++i) {
+        const int i0 = p.cell_start[b * 65 + c] + first, i1 = p.cell_start[b * 65 + c + 1];
+        for (int i = i0; i < i1; i += EACH) {
             float w[D][3], dw[D][3], X[D];
             if (!cell_particle<D>(p, sc, i, bb, l, w, dw, X)) continue;
             float mv[C];
@@ -1419,6 +1421,12 @@ __global__ __launch_bounds__(BWG) void k_p2g(KP p) {
 #pragma unroll
             for (int ch = 0; ch < C; ++ch) mine[ch * LTN + t] += acc[n][ch];
             MPM_STEP_FENCE();
+        }
+        if (SPLIT) {
+            __syncthreads();
+            store_wave_tiles<D, C>(p, b, tile_all[0]);
+            __syncthreads();
+            continue;
         }
         float* dst = p.tiles + (int64_t)b * C * TN;
         for (int t = c; t < C * TN; t += 64) {
@@ -3797,7 +3805,10 @@ template void launch_pack_write<3>(const KP&, hipStream_t, const PackArgs&);
 void launch_read_speeds(const KP& p, hipStream_t s, int* dst) { hipLaunchKernelGGL(k_read_speeds, dim3(1), dim3(WG), 0, s, p, dst); }
 void launch_poll(const KP& p, hipStream_t s, int* dst) { hipLaunchKernelGGL(k_poll, dim3(1), dim3(64), 0, s, p, dst); }
 template <int D> void launch_reorder(const KP& p, hipStream_t s, int grid) { hipLaunchKernelGGL(k_reorder<D>, dim3(grid), dim3(WG), 0, s, p); }
-template <int D> void launch_p2g(const KP& p, hipStream_t s, int grid) { hipLaunchKernelGGL(k_p2g<D>, dim3(grid), dim3(BWG), 0, s, p); }
+template <int D> void launch_p2g(const KP& p, hipStream_t s, int grid) {
+    if (p.split_p2g) hipLaunchKernelGGL((k_p2g<D, true>), dim3(grid), dim3(BWG), 0, s, p);
+    else hipLaunchKernelGGL((k_p2g<D, false>), dim3(grid), dim3(BWG), 0, s, p);
+}
 template <int D> void launch_normalize(const KP& p, hipStream_t s, int grid) { hipLaunchKernelGGL(k_normalize<D>, dim3(grid), dim3(WG), 0, s, p); }
 template <int D> void launch_init_volume(const KP& p, hipStream_t s, int grid) { hipLaunchKernelGGL(k_init_volume<D>, dim3(grid), dim3(BWG), 0, s, p); }
 template <int D> void launch_particle_force(const KP& p, hipStream_t s, int grid, bool constitutive, bool force) {
