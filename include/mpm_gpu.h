@@ -332,7 +332,7 @@ int mpm_measure_copy_bandwidth(int64_t bytes, int32_t reps, double* gbs);
  * with stats it waits and returns MPM_E_CAPACITY when the particles needed
  * more than MPM_NOALLOC_MAX_BLOCKS active blocks (the substep was then a
  * no-op) and MPM_E_NONFINITE as mpm_substep does.
- * Every working buffer lives in one static device array per GPU (40 MiB,
+ * Every working buffer lives in one static device array per GPU (46 MiB,
  * held until the process ends) that every call on that GPU shares and that
  * keeps the last call's contents: calls that overlap on one GPU race.  Sizes
  * beyond the limits are refused with MPM_E_CAPACITY before any GPU work;

@@ -114,6 +114,7 @@ mpm::SceneParams scene_params(const mpm_scene_desc& d, int slot_base, int nslots
 enum SizeClass { SIZE_ONE_LAUNCH, SIZE_SPLIT, SIZE_LARGE };
 SizeClass size_class(const mpm_context* c);
 
+int tile_nodes(int D) { return D == 3 ? 216 : 100; }
 mpm::KP make_kp(const mpm_context* c) {
     mpm::KP p{};
     p.scn = c->scn;
@@ -164,7 +165,7 @@ mpm::KP make_kp(const mpm_context* c) {
     p.g_flags = c->g_flags;
     p.gcap = c->gcap;
     p.tiles = c->tiles;
-    p.cg_tiles = c->cg_tiles;
+    p.cg_tiles = c->tiles + (int64_t)c->bcap * (c->D + 1) * tile_nodes(c->D);
     p.ctr = c->ctr;
     p.bsum = c->bsum;
     p.bmax = c->bmax;
@@ -636,8 +637,8 @@ void layout_buffers(mpm_context* c, Take&& take) {
     take(&c->block_full, bcap);
     take(&c->cell_count, nslots * 64);
     take(&c->cell_start, bcap * 65 + 1);
-    take(&c->tiles, bcap * (D + 1) * (D == 3 ? 216 : 100));
-    take(&c->cg_tiles, 2 * std::min(bcap, (size_t)mpm::CG_RESIDENT) * D * (D == 3 ? 216 : 100));
+    // (the second part is KP::cg_tiles: one allocation, they cost a tenth of a millisecond each)
+    take(&c->tiles, (bcap * (D + 1) + 2 * std::min(bcap, (size_t)mpm::CG_RESIDENT) * D) * tile_nodes((int)D));
     take(&c->scan_part, (size_t)2 * c->nparts);
     take(&c->g_m, gcap);
     take(&c->g_v, (size_t)D * gcap);

@@ -61,7 +61,6 @@ struct mpm_context {
     mpm::SceneState* sst = nullptr;
     mpm::CGState* cg = nullptr;
     int* slot_scene = nullptr;   // per slot: owning scene, -1 if free
-    float* cg_tiles = nullptr;
     double *bsum = nullptr, *bmax = nullptr, *bsq = nullptr;
     unsigned* bu = nullptr;
     int cg_predict = 0;    // the next solve's first launch batch: the last solve's iterations plus one
