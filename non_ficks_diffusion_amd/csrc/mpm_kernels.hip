@@ -2728,7 +2728,10 @@ __global__ __launch_bounds__(NGW, 6) void k_cg_node(KP p, int k) {
         __syncthreads();
         if (b >= 0 && RESTART) {
 #pragma unroll
-            for (int a = 0; a < D; ++a) p.g_r[a * p.gcap + b * 64 + lane] = v.s[a];
+            for (int a = 0; a < D; ++a) {
+                p.g_r[a * p.gcap + b * 64 + lane] = v.s[a];
+                if (sh_fin[head]) p.g_s[a * p.gcap + b * 64 + lane] = 0.0f;  // no direction was taken
+            }
         } else if (b >= 0 && !sh_fin[head] && v.interior) {
 #pragma unroll
             for (int a = 0; a < D; ++a)

@@ -7,6 +7,8 @@ must match the FP64 oracle to the one-substep bar, 1e-5 relative L2, per
 field.  The particles carry a velocity gradient, so the operator's result
 reaches every compared field.
 """
+import threading
+
 import numpy as np
 import pytest
 
@@ -150,3 +152,39 @@ def test_node_pass_work_groups(dim, counts, scenes, graph):
         assert np.array_equal(once[k]["ids"], want["ids"])
         for f in ("x", "v", "F", "Jp"):
             assert rel(once[k][f], want[f]) < 1e-5, (k, f)
+
+
+def test_solves_of_two_handles_at_once():
+    """Work-groups of two launches that each exchange sums share the device:
+    handles driven from two threads end as they do one after the other."""
+    parts = [scattered(3, 64, 66000, 50, 0.2, 0.8), scattered(3, 64, 66000, 51, 0.3, 0.7), scattered(3, 32, 4000, 52, 0.3, 0.7)]
+    dt = 0.5 * float(parts[0][0].max_dt)
+
+    def handle(q):
+        d, x, v, m = q
+        s = M.Scene(d, 3 * len(m))
+        s.upload(x, v, m)
+        s.initialize()
+        return s
+
+    def drive(s):
+        for _ in range(4):
+            s.substep(dt)
+
+    want = []
+    for q in parts:
+        s = handle(q)
+        drive(s)
+        want.append(s.download())
+        s.close()
+    scenes = [handle(q) for q in parts]
+    threads = [threading.Thread(target=drive, args=(s,)) for s in scenes]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for s, w in zip(scenes, want):
+        got = s.download()
+        s.close()
+        for f in ("x", "v", "F", "Jp", "ids"):
+            assert np.array_equal(got[f], w[f]), f
