@@ -295,11 +295,13 @@ static_assert(offsetof(mpm::Counters, nblocks) == 0 && offsetof(mpm::Counters, o
 
 // The solve in one launch (k_cg_solve) for handles of up to this many
 // particles (at eight a cell about 130 blocks that hold some, 350 with their
-// halo).  Measured per frame of 60 fps: 3.8k particles in 32^3 13.3 -> 7.7 ms
-// (captured), twelve scenes of 48k together 26 -> 19; above, more blocks of
-// particles meet in a work-group and the launched kernels win: two balls of
-// 243k 73 -> 104 ms, a dense slab of 333k 45 -> 81, four requests of 200k
-// together 139 either way.  The rule reads only what the caller uploaded, so
+// halo).  Measured per frame against the operator and the node pass launched
+// for every iteration: 20k particles of two balls 13.5 -> 9.9 ms, 60k 13.9 ->
+// 11.8, a slab of 60k 10.3 -> 8.4, captured 7.7 -> 6.0, the 2D scene of 3.0k
+// 19.7 -> 14.9, twelve scenes of together 48k 20.1 -> 19.2; equal at 80k (7.9 and
+// 7.8, 6.1 and 6.4, 3.9 and 3.7); above, more blocks of particles meet in a
+// work-group and the launches win: 120k 8.5 -> 9.4 and 7.1 -> 7.8, four requests
+// of together 200k 112 -> 124.  The rule reads only what the caller uploaded, so
 // launched, replayed and repeated substeps take the same kernels.
 constexpr int64_t CG_SOLVE_MAX_PARTICLES = 65536;
 // P2G with a work-group per block: per launch 18.0 -> 9.8 us for balls of 3.8k
