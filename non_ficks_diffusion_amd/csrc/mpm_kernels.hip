@@ -472,6 +472,59 @@ __device__ inline void load_slots(const KP& p, int base, int ns, int* act, int* 
     }
 }
 
+// The scan's totals: active blocks and particles (one thread).
+__device__ inline void record_totals(const KP& p, int ta, int tc) {
+    p.ctr->n_prev = p.ctr->n_live;
+    if (ta > p.bcap) {
+        // the substep becomes a no-op: particles keep their order and state
+        p.ctr->overflow = 1;
+        p.ctr->nblocks = 0;
+    } else {
+        p.ctr->overflow = 0;  // a binning that fits clears an earlier overflow
+        p.ctr->n_live = tc;
+        p.ctr->nblocks = ta;
+        p.block_pstart[ta] = tc;
+    }
+}
+
+// The slots of load_slots, ra blocks and rc particles before them (moved past
+// them): their blocks and active indices, and the binning's marks cleared.
+__device__ inline void apply_scan(const KP& p, int base, int ns, const int* act, const int* cnt, int& ra, int& rc, bool overflow) {
+    // after an overflow no block is set up, so the binning's cell counters of
+    // the touched slots are cleared here instead of by the block set-up
+    int sact[SCAN_PER_THREAD];
+#pragma unroll
+    for (int k = 0; k < SCAN_PER_THREAD; ++k) {
+        const int s = base + k;
+        sact[k] = act[k] ? ra : -1;
+        if (act[k] && s < ns) {
+            if (ra < p.bcap) {
+                p.block_slot[ra] = s;
+                p.block_pstart[ra] = rc;
+            }
+            if (overflow)
+                for (int cell = 0; cell < 64; ++cell) p.cell_count[s * 64 + cell] = 0;
+        }
+        ra += act[k];
+        rc += cnt[k];
+    }
+    if (base + SCAN_PER_THREAD <= ns) {
+        *reinterpret_cast<int4*>(p.slot_active + base) = make_int4(sact[0], sact[1], sact[2], sact[3]);
+        *reinterpret_cast<int4*>(p.slot_touched + base) = make_int4(0, 0, 0, 0);
+        *reinterpret_cast<int4*>(p.slot_count + base) = make_int4(0, 0, 0, 0);
+    } else {
+#pragma unroll
+        for (int k = 0; k < SCAN_PER_THREAD; ++k) {
+            const int s = base + k;
+            if (s < ns) {
+                p.slot_active[s] = sact[k];
+                p.slot_touched[s] = 0;
+                p.slot_count[s] = 0;
+            }
+        }
+    }
+}
+
 __global__ __launch_bounds__(WG) void k_scan_reduce(KP p) {
     const int ns = scanned_slots(p);
     if ((int64_t)blockIdx.x * SCAN_TILE >= ns) {  // beyond the scanned slots: empty part
@@ -522,19 +575,7 @@ __global__ __launch_bounds__(WG) void k_scan_top(KP p) {
             rc += vc;
         }
     }
-    if (threadIdx.x == 0) {
-        p.ctr->n_prev = p.ctr->n_live;
-        if (ta > p.bcap) {
-            // the substep becomes a no-op: particles keep their order and state
-            p.ctr->overflow = 1;
-            p.ctr->nblocks = 0;
-        } else {
-            p.ctr->overflow = 0;  // a binning that fits clears an earlier overflow
-            p.ctr->n_live = tc;
-            p.ctr->nblocks = ta;
-            p.block_pstart[ta] = tc;
-        }
-    }
+    if (threadIdx.x == 0) record_totals(p, ta, tc);
 }
 
 __global__ __launch_bounds__(WG) void k_scan_apply(KP p) {
@@ -553,41 +594,59 @@ __global__ __launch_bounds__(WG) void k_scan_apply(KP p) {
     int ta, tc;
     int ra = wg_exclusive_scan(sa, ta) + p.scan_part[blockIdx.x];
     int rc = wg_exclusive_scan(sc, tc) + p.scan_part[p.nparts + blockIdx.x];
-    // after an overflow no block is set up, so the binning's cell counters of
-    // the touched slots are cleared here instead of by the block set-up
-    const bool overflow = p.ctr->overflow != 0;
-    int sact[SCAN_PER_THREAD];
+    apply_scan(p, base, ns, act, cnt, ra, rc, p.ctr->overflow != 0);
+}
+
+// The whole scan in one work-group of SCAN_ONE threads, Q times
+// SCAN_PER_THREAD consecutive slots each, for up to 8,192 slots (grids of up to
+// 68 cells an axis in 3D).  Bound by latency: three launches of 2.9 to 4.5 us
+// there do almost nothing, this one takes 4.5 us (1,331 slots) and 4.6 us (6,859);
+// with 16 slots a thread (13,824) it took 11.8 us, as long as the three.
+constexpr int SCAN_ONE = 1024;
+template <int Q>
+__global__ __launch_bounds__(SCAN_ONE) void k_scan_one(KP p) {
+    __shared__ int wa[SCAN_ONE / 64], wc[SCAN_ONE / 64];
+    const int ns = scanned_slots(p), lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int base = (int)threadIdx.x * Q * SCAN_PER_THREAD;
+    int act[Q][SCAN_PER_THREAD], cnt[Q][SCAN_PER_THREAD], sa = 0, sc = 0;
 #pragma unroll
-    for (int k = 0; k < SCAN_PER_THREAD; ++k) {
-        const int s = base + k;
-        sact[k] = act[k] ? ra : -1;
-        if (act[k] && s < ns) {
-            if (ra < p.bcap) {
-                p.block_slot[ra] = s;
-                p.block_pstart[ra] = rc;
-            }
-            if (overflow)
-                for (int cell = 0; cell < 64; ++cell) p.cell_count[s * 64 + cell] = 0;
-        }
-        ra += act[k];
-        rc += cnt[k];
-    }
-    // the thread's slots: active index, and the binning's marks cleared
-    if (base + SCAN_PER_THREAD <= ns) {
-        *reinterpret_cast<int4*>(p.slot_active + base) = make_int4(sact[0], sact[1], sact[2], sact[3]);
-        *reinterpret_cast<int4*>(p.slot_touched + base) = make_int4(0, 0, 0, 0);
-        *reinterpret_cast<int4*>(p.slot_count + base) = make_int4(0, 0, 0, 0);
-    } else {
+    for (int q = 0; q < Q; ++q) load_slots(p, base + q * SCAN_PER_THREAD, ns, act[q], cnt[q]);
+#pragma unroll
+    for (int q = 0; q < Q; ++q)
 #pragma unroll
         for (int k = 0; k < SCAN_PER_THREAD; ++k) {
-            const int s = base + k;
-            if (s < ns) {
-                p.slot_active[s] = sact[k];
-                p.slot_touched[s] = 0;
-                p.slot_count[s] = 0;
-            }
+            act[q][k] = act[q][k] != 0;
+            sa += act[q][k];
+            sc += cnt[q][k];
+        }
+    // inclusive over the wave, then the waves before
+    int ia = sa, ic = sc;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int ua = __shfl_up(ia, off), uc = __shfl_up(ic, off);
+        if (lane >= off) {
+            ia += ua;
+            ic += uc;
         }
     }
+    if (lane == 63) {
+        wa[wv] = ia;
+        wc[wv] = ic;
+    }
+    __syncthreads();
+    int ra = ia - sa, rc = ic - sc, ta = 0, tc = 0;
+#pragma unroll
+    for (int w = 0; w < SCAN_ONE / 64; ++w) {
+        if (w < wv) {
+            ra += wa[w];
+            rc += wc[w];
+        }
+        ta += wa[w];
+        tc += wc[w];
+    }
+    if (threadIdx.x == 0) record_totals(p, ta, tc);
+#pragma unroll
+    for (int q = 0; q < Q; ++q) apply_scan(p, base + q * SCAN_PER_THREAD, ns, act[q], cnt[q], ra, rc, ta > p.bcap);
 }
 
 // Per active block (one wave, lane = cell): its scene, the neighbour table
@@ -3782,9 +3841,16 @@ void launch_copy(const float4* src, float4* dst, int64_t n4, hipStream_t s) {
     hipLaunchKernelGGL(k_copy, dim3((unsigned)((n4 + WG - 1) / WG)), dim3(WG), 0, s, src, dst, n4);
 }
 void launch_scan(const KP& p, hipStream_t s) {
-    hipLaunchKernelGGL(k_scan_reduce, dim3(p.nparts), dim3(WG), 0, s, p);
-    hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(WG), 0, s, p);
-    hipLaunchKernelGGL(k_scan_apply, dim3(p.nparts), dim3(WG), 0, s, p);
+    constexpr int EACH = SCAN_ONE * SCAN_PER_THREAD;
+    if (p.nslots <= EACH) {
+        hipLaunchKernelGGL(k_scan_one<1>, dim3(1), dim3(SCAN_ONE), 0, s, p);
+    } else if (p.nslots <= 2 * EACH) {
+        hipLaunchKernelGGL(k_scan_one<2>, dim3(1), dim3(SCAN_ONE), 0, s, p);
+    } else {
+        hipLaunchKernelGGL(k_scan_reduce, dim3(p.nparts), dim3(WG), 0, s, p);
+        hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(WG), 0, s, p);
+        hipLaunchKernelGGL(k_scan_apply, dim3(p.nparts), dim3(WG), 0, s, p);
+    }
 }
 template <int D> void launch_block_setup(const KP& p, hipStream_t s, int grid) { hipLaunchKernelGGL(k_block_setup<D>, dim3(grid), dim3(WG), 0, s, p); }
 void launch_setup_order(const KP& p, hipStream_t s, int cell_groups) {

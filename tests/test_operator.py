@@ -188,3 +188,30 @@ def test_solves_of_two_handles_at_once():
         s.close()
         for f in ("x", "v", "F", "Jp", "ids"):
             assert np.array_equal(got[f], w[f]), f
+
+
+# cells an axis around which the binning's scan changes form: up to 4,096 and
+# 8,192 slots (3D 52 and 68 cells; 2D 496 has 4,225), alone and in a batch
+@pytest.mark.parametrize("dim,counts", [(3, 48), (3, 52), (3, 56), (3, 68), (3, 72), (3, 88), (3, 92), (2, 496), (2, 504), (2, 1000)])
+def test_scan_by_number_of_slots(dim, counts):
+    parts = [scattered(dim, counts, n, 60 + n, 0.02, 0.98) for n in (400, 3)]
+    dt = 0.5 * float(parts[0][0].max_dt)
+    b = M.Batch([q[0] for q in parts[:1]], [2000])
+    two = M.Batch([q[0] for q in parts], [2000, 100])
+    for h, m in ((b, 1), (two, 2)):
+        for k in range(m):
+            h.upload(k, *parts[k][1:])
+        h.initialize()
+        h.substep(dt)
+    for k, (d, x, v, m) in enumerate(parts):
+        o = O.Oracle(d, 8, 4, O.DOT_FP64 | O.SVD_FP64)
+        o.set_particles(x, v, m)
+        o.initialize()
+        o.advance_step(dt)
+        want = o.particles()
+        for got in [two.download(k)] + ([b.download(0)] if k == 0 else []):
+            assert np.array_equal(got["ids"], want["ids"])
+            for f in ("x", "v", "F", "Jp"):
+                assert rel(got[f], want[f]) < 1e-5, (k, f)
+    b.close()
+    two.close()
