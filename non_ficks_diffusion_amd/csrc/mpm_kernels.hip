@@ -2835,8 +2835,20 @@ __global__ __launch_bounds__(WG) void k_read_speeds(KP p, int* dst) {
 // tiles, for the scene's partials of s.q and, with r of the tile's nodes, for
 // those of r.r.  Everything that travels is its own flag: a place holds a bit
 // pattern that no value has until it is written, and its owner puts the pattern
-// back once every reader is known to have passed (two places, by parity of the
-// iteration; it is back before the owner's next s.q is out).
+// back once every reader is known to have passed.  Stores to two places are not
+// ordered, so a wave that polls for the place's next value has to know something
+// that the owner published behind a wait for the emptying store; those waits
+// are the drains before every s.q:
+//   tiles, s.q  two places each, by parity of the iteration.  Those of k - 1 are
+//         emptied in iteration k before its s.q; the next values in their places
+//         are polled in k + 1, behind the test of r.r k, which follows s.q k.
+//   r.r   two places.  r.r k - 1 is emptied in iteration k behind the sum of s.q
+//         k, so before s.q k + 1, which all that poll for r.r k + 1 have seen.
+//   r     three places: a tile's waves poll for r k as soon as their operator of
+//         k is stored, when all they know is r.r k - 1 (its test opened iteration
+//         k), and so s.q k - 1.  The place's last value r k - 3 was emptied in
+//         iteration k - 2, before s.q k - 1.  (Of two places, r k - 2 would be
+//         emptied in k - 1 behind its s.q: nothing they know follows that.)
 // Otherwise: work-group r of G takes blocks [r n / G, (r + 1) n / G) and counts
 // itself in at its scenes' counters before each wait.
 //
@@ -2959,10 +2971,14 @@ __device__ inline void cg_solve_resident(const KP& p, int blk0, int blk1, Operat
     if (done == ALL) return;
     if (K == 1 && full) op.open(blk0);
     const SceneParams& sc = p.scn[si];
-    // r of iteration k travels in one of two arrays, by parity
-    // (an offset: a choice between the two pointers became a table in scratch)
-    const int64_t apart = (int64_t)(reinterpret_cast<uintptr_t>(p.g_s) - reinterpret_cast<uintptr_t>(p.g_r)) / (int64_t)sizeof(float);
-    const auto r_place = [&](int k) { return p.g_r + (k & 1) * apart; };
+    // r of iteration k travels in g_s, g_r or the first words of the tiles (idle
+    // here, and more than the nodes), in turn from k = -1; `turn` is that of r k
+    // (offsets: a choice between pointers became a table in scratch)
+    static_assert((D + 1) * TN >= D * 64, "a block's tile place holds its nodes' r");
+    const int64_t to_r = (int64_t)(reinterpret_cast<uintptr_t>(p.g_r) - reinterpret_cast<uintptr_t>(p.g_s)) / (int64_t)sizeof(float);
+    const int64_t to_t = (int64_t)(reinterpret_cast<uintptr_t>(p.tiles) - reinterpret_cast<uintptr_t>(p.g_s)) / (int64_t)sizeof(float);
+    const auto r_place = [&](int t) { return p.g_s + (t == 0 ? 0 : t == 1 ? to_r : to_t); };
+    int turn = 0;
     if (b >= 0) {
         const int lane = lane0, n = b * 64 + lane;
         b0 = p.sst[si].block_begin;
@@ -2976,13 +2992,14 @@ __device__ inline void cg_solve_resident(const KP& p, int blk0, int blk1, Operat
             nx[nw][a][lane] = p.g_vs[a * p.gcap + n];
             nr[nw][a][lane] = p.g_r[a * p.gcap + n];
             ns[nw][a][lane] = 0.0f;
-            st_agent(r_place(0) + a * p.gcap + n, __uint_as_float(CG_EMPTY_FLOAT));
+            st_agent(r_place(1) + a * p.gcap + n, __uint_as_float(CG_EMPTY_FLOAT));
+            st_agent(r_place(2) + a * p.gcap + n, __uint_as_float(CG_EMPTY_FLOAT));
         }
     }
     // iteration -1 is the restart: the operator on x, r = b - A x
     double rho = 0.0;
-    for (int k = -1;; ++k) {
-        const int par = (k & 1) * CG_RESIDENT;
+    for (int k = -1;; ++k, turn = turn == 2 ? 0 : turn + 1) {
+        const int par = (k & 1) * CG_RESIDENT, before = turn == 0 ? 2 : turn - 1;
         const int lane = opaque(lane0), n = b * 64 + lane;
         op.tid = opaque(op.tid);
         // r of tile node `node`
@@ -2992,7 +3009,7 @@ __device__ inline void cg_solve_resident(const KP& p, int blk0, int blk1, Operat
             do {
                 waiting = false;
 #pragma unroll
-                for (int a = 0; a < D; ++a) rn[a] = ld_agent(r_place(k - 1) + a * p.gcap + node);
+                for (int a = 0; a < D; ++a) rn[a] = ld_agent(r_place(before) + a * p.gcap + node);
 #pragma unroll
                 for (int a = 0; a < D; ++a) waiting |= is_empty(rn[a]);
                 if (waiting) __builtin_amdgcn_s_sleep(4);
@@ -3073,6 +3090,7 @@ __device__ inline void cg_solve_resident(const KP& p, int blk0, int blk1, Operat
                 }
                 if (zero) r[a] = 0.0f;
             }
+            drain_stores();  // the places emptied above: r 0 is polled by waves that know no more than r.r -1
         } else {
             const float beta = sh_beta[k & 1][nw];
             float s[D];
@@ -3099,7 +3117,7 @@ __device__ inline void cg_solve_resident(const KP& p, int blk0, int blk1, Operat
                 clear_partial(p.bmax + par + b);
             }
 #pragma unroll
-            for (int a = 0; a < D; ++a) st_agent(r_place(k - 1) + a * p.gcap + n, __uint_as_float(CG_EMPTY_FLOAT));
+            for (int a = 0; a < D; ++a) st_agent(r_place(before) + a * p.gcap + n, __uint_as_float(CG_EMPTY_FLOAT));
             const double alpha_d = cg_alpha(rho, sq);
             if (b == b0 && lane == 0) cg_record_alpha(p.cg[si], sq, alpha_d);
             const float alpha = (float)alpha_d;
@@ -3117,7 +3135,7 @@ __device__ inline void cg_solve_resident(const KP& p, int blk0, int blk1, Operat
         mx = 0.0;
 #pragma unroll
         for (int a = 0; a < D; ++a) {
-            st_agent(r_place(k) + a * p.gcap + n, flagged(r[a]));
+            st_agent(r_place(turn) + a * p.gcap + n, flagged(r[a]));
             if (interior) {
                 sum += (double)r[a] * ((double)r[a] * m);
                 mx += (double)r[a] * (double)r[a];

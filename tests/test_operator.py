@@ -215,3 +215,32 @@ def test_scan_by_number_of_slots(dim, counts):
                 assert rel(got[f], want[f]) < 1e-5, (k, f)
     b.close()
     two.close()
+
+
+@pytest.mark.parametrize("dim,counts,n", [(3, 64, 130), (2, 256, 250), (3, 64, 8)])
+def test_one_block_to_a_work_group_repeats(dim, counts, n):
+    """The one-launch solve with a block to a work-group, where waves poll for
+    their neighbours' r ahead of their scene's sum: launched and replayed over
+    many iterations, the same bit for bit whatever the work-groups' timing."""
+    d, x, v, m = scattered(dim, counts, n, 70)
+    dt = 0.5 * float(d.max_dt)
+    runs = []
+    for graph in (False, True, True):
+        s = M.Scene(d, 2 * n)
+        s.upload(x, v, m)
+        s.initialize()
+        s.use_graph(graph)
+        runs.append(s)
+    iterations = 0
+    for step in range(40):
+        stats = [s.substep(dt, stats=True) for s in runs]
+        iterations += stats[0]["cg_iterations"]
+        assert stats[0]["active_blocks"] <= 512
+        got = [s.download() for s in runs]
+        for k in (1, 2):
+            assert stats[k] == stats[0], step
+            for f in ("x", "v", "F", "Jp", "ids"):
+                assert np.array_equal(got[k][f], got[0][f]), (step, k, f)
+    assert iterations > 200
+    for s in runs:
+        s.close()
