@@ -2385,15 +2385,28 @@ struct NodeRows {
     }
 };
 
+// r = b - q, Project(r) at node n; r holds b (0 outside the interior)
+template <int D>
+__device__ inline void cg_restart_residual(const KP& p, const SceneParams& sc, int n, bool interior, const float* q, float* r) {
+    if (interior) {
+#pragma unroll
+        for (int a = 0; a < D; ++a) r[a] = r[a] - q[a];
+    }
+    if (project_zero<D>(p, sc, n)) {
+#pragma unroll
+        for (int a = 0; a < D; ++a) r[a] = 0.0f;
+    }
+}
+
 // CG restart of block b: q = dt^2/m q + x (Multiply_Helper), r = b - q,
-// Project(r); the block's r.r (M-weighted) and max |r|^2.  r goes to g_r and
-// s = 0, or with TO_S (where the pass may be taken again) r goes to g_s.
-template <int D, bool AGENT, bool TO_S>
-__device__ inline void cg_restart_block(const KP& p, const SceneParams& sc, int b, int lane, double& sum, double& mx) {
+// Project(r); the block's r.r (M-weighted) and max |r|^2.  STORE: q, r and s = 0
+// are stored, otherwise nothing is.
+template <int D, bool AGENT, bool STORE>
+__device__ inline void cg_restart_block(const KP& p, const SceneParams& sc, int b, int lane, float* q, double& sum, double& mx) {
     const int n = b * 64 + lane;
     const float sds = sc.dt * sc.dt;
     const bool interior = (p.g_flags[n] & MPM_FLAG_INTERIOR_DEV) != 0;
-    float q[D], rv[D];
+    float rv[D];
     gather_node_tiles<D, D, AGENT>(p, sc, n, q);
 #pragma unroll
     for (int a = 0; a < D; ++a) rv[a] = p.g_r[a * p.gcap + n];
@@ -2401,20 +2414,16 @@ __device__ inline void cg_restart_block(const KP& p, const SceneParams& sc, int 
     if (interior) {
         const float cm = sds / mn;
 #pragma unroll
+        for (int a = 0; a < D; ++a) q[a] = cm * q[a] + p.g_vs[a * p.gcap + n];
+    }
+    cg_restart_residual<D>(p, sc, n, interior, q, rv);
+    if (STORE) {
+#pragma unroll
         for (int a = 0; a < D; ++a) {
-            q[a] = cm * q[a] + p.g_vs[a * p.gcap + n];
-            rv[a] = rv[a] - q[a];
+            st<AGENT>(p.g_r + a * p.gcap + n, rv[a]);
+            st<AGENT>(p.g_s + a * p.gcap + n, 0.0f);
+            p.g_q[a * p.gcap + n] = q[a];
         }
-    }
-    if (project_zero<D>(p, sc, n)) {
-#pragma unroll
-        for (int a = 0; a < D; ++a) rv[a] = 0.0f;
-    }
-#pragma unroll
-    for (int a = 0; a < D; ++a) {
-        st<AGENT>((TO_S ? p.g_s : p.g_r) + a * p.gcap + n, rv[a]);
-        if (!TO_S) st<AGENT>(p.g_s + a * p.gcap + n, 0.0f);
-        p.g_q[a * p.gcap + n] = q[a];
     }
     sum = 0.0;
     mx = 0.0;
@@ -2429,14 +2438,14 @@ __device__ inline void cg_restart_block(const KP& p, const SceneParams& sc, int 
 }
 
 // Tile sum of the operator, q = dt^2/m q + s, Project(q) on block b; the
-// block's s.q.  FORM: this iteration's s = r + beta s is formed and stored
-// first (interior nodes).
+// block's s.q.  FORM: this iteration's s = r + beta s is formed and stored first
+// (interior nodes), and q is stored.
 template <int D, bool FORM, bool AGENT>
-__device__ inline void cg_product_block(const KP& p, const SceneParams& sc, int b, int lane, float beta, int k, double& sum) {
+__device__ inline void cg_product_block(const KP& p, const SceneParams& sc, int b, int lane, float beta, int k, float* q, double& sum) {
     const float sds = sc.dt * sc.dt;
     const int n = b * 64 + lane;
     const bool interior = (p.g_flags[n] & MPM_FLAG_INTERIOR_DEV) != 0;
-    float q[D], sv[D], rv[D];
+    float sv[D], rv[D];
     // s, r and m load alongside the flags and the tile gather (every node of
     // an active block has them; only interior ones use them)
     const float mn = p.g_m[n];
@@ -2461,8 +2470,10 @@ __device__ inline void cg_product_block(const KP& p, const SceneParams& sc, int 
 #pragma unroll
         for (int a = 0; a < D; ++a) q[a] = 0.0f;
     }
+    if (FORM) {
 #pragma unroll
-    for (int a = 0; a < D; ++a) p.g_q[a * p.gcap + n] = q[a];
+        for (int a = 0; a < D; ++a) p.g_q[a * p.gcap + n] = q[a];
+    }
     sum = 0.0;
     double mx = 0.0;
     if (interior) {
@@ -2502,7 +2513,11 @@ __device__ inline void cg_record_alpha(CGState& cg, double sq, double alpha) {
 // that has waited for too long while some are missing closes the doors.  Then
 // those that hold a ticket wait for one another, share all groups by ticket and
 // start again (the partials that are there already are the same), and those
-// that come later leave.  (A door is one word: tickets taken, and once it is
+// that come later leave.  They may come when the others have long finished, so
+// nothing is stored before the ticket is known; and a block that one ticket
+// holder has begun may end with another, on an XCD whose stores are not ordered
+// with the first one's, so what is stored before all are settled (q) is the
+// same whoever stores it.  (A door is one word: tickets taken, and once it is
 // closed a bit and how many had been taken by then.  The first door to close
 // does so while one of its tickets is missing, so that nobody ever sees all of
 // them taken; the others follow.)
@@ -2678,14 +2693,15 @@ __global__ __launch_bounds__(NGW, 6) void k_cg_node(KP p, int k) {
     NodeRows<D, false> v;
     double t[2];  // the scene's sum (a run's first wave)
     for (bool settled = false;; settled = true) {
-        // q and s.q (restart: r, kept in g_s, and r.r)
+        // q and s.q (restart: q and r.r)
         for (int g = first; g < end; g += step) {
             take(g);
+            float q[D];
             if (b >= 0) {
                 const SceneParams& sc = p.scn[si];
                 double sum, mx = 0.0;
-                if (RESTART) cg_restart_block<D, false, true>(p, sc, b, lane, sum, mx);
-                else cg_product_block<D, false, false>(p, sc, b, lane, 0.0f, k, sum);
+                if (RESTART) cg_restart_block<D, false, false>(p, sc, b, lane, q, sum, mx);
+                else cg_product_block<D, false, false>(p, sc, b, lane, 0.0f, k, q, sum);
                 if (lane == 0) {
                     ws[wv] = sum;
                     wm[wv] = mx;
@@ -2697,6 +2713,10 @@ __global__ __launch_bounds__(NGW, 6) void k_cg_node(KP p, int k) {
             }
             __syncthreads();
             if (sh_ticket >= CG_DOOR_CLOSED) return;
+            if (b >= 0) {
+#pragma unroll
+                for (int a = 0; a < D; ++a) p.g_q[a * p.gcap + b * 64 + lane] = q[a];
+            }
             if (b >= 0 && wv == head) publish(First{}, first_sums, g);
             __syncthreads();
         }
@@ -2786,10 +2806,11 @@ __global__ __launch_bounds__(NGW, 6) void k_cg_node(KP p, int k) {
         }
         __syncthreads();
         if (b >= 0 && RESTART) {
+            cg_restart_residual<D>(p, p.scn[si], b * 64 + lane, v.interior, v.q, v.r);
 #pragma unroll
             for (int a = 0; a < D; ++a) {
-                p.g_r[a * p.gcap + b * 64 + lane] = v.s[a];
-                if (sh_fin[head]) p.g_s[a * p.gcap + b * 64 + lane] = 0.0f;  // no direction was taken
+                p.g_r[a * p.gcap + b * 64 + lane] = v.r[a];
+                p.g_s[a * p.gcap + b * 64 + lane] = sh_fin[head] ? 0.0f : v.r[a];  // (done: no direction was taken)
             }
         } else if (b >= 0 && !sh_fin[head] && v.interior) {
 #pragma unroll
@@ -3236,8 +3257,9 @@ __device__ inline void cg_solve_shared(const KP& p, int w0, int w1, int n, int g
             for_runs(p, w0, w1, [&](int si, int e, int r, int b) {
                 if ((done >> r) & 1) return;
                 for (b += wv; b < e; b += CGW / 64) {
+                    float q[D];
                     double sum, mx;
-                    cg_restart_block<D, true, false>(p, p.scn[si], b, lane, sum, mx);
+                    cg_restart_block<D, true, true>(p, p.scn[si], b, lane, q, sum, mx);
                     if (lane == 0) {
                         st_agent(p.bsum + b, sum);
                         st_agent(p.bmax + b, mx);
@@ -3254,8 +3276,9 @@ __device__ inline void cg_solve_shared(const KP& p, int w0, int w1, int n, int g
             if ((done >> r) & 1) return;
             const float beta = (float)ld_agent(&p.cg[si].beta);
             for (b += wv; b < e; b += CGW / 64) {
+                float q[D];
                 double sum;
-                cg_product_block<D, true, true>(p, p.scn[si], b, lane, beta, k, sum);
+                cg_product_block<D, true, true>(p, p.scn[si], b, lane, beta, k, q, sum);
                 if (lane == 0) st_agent(p.bsq + b, sum);
             }
         });

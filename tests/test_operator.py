@@ -244,3 +244,64 @@ def test_one_block_to_a_work_group_repeats(dim, counts, n):
     assert iterations > 200
     for s in runs:
         s.close()
+
+
+@pytest.mark.parametrize("counts,scenes", [(128, [(66000, 0.35, 0.65)]), (64, [(500, 0.4, 0.6), (66000, 0.2, 0.8), (300, 0.45, 0.5)])])
+def test_node_pass_on_a_busy_device(counts, scenes):
+    """Another handle's work-groups, of thousands of particles each, hold the
+    device for longer than the wait limits, so that work-groups of a node pass
+    start when those that found a place have shared the groups and finished.
+    Particles, statistics and the solve's own arrays are those of an idle device
+    bit for bit."""
+    parts = [scattered(3, counts, n, 40 + k, lo, hi) for k, (n, lo, hi) in enumerate(scenes)]
+    dt = 0.5 * float(parts[0][0].max_dt)
+
+    def drive(limit):
+        if len(parts) == 1:
+            h = M.Scene(parts[0][0], 3 * len(parts[0][1]))
+            h.upload(*parts[0][1:])
+        else:
+            h = M.Batch([q[0] for q in parts], [3 * len(q[1]) for q in parts])
+            for k, q in enumerate(parts):
+                h.upload(k, *q[1:])
+        if limit is not None:
+            h.set_wait_limit(limit)
+        h.initialize()
+        h.use_graph(True)
+        out = []
+        for _ in range(4):
+            h.substep(dt)
+            if len(parts) == 1:
+                out.append([{**h.download(), "stats": h.stats(), "r": h.read_grid(M.CH_CG_R), "s": h.read_grid(M.CH_CG_S),
+                             "q": h.read_grid(M.CH_CG_Q)}])
+            else:
+                out.append([{**h.download(k), "stats": h.stats(k)} for k in range(len(parts))])
+        h.close()
+        return out
+
+    want = drive(None)
+    d, x, v, m = M.scene_generate("two_balls", 96, 5, 1_000_000)
+    busy = M.Scene(d, len(m))
+    busy.upload(x, v, m)
+    busy.initialize()
+    stop = threading.Event()
+
+    def hold():
+        while not stop.is_set():
+            busy.substep(0.1 * float(d.max_dt))
+
+    other = threading.Thread(target=hold)
+    other.start()
+    try:
+        got = [drive(None), drive(0)]
+    finally:
+        stop.set()
+        other.join()
+        busy.close()
+    for run, steps in enumerate(got):
+        for step, (a, b) in enumerate(zip(steps, want)):
+            for k in range(len(parts)):
+                assert a[k]["stats"] == b[k]["stats"], (run, step, k)
+                for f in a[k]:
+                    if f != "stats":
+                        assert np.array_equal(a[k][f], b[k][f]), (run, step, k, f)
