@@ -954,6 +954,10 @@ __device__ inline void quat_of(const float* U, float* q) {
     const float n = 1.0f / sqrtf(w * w + x * x + y * y + z * z);
     q[0] = w * n; q[1] = x * n; q[2] = y * n; q[3] = z * n;
 }
+// The operator's and the solve's arithmetic is compiled into several kernels and
+// forms: products and sums fuse as written (contract(on)) and not as each one's
+// code around them happens to allow, so that all of them round alike.
+#pragma clang fp contract(on)
 __device__ inline void rot_of(const float* q, float* U) {
     const float w = q[0], x = q[1], y = q[2], z = q[3];
     U[0] = 1.0f - 2.0f * (y * y + z * z); U[1] = 2.0f * (x * y - w * z);        U[2] = 2.0f * (x * z + w * y);
@@ -985,6 +989,8 @@ __device__ inline void rotate_out(const float* U, const float* Ah, float* out) {
 #pragma unroll
         for (int j = 0; j < 3; ++j) out[i * 3 + j] = t[i * 3 + 0] * U[j * 3 + 0] + t[i * 3 + 1] * U[j * 3 + 1] + t[i * 3 + 2] * U[j * 3 + 2];
 }
+
+#pragma clang fp contract(fast)
 
 // The record of particle i.  3D: in the frame of U (F = U S V^T, R = U V^T)
 // the reference's force map T -> A = V0 F dP(T^T F)^T of fixed-corotated
@@ -1043,6 +1049,7 @@ __device__ inline void store_operator(const KP& p, int i, const StressState<D>& 
     for (int k = 0; k < OpRec<D>::W / 4; ++k) dst[k] = make_float4(rec[4 * k], rec[4 * k + 1], rec[4 * k + 2], rec[4 * k + 3]);
 }
 
+#pragma clang fp contract(on)
 // The 2x2 block of pair (lo, hi) with third index k applied to
 // (Th_lo,hi, Th_hi,lo).
 __device__ inline void apply_pair(float A, float B, float slo, float shi, float sk, float tlh, float thl, float& alh,
@@ -1091,6 +1098,8 @@ __device__ inline void apply_operator(const float* rec, float scale, const float
     }
 }
 
+#pragma clang fp contract(fast)
+
 template <int D>
 __device__ inline void store_operator_eos(const KP& p, int i, float c, const float* xo) {
     float rec[OpRec<D>::W];
@@ -1114,6 +1123,7 @@ __device__ inline void store_operator_eos(const KP& p, int i, float c, const flo
     for (int k = 0; k < OpRec<D>::W / 4; ++k) dst[k] = make_float4(rec[4 * k], rec[4 * k + 1], rec[4 * k + 2], rec[4 * k + 3]);
 }
 
+#pragma clang fp contract(on)
 // ---------------------------------------------------------------------------
 // The CG operator's stencil in difference form.  Per axis the weights of the
 // three stencil nodes sum to one, so a field in a cell is
@@ -1385,6 +1395,8 @@ __device__ inline void add_cell_nodes(const float* M, int base, int lane, float*
         }
     }
 }
+
+#pragma clang fp contract(fast)
 
 // Weights of particle i; false if it is not in cell l of block bb (only after
 // particles moved without re-binning: the particle is skipped).
@@ -1886,6 +1898,7 @@ __global__ __launch_bounds__(WG) void k_grid_update(KP p) {
     }
 }
 
+#pragma clang fp contract(on)
 // ============================================================================
 // CG (Apply_Force's solve, MPM_Example.cpp:700-711) for every scene of the
 // batch at once: Hestenes-Stiefel CG in the M inner product with a restart
@@ -2233,47 +2246,43 @@ __device__ inline void wave_reduce2(double& sum, double& mx) {
     }
 }
 
-// Sum / max of `count` partials starting at `first`, in a fixed order
-// relative to `first`; the result is broadcast to every thread.
+// Sum / max of `count` partials starting at `first`, in await_partials' order (a
+// lane adds every 64th, then the lanes are added); the result is in every
+// thread.  buf: 2 NT doubles of LDS.
 template <int NT>
-__device__ inline void reduce_range(const double* sums, const double* maxs, int first, int count, double& sum,
+__device__ inline void reduce_range(const double* sums, const double* maxs, int first, int count, double* buf, double& sum,
                                     double& mx) {
     constexpr int U = 4;  // independent loads in flight per thread
-    double sa[U], ma[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) { sa[u] = 0.0; ma[u] = 0.0; }
-    for (int base = (int)threadIdx.x; base < count; base += U * NT) {
-        // the chunk's loads all go out before its first add (an index past
+    const int tid = (int)threadIdx.x, lane = tid & 63;
+    sum = 0.0;
+    mx = 0.0;
+    __syncthreads();
+    for (int base = 0; base < count; base += U * NT) {
+        // the round's loads all go out before its first add (an index past
         // the range reads the range's last entry and is not added)
         double vs[U], vm[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int j = min(base + u * NT, count - 1);
+            const int j = min(base + u * NT + tid, count - 1);
             vs[u] = ld_agent(sums + first + j);
             vm[u] = maxs ? ld_agent(maxs + first + j) : 0.0;
         }
 #pragma unroll
-        for (int u = 0; u < U; ++u)
-            if (base + u * NT < count) {
-                sa[u] += vs[u];
-                if (maxs) ma[u] = fmax(ma[u], vm[u]);
+        for (int u = 0; u < U; ++u) {
+            if (base + u * NT >= count) break;
+            const bool in = base + u * NT + tid < count;
+            buf[tid] = in ? vs[u] : 0.0;
+            buf[NT + tid] = in ? vm[u] : 0.0;
+            __syncthreads();
+#pragma unroll
+            for (int w = 0; w < NT / 64; ++w) {
+                sum += buf[w * 64 + lane];
+                mx = fmax(mx, buf[NT + w * 64 + lane]);
             }
+            __syncthreads();
+        }
     }
-    double s = 0.0, m = 0.0;
-#pragma unroll
-    for (int u = 0; u < U; ++u) { s += sa[u]; m = fmax(m, ma[u]); }
-    wave_reduce2(s, m);
-    __shared__ double ss[NT / 64], sm[NT / 64];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    __syncthreads();
-    if (lane == 0) { ss[wave] = s; sm[wave] = m; }
-    __syncthreads();
-    s = 0.0;
-    m = 0.0;
-#pragma unroll
-    for (int w = 0; w < NT / 64; ++w) { s += ss[w]; m = fmax(m, sm[w]); }
-    sum = s;
-    mx = m;
+    wave_reduce2(sum, mx);
 }
 
 // Convergence test of iteration k (Convergence_Norm, MPM_CG_System.h:241-249:
@@ -2838,9 +2847,9 @@ __global__ __launch_bounds__(WG) void k_read_speeds(KP p, int* dst) {
 // ============================================================================
 // The whole CG solve of every scene in one launch, for scenes too small to
 // fill the chip: there a launch's work is a few microseconds, and the launches
-// of an iteration cost more than it.  The iterations and their arithmetic are
-// those of the launched kernels (a partial per block, a scene's partials summed
-// in block order).
+// of an iteration cost more than it.  The iterations and a block's arithmetic are
+// those of the launched kernels; a scene's sums run over a partial per block, in
+// the order of await_partials whichever form is taken.
 //
 // Work-groups share the blocks and wait for one another.  No wait depends on a
 // work-group that might not run: they enter through a door (cg_enter) that the
@@ -3239,7 +3248,7 @@ __device__ inline void cg_solve_shared(const KP& p, int w0, int w1, int n, int g
                 const int b0 = p.sst[si].block_begin, b1 = p.sst[si].block_end;
                 const CGTestIn in = cg_test_in(p, si, k);
                 double rr, mx;
-                reduce_range<CGW>(p.bsum, p.bmax, b0, b1 - b0, rr, mx);
+                reduce_range<CGW>(p.bsum, p.bmax, b0, b1 - b0, reinterpret_cast<double*>(S.coef), rr, mx);
                 if (cg_test(p, si, k, rr, mx, b == b0 && threadIdx.x == 0, beta, in)) {
                     done |= 1ull << r;
                     return;
@@ -3289,14 +3298,9 @@ __device__ inline void cg_solve_shared(const KP& p, int w0, int w1, int n, int g
             const int b0 = p.sst[si].block_begin, b1 = p.sst[si].block_end;
             const double rho = ld_agent(&p.cg[si].rho_hist[k & 1]);
             double sq, unused;
-            reduce_range<CGW>(p.bsq, nullptr, b0, b1 - b0, sq, unused);
-            const double alpha = sq != 0.0 ? rho / sq : (double)FLT_MAX;
-            if (b == b0 && threadIdx.x == 0) {
-                CGState& cg = p.cg[si];
-                cg.sq = sq;
-                cg.alpha = alpha;
-                cg.multiplies += 1;
-            }
+            reduce_range<CGW>(p.bsq, nullptr, b0, b1 - b0, reinterpret_cast<double*>(S.coef), sq, unused);
+            const double alpha = cg_alpha(rho, sq);
+            if (b == b0 && threadIdx.x == 0) cg_record_alpha(p.cg[si], sq, alpha);
             for (b += wv; b < e; b += CGW / 64) {
                 double sum, mx;
                 NodeRows<D, true> v;
@@ -3346,6 +3350,8 @@ __global__ __launch_bounds__(CGW, 4) void k_cg_solve(KP p) {
         cg_solve_shared<D>(p, w0, w1, n, g, S);
     }
 }
+
+#pragma clang fp contract(fast)
 
 // ============================================================================
 // G2P (MPM_Example.cpp:631-660): PIC/FLIP velocity, F and X update, removal

@@ -305,3 +305,69 @@ def test_node_pass_on_a_busy_device(counts, scenes):
                 for f in a[k]:
                     if f != "stats":
                         assert np.array_equal(a[k][f], b[k][f]), (run, step, k, f)
+
+
+def solved(parts, graph, limit, steps):
+    """Particles, statistics and (one scene) the solve's arrays after each
+    substep, and the active blocks of all scenes after the first."""
+    dt = 0.5 * float(parts[0][0].max_dt)
+    if len(parts) == 1:
+        h = M.Scene(parts[0][0], 2 * len(parts[0][1]))
+        h.upload(*parts[0][1:])
+    else:
+        h = M.Batch([q[0] for q in parts], [2 * len(q[1]) for q in parts])
+        for k, q in enumerate(parts):
+            h.upload(k, *q[1:])
+    if limit is not None:
+        h.set_wait_limit(limit)
+    h.initialize()
+    h.use_graph(graph)
+    out = []
+    for _ in range(steps):
+        h.substep(dt)
+        if len(parts) == 1:
+            out.append([{**h.download(), "stats": h.stats(), "r": h.read_grid(M.CH_CG_R), "s": h.read_grid(M.CH_CG_S),
+                         "q": h.read_grid(M.CH_CG_Q)}])
+        else:
+            out.append([{**h.download(k), "stats": h.stats(k)} for k in range(len(parts))])
+    h.close()
+    return out, sum(o["stats"]["active_blocks"] for o in out[0])
+
+
+def assert_same_bits(got, want, where):
+    for f in set(got) & set(want):
+        if f == "stats":
+            assert got[f] == want[f], where
+        else:
+            assert np.array_equal(got[f], want[f]), (where, f)
+
+
+# (dimension, cells, particles of each scene, blocks): one scene with a block to a
+# work-group and with two, two and three scenes with two, and ranges of blocks
+@pytest.mark.parametrize("graph", [False, True])
+@pytest.mark.parametrize("dim,counts,sizes,blocks", [
+    (3, 64, [130], (1, 512)), (2, 256, [250], (1, 512)), (3, 64, [250], (513, 1024)), (3, 64, [130, 130], (513, 1024)),
+    (2, 256, [300, 3, 250], (513, 1024)), (3, 64, [250, 5, 300], (1025, 4096))])
+def test_one_launch_solve_with_few_work_groups(dim, counts, sizes, blocks, graph):
+    """With a wait limit of zero the solve's door closes on those that happen to
+    run: they share the blocks and end with the same bits."""
+    parts = [scattered(dim, counts, n, 80 + k) for k, n in enumerate(sizes)]
+    want, nb = solved(parts, graph, None, 3)
+    assert blocks[0] <= nb <= blocks[1]
+    got, _ = solved(parts, graph, 0, 3)
+    for step in range(3):
+        assert got[step][0]["stats"]["cg_iterations"] > 3
+        for k in range(len(parts)):
+            assert_same_bits(got[step][k], want[step][k], (step, k))
+
+
+@pytest.mark.parametrize("dim,counts,n", [(3, 64, 130), (2, 256, 250)])
+def test_one_and_two_blocks_to_a_work_group(dim, counts, n):
+    """A scene alone (a block to a work-group) and in a batch (two): the
+    same bits over many iterations."""
+    parts = [scattered(dim, counts, n, 70 + k) for k in range(2)]
+    alone, nb = solved(parts[:1], True, None, 30)
+    both, nb2 = solved(parts, True, None, 30)
+    assert nb <= 512 < nb2 <= 1024
+    for step in range(30):
+        assert_same_bits(both[step][0], alone[step][0], step)
