@@ -597,8 +597,8 @@ int fill_stats(mpm_context* c, int s, mpm_step_stats* out) {
 void size_context(mpm_context* c) {
     c->gcap = (int64_t)c->bcap * 64;
     c->nparts = (c->nslots + mpm::SCAN_TILE - 1) / mpm::SCAN_TILE;
-    // CG partials: one per block, or the node pass's pairs per group of blocks and scene
-    c->nred = (size_t)std::max(std::max(c->bcap, MAX_NODE_GROUPS), 2 * (c->bcap / 8 + 1 + c->nscenes));
+    // CG partials: one per block, or what the work-groups of a launch exchange
+    c->nred = (size_t)std::max(c->bcap, mpm::cg_exchange_places(c->bcap, c->nscenes));
     c->grid_particle = (int)std::min<int64_t>(((c->pcap + mpm::WG - 1) / mpm::WG + 7) / 8 * 8, 4096);
     c->grid_block = (int)std::min<int64_t>(((int64_t)c->bcap + 7) / 8 * 8, 8192);
     c->grid_op = c->grid_block;
@@ -1247,7 +1247,7 @@ int round8(int64_t v) { return (int)std::max<int64_t>(8, (v + 7) / 8 * 8); }
 
 int check_config(const mpm_context* c, const mpm_launch_config& g) {
     auto ok = [](int v, int hi) { return v >= 8 && v <= hi && v % 8 == 0; };
-    if (!ok(g.block_groups, 1 << 20) || !ok(g.node_groups, (int)std::min<size_t>(c->nred, MAX_NODE_GROUPS)) ||
+    if (!ok(g.block_groups, 1 << 20) || !ok(g.node_groups, MAX_NODE_GROUPS) ||
         !ok(g.particle_groups, 1 << 20) || !ok(g.operator_groups, 1 << 20))
         return mpm_set_error(MPM_E_INVALID, "launch config: work-group counts must be multiples of 8 in range "
                                             "(node_groups at most 2048)");
@@ -1389,7 +1389,7 @@ int autotune(mpm_context* c, const float* dts, mpm_launch_config& best) {
     }
     // per-node kernels
     cand.clear();
-    const int node_hi = (int)std::min<size_t>(c->nred, MAX_NODE_GROUPS);
+    const int node_hi = MAX_NODE_GROUPS;
     for (int g : {128, 256, 512, 1024, 2048})
         if (g <= node_hi && (g <= round8(h.nblocks / 4 + 8) || g == 128)) cand.push_back(g);
     if (std::find(cand.begin(), cand.end(), cur.node_groups) == cand.end()) cand.push_back(cur.node_groups);

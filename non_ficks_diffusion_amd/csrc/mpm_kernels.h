@@ -232,6 +232,19 @@ constexpr int CG_SOLVE_MAX_SCENES = 64;
 constexpr int CG_GROUPS = 512;     // its work-groups (two fit a CU)
 constexpr int CG_RESIDENT = 2 * CG_GROUPS;  // blocks up to which their state stays in the work-groups
 template <int D> void launch_cg_solve(const KP& p, hipStream_t s);
+
+// Places of what the CG's work-groups exchange (bsum, bmax and bsq hold as many):
+// the node pass's groups of NGB blocks, its partials (s.q; pairs of r.r and max
+// |r|^2), and the sums over chunks, a value and a pair for each of eight XCDs.
+constexpr int NGB = 8, CG_CHUNK_RUNS = 64;
+__host__ __device__ constexpr int cg_groups(int nblocks) { return (nblocks + NGB - 1) / NGB; }
+__host__ __device__ constexpr int cg_places(int ng, int nscenes) { return ng + nscenes; }
+__host__ __device__ constexpr int cg_chunk_places(int ng) { return (ng / (CG_CHUNK_RUNS / 2) + 17) / 16 * 16; }
+constexpr int cg_exchange_places(int bcap, int nscenes) {
+    const int ng = cg_groups(bcap), pairs = 2 * cg_places(ng, nscenes), chunks = 24 * cg_chunk_places(ng);
+    const int most = pairs > chunks ? pairs : chunks;
+    return most > 2 * CG_RESIDENT ? most : 2 * CG_RESIDENT;  // (k_cg_solve: a place per block and parity)
+}
 template <int D> void launch_g2p(const KP& p, hipStream_t s, int grid);
 template <int D> void launch_max_speed(const KP& p, hipStream_t s, int grid);
 template <int D> void launch_noalloc_load(const KP& p, hipStream_t s, int grid, const SceneParams& sp, const NoallocIn& a);

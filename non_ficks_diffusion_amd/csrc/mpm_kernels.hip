@@ -1919,12 +1919,10 @@ __device__ inline float cg_direction(float r, float s, float beta, int k) {
 //   bsum  the runs' partials of r.r and max |r|^2, in pairs,
 //   bmax  for scenes of many runs the sums over chunks of CG_CHUNK_RUNS of
 //         them, s.q and then the pairs, a copy per XCD.
-constexpr int NGW = 512, NGB = NGW / 64;
+constexpr int NGW = 512;
+static_assert(NGW == 64 * NGB, "a wave per block");
 constexpr int CG_NODE_GROUPS = 768;  // three of 512 threads a CU: all fit at once
-constexpr int CG_CHUNK_RUNS = 64, CG_DIRECT_RUNS = 192;  // (scenes of up to so many runs are summed directly)
-__device__ inline int cg_groups(int nblocks) { return (nblocks + NGB - 1) / NGB; }
-__device__ inline int cg_places(const KP& p, int ng) { return ng + p.nscenes; }
-__device__ inline int cg_chunk_places(int ng) { return (ng / (CG_CHUNK_RUNS / 2) + 17) / 16 * 16; }
+constexpr int CG_DIRECT_RUNS = 192;  // (scenes of up to so many runs are summed directly)
 
 // LDS of the CG operator's work-group of NT threads:
 //   coef  the block's coefficient rows, later the node contributions of every
@@ -2207,7 +2205,7 @@ __global__ __launch_bounds__(BWG, 4) void k_cg_force(KP p) {
         }
     }
     if (live <= 0) return;
-    const int ng = cg_groups(p.ctr->nblocks), places = cg_places(p, ng), chunks = 24 * cg_chunk_places(ng);
+    const int ng = cg_groups(p.ctr->nblocks), places = cg_places(ng, p.nscenes), chunks = 24 * cg_chunk_places(ng);
     for (int i = (int)blockIdx.x * BWG + (int)threadIdx.x; i < max(2 * places, chunks); i += (int)gridDim.x * BWG) {
         const double empty = __longlong_as_double((long long)CG_EMPTY);
         if (i < places) p.bsq[i] = empty;
