@@ -166,6 +166,7 @@ mpm::KP make_kp(const mpm_context* c) {
     p.gcap = c->gcap;
     p.tiles = c->tiles;
     p.cg_tiles = c->tiles + (int64_t)c->bcap * (c->D + 1) * tile_nodes(c->D);
+    p.cg_waits = reinterpret_cast<int*>(p.cg_tiles + 2 * (int64_t)std::min(c->bcap, mpm::CG_RESIDENT) * c->D * tile_nodes(c->D));
     p.ctr = c->ctr;
     p.bsum = c->bsum;
     p.bmax = c->bmax;
@@ -639,8 +640,8 @@ void layout_buffers(mpm_context* c, Take&& take) {
     take(&c->block_full, bcap);
     take(&c->cell_count, nslots * 64);
     take(&c->cell_start, bcap * 65 + 1);
-    // (the second part is KP::cg_tiles: one allocation, they cost a tenth of a millisecond each)
-    take(&c->tiles, (bcap * (D + 1) + 2 * std::min(bcap, (size_t)mpm::CG_RESIDENT) * D) * tile_nodes((int)D));
+    // (then KP::cg_tiles and cg_waits: one allocation, they cost a tenth of a millisecond each)
+    take(&c->tiles, (bcap * (D + 1) + 2 * std::min(bcap, (size_t)mpm::CG_RESIDENT) * D) * tile_nodes((int)D) + mpm::CG_WAIT_INTS);
     take(&c->scan_part, (size_t)2 * c->nparts);
     take(&c->g_m, gcap);
     take(&c->g_v, (size_t)D * gcap);

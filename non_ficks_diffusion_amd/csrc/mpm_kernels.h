@@ -143,6 +143,7 @@ struct KP {
     int64_t gcap;
     float* tiles;    // per active block, (D+1) * (B+2)^D floats
     float* cg_tiles;  // k_cg_solve: per block and parity of the iteration, D * (B+2)^D floats
+    int* cg_waits;    // k_cg_solve: CG_WAIT_INTS
     // control
     Counters* ctr;
     // partials of the CG: k_cg_solve a place per active block (r.r, max |r|^2,
@@ -231,6 +232,10 @@ template <int D> void launch_cg_node(const KP& p, hipStream_t s, int blocks, int
 constexpr int CG_SOLVE_MAX_SCENES = 64;
 constexpr int CG_GROUPS = 512;     // its work-groups (two fit a CU)
 constexpr int CG_RESIDENT = 2 * CG_GROUPS;  // blocks up to which their state stays in the work-groups
+// Counted waits of scenes that more than CG_WAIT_FLAT work-groups share: per set
+// eight counters, one over them and eight go-aheads, each on a line of its own.
+constexpr int CG_WAIT_FLAT = 64, CG_WAIT_LINE = 32, CG_WAIT_SET = 17 * CG_WAIT_LINE;
+constexpr int CG_WAIT_INTS = CG_GROUPS / CG_WAIT_FLAT * CG_WAIT_SET;
 template <int D> void launch_cg_solve(const KP& p, hipStream_t s);
 
 // Places of what the CG's work-groups exchange (bsum, bmax and bsq hold as many):
