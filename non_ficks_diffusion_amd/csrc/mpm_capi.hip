@@ -110,7 +110,8 @@ mpm::SceneParams scene_params(const mpm_scene_desc& d, int slot_base, int nslots
     return p;
 }
 
-// How many particles were uploaded: which forms of the kernels a substep takes.
+// Which forms of the kernels a substep takes: by how many particles were uploaded
+// and how many blocks the substep before the last had.
 enum SizeClass { SIZE_ONE_LAUNCH, SIZE_SPLIT, SIZE_LARGE };
 SizeClass size_class(const mpm_context* c);
 
@@ -172,6 +173,7 @@ mpm::KP make_kp(const mpm_context* c) {
     p.bmax = c->bmax;
     p.bsq = c->bsq;
     p.bu = c->bu;
+    p.blocks_out = c->blocks_out;
     return p;
 }
 
@@ -288,6 +290,7 @@ constexpr int CG_COVER = 1;
 // A done poll copies the first eight counters into a slot of POLL_INTS pinned
 // ints.
 constexpr int POLL_INTS = 8;
+constexpr int FDONE_INTS = offsetof(mpm::Counters, frame_ndone) / sizeof(int) + 1;
 enum { POLL_NBLOCKS = 0, POLL_OVERFLOW = 3, POLL_NDONE = 4, POLL_CG_ITERS = 7 };
 static_assert(offsetof(mpm::Counters, nblocks) == 0 && offsetof(mpm::Counters, overflow) == POLL_OVERFLOW * sizeof(int) &&
                   offsetof(mpm::Counters, cg_ndone) == POLL_NDONE * sizeof(int) &&
@@ -302,24 +305,39 @@ static_assert(offsetof(mpm::Counters, nblocks) == 0 && offsetof(mpm::Counters, o
 // 19.7 -> 14.9, twelve scenes of together 48k 20.1 -> 19.2; equal at 80k (7.9 and
 // 7.8, 6.1 and 6.4, 3.9 and 3.7); above, more blocks of particles meet in a
 // work-group and the launches win: 120k 8.5 -> 9.4 and 7.1 -> 7.8, four requests
-// of together 200k 112 -> 124.  The rule reads only what the caller uploaded, so
-// launched, replayed and repeated substeps take the same kernels.
+// of together 200k 112 -> 124.  And for up to the blocks that its work-groups keep
+// resident: beyond, where few particles lie scattered over many blocks, they
+// share ranges of blocks with counted waits, and the launches win (a substep of
+// 700 particles in 1,259 blocks 639 us launched, 1,156 in one launch; 2k in 1,646
+// 1,059 and 1,787; 60k in 13,670 6.5 and 12.6 ms).  The blocks are those of the
+// substep before the last, which the host knows without holding the device up
+// in launched and replayed substeps alike (choose_form): both take the same
+// kernels, and so does a repeated run.
 constexpr int64_t CG_SOLVE_MAX_PARTICLES = 65536;
 // P2G with a work-group per block: per launch 18.0 -> 9.8 us for balls of 3.8k
 // particles, 22.2 -> 11.1 fluid of 20k, 21.4 -> 16.4 two balls of 243k, 21.4 ->
 // 17.9 a dense slab of 333k; but 25.1 -> 28.6 for twelve scenes of together
 // 603k and 30.5 -> 37.2 for 1.0M, where the blocks alone fill the chip.
 constexpr int64_t P2G_SPLIT_MAX = 400000;
-SizeClass size_class(const mpm_context* c) {
+int64_t uploaded(const mpm_context* c, int& scenes) {
     int64_t n = 0;
-    int scenes = 0;
+    scenes = 0;
     for (int s = 0; s < c->nscenes; ++s) {
         if (c->pool && !c->entry_used[(size_t)s]) continue;
         n += c->sc[(size_t)s].n_uploaded;
         ++scenes;
     }
-    if (n <= CG_SOLVE_MAX_PARTICLES && scenes <= mpm::CG_SOLVE_MAX_SCENES) return SIZE_ONE_LAUNCH;
-    return n <= P2G_SPLIT_MAX ? SIZE_SPLIT : SIZE_LARGE;
+    return n;
+}
+// by its particles and scenes, whatever its blocks
+bool fits_one_launch(const mpm_context* c) {
+    int scenes;
+    return uploaded(c, scenes) <= CG_SOLVE_MAX_PARTICLES && scenes <= mpm::CG_SOLVE_MAX_SCENES;
+}
+SizeClass size_class(const mpm_context* c) {
+    if (fits_one_launch(c) && !c->many_blocks) return SIZE_ONE_LAUNCH;
+    int scenes;
+    return uploaded(c, scenes) <= P2G_SPLIT_MAX ? SIZE_SPLIT : SIZE_LARGE;
 }
 bool cg_in_one_launch(const mpm_context* c) { return size_class(c) == SIZE_ONE_LAUNCH; }
 
@@ -673,14 +691,16 @@ int allocate_context(mpm_context* c) {
     layout_buffers(c, [&](auto** ptr, size_t count) { A(dalloc(c, ptr, count)); });
     if (rc == MPM_OK) {
         void* hp = nullptr;
-        // coherent: k_poll and k_read_speeds store into it from the device
-        if (hipHostMalloc(&hp, (2 * POLL_INTS + 1 + (size_t)nscenes) * sizeof(int), hipHostMallocCoherent) != hipSuccess)
+        // coherent: k_poll, k_read_speeds and k_g2p_reduce store into it from the device
+        if (hipHostMalloc(&hp, (2 * POLL_INTS + 1 + (size_t)nscenes + 2) * sizeof(int), hipHostMallocCoherent) != hipSuccess)
             rc = mpm_set_error(MPM_E_HIP, "hipHostMalloc failed");
         c->h_done = (int*)hp;
         if (rc == MPM_OK && hipHostGetDevicePointer((void**)&c->d_done, hp, 0) != hipSuccess)
             rc = mpm_set_error(MPM_E_HIP, "hipHostGetDevicePointer failed");
         for (int k = 0; k < 2 && rc == MPM_OK; ++k)
-            if (hipEventCreateWithFlags(&c->done_ev[k], hipEventDisableTiming) != hipSuccess) rc = mpm_set_error(MPM_E_HIP, "hipEventCreate failed");
+            if (hipEventCreateWithFlags(&c->done_ev[k], hipEventDisableTiming) != hipSuccess ||
+                hipEventCreateWithFlags(&c->blocks_ev[k], hipEventDisableTiming) != hipSuccess)
+                rc = mpm_set_error(MPM_E_HIP, "hipEventCreate failed");
         hp = nullptr;
         if (rc == MPM_OK && hipHostMalloc(&hp, sizeof(float) * (size_t)nscenes, hipHostMallocDefault) != hipSuccess)
             rc = mpm_set_error(MPM_E_HIP, "hipHostMalloc failed");
@@ -688,8 +708,8 @@ int allocate_context(mpm_context* c) {
         if (rc == MPM_OK && hipEventCreateWithFlags(&c->dt_ev, hipEventDisableTiming) != hipSuccess)
             rc = mpm_set_error(MPM_E_HIP, "hipEventCreate failed");
         hp = nullptr;
-        // the overflow flag through the frame-done count (Counters::overflow .. frame_ndone)
-        if (rc == MPM_OK && hipHostMalloc(&hp, 4 * sizeof(int), hipHostMallocDefault) != hipSuccess)
+        // the active blocks through the frame-done count (Counters::nblocks .. frame_ndone)
+        if (rc == MPM_OK && hipHostMalloc(&hp, FDONE_INTS * sizeof(int), hipHostMallocDefault) != hipSuccess)
             rc = mpm_set_error(MPM_E_HIP, "hipHostMalloc failed");
         c->h_fdone = (int*)hp;
         if (rc == MPM_OK && hipEventCreateWithFlags(&c->fdone_ev, hipEventDisableTiming) != hipSuccess)
@@ -1073,6 +1093,28 @@ void invalidate_graphs(mpm_context* c) {
 // even, so a replay leaves the particle buffers at the parity it found.
 constexpr int FRAME_K = 4;
 
+// The form of the next substep's CG.  A replay's count is waited for until two
+// substeps later: by then the device has the next one queued.
+int choose_form(mpm_context* c) {
+    const int at = c->cur;
+    if (c->blocks_pending[at]) {
+        HIPCHECK(hipEventSynchronize(c->blocks_ev[at]));
+        c->blocks_pending[at] = false;
+        c->blocks_of[at] = c->h_done[2 * POLL_INTS + 1 + c->nscenes + at];
+    }
+    c->many_blocks = c->blocks_of[at] > mpm::CG_RESIDENT;
+    return MPM_OK;
+}
+// Both of the last substeps had so many blocks (the host has waited for them).
+void note_blocks(mpm_context* c, int blocks) {
+    for (int k = 0; k < 2; ++k) {
+        c->blocks_of[k] = blocks;
+        c->blocks_pending[k] = false;
+    }
+    c->blocks_seen = blocks;
+    c->many_blocks = blocks > mpm::CG_RESIDENT;
+}
+
 // The captured graph of a buffer parity: one for each size class.
 int graph_slot(const mpm_context* c, int parity) { return parity + 2 * size_class(c); }
 
@@ -1123,6 +1165,8 @@ int device_frames(mpm_context* c, const float* time, const float* target, float*
         ndone += st.done;
     }
     HIPCHECK(hipMemcpyAsync(c->frame, f.data(), sizeof(mpm::FrameState) * (size_t)n, hipMemcpyHostToDevice, c->stream));
+    const int rc = choose_form(c);
+    if (rc) return rc;
     while (ndone < n) {
         const int parity = c->cur;
         if (!c->fexec[graph_slot(c, parity)]) {
@@ -1133,15 +1177,14 @@ int device_frames(mpm_context* c, const float* time, const float* target, float*
         c->binned = false;
         c->ever_binned = true;
         c->stepped = true;
-        // one copy reads the overflow flag and the frame-done count
-        static_assert(offsetof(mpm::Counters, frame_ndone) == offsetof(mpm::Counters, overflow) + 3 * sizeof(int),
-                      "layout");
-        HIPCHECK(hipMemcpyAsync(c->h_fdone, &c->ctr->overflow, 4 * sizeof(int), hipMemcpyDeviceToHost, c->stream));
+        // one copy reads the active blocks, the overflow flag and the frame-done count
+        HIPCHECK(hipMemcpyAsync(c->h_fdone, &c->ctr->nblocks, FDONE_INTS * sizeof(int), hipMemcpyDeviceToHost, c->stream));
         HIPCHECK(hipEventRecord(c->fdone_ev, c->stream));
         HIPCHECK(hipEventSynchronize(c->fdone_ev));
         // a binning over the block capacity made the replayed substeps no-ops
-        if (c->h_fdone[0] != 0) return mpm_set_error(MPM_E_CAPACITY, "active blocks exceed the block capacity");
-        ndone = c->h_fdone[3];
+        if (c->h_fdone[POLL_OVERFLOW] != 0) return mpm_set_error(MPM_E_CAPACITY, "active blocks exceed the block capacity");
+        ndone = c->h_fdone[FDONE_INTS - 1];
+        note_blocks(c, c->h_fdone[POLL_NBLOCKS]);
     }
     HIPCHECK(hipMemcpy(f.data(), c->frame, sizeof(mpm::FrameState) * (size_t)n, hipMemcpyDeviceToHost));
     for (int s = 0; s < n; ++s) {
@@ -1168,11 +1211,13 @@ int graph_substep(mpm_context* c, const float* dts) {
     if (!c->gexec[graph_slot(c, parity)]) {
         const bool timing = c->timing;
         c->timing = false;
+        c->blocks_out = c->d_done + 2 * POLL_INTS + 1 + c->nscenes + parity;
         HIPCHECK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
         const int rc = c->D == 3 ? substep<3>(c, nullptr, true) : substep<2>(c, nullptr, true);
         hipGraph_t g = nullptr;
         const hipError_t e = hipStreamEndCapture(c->stream, &g);
         c->timing = timing;
+        c->blocks_out = nullptr;
         c->cur = parity;  // capture records launches only: the buffers have not moved
         if (rc != MPM_OK || e != hipSuccess) {
             if (g) (void)hipGraphDestroy(g);
@@ -1186,6 +1231,10 @@ int graph_substep(mpm_context* c, const float* dts) {
         }
     }
     HIPCHECK(hipGraphLaunch(c->gexec[graph_slot(c, parity)], c->stream));
+    if (fits_one_launch(c)) {
+        HIPCHECK(hipEventRecord(c->blocks_ev[parity], c->stream));
+        c->blocks_pending[parity] = true;
+    }
     c->cur = parity ^ 1;  // the replay binned once
     c->binned = false;
     c->ever_binned = true;
@@ -1199,11 +1248,13 @@ int do_substep(mpm_context* c, const float* dts) {
     int active = 0, last = -1;
     for (int s = 0; s < c->nscenes; ++s)
         if (dts[s] > 0.0f) { ++active; last = s; }
-    const bool small = cg_in_one_launch(c);
+    int rc = choose_form(c);
+    if (rc) return rc;
+    const int parity = c->cur;
+    const bool replay = c->graph && !c->emitted, small = cg_in_one_launch(c);
     const bool solo = !small && c->nscenes > 1 && active == 1 && c->sc[(size_t)last].n_uploaded >= SOLO_LAUNCHED_MIN;
-    int rc = c->graph && !c->emitted && !solo ? graph_substep(c, dts)
-             : c->D == 3                      ? substep<3>(c, dts)
-                                              : substep<2>(c, dts);
+    rc = replay && !solo ? graph_substep(c, dts) : c->D == 3 ? substep<3>(c, dts) : substep<2>(c, dts);
+    if (!replay || solo) c->blocks_of[parity] = c->blocks_seen;
     if (rc) return rc;
     for (int s = 0; s < c->nscenes; ++s)
         if (dts[s] > 0.0f) c->sc[(size_t)s].last_dt = dts[s];
@@ -1669,7 +1720,10 @@ int mpm_destroy(mpm_handle c) {
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     for (void* p : c->allocations) (void)hipFree(p);
     for (hipEvent_t e : c->ev) (void)hipEventDestroy(e);
-    for (int k = 0; k < 2; ++k) if (c->done_ev[k]) (void)hipEventDestroy(c->done_ev[k]);
+    for (int k = 0; k < 2; ++k) {
+        if (c->done_ev[k]) (void)hipEventDestroy(c->done_ev[k]);
+        if (c->blocks_ev[k]) (void)hipEventDestroy(c->blocks_ev[k]);
+    }
     if (c->h_done) (void)hipHostFree(c->h_done);
     invalidate_graphs(c);
     if (c->dt_ev) (void)hipEventDestroy(c->dt_ev);
@@ -1785,7 +1839,7 @@ int mpm_initialize(mpm_handle c) {
     mpm::Counters h{};
     rc = read_counters(c, h);
     if (rc) return rc;
-    c->blocks_seen = h.nblocks;
+    note_blocks(c, h.nblocks);
     // the particles need more active blocks than the handle stores: nothing
     // was built, and the handle waits for an upload that fits
     if (h.overflow) return mpm_set_error(MPM_E_CAPACITY, "mpm_initialize: active blocks exceed the block capacity");
@@ -2405,6 +2459,7 @@ int noalloc_substep(NoallocDevice& nd, const mpm_scene_desc& d, int64_t n, float
     c->graph = false;
     c->timing = false;
     c->blocks_seen = 0;
+    c->many_blocks = false;
     c->emitted = true;  // every call runs Process_Waiting_Particles for particles of volume 0
     c->ever_binned = true;
     size_t off = 0;

@@ -65,7 +65,8 @@ struct mpm_context {
     unsigned* bu = nullptr;
     int cg_predict = 0;    // the next solve's first launch batch: the last solve's iterations plus one
     // pinned: per poll slot (8 ints) Counters::nblocks .. cg_iters; then the
-    // overflow flag and every scene's max |V|^2 (max_velocities)
+    // overflow flag and every scene's max |V|^2 (max_velocities); then two places
+    // for the active blocks of a replayed substep
     int* h_done = nullptr;
     int* d_done = nullptr;  // the device's address of h_done
     bool overflow_seen = false;  // the last substep's poll saw a block-capacity overflow
@@ -76,6 +77,14 @@ struct mpm_context {
     bool poll_pending[2] = {false, false};
     int poll_boundary[2] = {0, 0};
     int poll_older = 0, poll_target = 1, poll_max_it = 0;
+    // active blocks of the substep before the last (by buffer parity: binning swaps
+    // the buffers), which choose the CG's form; those of a replay are pending in
+    // pinned memory until its event
+    int blocks_of[2] = {0, 0};
+    bool blocks_pending[2] = {false, false};
+    hipEvent_t blocks_ev[2] = {nullptr, nullptr};
+    bool many_blocks = false;   // more than the one-launch solve keeps resident
+    int* blocks_out = nullptr;  // KP::blocks_out of a substep being captured
     int blocks_seen = 0;   // active blocks of the last binning whose counters the host has read (0: none)
     int grid_particle = 0, grid_block = 0, grid_node = 0;
     int op_mode = 0, grid_op = 0;  // CG operator: its mode (0 or 1, one kernel serves both) and work-groups

@@ -151,6 +151,7 @@ struct KP {
     double* bsum;
     double* bmax;
     double* bsq;
+    int* blocks_out;  // where G2P's reduction notes the active blocks (pinned; null: nowhere)
     unsigned* bu;    // 2 * bcap: per block max |V|^2 bits | removals (G2P)
 };
 

@@ -3545,6 +3545,7 @@ __global__ __launch_bounds__(BWG) void k_g2p(KP p) {
 // Scenes that did not advance keep their values.
 __global__ __launch_bounds__(WG) void k_g2p_reduce(KP p) {
     const int si = blockIdx.x;
+    if (si == 0 && threadIdx.x == 0 && p.blocks_out) *p.blocks_out = p.ctr->nblocks;
     if (!p.scn[si].active) return;
     const int b0 = p.sst[si].block_begin, b1 = p.sst[si].block_end;
     constexpr int U = 8;

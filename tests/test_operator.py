@@ -371,3 +371,39 @@ def test_one_and_two_blocks_to_a_work_group(dim, counts, n):
     assert nb <= 512 < nb2 <= 1024
     for step in range(30):
         assert_same_bits(both[step][0], alone[step][0], step)
+
+
+@pytest.mark.parametrize("n,lo,hi,many", [(300, 0.3, 0.7, False), (900, 0.1, 0.9, True), (900, 0.28, 0.72, None)])
+def test_form_of_the_solve_by_blocks(n, lo, hi, many):
+    """Few particles over more blocks than the one-launch solve keeps resident
+    take the launched kernels: from the start, or (None) from the third substep
+    after the particles have spread over so many; replays take the same
+    kernels as launched substeps, bit for bit, across the change."""
+    d, x, v, m = scattered(3, 64, n, 90, lo, hi)
+    if many is None:
+        v = (60 * (x - 0.5)).astype(np.float32)
+    runs = []
+    for graph in (False, True):
+        s = M.Scene(d, 20 * n)
+        s.upload(x, v, m)
+        s.initialize()
+        s.use_graph(graph)
+        runs.append(s)
+    runs[0].enable_timing()
+    blocks, launched, nodes = [], [], 0
+    for step in range(16):
+        st = [s.substep(1e-3, stats=True) for s in runs]
+        assert st[0] == st[1], step
+        blocks.append(st[0]["active_blocks"])
+        now = runs[0].kernel_times()["cg_node"][1]
+        launched.append(now > nodes)
+        nodes = now
+        a, b = (s.download() for s in runs)
+        for f in ("x", "v", "F", "Jp", "ids"):
+            assert np.array_equal(a[f], b[f]), (step, f)
+    if many is None:
+        assert min(blocks) <= 1024 < max(blocks)
+    assert launched[2:] == [k > 1024 for k in blocks[:-2]]
+    assert many is None or launched == [many] * 16
+    for s in runs:
+        s.close()

@@ -152,3 +152,28 @@ def test_noalloc_refuses_sizes_beyond_its_limits():
     with pytest.raises(M.MPMError) as e:
         M.substep_noalloc(d, 100, fake, fake, None, None, fake, fake, fake, 1e-3)
     assert e.value.code == E_INVALID
+
+
+@pytest.mark.parametrize("n", [600, 1000])
+def test_noalloc_substep_of_scattered_particles(n):
+    """More active blocks than the solve's work-groups keep resident: they share
+    ranges of blocks, where a handle takes the launched kernels."""
+    r = np.random.default_rng(n)
+    d, _, _, _ = M.scene_generate("two_balls", 64, 0)
+    d.cg_max_iterations = 200
+    x = r.uniform(0.1, 0.9, (n, 3)).astype(np.float32)
+    v = ((x - 0.5) @ r.uniform(-1.0, 1.0, (3, 3)) + 0.5).astype(np.float32)
+    m = np.full(n, 400.0 / 64 ** 3 / 8, np.float32)
+    dt = 0.5 * float(d.max_dt)
+    want, st = handle_path(d, x, v, m, dt)
+    assert 1024 < st["active_blocks"] <= 2048
+    got, st_got = noalloc_path(d, x, v, m, dt, Hip(), True)
+    check(got, st_got, want, st, f"{n} scattered particles")
+
+
+def test_noalloc_substep_at_its_limits():
+    d, x, v, m = M.scene_generate("slab", M.NOALLOC_MAX_COUNTS, 3, M.NOALLOC_MAX_PARTICLES)
+    assert len(m) == M.NOALLOC_MAX_PARTICLES
+    want, st = handle_path(d, x, v, m, 1e-3)
+    got, st_got = noalloc_path(d, x, v, m, 1e-3, Hip(), True)
+    check(got, st_got, want, st, "the most particles and cells")
