@@ -110,10 +110,9 @@ mpm::SceneParams scene_params(const mpm_scene_desc& d, int slot_base, int nslots
     return p;
 }
 
-// Which forms of the kernels a substep takes: by how many particles were uploaded
-// and how many blocks the substep before the last had.
-enum SizeClass { SIZE_ONE_LAUNCH, SIZE_SPLIT, SIZE_LARGE };
-SizeClass size_class(const mpm_context* c);
+// The form of the CG: by how many particles were uploaded and how many blocks the
+// substep before the last had.
+bool cg_in_one_launch(const mpm_context* c);
 
 int tile_nodes(int D) { return D == 3 ? 216 : 100; }
 mpm::KP make_kp(const mpm_context* c) {
@@ -123,8 +122,7 @@ mpm::KP make_kp(const mpm_context* c) {
     p.cg = c->cg;
     p.slot_scene = c->slot_scene;
     p.nscenes = c->nscenes;
-    p.one_launch = size_class(c) == SIZE_ONE_LAUNCH ? 1 : 0;
-    p.split_p2g = size_class(c) != SIZE_LARGE ? 1 : 0;
+    p.one_launch = cg_in_one_launch(c) ? 1 : 0;
     p.one_active = c->one_active ? 1 : 0;
     p.door_ticks = c->door_ticks;
     p.pcur = c->pbuf[c->cur];
@@ -314,32 +312,18 @@ static_assert(offsetof(mpm::Counters, nblocks) == 0 && offsetof(mpm::Counters, o
 // in launched and replayed substeps alike (choose_form): both take the same
 // kernels, and so does a repeated run.
 constexpr int64_t CG_SOLVE_MAX_PARTICLES = 65536;
-// P2G with a work-group per block: per launch 18.0 -> 9.8 us for balls of 3.8k
-// particles, 22.2 -> 11.1 fluid of 20k, 21.4 -> 16.4 two balls of 243k, 21.4 ->
-// 17.9 a dense slab of 333k; but 25.1 -> 28.6 for twelve scenes of together
-// 603k and 30.5 -> 37.2 for 1.0M, where the blocks alone fill the chip.
-constexpr int64_t P2G_SPLIT_MAX = 400000;
-int64_t uploaded(const mpm_context* c, int& scenes) {
+// by its particles and scenes, whatever its blocks
+bool fits_one_launch(const mpm_context* c) {
     int64_t n = 0;
-    scenes = 0;
+    int scenes = 0;
     for (int s = 0; s < c->nscenes; ++s) {
         if (c->pool && !c->entry_used[(size_t)s]) continue;
         n += c->sc[(size_t)s].n_uploaded;
         ++scenes;
     }
-    return n;
+    return n <= CG_SOLVE_MAX_PARTICLES && scenes <= mpm::CG_SOLVE_MAX_SCENES;
 }
-// by its particles and scenes, whatever its blocks
-bool fits_one_launch(const mpm_context* c) {
-    int scenes;
-    return uploaded(c, scenes) <= CG_SOLVE_MAX_PARTICLES && scenes <= mpm::CG_SOLVE_MAX_SCENES;
-}
-SizeClass size_class(const mpm_context* c) {
-    if (fits_one_launch(c) && !c->many_blocks) return SIZE_ONE_LAUNCH;
-    int scenes;
-    return uploaded(c, scenes) <= P2G_SPLIT_MAX ? SIZE_SPLIT : SIZE_LARGE;
-}
-bool cg_in_one_launch(const mpm_context* c) { return size_class(c) == SIZE_ONE_LAUNCH; }
+bool cg_in_one_launch(const mpm_context* c) { return fits_one_launch(c) && !c->many_blocks; }
 
 int max_cg_iterations(const mpm_context* c) {
     if (c->pool) return c->pool_cg_max;
@@ -1073,7 +1057,7 @@ int download_scene(mpm_context* c, int s, int64_t cap, float* x, float* v, float
 }
 
 void invalidate_graphs(mpm_context* c) {
-    for (int k = 0; k < 6; ++k) {
+    for (int k = 0; k < 4; ++k) {
         if (c->gexec[k]) {
             (void)hipGraphExecDestroy(c->gexec[k]);
             c->gexec[k] = nullptr;
@@ -1115,8 +1099,8 @@ void note_blocks(mpm_context* c, int blocks) {
     c->many_blocks = blocks > mpm::CG_RESIDENT;
 }
 
-// The captured graph of a buffer parity: one for each size class.
-int graph_slot(const mpm_context* c, int parity) { return parity + 2 * size_class(c); }
+// The captured graph of a buffer parity: one for each form of the CG.
+int graph_slot(const mpm_context* c, int parity) { return parity + (cg_in_one_launch(c) ? 2 : 0); }
 
 int capture_frame_graph(mpm_context* c, int parity) {
     const bool timing = c->timing;

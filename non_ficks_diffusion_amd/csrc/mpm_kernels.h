@@ -95,7 +95,6 @@ struct KP {
     const int* slot_scene;  // per global slot: the scene that owns it, -1 if none
     int nscenes;
     int one_launch;  // the solve is k_cg_solve
-    int split_p2g;   // P2G takes a work-group per block
     int one_active;  // a launched batch substep of one scene (the others count no operator applications)
     int door_ticks;  // how long work-groups that exchange wait for the others to start (100 MHz clock)
     // particles: field-major arrays of capacity pcap

@@ -1420,14 +1420,20 @@ __device__ inline bool cell_particle(const KP& p, const SceneParams& sc, int i, 
 // One wave per block (the waves of a work-group take different blocks and share
 // nothing); SPLIT: a work-group per block, its waves taking every NW-th
 // particle of a cell, where there are too few blocks to fill the chip and the
-// fullest cell's particles, one after another, are the time (P2G_SPLIT_MAX).
+// fullest cell's particles, one after another, are the time.  Up to
+// P2G_SPLIT_BLOCKS active blocks, read here, so that launched and replayed
+// substeps agree: 3.8k particles in 72 blocks 24.5 us whole, 13.5 split, 200k in
+// 805 22.9 and 15.0, 390k in 1,415 24.3 and 22.9, 390k in 1,576 24.6 and 21.6, 1.0M
+// in 986 56 and 40; but 1.0k in 1,869 11.4 and 15.8, 320k in 2,724 25.7 and 29.9,
+// 1.0M in 3,347 33.2 and 39.7, 200k scattered over 20,490 56 and 140 (four tiles of
+// which most of the nodes are empty).
 // ============================================================================
+constexpr int P2G_SPLIT_BLOCKS = 1536;
 template <int D, bool SPLIT>
-__global__ __launch_bounds__(BWG) void k_p2g(KP p) {
+__device__ inline void p2g_blocks(const KP& p, float (*tile_all)[(D + 1) * Dims<D>::LTN]) {
     using Dm = Dims<D>;
     constexpr int LTN = Dm::LTN, C = D + 1, TN = Dm::TN, LX = Dm::LX, LY = Dm::LY;
     constexpr int NS = D == 3 ? 27 : 9, EACH = SPLIT ? NW : 1;
-    __shared__ float tile_all[NW][C * LTN];
     const int c = threadIdx.x & 63, first = SPLIT ? (int)(threadIdx.x >> 6) : 0;
     float* mine = tile_all[threadIdx.x >> 6];
     int l[D];
@@ -1508,6 +1514,12 @@ __global__ __launch_bounds__(BWG) void k_p2g(KP p) {
         }
         MPM_STEP_FENCE();
     }
+}
+template <int D>
+__global__ __launch_bounds__(BWG) void k_p2g(KP p) {
+    __shared__ float tile_all[NW][(D + 1) * Dims<D>::LTN];
+    if (p.ctr->nblocks <= P2G_SPLIT_BLOCKS) p2g_blocks<D, true>(p, tile_all);
+    else p2g_blocks<D, false>(p, tile_all);
 }
 
 // Tile sum of P2G + Flag_Setup_Helper (Flag_Setup_Helper.h:25-35) +
@@ -3946,8 +3958,7 @@ void launch_read_speeds(const KP& p, hipStream_t s, int* dst) { hipLaunchKernelG
 void launch_poll(const KP& p, hipStream_t s, int* dst) { hipLaunchKernelGGL(k_poll, dim3(1), dim3(64), 0, s, p, dst); }
 template <int D> void launch_reorder(const KP& p, hipStream_t s, int grid) { hipLaunchKernelGGL(k_reorder<D>, dim3(grid), dim3(WG), 0, s, p); }
 template <int D> void launch_p2g(const KP& p, hipStream_t s, int grid) {
-    if (p.split_p2g) hipLaunchKernelGGL((k_p2g<D, true>), dim3(grid), dim3(BWG), 0, s, p);
-    else hipLaunchKernelGGL((k_p2g<D, false>), dim3(grid), dim3(BWG), 0, s, p);
+    hipLaunchKernelGGL(k_p2g<D>, dim3(grid), dim3(BWG), 0, s, p);
 }
 template <int D> void launch_normalize(const KP& p, hipStream_t s, int grid) { hipLaunchKernelGGL(k_normalize<D>, dim3(grid), dim3(WG), 0, s, p); }
 template <int D> void launch_init_volume(const KP& p, hipStream_t s, int grid) { hipLaunchKernelGGL(k_init_volume<D>, dim3(grid), dim3(BWG), 0, s, p); }

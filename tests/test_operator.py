@@ -407,3 +407,23 @@ def test_form_of_the_solve_by_blocks(n, lo, hi, many):
     assert many is None or launched == [many] * 16
     for s in runs:
         s.close()
+
+
+# (dimension, cells, particles, blocks): either side of the number of blocks up to
+# which P2G takes a work-group per block
+@pytest.mark.parametrize("dim,counts,n,blocks", [(3, 64, 730, (1500, 1536)), (3, 64, 744, (1537, 1560)), (2, 512, 1400, (1400, 1536)),
+                                                 (2, 512, 1700, (1537, 1800))])
+def test_p2g_by_number_of_blocks(dim, counts, n, blocks):
+    d, x, v, m = scattered(dim, counts, n, 95, 0.1, 0.9)
+    s = M.Scene(d, 20 * n)
+    s.upload(x, v, m)
+    s.initialize()
+    assert blocks[0] <= s.stats()["active_blocks"] <= blocks[1]
+    mass, vel = s.read_grid(M.CH_MASS), s.read_grid(M.CH_VELOCITY)  # of the initialisation
+    s.close()
+    o = O.Oracle(d, 8, 4, O.DOT_FP64 | O.SVD_FP64)
+    o.set_particles(x, v, m)
+    o.initialize()
+    want = o.grid(M.CH_MASS)
+    assert rel(mass, want) < 1e-5
+    assert rel(mass[..., None] * vel, want[..., None] * o.grid(M.CH_VELOCITY)) < 1e-5
