@@ -133,14 +133,16 @@ typedef struct mpm_context* mpm_handle;
  * whose loops run on CPU threads).  Every count is a multiple of 8 (the
  * XCDs of an MI355X). */
 typedef struct mpm_launch_config {
-    int32_t block_groups;     /* work-groups of the per-block kernels (P2G, forces, CG operator, G2P);
-                                 each takes about active_blocks / block_groups 4^3 blocks */
-    int32_t node_groups;      /* work-groups of the per-node kernels (normalize, grid update, CG vector
-                                 updates), at most 2048 */
+    int32_t block_groups;     /* work-groups of the per-block kernels (P2G, forces, G2P); each takes
+                                 about active_blocks / block_groups 4^3 blocks.  Until a count is set or
+                                 tuned it follows the active blocks */
+    int32_t node_groups;      /* work-groups of the per-node kernels (normalize, grid update), at most
+                                 2048; the CG's node pass follows the active blocks */
     int32_t particle_groups;  /* work-groups of the per-particle kernels (binning, reorder); particles
                                  per thread = live particles / (256 particle_groups) */
     int32_t operator_mode;    /* CG operator: 0 or 1; kept for callers that set it, one kernel serves both */
-    int32_t operator_groups;  /* work-groups of the CG operator (a block each at a time) */
+    int32_t operator_groups;  /* work-groups of the CG operator (a block each at a time), as block_groups;
+                                 unused where the whole CG is one launch */
     int32_t from_cache;       /* mpm_autotune: 1 if taken from the size-bucket cache */
     float block_ms, node_ms, particle_ms, operator_ms;  /* mpm_autotune: the chosen shapes' timing sequences */
 } mpm_launch_config;
@@ -349,15 +351,16 @@ int mpm_substep_noalloc(const mpm_scene_desc* desc, int64_t n, float* x, float* 
 /* ---- launch shapes, autotuner, captured substeps ------------------------ */
 /* (No counterpart in the reference.)  Current launch shapes of a handle. */
 int mpm_get_launch_config(mpm_handle h, mpm_launch_config* cfg);
-/* Sets the launch shapes (results do not depend on them). */
+/* Sets the launch shapes (results do not depend on them).  A count set as it is
+ * reported stays what it was. */
 int mpm_set_launch_config(mpm_handle h, const mpm_launch_config* cfg);
 /* How long the CG's work-groups, which exchange sums within a launch, wait for
  * the last of their launch to start before those that run share its work (in
  * 10 ns; the default, 5000, is far above the time a free device takes).
  * Results do not depend on it. */
 int mpm_set_wait_limit(mpm_handle h, int32_t ticks);
-/* Autotuner: times candidate work-group counts for the per-block,
- * per-node and per-particle kernels on the handle's current particles
+/* Autotuner: times candidate work-group counts for the CG operator (where the CG
+ * is not one launch), the per-block, per-node and per-particle kernels on the handle's current particles
  * (re-binned, with the grid and CG set up for dt; nscenes dts, or one dt for
  * a single scene) and keeps the fastest of each.  Particle state is not
  * advanced; grid and CG buffers are left as scratch, so call it between

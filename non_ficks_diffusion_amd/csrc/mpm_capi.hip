@@ -5,6 +5,7 @@
 
 #include <algorithm>
 #include <cfloat>
+#include <climits>
 #include <cstddef>
 #include <map>
 #include <mutex>
@@ -226,25 +227,28 @@ void set_step(mpm_context* c, const float* dts, float dt_all, bool force_active,
     }
 }
 
-// Work-groups of the kernels that take a block each: no more than the blocks
-// of the last binning the host has seen (a done poll, or the initialisation)
-// with a quarter on top, four times them in a captured sequence, which keeps its
-// grid for later substeps.  More blocks than that are taken in further rounds,
-// so the count only matters for speed: the avalanche's 3,340 blocks leave 4,850
-// of 8,192 work-groups without one, which cost an operator launch 5 us.
-int block_groups(const mpm_context* c, int configured) {
-    if (c->blocks_seen <= 0) return configured;
+// Work-groups of the kernels that take a block each, unless they were chosen: no
+// more than the blocks of the last binning the host has seen (a done poll, a
+// replay's note, the initialisation) with a quarter on top, four times them in a
+// captured sequence, which keeps its grid until the blocks outgrow it.  More
+// blocks than that are taken in further rounds, so the count only matters for
+// speed: the avalanche's 3,340 blocks leave 4,850 of 8,192 work-groups without
+// one, which cost an operator launch 5 us.
+int groups_for_blocks(const mpm_context* c, int most) {
+    if (c->blocks_seen <= 0) return most;
     const int64_t want = c->capturing ? 4 * (int64_t)c->blocks_seen + 256 : c->blocks_seen + c->blocks_seen / 4 + 64;
-    return (int)std::min<int64_t>(configured, (want + 7) / 8 * 8);
+    return (int)std::min<int64_t>(most, (want + 7) / 8 * 8);
 }
+int block_groups(const mpm_context* c) { return c->block_set ? c->grid_block : groups_for_blocks(c, c->grid_block); }
+int operator_groups(const mpm_context* c) { return c->op_set ? c->grid_op : groups_for_blocks(c, c->grid_op); }
 
 template <int D>
 void launch_operator(const mpm_context* c, const mpm::KP& p, bool restart) {
-    mpm::launch_cg_force<D>(p, c->stream, block_groups(c, c->grid_op), restart);
+    mpm::launch_cg_force<D>(p, c->stream, operator_groups(c), restart);
 }
 template <int D>
 void launch_node_pass(const mpm_context* c, const mpm::KP& p, int k, bool restart) {
-    mpm::launch_cg_node<D>(p, c->stream, block_groups(c, c->bcap), k, restart);
+    mpm::launch_cg_node<D>(p, c->stream, groups_for_blocks(c, c->bcap), k, restart);
 }
 
 // ---- stage sequences --------------------------------------------------------
@@ -254,7 +258,7 @@ void stage_bin(mpm_context* c) {
     timed(c, KC_BIN, [&] { mpm::launch_bin<D>(p, c->stream, c->grid_particle); });
     timed(c, KC_SCAN, [&] { mpm::launch_scan(p, c->stream); });
     timed(c, KC_SETUP, [&] {
-        mpm::launch_block_setup<D>(p, c->stream, block_groups(c, c->grid_block));
+        mpm::launch_block_setup<D>(p, c->stream, block_groups(c));
         mpm::launch_setup_order(p, c->stream, c->grid_particle);
     });
     timed(c, KC_REORDER, [&] { mpm::launch_reorder<D>(p, c->stream, c->grid_particle); });
@@ -267,14 +271,14 @@ void stage_bin(mpm_context* c) {
 template <int D>
 void stage_p2g(mpm_context* c) {
     mpm::KP p = make_kp(c);
-    timed(c, KC_P2G, [&] { mpm::launch_p2g<D>(p, c->stream, block_groups(c, c->grid_block)); });
+    timed(c, KC_P2G, [&] { mpm::launch_p2g<D>(p, c->stream, block_groups(c)); });
     timed(c, KC_NORMALIZE, [&] { mpm::launch_normalize<D>(p, c->stream, c->grid_node); });
 }
 
 template <int D>
 void stage_waiting(mpm_context* c) {
     mpm::KP p = make_kp(c);
-    timed(c, KC_INIT_VOLUME, [&] { mpm::launch_init_volume<D>(p, c->stream, block_groups(c, c->grid_block)); });
+    timed(c, KC_INIT_VOLUME, [&] { mpm::launch_init_volume<D>(p, c->stream, block_groups(c)); });
 }
 
 // particles from which a batch substep with one active scene is launched
@@ -447,7 +451,7 @@ int finish_cg_poll(mpm_context* c) {
 template <int D>
 void stage_g2p(mpm_context* c) {
     mpm::KP p = make_kp(c);
-    timed(c, KC_G2P, [&] { mpm::launch_g2p<D>(p, c->stream, block_groups(c, c->grid_block)); });
+    timed(c, KC_G2P, [&] { mpm::launch_g2p<D>(p, c->stream, block_groups(c)); });
     c->binned = false;
 }
 
@@ -464,11 +468,11 @@ int run_stage(mpm_context* c, int stage, float dt) {
             set_step(c, nullptr, dt, true, true);
             break;
         case MPM_STAGE_CONSTITUTIVE:
-            timed(c, KC_PFORCE, [&] { mpm::launch_particle_force<D>(p, c->stream, block_groups(c, c->grid_block), true, false); });
+            timed(c, KC_PFORCE, [&] { mpm::launch_particle_force<D>(p, c->stream, block_groups(c), true, false); });
             c->records_fresh = c->binned;
             break;
         case MPM_STAGE_EXPLICIT_FORCE:
-            timed(c, KC_PFORCE, [&] { mpm::launch_particle_force<D>(p, c->stream, block_groups(c, c->grid_block), false, true); });
+            timed(c, KC_PFORCE, [&] { mpm::launch_particle_force<D>(p, c->stream, block_groups(c), false, true); });
             timed(c, KC_GRID, [&] { mpm::launch_grid_update<D>(p, c->stream, c->grid_node, true, false, false, true); });
             break;
         case MPM_STAGE_COLLISION:
@@ -513,7 +517,7 @@ int substep(mpm_context* c, const float* dts, bool capture = false) {
     if (c->pool || c->emitted) {
         // scenes attached or particles added since the last substep:
         // Process_Waiting_Particles (every other scene's blocks return at once)
-        timed(c, KC_INIT_VOLUME, [&] { mpm::launch_init_volume<D>(p, c->stream, block_groups(c, c->grid_block)); });
+        timed(c, KC_INIT_VOLUME, [&] { mpm::launch_init_volume<D>(p, c->stream, block_groups(c)); });
         mpm::launch_clear_waiting(p, c->stream);
         if (!capture) {
             c->emitted = false;
@@ -523,7 +527,7 @@ int substep(mpm_context* c, const float* dts, bool capture = false) {
             }
         }
     }
-    timed(c, KC_PFORCE, [&] { mpm::launch_particle_force<D>(p, c->stream, block_groups(c, c->grid_block), true, true); });
+    timed(c, KC_PFORCE, [&] { mpm::launch_particle_force<D>(p, c->stream, block_groups(c), true, true); });
     c->records_fresh = true;
     timed(c, KC_GRID, [&] { mpm::launch_grid_update<D>(p, c->stream, c->grid_node, true, true, true, false); });
     int rc = stage_cg<D>(c, false, capture);
@@ -679,6 +683,7 @@ int allocate_context(mpm_context* c) {
         if (hipHostMalloc(&hp, (2 * POLL_INTS + 1 + (size_t)nscenes + 2) * sizeof(int), hipHostMallocCoherent) != hipSuccess)
             rc = mpm_set_error(MPM_E_HIP, "hipHostMalloc failed");
         c->h_done = (int*)hp;
+        if (rc == MPM_OK) std::memset(hp, 0, (2 * POLL_INTS + 1 + (size_t)nscenes + 2) * sizeof(int));
         if (rc == MPM_OK && hipHostGetDevicePointer((void**)&c->d_done, hp, 0) != hipSuccess)
             rc = mpm_set_error(MPM_E_HIP, "hipHostGetDevicePointer failed");
         for (int k = 0; k < 2 && rc == MPM_OK; ++k)
@@ -1152,12 +1157,12 @@ int device_frames(mpm_context* c, const float* time, const float* target, float*
     const int rc = choose_form(c);
     if (rc) return rc;
     while (ndone < n) {
-        const int parity = c->cur;
-        if (!c->fexec[graph_slot(c, parity)]) {
+        const int parity = c->cur, at = graph_slot(c, parity);
+        if (!c->fexec[at]) {
             const int rc = capture_frame_graph(c, parity);
             if (rc) return rc;
         }
-        HIPCHECK(hipGraphLaunch(c->fexec[graph_slot(c, parity)], c->stream));
+        HIPCHECK(hipGraphLaunch(c->fexec[at], c->stream));
         c->binned = false;
         c->ever_binned = true;
         c->stepped = true;
@@ -1191,8 +1196,8 @@ int graph_substep(mpm_context* c, const float* dts) {
     HIPCHECK(hipMemcpyAsync(c->d_dt, c->h_dt, sizeof(float) * (size_t)c->nscenes, hipMemcpyHostToDevice, c->stream));
     HIPCHECK(hipEventRecord(c->dt_ev, c->stream));
     c->dt_pending = true;
-    const int parity = c->cur;
-    if (!c->gexec[graph_slot(c, parity)]) {
+    const int parity = c->cur, at = graph_slot(c, parity);
+    if (!c->gexec[at]) {
         const bool timing = c->timing;
         c->timing = false;
         c->blocks_out = c->d_done + 2 * POLL_INTS + 1 + c->nscenes + parity;
@@ -1207,14 +1212,14 @@ int graph_substep(mpm_context* c, const float* dts) {
             if (g) (void)hipGraphDestroy(g);
             return rc != MPM_OK ? rc : mpm_set_error(MPM_E_HIP, std::string("hipStreamEndCapture: ") + hipGetErrorString(e));
         }
-        const hipError_t ei = hipGraphInstantiate(&c->gexec[graph_slot(c, parity)], g, nullptr, nullptr, 0);
+        const hipError_t ei = hipGraphInstantiate(&c->gexec[at], g, nullptr, nullptr, 0);
         (void)hipGraphDestroy(g);
         if (ei != hipSuccess) {
-            c->gexec[graph_slot(c, parity)] = nullptr;
+            c->gexec[at] = nullptr;
             return mpm_set_error(MPM_E_HIP, std::string("hipGraphInstantiate: ") + hipGetErrorString(ei));
         }
     }
-    HIPCHECK(hipGraphLaunch(c->gexec[graph_slot(c, parity)], c->stream));
+    HIPCHECK(hipGraphLaunch(c->gexec[at], c->stream));
     if (fits_one_launch(c)) {
         HIPCHECK(hipEventRecord(c->blocks_ev[parity], c->stream));
         c->blocks_pending[parity] = true;
@@ -1294,23 +1299,26 @@ int check_config(const mpm_context* c, const mpm_launch_config& g) {
 
 mpm_launch_config current_config(const mpm_context* c) {
     mpm_launch_config g{};
-    g.block_groups = c->grid_block;
+    g.block_groups = block_groups(c);
     g.node_groups = c->grid_node;
     g.particle_groups = c->grid_particle;
     g.operator_mode = c->op_mode;
-    g.operator_groups = c->grid_op;
+    g.operator_groups = operator_groups(c);
     return g;
 }
 
+// (counts that are set as they are reported stay as they were: fitted to the
+// blocks where nothing else was chosen)
 void apply_config(mpm_context* c, const mpm_launch_config& g) {
-    if (g.block_groups != c->grid_block || g.node_groups != c->grid_node || g.particle_groups != c->grid_particle ||
-        g.operator_mode != c->op_mode || g.operator_groups != c->grid_op)
-        invalidate_graphs(c);
-    c->grid_block = g.block_groups;
+    const bool block = g.block_groups != block_groups(c), op = g.operator_groups != operator_groups(c);
+    if (block || op || g.node_groups != c->grid_node || g.particle_groups != c->grid_particle) invalidate_graphs(c);
+    if (block) c->grid_block = g.block_groups;
+    if (op) c->grid_op = g.operator_groups;
+    c->block_set = c->block_set || block;
+    c->op_set = c->op_set || op;
     c->grid_node = g.node_groups;
     c->grid_particle = g.particle_groups;
     c->op_mode = g.operator_mode;
-    c->grid_op = g.operator_groups;
 }
 
 // Re-opens every scene's CG solve so that operator launches do work.
@@ -1357,8 +1365,9 @@ int time_median(mpm_context* c, Prep&& prep, Seq&& seq, float& ms_out) {
 
 // Times each candidate work-group count on a sequence of the kernels it
 // shapes, weighted as in a substep of a few CG iterations:
-//   per-block:    P2G + particle force + 8 CG operator applications;
-//   per-node:     normalize + grid update + 8 CG restart node passes;
+//   operator:     8 CG operator applications (not where the CG is one launch);
+//   per-block:    P2G + particle force;
+//   per-node:     normalize + grid update;
 //   per-particle: binning (bin, scan, block set-up, reorder) twice.
 // Every kernel of a sequence is idempotent on the binned particles, so the
 // particle state does not change.
@@ -1381,9 +1390,9 @@ int autotune(mpm_context* c, const float* dts, mpm_launch_config& best) {
     // a grid and CG set-up on the binned particles
     {
         mpm::KP p = make_kp(c);
-        mpm::launch_p2g<D>(p, c->stream, block_groups(c, c->grid_block));
+        mpm::launch_p2g<D>(p, c->stream, block_groups(c));
         mpm::launch_normalize<D>(p, c->stream, c->grid_node);
-        mpm::launch_particle_force<D>(p, c->stream, block_groups(c, c->grid_block), false, true);
+        mpm::launch_particle_force<D>(p, c->stream, block_groups(c), false, true);
         mpm::launch_grid_update<D>(p, c->stream, c->grid_node, true, true, true, false);
         launch_operator<D>(c, p, true);
         launch_node_pass<D>(c, p, 0, true);
@@ -1398,6 +1407,7 @@ int autotune(mpm_context* c, const float* dts, mpm_launch_config& best) {
     std::vector<int> ops = cand;
     if (std::find(ops.begin(), ops.end(), cur.operator_groups) == ops.end()) ops.push_back(cur.operator_groups);
     float best_ms = FLT_MAX;
+    if (cg_in_one_launch(c)) ops.clear();
     for (int g : ops) {
         const mpm::KP p = make_kp(c);
         float ms = 0.0f;

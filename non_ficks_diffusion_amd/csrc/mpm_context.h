@@ -88,6 +88,7 @@ struct mpm_context {
     int blocks_seen = 0;   // active blocks of the last binning whose counters the host has read (0: none)
     int grid_particle = 0, grid_block = 0, grid_node = 0;
     int op_mode = 0, grid_op = 0;  // CG operator: its mode (0 or 1, one kernel serves both) and work-groups
+    bool block_set = false, op_set = false;  // grid_block, grid_op were chosen (by the caller or the tuner)
     size_t nred = 0;           // entries of the reduction partial arrays
     // captured substeps: one graph per particle-buffer parity
     bool graph = false;

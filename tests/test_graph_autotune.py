@@ -265,3 +265,73 @@ def test_stage_timing_leaves_the_state_as_it_was():
     assert_same(a1, a0, "substep after stage timing")
     assert n1 == n0 and abs(t1 - t0) <= 1e-6 * t0, (n1, n0, t1, t0)
     assert_same(f1, f0, "frame after stage timing")
+
+
+def launched_cg_handle(n=66000, counts=64):
+    """A scene above the size whose CG is one launch."""
+    r = np.random.default_rng(11)
+    d, _, _, _ = M.scene_generate("two_balls", counts, 0)
+    d.cg_max_iterations = 30
+    x = r.uniform(0.3, 0.7, (n, 3)).astype(np.float32)
+    v = ((x - 0.5) @ r.uniform(-1.0, 1.0, (3, 3)) + 0.5).astype(np.float32)
+    s = M.Scene(d, n)
+    s.upload(x, v, np.full(n, 400.0 / counts ** 3 / 8, np.float32))
+    s.initialize()
+    return s, 0.3 * float(d.max_dt)
+
+
+def test_counts_follow_the_blocks_until_they_are_chosen():
+    s, dt = launched_cg_handle()
+    blocks = s.stats()["active_blocks"]
+    cfg = s.launch_config()
+    for key in ("block_groups", "operator_groups"):
+        assert blocks <= cfg[key] <= 1.25 * blocks + 72 and cfg[key] % 8 == 0, key
+    # set as reported: still following
+    s.set_launch_config(cfg["block_groups"], cfg["node_groups"], cfg["particle_groups"], operator_groups=cfg["operator_groups"])
+    s.use_graph(True)
+    s.substep(dt)
+    s.use_graph(False)
+    s.substep(dt)
+    assert s.launch_config()["block_groups"] <= 1.25 * s.stats()["active_blocks"] + 72
+    # chosen: as chosen
+    s.set_launch_config(4096, cfg["node_groups"], cfg["particle_groups"], operator_groups=40)
+    s.substep(dt)
+    got = s.launch_config()
+    assert got["block_groups"] == 4096 and got["operator_groups"] == 40
+    s.close()
+
+
+def test_autotune_times_the_operator_where_it_is_launched():
+    s, dt = launched_cg_handle()
+    cfg = s.autotune(dt)
+    assert cfg["operator_ms"] > 0
+    got = s.launch_config()
+    for key in ("block_groups", "node_groups", "particle_groups", "operator_groups"):
+        assert got[key] == cfg[key], key
+    s.close()
+    d, x, v, m = M.scene_generate("two_balls", 32, 0)
+    s = M.Scene(d, len(m))
+    s.upload(x, v, m)
+    s.initialize()
+    cfg = s.autotune(dt)  # its CG is one launch
+    assert cfg["operator_ms"] == 0 and cfg["block_ms"] > 0
+    s.close()
+
+
+@pytest.mark.parametrize("graph", [False, True])
+def test_launched_operator_with_fewer_groups_than_blocks(graph):
+    """A launched CG whose operator takes several blocks to a work-group."""
+    runs = []
+    for groups in (None, 24):
+        s, dt = launched_cg_handle()
+        if groups:
+            cfg = s.launch_config()
+            s.set_launch_config(groups, 64, cfg["particle_groups"], operator_groups=groups)
+            assert groups < s.stats()["active_blocks"] // 8
+        s.use_graph(graph)
+        for _ in range(3):
+            s.substep(dt)
+        runs.append(s)
+    assert_identical(runs[1].download(), runs[0].download(), groups)
+    for s in runs:
+        s.close()
