@@ -1099,9 +1099,24 @@ void note_blocks(mpm_context* c, int blocks) {
     for (int k = 0; k < 2; ++k) {
         c->blocks_of[k] = blocks;
         c->blocks_pending[k] = false;
+        c->h_done[2 * POLL_INTS + 1 + c->nscenes + k] = 0;
     }
     c->blocks_seen = blocks;
     c->many_blocks = blocks > mpm::CG_RESIDENT;
+}
+
+// Gives up a captured graph whose grids were made for far fewer blocks than the
+// last ones seen.
+int drop_outgrown(mpm_context* c, hipGraphExec_t& exec, int made_for) {
+    if (!exec || made_for <= 0 || c->blocks_seen <= made_for) return MPM_OK;
+    HIPCHECK(hipStreamSynchronize(c->stream));
+    (void)hipGraphExecDestroy(exec);
+    exec = nullptr;
+    return MPM_OK;
+}
+// The blocks that grids captured now are made for (0: any number).
+int capture_blocks(const mpm_context* c) {
+    return c->blocks_seen <= 0 ? 0 : (int)std::min<int64_t>(4 * (int64_t)c->blocks_seen + 256, INT_MAX);
 }
 
 // The captured graph of a buffer parity: one for each form of the CG.
@@ -1158,8 +1173,11 @@ int device_frames(mpm_context* c, const float* time, const float* target, float*
     if (rc) return rc;
     while (ndone < n) {
         const int parity = c->cur, at = graph_slot(c, parity);
+        int rc = drop_outgrown(c, c->fexec[at], c->fblocks[at]);
+        if (rc) return rc;
         if (!c->fexec[at]) {
-            const int rc = capture_frame_graph(c, parity);
+            c->fblocks[at] = capture_blocks(c);
+            rc = capture_frame_graph(c, parity);
             if (rc) return rc;
         }
         HIPCHECK(hipGraphLaunch(c->fexec[at], c->stream));
@@ -1197,7 +1215,14 @@ int graph_substep(mpm_context* c, const float* dts) {
     HIPCHECK(hipEventRecord(c->dt_ev, c->stream));
     c->dt_pending = true;
     const int parity = c->cur, at = graph_slot(c, parity);
+    // (as far as the replays before have noted it: only speed depends on it)
+    const volatile int* const noted = c->h_done + 2 * POLL_INTS + 1 + c->nscenes;
+    for (int k = 0; k < 2; ++k)
+        if (noted[k] > 0) c->blocks_seen = noted[k];
+    const int rc_drop = drop_outgrown(c, c->gexec[at], c->gblocks[at]);
+    if (rc_drop) return rc_drop;
     if (!c->gexec[at]) {
+        c->gblocks[at] = capture_blocks(c);
         const bool timing = c->timing;
         c->timing = false;
         c->blocks_out = c->d_done + 2 * POLL_INTS + 1 + c->nscenes + parity;

@@ -93,8 +93,9 @@ struct mpm_context {
     // captured substeps: one graph per particle-buffer parity
     bool graph = false;
     bool capturing = false;  // the launches are being captured (or stand for any later state)
-    // (two for each form of the CG)
+    // (two for each form of the CG), and the blocks its grids were made for
     hipGraphExec_t gexec[4] = {};
+    int gblocks[4] = {};
     float* d_dt = nullptr;     // per-scene dt read by a replayed graph
     float* h_dt = nullptr;     // pinned staging of d_dt
     hipEvent_t dt_ev = nullptr;
@@ -103,6 +104,7 @@ struct mpm_context {
     // buffer parity, pinned read-back of the frame-done count
     mpm::FrameState* frame = nullptr;
     hipGraphExec_t fexec[4] = {};
+    int fblocks[4] = {};
     int* h_fdone = nullptr;
     hipEvent_t fdone_ev = nullptr;
     // serving arena: scenes attach to free entries, slot ranges and particle space
