@@ -44,3 +44,46 @@ def test_download_is_the_upload_by_id(dim, n):
         with pytest.raises(M.MPMError):
             b.download(1, cap=len(keep) - 1)
     b.close()
+
+
+@pytest.mark.parametrize("dim", [2, 3])
+def test_download_with_ids_past_the_capacity(dim):
+    """Ids are not reused, so a scene that keeps losing and gaining particles
+    passes its capacity: the download then orders on the host, with the same
+    result."""
+    r = np.random.default_rng(dim)
+    d, _, _, _ = M.scene_generate("disk2d" if dim == 2 else "two_balls", 32, 0)
+    d.gravity[:] = (0.0,) * len(d.gravity)
+    d.nplanes = 0
+    dt = float(d.max_dt)
+    cap, stay, leave = 200, 10, 50
+    s = M.Scene(d, cap)
+    mass, x_of, alive = {}, {}, []
+    ids = 0
+    for step in range(6):
+        n = stay + leave
+        x = r.uniform(0.3, 0.7, (n, dim)).astype(np.float32)
+        v = np.zeros((n, dim), np.float32)
+        v[stay:] = 2.0 / dt  # leaves the domain in the substep
+        m = r.uniform(0.5, 1.0, n).astype(np.float32)
+        x[stay:] = 0.9 + 0.001 * (x[stay:] - 0.5)  # away from those that stay
+        if step == 0:
+            s.upload(x, v, m)
+            s.initialize()
+        else:
+            s.add_particles(x, v, m)
+        mass.update(zip(range(ids, ids + n), m))
+        x_of.update(zip(range(ids, ids + n), x))
+        alive += range(ids, ids + stay)
+        ids += n
+        s.substep(dt)
+        got = s.download()
+        assert got["ids"].tolist() == alive
+        assert np.array_equal(got["mass"], np.array([mass[k] for k in alive]))
+        assert np.abs(got["x"] - np.array([x_of[k] for k in alive])).max() < 1e-3
+        assert np.all(got["volume"] > 0) and not got["material"].any()
+        assert np.abs(got["F"] - np.eye(dim)).max() < 0.1 and np.abs(got["Jp"] - 1).max() < 0.1
+    assert ids > cap
+    with pytest.raises(M.MPMError):
+        s.download(cap=len(alive) - 1)
+    s.close()
