@@ -372,9 +372,9 @@ int mpm_set_wait_limit(mpm_handle h, int32_t ticks);
 int mpm_autotune(mpm_handle h, const float* dt, int32_t flags, mpm_launch_config* out);
 /* Captured substeps: with on != 0 every substep replays a HIP graph of its
  * whole launch sequence (captured at the first such substep, one graph per
- * particle-buffer parity), the CG with a fixed count of max(cg_max_iterations)
- * iterations whose kernels return at once for finished solves, and dts read
- * from device memory.  Results equal the launched substep's.  Needs CG caps
+ * particle-buffer parity and form of the CG), the CG as one launch or with a
+ * fixed count of max(cg_max_iterations) iterations whose kernels return at once
+ * for finished solves, and dts read from device memory.  Results equal the launched substep's.  Needs CG caps
  * of at most 256 iterations. */
 int mpm_set_graph(mpm_handle h, int32_t on);
 
@@ -433,7 +433,8 @@ typedef struct mpm_serve_config {
     int32_t max_scenes;          /* resident scenes at most */
     int32_t max_counts;          /* largest grid of a request, cells per axis */
     int32_t cg_max_iterations;   /* CG cap every request must stay within (<= 256) */
-    int64_t hbm_budget_bytes;    /* the arena is sized from it; admission stays within it */
+    int64_t hbm_budget_bytes;    /* the arena is sized from it (up to 6 MB that do not grow with it are
+                                    not counted); admission stays within it */
     int32_t graph;               /* replay captured substeps */
     int32_t keep_results;        /* keep finished requests' particles for mpm_serve_download */
     int32_t max_tick_substeps;   /* > 0: a tick also ends after this many substeps */

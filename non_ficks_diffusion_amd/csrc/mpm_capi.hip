@@ -338,9 +338,8 @@ int max_cg_iterations(const mpm_context* c) {
 
 // Apply_Force's implicit solve (MPM_Example.cpp:700-711) for every active
 // scene: CG set-up, restart (r = b - A x, Project) and iterations until every
-// scene's solve is done (converged or at its cap).  Batches reduce each
-// scene's block partials in per-scene kernels (five launches per iteration);
-// one scene needs no reducer launches (four per iteration).
+// scene's solve is done (converged or at its cap): one launch (cg_in_one_launch),
+// or two for the restart and two per iteration, the operator and the node pass.
 template <int D>
 int stage_cg(mpm_context* c, bool do_init, bool fixed = false) {
     mpm::KP p = make_kp(c);

@@ -20,10 +20,10 @@
 // sums, for every node, the (at most 2^D) tiles that cover it in a fixed
 // order.  There are no global atomics on the scatter path, and the
 // cross-block sum is deterministic.  Gathers load the tile once from the
-// 3^D neighbour blocks.  Node kernels run one wave per block; reductions
-// (CG dot products and norms, G2P's max speed) write one partial per block,
-// and a one-work-group-per-scene kernel sums a scene's block partials in a
-// fixed order.
+// 3^D neighbour blocks.  Node kernels run one wave per block.  Reductions sum a
+// scene's partials in a fixed order: G2P's max speed in a kernel of one
+// work-group per scene, the CG's dot products and norms within the launch that
+// forms them (k_cg_node, k_cg_solve).
 #include "mpm_kernels.h"
 #include <algorithm>
 
