@@ -955,14 +955,30 @@ __device__ inline void quat_of(const float* U, float* q) {
     q[0] = w * n; q[1] = x * n; q[2] = y * n; q[3] = z * n;
 }
 // The operator's and the solve's arithmetic is compiled into several kernels and
-// forms: products and sums fuse as written (contract(on)) and not as each one's
-// code around them happens to allow, so that all of them round alike.
+// forms: products and sums fuse as written (contract(on), and fmaf where the order
+// matters) and not as each one's code around them happens to allow, so that a
+// form and its fallback round alike.
 #pragma clang fp contract(on)
-__device__ inline void rot_of(const float* q, float* U) {
+// Which product of a rotation's sums of two is rounded on its own: the launched
+// operator and the one-launch solve with one and with two blocks to a work-group
+// each came to differ in this, and keep it, so that a scene's results stay what
+// they were.  (The solve's fallback, ROUND_EITHER, is told whose it is.)
+enum Rounding { ROUND_LAUNCHED, ROUND_ONE, ROUND_TWO, ROUND_EITHER };
+template <int R>
+__device__ inline void rot_of(const float* q, bool two, float* U) {
+    constexpr bool SOLVE = R != ROUND_LAUNCHED;
     const float w = q[0], x = q[1], y = q[2], z = q[3];
-    U[0] = 1.0f - 2.0f * (y * y + z * z); U[1] = 2.0f * (x * y - w * z);        U[2] = 2.0f * (x * z + w * y);
-    U[3] = 2.0f * (x * y + w * z);        U[4] = 1.0f - 2.0f * (x * x + z * z); U[5] = 2.0f * (y * z - w * x);
-    U[6] = 2.0f * (x * z - w * y);        U[7] = 2.0f * (y * z + w * x);        U[8] = 1.0f - 2.0f * (x * x + y * y);
+    const bool xy = R == ROUND_TWO || (R == ROUND_EITHER && two);
+    const float a = xy ? x : y, b = xy ? y : x;
+    U[0] = fmaf(-2.0f, SOLVE ? fmaf(y, y, z * z) : fmaf(z, z, y * y), 1.0f);
+    U[1] = 2.0f * fmaf(x, y, -(w * z));
+    U[2] = 2.0f * fmaf(x, z, w * y);
+    U[3] = 2.0f * fmaf(x, y, w * z);
+    U[4] = fmaf(-2.0f, SOLVE ? fmaf(x, x, z * z) : fmaf(z, z, x * x), 1.0f);
+    U[5] = 2.0f * (SOLVE ? fmaf(-w, x, y * z) : fmaf(y, z, -(w * x)));
+    U[6] = 2.0f * fmaf(x, z, -(w * y));
+    U[7] = 2.0f * (SOLVE ? fmaf(w, x, y * z) : fmaf(y, z, w * x));
+    U[8] = fmaf(-2.0f, fmaf(a, a, b * b), 1.0f);
 }
 
 // Ahat = U^T A U (3x3)
@@ -983,7 +999,10 @@ __device__ inline void rotate_out(const float* U, const float* Ah, float* out) {
 #pragma unroll
     for (int i = 0; i < 3; ++i)
 #pragma unroll
-        for (int j = 0; j < 3; ++j) t[i * 3 + j] = U[i * 3 + 0] * Ah[0 * 3 + j] + U[i * 3 + 1] * Ah[1 * 3 + j] + U[i * 3 + 2] * Ah[2 * 3 + j];
+        for (int j = 0; j < 3; ++j) {
+            const float u0 = U[i * 3], u1 = U[i * 3 + 1], a0 = Ah[j], a1 = Ah[3 + j];
+            t[i * 3 + j] = fmaf(U[i * 3 + 2], Ah[6 + j], j == 0 ? fmaf(u1, a1, u0 * a0) : fmaf(u0, a0, u1 * a1));
+        }
 #pragma unroll
     for (int i = 0; i < 3; ++i)
 #pragma unroll
@@ -1051,35 +1070,36 @@ __device__ inline void store_operator(const KP& p, int i, const StressState<D>& 
 
 #pragma clang fp contract(on)
 // The 2x2 block of pair (lo, hi) with third index k applied to
-// (Th_lo,hi, Th_hi,lo).
+// (Th_lo,hi, Th_hi,lo).  FIRST: the pair (0, 1).
+template <bool FIRST>
 __device__ inline void apply_pair(float A, float B, float slo, float shi, float sk, float tlh, float thl, float& alh,
                                   float& ahl) {
     const float sm = slo + shi;
     const float inv = __builtin_amdgcn_rcpf(sm);
     const float g = A * (sm - 1.0f) * inv;
     const float a = g * slo * slo, c = g * shi * shi;
-    const float b = slo * shi * (A * inv - B * sk);
-    alh = a * tlh + b * thl;
-    ahl = b * tlh + c * thl;
+    const float b = slo * shi * fmaf(A, inv, -(B * sk));
+    alh = FIRST ? fmaf(b, thl, a * tlh) : fmaf(a, tlh, b * thl);
+    ahl = fmaf(b, tlh, c * thl);
 }
 
 // A = scale L T from a particle's operator record (in registers)
-template <int D>
-__device__ inline void apply_operator(const float* rec, float scale, const float* T, float* A) {
+template <int D, int R>
+__device__ inline void apply_operator(const float* rec, float scale, bool two, const float* T, float* A) {
     constexpr int DD = D * D;
     if constexpr (D == 3) {
         const float s0 = rec[7], s1 = rec[8], s2 = rec[9];
         const float a2 = scale * rec[10], bl = scale * rec[11], pj = scale * rec[12], kappa = fmaf(scale, rec[13], pj);
         float U[9], Th[9], Ah[9];
-        rot_of(rec + 3, U);
+        rot_of<R>(rec + 3, two, U);
         rotate_in(U, T, Th);
         const float tr = kappa * (Th[0] + Th[4] + Th[8]);
         Ah[0] = fmaf(fmaf(a2 * s0, s0, -pj), Th[0], tr);
         Ah[4] = fmaf(fmaf(a2 * s1, s1, -pj), Th[4], tr);
         Ah[8] = fmaf(fmaf(a2 * s2, s2, -pj), Th[8], tr);
-        apply_pair(a2, bl, s0, s1, s2, Th[1], Th[3], Ah[1], Ah[3]);
-        apply_pair(a2, bl, s0, s2, s1, Th[2], Th[6], Ah[2], Ah[6]);
-        apply_pair(a2, bl, s1, s2, s0, Th[5], Th[7], Ah[5], Ah[7]);
+        apply_pair<true>(a2, bl, s0, s1, s2, Th[1], Th[3], Ah[1], Ah[3]);
+        apply_pair<false>(a2, bl, s0, s2, s1, Th[2], Th[6], Ah[2], Ah[6]);
+        apply_pair<false>(a2, bl, s1, s2, s0, Th[5], Th[7], Ah[5], Ah[7]);
         rotate_out(U, Ah, A);
     } else {
         const float* tri = rec + D;
@@ -1307,7 +1327,9 @@ __device__ inline void add_force_moments(const PackedForce<D>& f4, float* M) {
                 float* k = M + (i * 3 + j) * 3;
                 if (i != 1 || j != 1) {
                     k[0] = fmaf(a.w, z[j], fmaf(p.z, y[j], k[0]));
-                    k[1] += y[j];
+                    if (i == 1) k[1] = fmaf(j == 0 ? r.w : d2y, f[1], k[1]);
+                    else if (j == 1) k[1] = fmaf(i == 0 ? p.w : d2x, a.x, k[1]);
+                    else k[1] += y[j];
                     k[2] = fmaf(d2z, z[j], fmaf(r.z, y[j], k[2]));
                 } else {
                     k[0] = fmaf(a.w, z[j], k[0]);
@@ -1325,7 +1347,7 @@ __device__ inline void add_force_moments(const PackedForce<D>& f4, float* M) {
             float* k = M + i * 3;
             if (i != 1) {
                 k[0] = fmaf(a.w, f[i], fmaf(p.y, e[i], k[0]));
-                k[1] += e[i];
+                k[1] = fmaf(i == 0 ? a.z : d2x, a.x, k[1]);
                 k[2] = fmaf(d2y, f[i], fmaf(p.w, e[i], k[2]));
             } else {
                 k[0] = fmaf(a.w, f[i], k[0]);
@@ -1999,7 +2021,7 @@ __device__ inline void sort_cells(int n, int lane, int* hist, unsigned char* per
 // particle and only these 70 operations wait for the fullest cell of the
 // wave; the cells are dealt to the waves by descending count, so that a
 // wave's cells are alike.
-template <int D, int NT>
+template <int D, int NT, int R>
 struct BlockOperator {
     using CS = CellStencil<D>;
     using Dm = Dims<D>;
@@ -2016,8 +2038,10 @@ struct BlockOperator {
     int chunks;  // particle p0 + t chunks + c sits at place t of chunk c
     int li, node;  // tile node tid: its LDS index and grid node (-1: none)
 
-    __device__ BlockOperator(const KP& kp, L& lds)
-        : p(kp), S(lds), rec4(reinterpret_cast<const float4*>(kp.pop)), tid(threadIdx.x), lane(tid & 63), wv(tid >> 6) {
+    const bool two;  // (ROUND_EITHER)
+
+    __device__ BlockOperator(const KP& kp, L& lds, bool round_two = false)
+        : p(kp), S(lds), rec4(reinterpret_cast<const float4*>(kp.pop)), tid(threadIdx.x), lane(tid & 63), wv(tid >> 6), two(round_two) {
         int l[D], off0[D];
         local_coords<D>(lane, l);
         base = tile_index<D>(l, 0, off0);  // cell `lane`'s stencil corner
@@ -2102,7 +2126,7 @@ struct BlockOperator {
                 const OuterWeights<D> g(rec);
                 float T[DD], A[DD];  // A = V0 F dP(T^T F)^T
                 stencil_gradient<D>(g, S.coef, S.cell[tid], T);
-                apply_operator<D>(rec, scale, T, A);
+                apply_operator<D, R>(rec, scale, two, T, A);
                 pack_particle<D>(g, A, pack + tid * CS::PACK);
             }
             __syncthreads();
@@ -2172,9 +2196,9 @@ struct BlockOperator {
 };
 
 // load(a, n): channel a of node n
-template <int D, int NT, bool AGENT, class Load>
-__device__ inline void operator_block(const KP& p, int b, float inv_dx, OperatorLds<D, NT>& S, Load&& load) {
-    BlockOperator<D, NT> op(p, S);
+template <int D, int NT, int R, bool AGENT, class Load>
+__device__ inline void operator_block(const KP& p, int b, float inv_dx, bool two, OperatorLds<D, NT>& S, Load&& load) {
+    BlockOperator<D, NT, R> op(p, S, two);
     op.open(b);
     float u[D];
 #pragma unroll
@@ -2231,7 +2255,7 @@ __global__ __launch_bounds__(BWG, 4) void k_cg_force(KP p) {
         const int si = p.nscenes == 1 ? 0 : p.block_scene[b];
         const SceneParams& sc = p.scn[si];
         if (!sc.active || (p.nscenes > 1 && p.cg[si].done) || block_empty(p, b)) continue;
-        operator_block<D, BWG, false>(p, b, sc.inv_dx, S, [&](int a, int64_t n) {
+        operator_block<D, BWG, ROUND_LAUNCHED, false>(p, b, sc.inv_dx, false, S, [&](int a, int64_t n) {
             return RESTART ? p.g_vs[a * p.gcap + n] : p.g_s[a * p.gcap + n];
         });
     }
@@ -2989,7 +3013,7 @@ __device__ inline void cg_solve_resident(const KP& p, int blk0, int blk1, Operat
     __shared__ float nx[K][D][64], nr[K][D][64], ns[K][D][64], nm[K][64], ts[K][D][TN];
     // the wave's number as a scalar: its block's and scene's data stay scalar
     const int lane0 = threadIdx.x & 63, nw = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) - NODES;
-    BlockOperator<D, CGW> op(p, S);
+    BlockOperator<D, CGW, K == 1 ? ROUND_ONE : ROUND_TWO> op(p, S);
     // wave NODES + j: the nodes of block j; tile threads: their node's s in
     // every tile.  full, done: a bit per block.
     unsigned long long interiors = 0, zeros = 0;  // a bit per lane (scalar)
@@ -3291,7 +3315,7 @@ __device__ inline void cg_solve_shared(const KP& p, int w0, int w1, int n, int g
             }
             for (; b < e; ++b)
                 if (!block_empty(p, b))
-                    operator_block<D, CGW, true>(p, b, p.scn[si].inv_dx, S, [&](int a, int64_t nd) {
+                    operator_block<D, CGW, ROUND_EITHER, true>(p, b, p.scn[si].inv_dx, n > CG_GROUPS, S, [&](int a, int64_t nd) {
                         return k < 0 ? p.g_vs[a * p.gcap + nd]
                                      : cg_direction(ld_agent(p.g_r + a * p.gcap + nd), ld_agent(p.g_s + a * p.gcap + nd), beta, k);
                     });

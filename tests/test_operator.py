@@ -7,6 +7,7 @@ must match the FP64 oracle to the one-substep bar, 1e-5 relative L2, per
 field.  The particles carry a velocity gradient, so the operator's result
 reaches every compared field.
 """
+import contextlib
 import threading
 
 import numpy as np
@@ -246,6 +247,30 @@ def test_one_block_to_a_work_group_repeats(dim, counts, n):
         s.close()
 
 
+@contextlib.contextmanager
+def busy_device():
+    """Another handle's substeps, of work-groups of thousands of particles each,
+    run meanwhile."""
+    d, x, v, m = M.scene_generate("two_balls", 96, 5, 1_000_000)
+    busy = M.Scene(d, len(m))
+    busy.upload(x, v, m)
+    busy.initialize()
+    stop = threading.Event()
+
+    def hold():
+        while not stop.is_set():
+            busy.substep(0.1 * float(d.max_dt))
+
+    other = threading.Thread(target=hold)
+    other.start()
+    try:
+        yield
+    finally:
+        stop.set()
+        other.join()
+        busy.close()
+
+
 @pytest.mark.parametrize("counts,scenes", [(128, [(66000, 0.35, 0.65)]), (64, [(500, 0.4, 0.6), (66000, 0.2, 0.8), (300, 0.45, 0.5)])])
 def test_node_pass_on_a_busy_device(counts, scenes):
     """Another handle's work-groups, of thousands of particles each, hold the
@@ -280,24 +305,8 @@ def test_node_pass_on_a_busy_device(counts, scenes):
         return out
 
     want = drive(None)
-    d, x, v, m = M.scene_generate("two_balls", 96, 5, 1_000_000)
-    busy = M.Scene(d, len(m))
-    busy.upload(x, v, m)
-    busy.initialize()
-    stop = threading.Event()
-
-    def hold():
-        while not stop.is_set():
-            busy.substep(0.1 * float(d.max_dt))
-
-    other = threading.Thread(target=hold)
-    other.start()
-    try:
+    with busy_device():
         got = [drive(None), drive(0)]
-    finally:
-        stop.set()
-        other.join()
-        busy.close()
     for run, steps in enumerate(got):
         for step, (a, b) in enumerate(zip(steps, want)):
             for k in range(len(parts)):
@@ -349,28 +358,19 @@ def assert_same_bits(got, want, where):
     (3, 64, [130], (1, 512)), (2, 256, [250], (1, 512)), (3, 64, [250], (513, 1024)), (3, 64, [130, 130], (513, 1024)),
     (2, 256, [300, 3, 250], (513, 1024)), (3, 64, [250, 5, 300], (1025, 4096))])
 def test_one_launch_solve_with_few_work_groups(dim, counts, sizes, blocks, graph):
-    """With a wait limit of zero the solve's door closes on those that happen to
-    run: they share the blocks and end with the same bits."""
+    """Beside another handle's long work-groups, and with a wait limit of zero, the
+    solve's door closes on those that happen to run: they share the blocks and
+    end with the same bits as all of them on an idle device."""
     parts = [scattered(dim, counts, n, 80 + k) for k, n in enumerate(sizes)]
-    want, nb = solved(parts, graph, None, 3)
+    want, nb = solved(parts, graph, None, 6)
     assert blocks[0] <= nb <= blocks[1]
-    got, _ = solved(parts, graph, 0, 3)
-    for step in range(3):
-        assert got[step][0]["stats"]["cg_iterations"] > 3
-        for k in range(len(parts)):
-            assert_same_bits(got[step][k], want[step][k], (step, k))
-
-
-@pytest.mark.parametrize("dim,counts,n", [(3, 64, 130), (2, 256, 250)])
-def test_one_and_two_blocks_to_a_work_group(dim, counts, n):
-    """A scene alone (a block to a work-group) and in a batch (two): the
-    same bits over many iterations."""
-    parts = [scattered(dim, counts, n, 70 + k) for k in range(2)]
-    alone, nb = solved(parts[:1], True, None, 30)
-    both, nb2 = solved(parts, True, None, 30)
-    assert nb <= 512 < nb2 <= 1024
-    for step in range(30):
-        assert_same_bits(both[step][0], alone[step][0], step)
+    with busy_device():
+        runs = [solved(parts, graph, limit, 6)[0] for limit in (0, None)]
+    for got in runs:
+        for step in range(6):
+            assert got[step][0]["stats"]["cg_iterations"] > 3
+            for k in range(len(parts)):
+                assert_same_bits(got[step][k], want[step][k], (step, k))
 
 
 @pytest.mark.parametrize("n,lo,hi,many", [(300, 0.3, 0.7, False), (900, 0.1, 0.9, True), (900, 0.28, 0.72, None)])
