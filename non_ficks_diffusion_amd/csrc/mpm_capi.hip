@@ -686,9 +686,7 @@ int allocate_context(mpm_context* c) {
         if (rc == MPM_OK && hipHostGetDevicePointer((void**)&c->d_done, hp, 0) != hipSuccess)
             rc = mpm_set_error(MPM_E_HIP, "hipHostGetDevicePointer failed");
         for (int k = 0; k < 2 && rc == MPM_OK; ++k)
-            if (hipEventCreateWithFlags(&c->done_ev[k], hipEventDisableTiming) != hipSuccess ||
-                hipEventCreateWithFlags(&c->blocks_ev[k], hipEventDisableTiming) != hipSuccess)
-                rc = mpm_set_error(MPM_E_HIP, "hipEventCreate failed");
+            if (hipEventCreateWithFlags(&c->done_ev[k], hipEventDisableTiming) != hipSuccess) rc = mpm_set_error(MPM_E_HIP, "hipEventCreate failed");
         hp = nullptr;
         if (rc == MPM_OK && hipHostMalloc(&hp, sizeof(float) * (size_t)nscenes, hipHostMallocDefault) != hipSuccess)
             rc = mpm_set_error(MPM_E_HIP, "hipHostMalloc failed");
@@ -1081,13 +1079,29 @@ void invalidate_graphs(mpm_context* c) {
 // even, so a replay leaves the particle buffers at the parity it found.
 constexpr int FRAME_K = 4;
 
-// The form of the next substep's CG.  A replay's count is waited for until two
-// substeps later: by then the device has the next one queued.
+// The staging buffer of the dts is free once their last copy has run, which
+// comes after the replay before.
+int await_dt_copy(mpm_context* c) {
+    if (!c->dt_pending) return MPM_OK;
+    HIPCHECK(hipEventSynchronize(c->dt_ev));
+    c->dt_pending = false;
+    c->replays_run = std::max(c->replays_run, c->replays - 1);
+    return MPM_OK;
+}
+
+// The form of the next substep's CG.  The replay before the last has run when
+// the dts of the last are copied, which a replay waits for anyway (an event of
+// its own took 3 to 5 us of every replay).
 int choose_form(mpm_context* c) {
     const int at = c->cur;
     if (c->blocks_pending[at]) {
-        HIPCHECK(hipEventSynchronize(c->blocks_ev[at]));
-        c->blocks_pending[at] = false;
+        const int rc = await_dt_copy(c);
+        if (rc) return rc;
+        if (c->replays_run < c->blocks_pending[at]) {  // binned stage by stage in between
+            HIPCHECK(hipStreamSynchronize(c->stream));
+            c->replays_run = c->replays;
+        }
+        c->blocks_pending[at] = 0;
         c->blocks_of[at] = c->h_done[2 * POLL_INTS + 1 + c->nscenes + at];
     }
     c->many_blocks = c->blocks_of[at] > mpm::CG_RESIDENT;
@@ -1097,7 +1111,7 @@ int choose_form(mpm_context* c) {
 void note_blocks(mpm_context* c, int blocks) {
     for (int k = 0; k < 2; ++k) {
         c->blocks_of[k] = blocks;
-        c->blocks_pending[k] = false;
+        c->blocks_pending[k] = 0;
         c->h_done[2 * POLL_INTS + 1 + c->nscenes + k] = 0;
     }
     c->blocks_seen = blocks;
@@ -1205,10 +1219,8 @@ int device_frames(mpm_context* c, const float* time, const float* target, float*
 // One substep as a graph replay: the dts go to d_dt through pinned staging,
 // then the graph of the current buffer parity (captured on first use) runs.
 int graph_substep(mpm_context* c, const float* dts) {
-    if (c->dt_pending) {  // the staging buffer is free once the last copy ran
-        HIPCHECK(hipEventSynchronize(c->dt_ev));
-        c->dt_pending = false;
-    }
+    const int rc_dt = await_dt_copy(c);
+    if (rc_dt) return rc_dt;
     std::memcpy(c->h_dt, dts, sizeof(float) * (size_t)c->nscenes);
     HIPCHECK(hipMemcpyAsync(c->d_dt, c->h_dt, sizeof(float) * (size_t)c->nscenes, hipMemcpyHostToDevice, c->stream));
     HIPCHECK(hipEventRecord(c->dt_ev, c->stream));
@@ -1244,10 +1256,8 @@ int graph_substep(mpm_context* c, const float* dts) {
         }
     }
     HIPCHECK(hipGraphLaunch(c->gexec[at], c->stream));
-    if (fits_one_launch(c)) {
-        HIPCHECK(hipEventRecord(c->blocks_ev[parity], c->stream));
-        c->blocks_pending[parity] = true;
-    }
+    ++c->replays;
+    c->blocks_pending[parity] = fits_one_launch(c) ? c->replays : 0;
     c->cur = parity ^ 1;  // the replay binned once
     c->binned = false;
     c->ever_binned = true;
@@ -1738,10 +1748,7 @@ int mpm_destroy(mpm_handle c) {
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     for (void* p : c->allocations) (void)hipFree(p);
     for (hipEvent_t e : c->ev) (void)hipEventDestroy(e);
-    for (int k = 0; k < 2; ++k) {
-        if (c->done_ev[k]) (void)hipEventDestroy(c->done_ev[k]);
-        if (c->blocks_ev[k]) (void)hipEventDestroy(c->blocks_ev[k]);
-    }
+    for (int k = 0; k < 2; ++k) if (c->done_ev[k]) (void)hipEventDestroy(c->done_ev[k]);
     if (c->h_done) (void)hipHostFree(c->h_done);
     invalidate_graphs(c);
     if (c->dt_ev) (void)hipEventDestroy(c->dt_ev);

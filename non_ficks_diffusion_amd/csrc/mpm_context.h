@@ -78,11 +78,11 @@ struct mpm_context {
     int poll_boundary[2] = {0, 0};
     int poll_older = 0, poll_target = 1, poll_max_it = 0;
     // active blocks of the substep before the last (by buffer parity: binning swaps
-    // the buffers), which choose the CG's form; those of a replay are pending in
-    // pinned memory until its event
+    // the buffers), which choose the CG's form; those of replay number
+    // blocks_pending (0: none) are in pinned memory once it has run
     int blocks_of[2] = {0, 0};
-    bool blocks_pending[2] = {false, false};
-    hipEvent_t blocks_ev[2] = {nullptr, nullptr};
+    int64_t blocks_pending[2] = {0, 0};
+    int64_t replays = 0, replays_run = 0;  // launched, and those the host knows to have run
     bool many_blocks = false;   // more than the one-launch solve keeps resident
     int* blocks_out = nullptr;  // KP::blocks_out of a substep being captured
     int blocks_seen = 0;   // active blocks of the last binning whose counters the host has read (0: none)
