@@ -2921,7 +2921,7 @@ __global__ __launch_bounds__(WG) void k_read_speeds(KP p, int* dst) {
 // exchanges of a store and a load that has to find it).  Two balls of 3.8k
 // particles, captured, a frame: 18.1 ms with launched kernels, 7.7 resident with
 // a flag per force tile and r waited for before r.r goes out (stores drained,
-// then the flag, then the values: three round trips for one), 7.2 now; 2D scene
+// then the flag, then the values: three round trips for one), 6.9 now; 2D scene
 // of 3.0k 18.3 -> 17.0, twelve scenes of 48k 19.3 -> 18.6, and the disk of 512
 // 0.77 -> 0.74 ms for four substeps.
 // ============================================================================
